@@ -146,6 +146,63 @@ def run(s):
     return (y.detach(), *torch.autograd.grad(y, s["wanted"], s["dy"]))
 
 
+def exact(case, seed):
+    """The same outputs from plain torch in float64: one shifted product per tap, products across a boundary dropped."""
+    s = prepare(case, seed)
+    x, conv, K, res = s["x"], s["conv"], case["K"], case["residual"]
+    leaves = [t.detach().double().requires_grad_(case["train"]) for t in s["wanted"]]
+    X, W, B = leaves[0].reshape(-1, x.shape[-1]), leaves[1], leaves[2]
+    T, P = X.shape[0], (K - 1) // 2
+    rows = torch.arange(T, device=DEV)
+    if case["form"] == "padded":
+        row_in = torch.arange(512, device=DEV)[None, :]
+        seq = 2 * torch.arange(T // 512, device=DEV)[:, None] + (row_in >= s["mask"].sum(1)[:, None])
+        seq = seq.reshape(-1)
+    else:
+        seq = torch.searchsorted(s["cu"].long(), rows, right=True)
+    if case["form"] == "ln":
+        mean = X.mean(1, keepdim=True)
+        h = (X - mean) * torch.rsqrt((X - mean).pow(2).mean(1, keepdim=True) + s["norm"].eps) * leaves[3] + leaves[4]
+    elif case["form"] == "gated":
+        h = X[:, :case["C"]] * X[:, case["C"]:] * torch.sigmoid(X[:, case["C"]:])
+    else:
+        h = X
+    valid = [None] * K
+    y = torch.zeros_like(h.detach())
+
+    def spans(d):               # output rows and input rows of the tap d rows away
+        return slice(max(0, -d), T - max(0, d)), slice(max(0, d), T - max(0, -d))
+
+    hd, wd = h.detach(), W.detach()
+    for k in range(K):
+        if abs(k - P) >= T:
+            continue
+        o, i = spans(k - P)
+        valid[k] = (seq[o] == seq[i])[:, None]
+        y[o] += torch.where(valid[k], hd[i] * wd[:, k], 0.0)
+    y += B.detach()
+    if res:
+        y += X.detach()
+    if not case["train"]:
+        return y.reshape(*x.shape[:-1], case["C"])
+    dy = s["dy"].double()
+    dh, dw = torch.zeros_like(hd), torch.zeros_like(wd)
+    for k in range(K):
+        if valid[k] is None:
+            continue
+        o, i = spans(k - P)
+        g = torch.where(valid[k], dy[o], 0.0)
+        dh[i] += g * wd[:, k]
+        dw[:, k] = (g * hd[i]).sum(0)
+    dx, rest = dh, []
+    if case["form"] in ("ln", "gated"):
+        inner = [leaves[0]] + leaves[3:]
+        dx, *rest = torch.autograd.grad(h, inner, dh)
+    if res:
+        dx = dx + dy
+    return (y, dx, dw, dy.sum(0), *rest)
+
+
 def work(case):
     """Bytes: every input read once and every output written once, in each direction (the backward reads x again). Operations:
     two per tap and element forward, four backward (dx and dw), one for db, and the gate's or the norm's few."""
