@@ -19,7 +19,8 @@
  *
  *   Kernel sizes: K = 3, 5, 7, 9, 15 and 31 have kernels of their own. Any other odd K <= 31 runs on the
  *   kernels of the next of 3, 15, 31 with zero taps on either side (w and dw keep rows of K taps; the
- *   workspace holds slabs of that size): for finite inputs the same sums with exact zeros added, so the
+ *   workspace holds slabs of that size; K = 11 and 17 .. 21 leave part of the zero taps out where a call
+ *   takes LDS-staged kernels): for finite inputs the same sums with exact zeros added, so the
  *   same results; a NaN/Inf in x or dy then reaches the rows within that larger half-width of its own
  *   sequence (0 * Inf), never another sequence, and never a tap of dw that its products do not belong
  *   to. Odd K from 33 to NPLM_DWCONV_MAX_K run untuned kernels (one wave per row). The gated entry

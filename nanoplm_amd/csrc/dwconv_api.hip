@@ -41,6 +41,15 @@ bool specialised_k(int K) { return K == 3 || K == 5 || K == 7 || K == 9 || K == 
 // Runtime-K kernels (one wave per row) remain for K > 31.
 int exec_kernel_size(int K) { return K > 31 || specialised_k(K) ? K : K < 3 ? 3 : K < 15 ? 15 : 31; }
 
+// The number of taps the LDS-staged and role-split kernels run such a size with: they are built for 11 and 21 taps as well,
+// so K = 11 and K = 17 .. 21 leave out zero taps (and halo rows) of the 15 and 31 that plans and workspaces are made for.
+// Tiles, token blocks and the order of every sum are those of exec_kernel_size(K); a slab is shorter and fits its place.
+// Measured at C=2048, T=65536, log-normal lengths, bf16, whole calls, running as 15 / 31 -> this (us): K=11 forward 111 -> 93,
+// with backward 304 -> 262; K=17 130 -> 104, 379 -> 313; K=21 133 -> 108, 379 -> 318; gated K=11 191 -> 185, 457 -> 427, K=21
+// 226 -> 199, 588 -> 504; fp32 forward and backward 455 -> 446 (K=11), 544 -> 492 (K=21). A form of 13 taps would save two of 15
+// taps where 11 saves four, one of 25 six of 31: neither is built.
+int lds_taps(int K) { return K == 11 ? 11 : K >= 17 && K <= 21 ? 21 : exec_kernel_size(K); }
+
 int pow2_floor(int v) { int p = 1; while (p * 2 <= v) p *= 2; return p; }
 int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
@@ -256,6 +265,7 @@ hipError_t launch_fwd_lds(int K, const LdsPlan& p, const ConvPtrs& a, const LdsG
         case 5: return launch_fwd_lds_k5(p.sh, a, g, grid, s);
         case 7: return launch_fwd_lds_k7(p.sh, a, g, grid, s);
         case 9: return launch_fwd_lds_k9(p.sh, a, g, grid, s);
+        case 11: return launch_fwd_lds_k11(p.sh, a, g, grid, s);
         case 15: return launch_fwd_lds_k15(p.sh, a, g, grid, s);
         case 31: return launch_fwd_lds_k31(p.sh, a, g, grid, s);
     }
@@ -275,7 +285,23 @@ hipError_t launch_bwd_lds(int K, const LdsPlan& p, bool wdx, bool wdw, const Con
     return hipErrorInvalidConfiguration;
 }
 
-// ---- role-split LDS-staged kernels at K = 31 and 15 (dwconv_lds_split_kernels.h) ---------------------
+// ---- role-split LDS-staged kernels at K = 31 and 15 (dwconv_lds_split_kernels.h), run with lds_taps() taps ---
+#define NPLM_LAUNCH_SPLIT(NAME)                                                                          \
+    hipError_t NAME(int taps, bool bf16, const ConvPtrs& a, const LdsGeo& g, dim3 grid, hipStream_t s) { \
+        switch (taps) {                                                                                  \
+            case 11: return NAME##_k11(bf16, a, g, grid, s);                                             \
+            case 15: return NAME##_k15(bf16, a, g, grid, s);                                             \
+            case 21: return NAME##_k21(bf16, a, g, grid, s);                                             \
+            case 31: return NAME##_k31(bf16, a, g, grid, s);                                             \
+        }                                                                                                \
+        return hipErrorInvalidConfiguration;                                                             \
+    }
+NPLM_LAUNCH_SPLIT(launch_fwd_split)
+NPLM_LAUNCH_SPLIT(launch_bwd_split)
+NPLM_LAUNCH_SPLIT(launch_fwd_split_gated)
+NPLM_LAUNCH_SPLIT(launch_bwd_split_gated)
+#undef NPLM_LAUNCH_SPLIT
+
 bool split_eligible(bool bf16, long long T, int C, int K, uintptr_t align_bits) {
     const int E = bf16 ? 2 : 4;
     if (!lds_split_kernel_size(K) || T < 1) return false;
@@ -401,7 +427,8 @@ int fwd_impl(const void* x, const int32_t* cu, const void* w, const void* b, voi
     if (flags & ~(uint32_t)NPLM_DWCONV_RESIDUAL) return -NPLM_DWCONV_EFLAGS;
     if (T == 0) return 0;
     if (!x || !cu || !w || !y) return -NPLM_DWCONV_ENULL;
-    const int tap_off = (exec_kernel_size(K) - K) / 2;
+    const int taps = lds_taps(K), tap_off = (exec_kernel_size(K) - K) / 2;
+    const int lds_w_flags = kernel_w_flags(w_dtype, flags) | ((taps - K) / 2 << W_TAP_OFF_SHIFT);
     K = exec_kernel_size(K);        // from here on the kernel size that runs
     const int w_flags = kernel_w_flags(w_dtype, flags) | (tap_off << W_TAP_OFF_SHIFT);
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
@@ -418,16 +445,17 @@ int fwd_impl(const void* x, const int32_t* cu, const void* w, const void* b, voi
         rc = make_split_plan(true, bf16, T, C, K, tune, &lp);
         if (rc) return rc;
         const ConvPtrs la{x, nullptr, cu, w, b, y, nullptr};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, w_flags);
-        return (int)(K == 31 ? launch_fwd_split_k31(bf16, la, lg, dim3(lp.ncb * lp.nbt), s)
-                             : launch_fwd_split_k15(bf16, la, lg, dim3(lp.ncb * lp.nbt), s));
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, lds_w_flags);
+        return (int)launch_fwd_split(taps, bf16, la, lg, dim3(lp.ncb * lp.nbt), s);
     }
     if (algo == 2) {
+        // of the shorter forms the loader-wave forward has the one of 11 taps; shape overrides name shapes of K
+        const int lds_k = (taps == 11 && !tune) ? taps : K;
         LdsPlan lp;
-        rc = make_lds_plan(false, bf16, T, C, K, tune, &lp);
+        rc = make_lds_plan(false, bf16, T, C, lds_k, tune, &lp);
         if (rc) return rc;
         const ConvPtrs la{x, nullptr, cu, w, b, y, nullptr};
-        const hipError_t e = launch_fwd_lds(K, lp, la, make_lds_geo(lp, T, C, S, w_flags), s);
+        const hipError_t e = launch_fwd_lds(lds_k, lp, la, make_lds_geo(lp, T, C, S, lds_k == K ? w_flags : lds_w_flags), s);
         if (e == hipErrorInvalidConfiguration && tune) return -NPLM_DWCONV_ETUNING;
         return (int)e;
     }
@@ -466,7 +494,7 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
         if (e == hipSuccess) e = out_bf16 ? fill_zero16(db, C, s) : fill_zero(db, C, s);
         return (int)e;
     }
-    const int tap_off = (exec_kernel_size(K) - K) / 2;
+    const int taps = lds_taps(K), lds_tap_off = (taps - K) / 2, tap_off = (exec_kernel_size(K) - K) / 2;
     K = exec_kernel_size(K);        // from here on the kernel size that runs (slabs of K + 1 rows; dw rows stay the caller's)
     const int w_flags = kernel_w_flags(w_dtype, flags) | (tap_off << W_TAP_OFF_SHIFT);
     if (!dx && !want_red) return 0;
@@ -493,17 +521,17 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
             return -NPLM_DWCONV_EWORKSPACE;
         float* part = reinterpret_cast<float*>(workspace);
         const ConvPtrs la{x, dy, cu, w, nullptr, dx, part};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, w_flags);
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | (lds_tap_off << W_TAP_OFF_SHIFT));
         const dim3 grid(lp.ncb * lp.nbt);
-        hipError_t e = K == 31 ? launch_bwd_split_k31(bf16, la, lg, grid, s) : launch_bwd_split_k15(bf16, la, lg, grid, s);
+        hipError_t e = launch_bwd_split(taps, bf16, la, lg, grid, s);
         if (e != hipSuccess) return (int)e;
         if (tune && tune->mid_event) {
             e = hipEventRecord((hipEvent_t)tune->mid_event, s);
             if (e != hipSuccess) return (int)e;
         }
-        const long long n_out = (long long)(K + 1) * C;
+        const long long n_out = (long long)(taps + 1) * C;
         hipLaunchKernelGGL(dwconv_finalize_kernel<FIN_SPLIT>, dim3((unsigned)((n_out + 63) / 64)), dim3(64 * FIN_SPLIT), 0,
-                           s, (const float*)part, lp.nbt, C, K, dw, db, out_bf16, tap_off);
+                           s, (const float*)part, lp.nbt, C, taps, dw, db, out_bf16, lds_tap_off);
         return (int)hipGetLastError();
     }
     if (algo == 2) {
@@ -698,6 +726,7 @@ int nplm_dwconv_gated_fwd(const void* z, const int32_t* cu, const void* w, const
     if (flags & ~(uint32_t)NPLM_DWCONV_RESIDUAL) return -NPLM_DWCONV_EFLAGS;
     if (T == 0) return 0;
     if (!z || !cu || !w || !y) return -NPLM_DWCONV_ENULL;
+    const int taps = lds_taps(K), lds_tap_flags = (taps - K) / 2 << W_TAP_OFF_SHIFT;
     const int tap_flags = ((exec_kernel_size(K) - K) / 2) << W_TAP_OFF_SHIFT;
     K = exec_kernel_size(K);        // from here on the kernel size that runs
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
@@ -709,10 +738,9 @@ int nplm_dwconv_gated_fwd(const void* z, const int32_t* cu, const void* w, const
         rc = make_split_plan(true, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;
         const ConvPtrs la{z, nullptr, cu, w, b, y, nullptr};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | tap_flags);
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | lds_tap_flags);
         const dim3 grid(lp.ncb * lp.nbt);
-        return (int)(K == 31 ? launch_fwd_split_gated_k31(bf16, la, lg, grid, (hipStream_t)stream)
-                             : launch_fwd_split_gated_k15(bf16, la, lg, grid, (hipStream_t)stream));
+        return (int)launch_fwd_split_gated(taps, bf16, la, lg, grid, (hipStream_t)stream);
     }
     rc = make_lds_plan(false, bf16, T, C, K, nullptr, &lp, true);
     if (rc) return rc == -NPLM_DWCONV_ETUNING ? -NPLM_DWCONV_EUNSUPPORTED : rc;
@@ -973,6 +1001,7 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
         return (int)e;
     }
     if (!z || !dy || !cu || !w || !dz) return -NPLM_DWCONV_ENULL;
+    const int taps = lds_taps(K), lds_tap_off = (taps - K) / 2;
     const int tap_off = (exec_kernel_size(K) - K) / 2, tap_flags = tap_off << W_TAP_OFF_SHIFT;
     K = exec_kernel_size(K);        // from here on the kernel size that runs (slabs of K + 1 rows; dw rows stay the caller's)
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
@@ -986,13 +1015,13 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
         if (!workspace || (uintptr_t)workspace % 256 || workspace_bytes < slab * (size_t)lp.nbt) return -NPLM_DWCONV_EWORKSPACE;
         float* part = reinterpret_cast<float*>(workspace);
         const ConvPtrs la{z, dy, cu, w, nullptr, dz, part};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | tap_flags);
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | (lds_tap_off << W_TAP_OFF_SHIFT));
         const dim3 grid(lp.ncb * lp.nbt);
-        hipError_t e = K == 31 ? launch_bwd_split_gated_k31(bf16, la, lg, grid, s) : launch_bwd_split_gated_k15(bf16, la, lg, grid, s);
+        hipError_t e = launch_bwd_split_gated(taps, bf16, la, lg, grid, s);
         if (e != hipSuccess) return (int)e;
-        const long long n_out = (long long)(K + 1) * C;
+        const long long n_out = (long long)(taps + 1) * C;
         hipLaunchKernelGGL(dwconv_finalize_kernel<FIN_SPLIT>, dim3((unsigned)((n_out + 63) / 64)), dim3(64 * FIN_SPLIT), 0, s,
-                           (const float*)part, lp.nbt, C, K, dw, db, out_bf16, tap_off);
+                           (const float*)part, lp.nbt, C, taps, dw, db, out_bf16, lds_tap_off);
         return (int)hipGetLastError();
     }
     if (long_gated_bwd_supported(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {

@@ -117,16 +117,18 @@ hipError_t launch_bwd_gated_k31(bool bf16, int unroll, int maxt, const ConvPtrs&
 // and LDS-staged forward with the gate formed in LDS by the loader waves (rows the role-split forward does not take)
 hipError_t launch_fwd_lds_gated_k15(bool bf16, bool narrow, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 hipError_t launch_fwd_lds_gated_k31(bool bf16, bool narrow, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-// role-split LDS kernels at K = 31 and 15 (fixed shape per dtype, see lds_split_shape())
-hipError_t launch_bwd_split_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-hipError_t launch_fwd_split_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-hipError_t launch_bwd_split_k15(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-// gated role-split forward (z = [u | g] in, y out), see lds_split_gated_fwd_shape()
-hipError_t launch_fwd_split_gated_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-hipError_t launch_fwd_split_gated_k15(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-// gated role-split backward (z = [u | g] in, dz out), see lds_split_gated_shape()
-hipError_t launch_bwd_split_gated_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
-hipError_t launch_bwd_split_gated_k15(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
+// role-split LDS kernels (fixed shape per dtype, see lds_split_shape()); gated: z = [u | g] in, y or dz out, see
+// lds_split_gated_fwd_shape() and lds_split_gated_shape()
+#define NPLM_DECLARE_SPLIT_K(KK)                                                                                        \
+    hipError_t launch_fwd_split_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);       \
+    hipError_t launch_bwd_split_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);       \
+    hipError_t launch_fwd_split_gated_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s); \
+    hipError_t launch_bwd_split_gated_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
+NPLM_DECLARE_SPLIT_K(11)
+NPLM_DECLARE_SPLIT_K(15)
+NPLM_DECLARE_SPLIT_K(21)
+NPLM_DECLARE_SPLIT_K(31)
+#undef NPLM_DECLARE_SPLIT_K
 // LayerNorm-fused forward (dwconv_ln_kernels.h), K <= 9, fixed shape per dtype, see lds_ln_shape()
 hipError_t launch_ln_fwd_k3(bool bf16, const ConvPtrs& p, const LnArgs& ln, const LdsGeo& g, dim3 grid, hipStream_t s);
 hipError_t launch_ln_fwd_k5(bool bf16, const ConvPtrs& p, const LnArgs& ln, const LdsGeo& g, dim3 grid, hipStream_t s);
@@ -180,11 +182,11 @@ hipError_t launch_ln_bwd_k3(bool bf16, const ConvPtrs& p, const LnSide& ln, cons
 hipError_t launch_ln_bwd_k5(bool bf16, const ConvPtrs& p, const LnSide& ln, const LdsGeo& g, dim3 grid, hipStream_t s);
 hipError_t launch_ln_bwd_k7(bool bf16, const ConvPtrs& p, const LnSide& ln, const LdsGeo& g, dim3 grid, hipStream_t s);
 hipError_t launch_ln_bwd_k9(bool bf16, const ConvPtrs& p, const LnSide& ln, const LdsGeo& g, dim3 grid, hipStream_t s);
-hipError_t launch_fwd_split_k15(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 NPLM_DECLARE_LDS_K(3)
 NPLM_DECLARE_LDS_K(5)
 NPLM_DECLARE_LDS_K(7)
 NPLM_DECLARE_LDS_K(9)
+hipError_t launch_fwd_lds_k11(const LdsShapeSel& sh, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 NPLM_DECLARE_LDS_K(15)
 NPLM_DECLARE_LDS_K(31)
 #undef NPLM_DECLARE_LDS_K
@@ -257,7 +259,7 @@ constexpr SplitShapeSel lds_split_shape(bool fwd, bool bf16, int K) {
 // per lane in 256-byte blocks with 16, 20, 24 rows per wave 784 / 732, 765 / 718, 771 / 702: rows per wave count, tile
 // length does not. Both roles evaluate the gate's sigmoid (two quarter-rate instructions per element and role),
 // which is what the kernel costs over the plain one (510 us).
-constexpr SplitShapeSel lds_split_gated_shape(bool bf16, int K) { return SplitShapeSel{bf16 ? 2 : 1, K >= 31 ? 10 : 12, 4, 2}; }
+constexpr SplitShapeSel lds_split_gated_shape(bool bf16, int K) { return SplitShapeSel{bf16 ? 2 : 1, K >= 17 ? 10 : 12, 4, 2}; }
 // Gated role-split forward (K = 31, 15): a buffer holds a u tile and a g tile of R + K-1 rows each, which the waves turn
 // into one fp32 h tile in place before the row schedules run. 256-byte column blocks (one wave-column) with 16 row
 // groups of 8 rows: two buffers of 2 x 158 rows x 256 bytes = 158 KiB at K = 31. Measured at T=131072, C=2048, bf16

@@ -1,0 +1,3 @@
+// LDS-staged forward and role-split kernels of 11 taps (K = 11).
+#define NPLM_K 11
+#include "dwconv_lds_inst.inc"

@@ -226,6 +226,17 @@ def test_kernel_sizes_without_kernels_of_their_own_run_as_the_next_size_with_zer
     assert torch.equal(dw1, dw1x[:, off:off + K]) and torch.equal(db1, db1x)
 
 
+@pytest.mark.parametrize("K,C,dt,wdt", [(11, 1000, torch.bfloat16, torch.float32), (11, 264, torch.float32, torch.float32),
+                                        (17, 520, torch.bfloat16, torch.bfloat16), (19, 132, torch.float32, torch.float32),
+                                        (21, 1000, torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("lens", [[1], [10, 11, 12], [127, 2, 129], [700]])
+def test_kernels_of_11_and_21_taps_around_tile_edges(K, C, dt, wdt, lens):
+    """Rows that leave the last column block partly empty, sequences around the halo and around the tiles of 32, 64 and
+    128 rows."""
+    print(f"[case] K={K} C={C} {dt} w {wdt} {lens}", flush=True)
+    _check_case(*_random_case(lens, C, K, dt, wdt, seed=K + C + len(lens)), f"K={K} C={C} {lens}")
+
+
 @pytest.mark.parametrize("C", [1, 7, 8, 24, 64, 72, 100, 128, 130, 384, 520, 576, 640, 768, 1000, 1024, 1152, 1280, 2048,
                                2560, 4104])
 def test_channel_counts(C):
