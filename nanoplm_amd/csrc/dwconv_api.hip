@@ -389,6 +389,31 @@ hipError_t fill_zero(float* p, long long n, hipStream_t s) {
     return hipGetLastError();
 }
 
+// cu_seqlens [2B+1] of a right-padded mask [B, L] over the flat rows: block b sums row b of the mask (each value taken as
+// int32, sums wrap in 32 bits) and writes b * L and b * L + that sum; the last entry is B * L. Bound by its launch: a
+// block per row has 256 loads of the row in flight, and 32 rows of 512 int64 are 128 KiB. It takes the place of
+// eight elementwise and reduction launches (sum, arange, mul, add, stack, full, cat and a copy): a padded call of 32 x 512
+// rows at C=768 goes from 65 to 25 us, of which the conv kernel is 13.
+template <typename V>
+__global__ void __launch_bounds__(256) mask_cu_kernel(const V* __restrict__ mask, long long row_stride, long long L, unsigned B,
+                                                      int32_t* __restrict__ cu) {
+    __shared__ unsigned part[4];
+    const unsigned b = blockIdx.x;
+    const V* row = mask + (size_t)b * (size_t)row_stride;
+    unsigned n = 0;
+    for (long long i = threadIdx.x; i < L; i += 256) n += (unsigned)(int32_t)row[i];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) n += (unsigned)__shfl_xor((int)n, d, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned start = b * (unsigned)L;
+        cu[2 * (size_t)b] = (int32_t)start;
+        cu[2 * (size_t)b + 1] = (int32_t)(start + part[0] + part[1] + part[2] + part[3]);
+        if (b + 1 == B) cu[2 * (size_t)B] = (int32_t)(B * (unsigned)L);
+    }
+}
+
 // launch flags of the kernels (W_BF16 | W_RESIDUAL) from the ABI's weight dtype and flags
 // Shapes the gated (z = [u | g]) kernels are built for.
 bool gated_supported(bool bwd, bool bf16, long long T, int C, int K, uintptr_t align_bits) {
@@ -1123,6 +1148,20 @@ size_t nplm_dwconv_bwd_workspace_bytes(int64_t T, int32_t C, int32_t K, int32_t 
     }
     const size_t bytes = (size_t)slabs * (K + 1) * C * sizeof(float);
     return (bytes + 255) & ~(size_t)255;
+}
+
+int nplm_dwconv_mask_cu(const void* mask, int32_t kind, int64_t row_stride, int64_t B, int64_t L, int32_t* cu, void* stream) {
+    if (B < 1 || B > kMaxRows || L < 1 || L > kMaxRows || row_stride < 0) return -NPLM_DWCONV_ESHAPE;
+    if (!mask || !cu) return -NPLM_DWCONV_ENULL;
+    const dim3 grid((unsigned)B), block(256);
+    hipStream_t s = (hipStream_t)stream;
+    switch (kind) {
+        case 0: hipLaunchKernelGGL(mask_cu_kernel<uint8_t>, grid, block, 0, s, (const uint8_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        case 1: hipLaunchKernelGGL(mask_cu_kernel<int32_t>, grid, block, 0, s, (const int32_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        case 2: hipLaunchKernelGGL(mask_cu_kernel<int64_t>, grid, block, 0, s, (const int64_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        default: return -NPLM_DWCONV_EDTYPE;
+    }
+    return (int)hipGetLastError();
 }
 
 int32_t nplm_dwconv_exec_kernel_size(int32_t K) { return exec_kernel_size(K); }

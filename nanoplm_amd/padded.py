@@ -21,7 +21,10 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from .dwconv import varlen_dwconv
+from . import _lib
+from .dwconv import _launch_on, varlen_dwconv
+
+_MASK_KINDS = {torch.bool: 0, torch.uint8: 0, torch.int32: 1, torch.int64: 2}
 
 
 def right_padded_cu_seqlens(attention_mask: torch.Tensor) -> torch.Tensor:
@@ -37,6 +40,21 @@ def right_padded_cu_seqlens(attention_mask: torch.Tensor) -> torch.Tensor:
     inner = torch.stack((starts, starts + seqlens), dim=1).flatten()
     end = torch.full((1,), B * L, device=attention_mask.device, dtype=torch.int32)
     return torch.cat((inner, end))
+
+
+def _flat_cu_seqlens(mask: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """:func:`right_padded_cu_seqlens` for a call that runs the kernels at once: one launch for a bool or integer mask
+    with adjacent row elements on x's device, the elementwise operations for any other and while tracing."""
+    kind = _MASK_KINDS.get(mask.dtype)
+    if (torch.compiler.is_compiling() or type(mask) is not torch.Tensor or kind is None or not x.is_cuda
+            or mask.device != x.device or mask.numel() == 0 or (mask.shape[1] > 1 and mask.stride(1) != 1)):
+        return right_padded_cu_seqlens(mask)
+    B, L = mask.shape
+    cu = torch.empty((2 * B + 1,), dtype=torch.int32, device=mask.device)
+    with _launch_on(mask) as dev:
+        rc = _lib.load().nplm_dwconv_mask_cu(mask.data_ptr(), kind, mask.stride(0), B, L, cu.data_ptr(), dev.stream)
+    _lib.check(rc, "nplm_dwconv_mask_cu")
+    return cu
 
 
 def is_right_padded(attention_mask: torch.Tensor) -> torch.Tensor:
@@ -77,7 +95,7 @@ def padded_dwconv(x: torch.Tensor, attention_mask: torch.Tensor, weight: torch.T
         raise ValueError("x must be [B, L, C] and attention_mask [B, L]")
     B, L, C = x.shape
     if assume_right_padded:
-        cu = right_padded_cu_seqlens(attention_mask)
+        cu = _flat_cu_seqlens(attention_mask, x)
         y = varlen_dwconv(x.reshape(B * L, C), cu, weight, bias, residual)
         return y.view(B, L, C)
     indices, cu, _ = unpad_input(attention_mask)

@@ -46,6 +46,19 @@ def test_right_padded_batch_in_place(residual):
     assert torch.equal(y[~md], y2[~md])
 
 
+@pytest.mark.parametrize("dt", [torch.bool, torch.uint8, torch.int32, torch.int64, torch.float32])
+@pytest.mark.parametrize("B,L", [(1, 1), (3, 64), (5, 255), (2, 257), (300, 7), (0, 8), (4, 0)])
+def test_boundaries_in_one_launch_equal_the_elementwise_ones(B, L, dt):
+    """Masks around the 256 threads of a block, with rows that are a slice of a wider tensor and transposed ones (which
+    take the elementwise operations), against the boundaries formed on the CPU; not every row is right-padded."""
+    from nanoplm_amd.padded import _flat_cu_seqlens
+    wide = (torch.rand(B, L + 3, generator=torch.Generator().manual_seed(B * L)) > 0.3).to(dt)
+    x = torch.zeros(1, device=DEV)
+    d = wide.to(DEV)
+    assert torch.equal(_flat_cu_seqlens(d[:, 1:L + 1], x).cpu(), npa.right_padded_cu_seqlens(wide[:, 1:L + 1]))
+    assert torch.equal(_flat_cu_seqlens(d.t(), x).cpu(), npa.right_padded_cu_seqlens(wide.t()))
+
+
 def test_arbitrary_mask_goes_through_gather_and_scatter():
     g = torch.Generator().manual_seed(2)
     B, L, C = 5, 64, 256
