@@ -20,6 +20,7 @@ from typing import Optional, Tuple
 
 import torch
 import torch.nn.functional as F
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 
 from . import _lib
 from .dwconv import _launch_on, varlen_dwconv
@@ -42,11 +43,18 @@ def right_padded_cu_seqlens(attention_mask: torch.Tensor) -> torch.Tensor:
     return torch.cat((inner, end))
 
 
+def _operations_are_recorded() -> bool:
+    """Something sees this call's torch operations and not the library's launches: ``torch.compile`` and ``torch.export``,
+    ``torch.jit.trace``, a dispatch mode (``make_fx``, fake tensors, counters)."""
+    return torch.compiler.is_compiling() or torch.jit.is_tracing() or is_in_torch_dispatch_mode()
+
+
 def _flat_cu_seqlens(mask: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """:func:`right_padded_cu_seqlens` for a call that runs the kernels at once: one launch for a bool or integer mask
-    with adjacent row elements on x's device, the elementwise operations for any other and while tracing."""
+    with adjacent row elements on x's device, the elementwise operations for any other and wherever operations are
+    recorded (a recorded launch would be an ``empty`` that nothing fills)."""
     kind = _MASK_KINDS.get(mask.dtype)
-    if (torch.compiler.is_compiling() or type(mask) is not torch.Tensor or kind is None or not x.is_cuda
+    if (_operations_are_recorded() or type(mask) is not torch.Tensor or kind is None or not x.is_cuda
             or mask.device != x.device or mask.numel() == 0 or (mask.shape[1] > 1 and mask.stride(1) != 1)):
         return right_padded_cu_seqlens(mask)
     B, L = mask.shape

@@ -59,6 +59,16 @@ def test_boundaries_in_one_launch_equal_the_elementwise_ones(B, L, dt):
     assert torch.equal(_flat_cu_seqlens(d.t(), x).cpu(), npa.right_padded_cu_seqlens(wide.t()))
 
 
+def test_traced_door_follows_the_mask_of_the_replay():
+    """torch.jit.trace of the padded door with one mask, replayed with another, gives what the eager call gives."""
+    x, first, w, bias = _padded_case([37, 128, 0, 1], 128, 512, 7, torch.bfloat16, seed=4)
+    second = _padded_case([5, 0, 128, 90], 128, 512, 7, torch.bfloat16, seed=4)[1]
+    xd, wd, bd, m1, m2 = (t.to(DEV) for t in (x, w, bias, first, second))
+    traced = torch.jit.trace(lambda xx, mm: npa.padded_dwconv(xx, mm, wd, bd), (xd, m1))
+    for m in (m1, m2, m1):
+        assert torch.equal(traced(xd, m), npa.padded_dwconv(xd, m, wd, bd))
+
+
 def test_arbitrary_mask_goes_through_gather_and_scatter():
     g = torch.Generator().manual_seed(2)
     B, L, C = 5, 64, 256

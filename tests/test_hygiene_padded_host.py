@@ -1,9 +1,16 @@
 """Host-side logic around the op (no GPU): padded-batch boundaries, un/pad helpers, and how the
 module's parameters are seen by the reference's optimizer grouping rules."""
+import contextlib
+import ctypes
+from types import SimpleNamespace
+
+import pytest
 import torch
 from torch import nn
+from torch.fx.experimental.proxy_tensor import make_fx
 
 import nanoplm_amd as npa
+from nanoplm_amd import padded
 
 
 # ---- padded batches -----------------------------------------------------------------------------------
@@ -16,6 +23,34 @@ def test_right_padded_cu_seqlens_lists_real_and_pad_runs():
     assert not bool(npa.is_right_padded(torch.tensor([[0, 1, 1], [1, 1, 0]])))
     # fixed length 2B+1 whatever the lengths are (static shapes for torch.compile(dynamic=False))
     assert npa.right_padded_cu_seqlens(torch.ones(7, 9, dtype=torch.bool)).numel() == 15
+
+
+class _HostMaskCu:
+    """nplm_dwconv_mask_cu on host memory for a contiguous int64 mask, so that the one-launch route runs without a GPU."""
+    calls = 0
+
+    def nplm_dwconv_mask_cu(self, mask, kind, row_stride, B, L, cu, stream):
+        self.calls += 1
+        rows = (ctypes.c_int64 * (B * L)).from_address(mask)
+        out = (ctypes.c_int32 * (2 * B + 1)).from_address(cu)
+        for b in range(B):
+            out[2 * b], out[2 * b + 1] = b * L, b * L + sum(rows[b * L:(b + 1) * L])
+        out[2 * B] = B * L
+        return 0
+
+
+@pytest.mark.parametrize("record", [lambda f, m: torch.jit.trace(f, (m,)), lambda f, m: make_fx(f)(m)], ids=["jit.trace", "make_fx"])
+def test_recorded_boundaries_follow_the_mask_of_the_replay(monkeypatch, record):
+    """The library's launch is invisible to whatever records torch operations, so a recorded call has to hold the
+    elementwise operations: recorded with one mask and replayed with another it gives the other's boundaries."""
+    lib = _HostMaskCu()
+    monkeypatch.setattr(padded._lib, "load", lambda: lib)
+    monkeypatch.setattr(padded, "_launch_on", lambda t: contextlib.nullcontext(SimpleNamespace(stream=None)))
+    x = SimpleNamespace(is_cuda=True, device=torch.device("cpu"))
+    first, second = torch.tensor([[1, 0, 0, 0], [1, 1, 1, 0]]), torch.tensor([[1, 1, 0, 0], [1, 1, 1, 1]])
+    assert padded._flat_cu_seqlens(first, x).tolist() == [0, 1, 4, 7, 8] and lib.calls == 1
+    recorded = record(lambda m: padded._flat_cu_seqlens(m, x), first)
+    assert recorded(second).tolist() == [0, 2, 4, 8, 8]
 
 
 def test_unpad_and_pad_follow_the_reference_contracts():
