@@ -389,19 +389,19 @@ hipError_t fill_zero(float* p, long long n, hipStream_t s) {
     return hipGetLastError();
 }
 
-// cu_seqlens [2B+1] of a right-padded mask [B, L] over the flat rows: block b sums row b of the mask (each value taken as
-// int32, sums wrap in 32 bits) and writes b * L and b * L + that sum; the last entry is B * L. Bound by its launch: a
+// cu_seqlens [2B+1] of a right-padded mask [B, L] over the flat rows: block b sums row b of the mask (a bool counts as one
+// whatever its byte if that is not zero, any other value is taken as int32, sums wrap in 32 bits) and writes b * L and b * L + that sum; the last entry is B * L. Bound by its launch: a
 // block per row has 256 loads of the row in flight, and 32 rows of 512 int64 are 128 KiB. It takes the place of
 // eight elementwise and reduction launches (sum, arange, mul, add, stack, full, cat and a copy): a padded call of 32 x 512
 // rows at C=768 goes from 65 to 25 us, of which the conv kernel is 13.
-template <typename V>
+template <typename V, bool BOOL>
 __global__ void __launch_bounds__(256) mask_cu_kernel(const V* __restrict__ mask, long long row_stride, long long L, unsigned B,
                                                       int32_t* __restrict__ cu) {
     __shared__ unsigned part[4];
     const unsigned b = blockIdx.x;
     const V* row = mask + (size_t)b * (size_t)row_stride;
     unsigned n = 0;
-    for (long long i = threadIdx.x; i < L; i += 256) n += (unsigned)(int32_t)row[i];
+    for (long long i = threadIdx.x; i < L; i += 256) n += BOOL ? (unsigned)(row[i] != 0) : (unsigned)(int32_t)row[i];
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) n += (unsigned)__shfl_xor((int)n, d, 64);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
@@ -1156,9 +1156,10 @@ int nplm_dwconv_mask_cu(const void* mask, int32_t kind, int64_t row_stride, int6
     const dim3 grid((unsigned)B), block(256);
     hipStream_t s = (hipStream_t)stream;
     switch (kind) {
-        case 0: hipLaunchKernelGGL(mask_cu_kernel<uint8_t>, grid, block, 0, s, (const uint8_t*)mask, row_stride, L, (unsigned)B, cu); break;
-        case 1: hipLaunchKernelGGL(mask_cu_kernel<int32_t>, grid, block, 0, s, (const int32_t*)mask, row_stride, L, (unsigned)B, cu); break;
-        case 2: hipLaunchKernelGGL(mask_cu_kernel<int64_t>, grid, block, 0, s, (const int64_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        case 0: hipLaunchKernelGGL((mask_cu_kernel<uint8_t, true>), grid, block, 0, s, (const uint8_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        case 1: hipLaunchKernelGGL((mask_cu_kernel<int32_t, false>), grid, block, 0, s, (const int32_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        case 2: hipLaunchKernelGGL((mask_cu_kernel<int64_t, false>), grid, block, 0, s, (const int64_t*)mask, row_stride, L, (unsigned)B, cu); break;
+        case 3: hipLaunchKernelGGL((mask_cu_kernel<uint8_t, false>), grid, block, 0, s, (const uint8_t*)mask, row_stride, L, (unsigned)B, cu); break;
         default: return -NPLM_DWCONV_EDTYPE;
     }
     return (int)hipGetLastError();

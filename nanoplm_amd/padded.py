@@ -25,7 +25,7 @@ from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 from . import _lib
 from .dwconv import _launch_on, varlen_dwconv
 
-_MASK_KINDS = {torch.bool: 0, torch.uint8: 0, torch.int32: 1, torch.int64: 2}
+_MASK_KINDS = {torch.bool: 0, torch.int32: 1, torch.int64: 2, torch.uint8: 3}
 
 
 def right_padded_cu_seqlens(attention_mask: torch.Tensor) -> torch.Tensor:

@@ -59,6 +59,16 @@ def test_boundaries_in_one_launch_equal_the_elementwise_ones(B, L, dt):
     assert torch.equal(_flat_cu_seqlens(d.t(), x).cpu(), npa.right_padded_cu_seqlens(wide.t()))
 
 
+def test_boundaries_of_a_bool_mask_that_is_a_view_of_bytes():
+    """A bool counts as one whatever its byte holds if that is not zero (what torch's sum does); a uint8 counts as its value."""
+    from nanoplm_amd.padded import _flat_cu_seqlens
+    x = torch.zeros(1, device=DEV)
+    raw = torch.zeros(4, 300, dtype=torch.uint8)
+    raw[0, :2], raw[1, :300], raw[3, :7] = 255, 2, torch.arange(1, 8, dtype=torch.uint8)
+    assert _flat_cu_seqlens(raw.to(DEV).view(torch.bool), x).tolist() == [0, 2, 300, 600, 600, 600, 900, 907, 1200]
+    assert _flat_cu_seqlens(raw.to(DEV), x).tolist() == [0, 510, 300, 900, 600, 600, 900, 928, 1200]
+
+
 def test_traced_door_follows_the_mask_of_the_replay():
     """torch.jit.trace of the padded door with one mask, replayed with another, gives what the eager call gives."""
     x, first, w, bias = _padded_case([37, 128, 0, 1], 128, 512, 7, torch.bfloat16, seed=4)
