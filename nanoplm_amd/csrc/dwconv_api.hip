@@ -389,29 +389,68 @@ hipError_t fill_zero(float* p, long long n, hipStream_t s) {
     return hipGetLastError();
 }
 
-// cu_seqlens [2B+1] of a right-padded mask [B, L] over the flat rows: block b sums row b of the mask (a bool counts as one
-// whatever its byte if that is not zero, any other value is taken as int32, sums wrap in 32 bits) and writes b * L and b * L + that sum; the last entry is B * L. Bound by its launch: a
-// block per row has 256 loads of the row in flight, and 32 rows of 512 int64 are 128 KiB. It takes the place of
-// eight elementwise and reduction launches (sum, arange, mul, add, stack, full, cat and a copy): a padded call of 32 x 512
-// rows at C=768 goes from 65 to 25 us, of which the conv kernel is 13.
-template <typename V, bool BOOL>
-__global__ void __launch_bounds__(256) mask_cu_kernel(const V* __restrict__ mask, long long row_stride, long long L, unsigned B,
-                                                      int32_t* __restrict__ cu) {
-    __shared__ unsigned part[4];
-    const unsigned b = blockIdx.x;
-    const V* row = mask + (size_t)b * (size_t)row_stride;
+// cu_seqlens [2B+1] of a right-padded mask [B, L] over the flat rows: G threads sum a row of the mask (a bool counts as one
+// whatever its byte if that is not zero, any other value is taken as int32, sums wrap in 32 bits) and write b * L and
+// b * L + that sum; the last entry is B * L. It takes the place of eight elementwise and reduction launches (sum, arange, mul,
+// add, stack, full, cat and a copy): a padded call of 32 x 512 rows at C=768 goes from 65 to 25 us, of which the conv kernel is
+// 13. Short rows are bound by the launch and by how many blocks it starts, so several rows share a block; a long row is bound by
+// the loads that its threads have in flight, so G grows with L and a thread issues eight loads at once. Time on the device,
+// elementwise / 256 threads per row and one load at a time / this (us, int64): B=32, L=512 17.6 / 2.5 / 2.3; B=65536, L=8
+// 24.7 / 24.8 / 2.5; B=2^20, L=8 77 / 399 / 18; B=1, L=16384 20.4 / 9.8 / 3.8; B=1, L=65536 26.7 / 34.7 / 9.5; B=1024, L=16384
+// 63 / 23.1 / 20.3.
+template <typename V, bool BOOL, int G>
+__global__ void __launch_bounds__(G > 256 ? G : 256) mask_cu_kernel(const V* __restrict__ mask, long long row_stride, int L, unsigned B,
+                                                                   int32_t* __restrict__ cu) {
+    constexpr int NT = G > 256 ? G : 256;
+    const unsigned b = blockIdx.x * (NT / G) + threadIdx.x / G;
+    const int lane = threadIdx.x % G;
     unsigned n = 0;
-    for (long long i = threadIdx.x; i < L; i += 256) n += BOOL ? (unsigned)(row[i] != 0) : (unsigned)(int32_t)row[i];
+    if (b < B) {
+        const V* row = mask + (size_t)b * (size_t)row_stride;
+        auto count = [](V v) { return BOOL ? (unsigned)(v != 0) : (unsigned)(int32_t)v; };
+        int i = lane;
+        for (; i + 7 * G < L; i += 8 * G) {
+            V v[8];
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) n += (unsigned)__shfl_xor((int)n, d, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
-    __syncthreads();
-    if (threadIdx.x == 0) {
+            for (int u = 0; u < 8; ++u) v[u] = row[i + u * G];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) n += count(v[u]);
+        }
+        for (; i < L; i += G) n += count(row[i]);
+    }
+#pragma unroll
+    for (int d = (G < 64 ? G : 64) / 2; d > 0; d >>= 1) n += (unsigned)__shfl_xor((int)n, d, 64);
+    if constexpr (G > 64) {
+        __shared__ unsigned part[G / 64];
+        if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = n;
+        __syncthreads();
+        n = 0;
+#pragma unroll
+        for (int i = 0; i < G / 64; ++i) n += part[i];
+    }
+    if (lane == 0 && b < B) {
         const unsigned start = b * (unsigned)L;
         cu[2 * (size_t)b] = (int32_t)start;
-        cu[2 * (size_t)b + 1] = (int32_t)(start + part[0] + part[1] + part[2] + part[3]);
+        cu[2 * (size_t)b + 1] = (int32_t)(start + n);
         if (b + 1 == B) cu[2 * (size_t)B] = (int32_t)(B * (unsigned)L);
     }
+}
+template <typename V, bool BOOL, int G>
+hipError_t launch_mask_cu_g(const void* mask, long long row_stride, int L, unsigned B, int32_t* cu, hipStream_t s) {
+    constexpr unsigned NT = G > 256 ? G : 256, rows = NT / G;
+    hipLaunchKernelGGL((mask_cu_kernel<V, BOOL, G>), dim3((B + rows - 1) / rows), dim3(NT), 0, s, (const V*)mask, row_stride, L, B, cu);
+    return hipGetLastError();
+}
+// Threads per row by its length. Measured with 8 / 64 / 256 / 1024 (us, int64): 65536 rows of 64 6.0 / 10.2 / 28.9 / 120, of 128
+// 11.2 / 14.1 / 31.3 / 122, of 256 20.6 / 22.0 / 34.3 / 120 (1024 rows of 256 3.8 / 2.5 / 2.5 / 3.7); 16384 rows of 1024 33.5 /
+// 20.1 / 21.6 / 40.1; 32 rows of 2048 16.1 / 3.0 / 2.5 / 2.6, of 8192 58.7 / 6.0 / 3.5 / 3.3; one row of 16384 37 / 7.2 / 4.4 / 3.8,
+// of 65536 - / 24.1 / 12.4 / 9.5.
+template <typename V, bool BOOL>
+hipError_t launch_mask_cu(const void* mask, long long row_stride, int L, unsigned B, int32_t* cu, hipStream_t s) {
+    if (L <= 128) return launch_mask_cu_g<V, BOOL, 8>(mask, row_stride, L, B, cu, s);
+    if (L <= 1024) return launch_mask_cu_g<V, BOOL, 64>(mask, row_stride, L, B, cu, s);
+    if (L <= 8192) return launch_mask_cu_g<V, BOOL, 256>(mask, row_stride, L, B, cu, s);
+    return launch_mask_cu_g<V, BOOL, 1024>(mask, row_stride, L, B, cu, s);
 }
 
 // launch flags of the kernels (W_BF16 | W_RESIDUAL) from the ABI's weight dtype and flags
@@ -1151,18 +1190,16 @@ size_t nplm_dwconv_bwd_workspace_bytes(int64_t T, int32_t C, int32_t K, int32_t 
 }
 
 int nplm_dwconv_mask_cu(const void* mask, int32_t kind, int64_t row_stride, int64_t B, int64_t L, int32_t* cu, void* stream) {
-    if (B < 1 || B > kMaxRows || L < 1 || L > kMaxRows || row_stride < 0) return -NPLM_DWCONV_ESHAPE;
+    if (B < 1 || B > 1 << 28 || L < 1 || L > kMaxRows / B || row_stride < 0) return -NPLM_DWCONV_ESHAPE;    // a grid has fewer than 2^32 threads
     if (!mask || !cu) return -NPLM_DWCONV_ENULL;
-    const dim3 grid((unsigned)B), block(256);
     hipStream_t s = (hipStream_t)stream;
     switch (kind) {
-        case 0: hipLaunchKernelGGL((mask_cu_kernel<uint8_t, true>), grid, block, 0, s, (const uint8_t*)mask, row_stride, L, (unsigned)B, cu); break;
-        case 1: hipLaunchKernelGGL((mask_cu_kernel<int32_t, false>), grid, block, 0, s, (const int32_t*)mask, row_stride, L, (unsigned)B, cu); break;
-        case 2: hipLaunchKernelGGL((mask_cu_kernel<int64_t, false>), grid, block, 0, s, (const int64_t*)mask, row_stride, L, (unsigned)B, cu); break;
-        case 3: hipLaunchKernelGGL((mask_cu_kernel<uint8_t, false>), grid, block, 0, s, (const uint8_t*)mask, row_stride, L, (unsigned)B, cu); break;
-        default: return -NPLM_DWCONV_EDTYPE;
+        case 0: return (int)launch_mask_cu<uint8_t, true>(mask, row_stride, (int)L, (unsigned)B, cu, s);
+        case 1: return (int)launch_mask_cu<int32_t, false>(mask, row_stride, (int)L, (unsigned)B, cu, s);
+        case 2: return (int)launch_mask_cu<int64_t, false>(mask, row_stride, (int)L, (unsigned)B, cu, s);
+        case 3: return (int)launch_mask_cu<uint8_t, false>(mask, row_stride, (int)L, (unsigned)B, cu, s);
     }
-    return (int)hipGetLastError();
+    return -NPLM_DWCONV_EDTYPE;
 }
 
 int32_t nplm_dwconv_exec_kernel_size(int32_t K) { return exec_kernel_size(K); }

@@ -52,7 +52,7 @@ int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype
 // The kernel size K' a plain or gated conv of K taps runs as (K itself for 3, 5, 7, 9, 15, 31 and above 31).
 int32_t nplm_dwconv_exec_kernel_size(int32_t K);
 
-// cu [2B+1] = 0, len_0, L, L + len_1, 2L, ..., B*L of a right-padded mask [B, L] in device memory (B, L >= 1): kind 0 = bool
+// cu [2B+1] = 0, len_0, L, L + len_1, 2L, ..., B*L of a right-padded mask [B, L] in device memory (B, L >= 1; B <= 2^28): kind 0 = bool
 // (any non-zero byte counts as one), 1 = int32, 2 = int64, 3 = uint8; row_stride in elements, the elements of a row adjacent.
 int nplm_dwconv_mask_cu(const void* mask, int32_t kind, int64_t row_stride, int64_t B, int64_t L, int32_t* cu, void* stream);
 

@@ -49,13 +49,20 @@ def _operations_are_recorded() -> bool:
     return torch.compiler.is_compiling() or torch.jit.is_tracing() or is_in_torch_dispatch_mode()
 
 
+def _one_launch_pays(B: int, L: int) -> bool:
+    """The one launch has one block for a long row, where the elementwise operations spread it over the chip. Time on the
+    device, one launch / elementwise (us, int64): B=32, L=512 2.3 / 17.8; B=1, L=65536 9.5 / 26.7, L=131072 17.7 / 25.3,
+    L=262144 32.9 / 26.0; B=256, L=65536 20.3 / 59; B=2^20, L=1 13.2 / 38.8, the most rows that were timed."""
+    return 0 < B <= 1 << 20 and 0 < L <= 1 << 17
+
+
 def _flat_cu_seqlens(mask: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """:func:`right_padded_cu_seqlens` for a call that runs the kernels at once: one launch for a bool or integer mask
-    with adjacent row elements on x's device, the elementwise operations for any other and wherever operations are
-    recorded (a recorded launch would be an ``empty`` that nothing fills)."""
+    with adjacent row elements on x's device, the elementwise operations for any other, for the sizes at which they may be
+    the faster way and wherever operations are recorded (a recorded launch would be an ``empty`` that nothing fills)."""
     kind = _MASK_KINDS.get(mask.dtype)
     if (_operations_are_recorded() or type(mask) is not torch.Tensor or kind is None or not x.is_cuda
-            or mask.device != x.device or mask.numel() == 0 or (mask.shape[1] > 1 and mask.stride(1) != 1)):
+            or mask.device != x.device or not _one_launch_pays(*mask.shape) or (mask.shape[1] > 1 and mask.stride(1) != 1)):
         return right_padded_cu_seqlens(mask)
     B, L = mask.shape
     cu = torch.empty((2 * B + 1,), dtype=torch.int32, device=mask.device)

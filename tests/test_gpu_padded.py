@@ -47,10 +47,13 @@ def test_right_padded_batch_in_place(residual):
 
 
 @pytest.mark.parametrize("dt", [torch.bool, torch.uint8, torch.int32, torch.int64, torch.float32])
-@pytest.mark.parametrize("B,L", [(1, 1), (3, 64), (5, 255), (2, 257), (300, 7), (0, 8), (4, 0)])
+@pytest.mark.parametrize("B,L", [(1, 1), (33, 63), (31, 65), (32, 128), (5, 129), (3, 640), (6, 1024), (2, 1025), (2, 8192), (1, 8193),
+                                 (2, 9000), (1, 1 << 17), (1, (1 << 17) + 1), (65537, 2), (0, 8), (4, 0)])
 def test_boundaries_in_one_launch_equal_the_elementwise_ones(B, L, dt):
-    """Masks around the 256 threads of a block, with rows that are a slice of a wider tensor and transposed ones (which
-    take the elementwise operations), against the boundaries formed on the CPU; not every row is right-padded."""
+    """Row lengths around those at which more threads share a row (128, 1024, 8192) and their passes of eight loads, numbers
+    of rows around those of a block, the longest row of the one launch, rows that are a slice of a wider tensor and
+    transposed ones (which take the elementwise operations), against the boundaries formed on the CPU; not every row is
+    right-padded."""
     from nanoplm_amd.padded import _flat_cu_seqlens
     wide = (torch.rand(B, L + 3, generator=torch.Generator().manual_seed(B * L)) > 0.3).to(dt)
     x = torch.zeros(1, device=DEV)

@@ -39,18 +39,33 @@ class _HostMaskCu:
         return 0
 
 
+_ON_THE_MASKS_DEVICE = SimpleNamespace(is_cuda=True, device=torch.device("cpu"))
+
+
+def _play_the_launch_on_the_host(monkeypatch):
+    lib = _HostMaskCu()
+    monkeypatch.setattr(padded._lib, "load", lambda: lib)
+    monkeypatch.setattr(padded, "_launch_on", lambda t: contextlib.nullcontext(SimpleNamespace(stream=None)))
+    return lib
+
+
 @pytest.mark.parametrize("record", [lambda f, m: torch.jit.trace(f, (m,)), lambda f, m: make_fx(f)(m)], ids=["jit.trace", "make_fx"])
 def test_recorded_boundaries_follow_the_mask_of_the_replay(monkeypatch, record):
     """The library's launch is invisible to whatever records torch operations, so a recorded call has to hold the
     elementwise operations: recorded with one mask and replayed with another it gives the other's boundaries."""
-    lib = _HostMaskCu()
-    monkeypatch.setattr(padded._lib, "load", lambda: lib)
-    monkeypatch.setattr(padded, "_launch_on", lambda t: contextlib.nullcontext(SimpleNamespace(stream=None)))
-    x = SimpleNamespace(is_cuda=True, device=torch.device("cpu"))
+    lib, x = _play_the_launch_on_the_host(monkeypatch), _ON_THE_MASKS_DEVICE
     first, second = torch.tensor([[1, 0, 0, 0], [1, 1, 1, 0]]), torch.tensor([[1, 1, 0, 0], [1, 1, 1, 1]])
     assert padded._flat_cu_seqlens(first, x).tolist() == [0, 1, 4, 7, 8] and lib.calls == 1
     recorded = record(lambda m: padded._flat_cu_seqlens(m, x), first)
     assert recorded(second).tolist() == [0, 2, 4, 8, 8]
+
+
+@pytest.mark.parametrize("B,L,launches", [(1, 1 << 17, 1), (1, (1 << 17) + 1, 0), (1 << 20, 1, 1), ((1 << 20) + 1, 1, 0), (3, 0, 0), (0, 3, 0)])
+def test_long_rows_and_very_many_rows_keep_the_elementwise_boundaries(monkeypatch, B, L, launches):
+    lib = _play_the_launch_on_the_host(monkeypatch)
+    mask = (torch.arange(L)[None, :] < 1 + torch.arange(B)[:, None]).to(torch.int64)
+    assert torch.equal(padded._flat_cu_seqlens(mask, _ON_THE_MASKS_DEVICE), npa.right_padded_cu_seqlens(mask))
+    assert lib.calls == launches
 
 
 def test_unpad_and_pad_follow_the_reference_contracts():
