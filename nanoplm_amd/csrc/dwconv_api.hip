@@ -35,11 +35,11 @@ constexpr long long kMaxRows = (long long)INT_MAX - (1 << 20);   // row arithmet
 constexpr int kMaxTileRows = 1 << 16;
 constexpr size_t kSlabBudgetBytes = 16u << 20;   // cap on dw/db partials (written once, read once)
 
-bool specialised_k(int K) { return K == 3 || K == 5 || K == 7 || K == 9 || K == 15 || K == 31; }
+constexpr bool specialised_k(int K) { return K == 3 || K == 5 || K == 7 || K == 9 || K == 15 || K == 31; }
 // The kernel size a plain conv of K taps runs as: an odd K below 31 without kernels of its own takes the next size that
 // has them, with (exec - K) / 2 zero taps on either side (W_TAP_OFF_SHIFT); the caller's weight and dw rows stay K long.
 // Runtime-K kernels (one wave per row) remain for K > 31.
-int exec_kernel_size(int K) { return K > 31 || specialised_k(K) ? K : K < 3 ? 3 : K < 15 ? 15 : 31; }
+constexpr int exec_kernel_size(int K) { return K > 31 || specialised_k(K) ? K : K < 3 ? 3 : K < 15 ? 15 : 31; }
 
 // The number of taps the LDS-staged and role-split kernels run such a size with: they are built for 11 and 21 taps as well,
 // so K = 11 and K = 17 .. 21 leave out zero taps (and halo rows) of the 15 and 31 that plans and workspaces are made for.
@@ -48,7 +48,23 @@ int exec_kernel_size(int K) { return K > 31 || specialised_k(K) ? K : K < 3 ? 3 
 // with backward 304 -> 262; K=17 130 -> 104, 379 -> 313; K=21 133 -> 108, 379 -> 318; gated K=11 191 -> 185, 457 -> 427, K=21
 // 226 -> 199, 588 -> 504; fp32 forward and backward 455 -> 446 (K=11), 544 -> 492 (K=21). A form of 13 taps would save two of 15
 // taps where 11 saves four, one of 25 six of 31: neither is built.
-int lds_taps(int K) { return K == 11 ? 11 : K >= 17 && K <= 21 ? 21 : exec_kernel_size(K); }
+constexpr int lds_taps(int K) { return K == 11 ? 11 : K >= 17 && K <= 21 ? 21 : exec_kernel_size(K); }
+
+// A role-split call is planned (tiles, column blocks) with the shape of exec_kernel_size(K) and launched with the kernel's own
+// shape at lds_taps(K): they have to be one shape for every K, else rows would be left out or computed twice.
+constexpr bool split_plans_fit_their_kernels() {
+    for (int K = 1; K <= 31; K += 2)
+        for (int v = 0; v < 4; ++v) {
+            const bool fwd = v & 1, bf16 = v & 2;
+            const int plan = exec_kernel_size(K), run = lds_taps(K);
+            if (!lds_split_kernel_size(plan)) continue;
+            if (lds_split_shape(fwd, bf16, plan) != lds_split_shape(fwd, bf16, run)) return false;
+            if (lds_split_gated_shape(bf16, plan) != lds_split_gated_shape(bf16, run)) return false;
+            if (lds_split_gated_fwd_shape(bf16, plan) != lds_split_gated_fwd_shape(bf16, run)) return false;
+        }
+    return true;
+}
+static_assert(split_plans_fit_their_kernels(), "a role-split plan and the kernel it launches differ in shape");
 
 int pow2_floor(int v) { int p = 1; while (p * 2 <= v) p *= 2; return p; }
 int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }

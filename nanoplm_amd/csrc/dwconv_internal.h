@@ -249,6 +249,7 @@ constexpr LdsShapeSel lds_default_shape(bool bwd, bool bf16, int K) {
 //     at K = 31 only: at K = 15 the forward with loader waves is faster (C=2048: 190 against 203 us).
 struct SplitShapeSel {
     int vec, rw, nrg, ncw;
+    constexpr bool operator!=(const SplitShapeSel& o) const { return vec != o.vec || rw != o.rw || nrg != o.nrg || ncw != o.ncw; }
 };
 constexpr bool lds_split_kernel_size(int K) { return K == 31 || K == 15; }
 constexpr SplitShapeSel lds_split_shape(bool fwd, bool bf16, int K) {
