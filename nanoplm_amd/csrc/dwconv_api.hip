@@ -312,11 +312,20 @@ hipError_t launch_bwd_lds(int K, const LdsPlan& p, bool wdx, bool wdw, const Con
         }                                                                                                \
         return hipErrorInvalidConfiguration;                                                             \
     }
-NPLM_LAUNCH_SPLIT(launch_fwd_split)
 NPLM_LAUNCH_SPLIT(launch_bwd_split)
 NPLM_LAUNCH_SPLIT(launch_fwd_split_gated)
 NPLM_LAUNCH_SPLIT(launch_bwd_split_gated)
 #undef NPLM_LAUNCH_SPLIT
+// The library takes the plain forward of up to 15 taps to the kernels with loader waves (choose_algo()); of the role-split
+// ones only the size that shape overrides may name is built, and calls of 11 taps run there with 15.
+hipError_t launch_fwd_split(int taps, bool bf16, const ConvPtrs& a, const LdsGeo& g, dim3 grid, hipStream_t s) {
+    switch (taps) {
+        case 15: return launch_fwd_split_k15(bf16, a, g, grid, s);
+        case 21: return launch_fwd_split_k21(bf16, a, g, grid, s);
+        case 31: return launch_fwd_split_k31(bf16, a, g, grid, s);
+    }
+    return hipErrorInvalidConfiguration;
+}
 
 bool split_eligible(bool bf16, long long T, int C, int K, uintptr_t align_bits) {
     const int E = bf16 ? 2 : 4;
@@ -525,8 +534,9 @@ int fwd_impl(const void* x, const int32_t* cu, const void* w, const void* b, voi
         rc = make_split_plan(true, bf16, T, C, K, tune, &lp);
         if (rc) return rc;
         const ConvPtrs la{x, nullptr, cu, w, b, y, nullptr};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, lds_w_flags);
-        return (int)launch_fwd_split(taps, bf16, la, lg, dim3(lp.ncb * lp.nbt), s);
+        const int run = K == 31 ? taps : K;
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, run == K ? w_flags : lds_w_flags);
+        return (int)launch_fwd_split(run, bf16, la, lg, dim3(lp.ncb * lp.nbt), s);
     }
     if (algo == 2) {
         // of the shorter forms the loader-wave forward has the one of 11 taps; shape overrides name shapes of K

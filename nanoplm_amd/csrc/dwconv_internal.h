@@ -124,7 +124,6 @@ hipError_t launch_fwd_lds_gated_k31(bool bf16, bool narrow, const ConvPtrs& p, c
 // role-split LDS kernels (fixed shape per dtype, see lds_split_shape()); gated: z = [u | g] in, y or dz out, see
 // lds_split_gated_fwd_shape() and lds_split_gated_shape()
 #define NPLM_DECLARE_SPLIT_K(KK)                                                                                        \
-    hipError_t launch_fwd_split_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);       \
     hipError_t launch_bwd_split_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);       \
     hipError_t launch_fwd_split_gated_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s); \
     hipError_t launch_bwd_split_gated_k##KK(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
@@ -132,6 +131,9 @@ NPLM_DECLARE_SPLIT_K(11)
 NPLM_DECLARE_SPLIT_K(15)
 NPLM_DECLARE_SPLIT_K(21)
 NPLM_DECLARE_SPLIT_K(31)
+hipError_t launch_fwd_split_k15(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
+hipError_t launch_fwd_split_k21(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
+hipError_t launch_fwd_split_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 #undef NPLM_DECLARE_SPLIT_K
 // LayerNorm-fused forward (dwconv_ln_kernels.h), K <= 9, fixed shape per dtype, see lds_ln_shape()
 hipError_t launch_ln_fwd_k3(bool bf16, const ConvPtrs& p, const LnArgs& ln, const LdsGeo& g, dim3 grid, hipStream_t s);

@@ -1,3 +1,3 @@
-// LDS-staged forward and role-split kernels of 11 taps (K = 11).
+// LDS-staged forward, role-split backward and gated kernels of 11 taps (K = 11).
 #define NPLM_K 11
 #include "dwconv_lds_inst.inc"
