@@ -60,14 +60,15 @@ def _flat_cu_seqlens(mask: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """:func:`right_padded_cu_seqlens` for a call that runs the kernels at once: one launch for a bool or integer mask
     with adjacent row elements on x's device, the elementwise operations for any other, for the sizes at which they may be
     the faster way and wherever operations are recorded (a recorded launch would be an ``empty`` that nothing fills)."""
-    kind = _MASK_KINDS.get(mask.dtype)
-    if (_operations_are_recorded() or type(mask) is not torch.Tensor or kind is None or not x.is_cuda
-            or mask.device != x.device or not _one_launch_pays(*mask.shape) or (mask.shape[1] > 1 and mask.stride(1) != 1)):
+    if _operations_are_recorded() or type(mask) is not torch.Tensor or not x.is_cuda:
         return right_padded_cu_seqlens(mask)
-    B, L = mask.shape
-    cu = torch.empty((2 * B + 1,), dtype=torch.int32, device=mask.device)
+    (B, L), (row_stride, step) = mask.shape, mask.stride()
+    kind, device = _MASK_KINDS.get(mask.dtype), mask.device
+    if kind is None or device != x.device or not _one_launch_pays(B, L) or (step != 1 and L > 1):
+        return right_padded_cu_seqlens(mask)
+    cu = torch.empty(2 * B + 1, dtype=torch.int32, device=device)
     with _launch_on(mask) as dev:
-        rc = _lib.load().nplm_dwconv_mask_cu(mask.data_ptr(), kind, mask.stride(0), B, L, cu.data_ptr(), dev.stream)
+        rc = _lib.load().nplm_dwconv_mask_cu(mask.data_ptr(), kind, row_stride, B, L, cu.data_ptr(), dev.stream)
     _lib.check(rc, "nplm_dwconv_mask_cu")
     return cu
 
