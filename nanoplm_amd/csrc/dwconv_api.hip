@@ -43,11 +43,13 @@ constexpr int exec_kernel_size(int K) { return K > 31 || specialised_k(K) ? K : 
 
 // The number of taps the LDS-staged and role-split kernels run such a size with: they are built for 11 and 21 taps as well,
 // so K = 11 and K = 17 .. 21 leave out zero taps (and halo rows) of the 15 and 31 that plans and workspaces are made for.
-// Tiles, token blocks and the order of every sum are those of exec_kernel_size(K); a slab is shorter and fits its place.
+// The role-split kernels' tiles and token blocks and the order of every sum are those of exec_kernel_size(K); a slab holds
+// lds_taps(K) + 1 rows and fits its place.
 // Measured at C=2048, T=65536, log-normal lengths, bf16, whole calls, running as 15 / 31 -> this (us): K=11 forward 111 -> 93,
 // with backward 304 -> 262; K=17 130 -> 104, 379 -> 313; K=21 133 -> 108, 379 -> 318; gated K=11 191 -> 185, 457 -> 427, K=21
-// 226 -> 199, 588 -> 504; fp32 forward and backward 455 -> 446 (K=11), 544 -> 492 (K=21). A form of 13 taps would save two of 15
-// taps where 11 saves four, one of 25 six of 31: neither is built.
+// 226 -> 199, 588 -> 504; fp32 forward and backward 455 -> 446 (K=11), 544 -> 492 (K=21). Forms of 13 and 25 taps, which are not
+// built, would give (forward / backward alone, same sizes): K=13 107 / 170 -> 93 / 163, gated 185 / 264 -> 180 / 258, fp32 179 / 271
+// -> 173 / 269; K=23 and 25 136 / 249 -> 118 / 221, gated 229 / 361 -> 210 / 327, fp32 205 / 340 -> 207 / 305.
 constexpr int lds_taps(int K) { return K == 11 ? 11 : K >= 17 && K <= 21 ? 21 : exec_kernel_size(K); }
 
 // A role-split call is planned (tiles, column blocks) with the shape of exec_kernel_size(K) and launched with the kernel's own
@@ -478,7 +480,6 @@ hipError_t launch_mask_cu(const void* mask, long long row_stride, int L, unsigne
     return launch_mask_cu_g<V, BOOL, 1024>(mask, row_stride, L, B, cu, s);
 }
 
-// launch flags of the kernels (W_BF16 | W_RESIDUAL) from the ABI's weight dtype and flags
 // Shapes the gated (z = [u | g]) kernels are built for.
 bool gated_supported(bool bwd, bool bf16, long long T, int C, int K, uintptr_t align_bits) {
     const int E = bf16 ? 2 : 4;
@@ -504,6 +505,7 @@ int make_long_gated_plan(bool bf16, long long T, int C, int K, Plan* out) {
     return make_plan(true, bf16, T, C, K, 0, &t, out);
 }
 
+// launch flags of the kernels (W_BF16 | W_RESIDUAL) from the ABI's weight dtype and flags
 int kernel_w_flags(int32_t w_dtype, uint32_t flags) {
     return (w_dtype == NPLM_DWCONV_BF16 ? W_BF16 : 0) | ((flags & NPLM_DWCONV_RESIDUAL) ? W_RESIDUAL : 0);
 }
@@ -585,7 +587,7 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
         return (int)e;
     }
     const int taps = lds_taps(K), lds_tap_off = (taps - K) / 2, tap_off = (exec_kernel_size(K) - K) / 2;
-    K = exec_kernel_size(K);        // from here on the kernel size that runs (slabs of K + 1 rows; dw rows stay the caller's)
+    K = exec_kernel_size(K);        // from here on the kernel size that runs (workspace for slabs of K + 1 rows; dw rows stay the caller's)
     const int w_flags = kernel_w_flags(w_dtype, flags) | (tap_off << W_TAP_OFF_SHIFT);
     if (!dx && !want_red) return 0;
     if (!dy || !cu || !w || (want_red && !x)) return -NPLM_DWCONV_ENULL;
@@ -1093,7 +1095,7 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
     if (!z || !dy || !cu || !w || !dz) return -NPLM_DWCONV_ENULL;
     const int taps = lds_taps(K), lds_tap_off = (taps - K) / 2;
     const int tap_off = (exec_kernel_size(K) - K) / 2, tap_flags = tap_off << W_TAP_OFF_SHIFT;
-    K = exec_kernel_size(K);        // from here on the kernel size that runs (slabs of K + 1 rows; dw rows stay the caller's)
+    K = exec_kernel_size(K);        // from here on the kernel size that runs (workspace for slabs of K + 1 rows; dw rows stay the caller's)
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;

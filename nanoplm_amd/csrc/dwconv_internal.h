@@ -49,7 +49,8 @@ int nplm_dwconv_bwd_tuned(const void* x, const void* dy, const int32_t* cu, cons
 // Token-blocks (= workspace slabs of (K'+1)*C floats, K' the kernel size that runs: K, or for an odd K <= 31 without
 // kernels of its own the next of 3, 15, 31) a backward launch with these overrides uses.
 int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype, const nplm_dwconv_tuning* tune);
-// The kernel size K' a plain or gated conv of K taps runs as (K itself for 3, 5, 7, 9, 15, 31 and above 31).
+// The kernel size K' a plain or gated conv of K taps is planned as, and its workspace made for (K itself for 3, 5, 7, 9, 15, 31
+// and above 31); K = 11 and 17 .. 21 run kernels of 11 and 21 taps where they take LDS-staged or role-split ones.
 int32_t nplm_dwconv_exec_kernel_size(int32_t K);
 
 // cu [2B+1] = 0, len_0, L, L + len_1, 2L, ..., B*L of a right-padded mask [B, L] in device memory (B, L >= 1; B <= 2^28): kind 0 = bool

@@ -121,8 +121,9 @@ def bwd_workspace_bytes(T: int, C: int, K: int, dtype: torch.dtype) -> int:
 
 
 def exec_kernel_size(K: int) -> int:
-    """The kernel size a plain conv of K taps runs as: an odd K <= 31 that has no kernels of its own takes the next
-    size that has, with zero taps on either side; its dw/db slabs have that many rows."""
+    """The kernel size a plain conv of K taps is planned as, and its workspace made for: an odd K <= 31 that has no
+    kernels of its own takes the next size that has, with zero taps on either side (K = 11 and 17 .. 21 with fewer of
+    them on the LDS-staged and role-split kernels, whose slabs then fill part of their place)."""
     return int(_lib.load().nplm_dwconv_exec_kernel_size(K))
 
 

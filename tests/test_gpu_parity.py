@@ -55,8 +55,9 @@ def test_configuration_matches_oracle(index):
 
 @pytest.mark.parametrize("K", [11, 21])
 def test_headline_size_with_a_kernel_size_served_by_the_next_built_size(K):
-    """Configuration 3's tokens, lengths and width (T=131072, C=1024, bf16) with K = 11 (runs as 15) and K = 21 (runs as
-    31, the role-split kernels: every block walks 16 forward and 32 backward tiles) against the C oracle, and run twice."""
+    """Configuration 3's tokens, lengths and width (T=131072, C=1024, bf16) with K = 11 (planned as 15, on kernels
+    of 11 taps) and K = 21 (planned as 31, on the role-split kernels of 21 taps: every block walks 16 forward and 32
+    backward tiles) against the C oracle, and run twice."""
     print(f"[case] configuration 3 with K={K}", flush=True)
     wl = make_workload(3, with_dy=True)
     g = torch.Generator().manual_seed(K)
