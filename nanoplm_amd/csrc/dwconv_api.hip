@@ -318,8 +318,8 @@ NPLM_LAUNCH_SPLIT(launch_bwd_split)
 NPLM_LAUNCH_SPLIT(launch_fwd_split_gated)
 NPLM_LAUNCH_SPLIT(launch_bwd_split_gated)
 #undef NPLM_LAUNCH_SPLIT
-// The library takes the plain forward of up to 15 taps to the kernels with loader waves (choose_algo()); of the role-split
-// ones only the size that shape overrides may name is built, and calls of 11 taps run there with 15.
+// The library takes a plain forward of up to 15 taps to the matrix cores or to the kernels with loader waves (choose_algo());
+// of the role-split ones only the size that shape overrides may name is built, and calls of 11 taps run there with 15.
 hipError_t launch_fwd_split(int taps, bool bf16, const ConvPtrs& a, const LdsGeo& g, dim3 grid, hipStream_t s) {
     switch (taps) {
         case 15: return launch_fwd_split_k15(bf16, a, g, grid, s);
@@ -329,6 +329,19 @@ hipError_t launch_fwd_split(int taps, bool bf16, const ConvPtrs& a, const LdsGeo
     return hipErrorInvalidConfiguration;
 }
 
+#define NPLM_LAUNCH_MFMA(NAME)                                                                \
+    hipError_t NAME(int taps, const ConvPtrs& a, const LdsGeo& g, dim3 grid, hipStream_t s) { \
+        switch (taps) {                                                                       \
+            case 11: return NAME##_k11(a, g, grid, s);                                        \
+            case 15: return NAME##_k15(a, g, grid, s);                                        \
+            case 21: return NAME##_k21(a, g, grid, s);                                        \
+            case 31: return NAME##_k31(a, g, grid, s);                                        \
+        }                                                                                     \
+        return hipErrorInvalidConfiguration;                                                  \
+    }
+NPLM_LAUNCH_MFMA(launch_fwd_mfma)
+#undef NPLM_LAUNCH_MFMA
+
 bool split_eligible(bool bf16, long long T, int C, int K, uintptr_t align_bits) {
     const int E = bf16 ? 2 : 4;
     if (!lds_split_kernel_size(K) || T < 1) return false;
@@ -336,8 +349,13 @@ bool split_eligible(bool bf16, long long T, int C, int K, uintptr_t align_bits) 
     const SplitShapeSel sh = lds_split_shape(false, bf16, K);      // the column block is the same in both passes
     return (long long)C * E >= (long long)sh.ncw * 64 * sh.vec * E;
 }
+// The matrix-core kernels (dwconv_mfma_kernels.h) have the column blocks of the role-split ones in bf16.
+bool mfma_eligible(bool bf16, bool w_bf16, long long T, int C, int K, uintptr_t align_bits) {
+    return bf16 && w_bf16 && split_eligible(bf16, T, C, K, align_bits);
+}
+constexpr long long kMfmaMinRows = 4096;
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
-                    bool gated = false) {
+                    bool gated = false, int tile_rows = 0) {
     LdsPlan p{};
     nplm_dwconv_tuning z{};
     if (!tune) tune = &z;
@@ -345,7 +363,7 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
     const SplitShapeSel sh = !gated ? lds_split_shape(fwd, bf16, K) : fwd ? lds_split_gated_fwd_shape(bf16, K) : lds_split_gated_shape(bf16, K);
     const long long cb_bytes = (long long)sh.ncw * 64 * sh.vec * E;
     const long long row_bytes = (long long)C * E;
-    p.R = sh.rw * sh.nrg;
+    p.R = tile_rows ? tile_rows : sh.rw * sh.nrg;
     if ((long long)(p.R + K) * row_bytes * (gated ? 2 : 1) + 2 * row_bytes >= INT_MAX) return -NPLM_DWCONV_ESHAPE;
     p.ncb = ceil_div(row_bytes, cb_bytes);
     p.ntiles = ceil_div(T, p.R);
@@ -367,20 +385,30 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
     return 0;
 }
 
-// algo requested by the caller (0 = library's choice) -> 1 sliding-window, 2 LDS-staged, 3 role-split LDS-staged.
-// Measured on MI355X, bf16, T=131072:
+// algo requested by the caller (0 = library's choice) -> 1 sliding-window, 2 LDS-staged, 3 role-split LDS-staged, 4 matrix
+// cores. Measured on MI355X, bf16, T=131072:
 //   K=7, C=1024: both passes are fastest LDS-staged (the chip sweeps one compact window of rows with every load of a
 //     tile issued at once).
-//   K=31 and K=15 backward (ALU-bound; one wave cannot hold the fused backward's registers): the role-split kernel,
-//     when every output is asked for - C=2048, K=31: 510 us against 720 sliding-window on the log-normal length mix;
+//   11 to 31 taps, bf16 weights too, forward: matrix cores. On the vector ALU these sizes are bound by their FMAs (K=31, one
+//     sequence: 248 us where a copy of the same bytes takes 208); in us, matrix cores against the best of the others:
+//     K=31 C=2048: 202 against 260 (log-normal lengths), 184 / 248 (one sequence), 250 / 289 (20 to 128 residues);
+//     K=21 C=1024: 102 / 112; K=15: 182 / 192 at C=2048, 97 / 101 at C=1024; K=11 C=1024: 95 / 100;
+//     T=16384 C=1024: 24.6 / 28.6 at K=31, 17.7 / 21.4 at K=11. From kMfmaMinRows rows on: below, every block has a tile
+//     or two and what is measured is the launch (2048 rows, C=1024: K=31 11.8 / 12.5, K=15 10.0 / 10.2; 600 rows, C=512:
+//     12.2 / 11.8), while the others' sums are those of the sliding-window kernels bit for bit.
+//     fp32 weights would take three bf16 terms each: 280 us against 265 (K=31, C=2048), so they stay on the vector ALU.
+//   K=31 and K=15 backward (ALU-bound; one wave cannot hold the fused backward's registers): the role-split
+//     kernel, when every output is asked for - C=2048, K=31: 510 us against 720 sliding-window on the log-normal length mix;
 //     K=15: 345 against 385 (C=1024: 177 against 205). A backward asked for dx alone or dw/db alone takes the
 //     sliding-window kernel, like everything the LDS kernels are not built for (other sizes, narrow or unaligned rows).
-//   K=31 forward: the role-split kernel's dx role on every wave, 262 us against 299 LDS-staged with loader waves (C=2048).
-//   K=15 forward: LDS-staged with loader waves, 190 us against 203 role-split and 227 sliding-window (C=2048).
-int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, long long T, int C, int K, uintptr_t align_bits) {
+//   K=31 forward of fp32 weights: the role-split kernel's dx role on every wave, 262 us against 299 LDS-staged with loader
+//     waves (C=2048); K=15: LDS-staged with loader waves, 190 us against 203 role-split and 227 sliding-window (C=2048).
+int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, bool w_bf16, long long T, int C, int K, uintptr_t align_bits) {
+    if (tune && tune->algo == 4) return !bwd && mfma_eligible(bf16, w_bf16, T, C, K, align_bits) ? 4 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 3) return split_eligible(bf16, T, C, K, align_bits) ? 3 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 2) return lds_eligible(bf16, T, C, K, align_bits) ? 2 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 1) return 1;
+    if (mfma_eligible(bf16, w_bf16, T, C, K, align_bits) && T >= kMfmaMinRows && !bwd) return 4;
     if (split_eligible(bf16, T, C, K, align_bits) && (bwd || K == 31)) return 3;
     return lds_preferred(bwd, bf16, T, C, K, align_bits) ? 2 : 1;
 }
@@ -529,13 +557,14 @@ int fwd_impl(const void* x, const int32_t* cu, const void* w, const void* b, voi
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if (((uintptr_t)w | (uintptr_t)b) % WE || (uintptr_t)cu % 4) return -NPLM_DWCONV_EALIGN;
     hipStream_t s = (hipStream_t)stream;
-    const int algo = choose_algo(false, tune, bf16, T, C, K, bits);
+    const int algo = choose_algo(false, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, bits);
     if (algo < 0) return algo;
-    if (algo == 3) {
+    if (algo == 3 || algo == 4) {
         LdsPlan lp;
-        rc = make_split_plan(true, bf16, T, C, K, tune, &lp);
+        rc = make_split_plan(true, bf16, T, C, K, tune, &lp, false, algo == 4 ? kMfmaFwdRows : 0);
         if (rc) return rc;
         const ConvPtrs la{x, nullptr, cu, w, b, y, nullptr};
+        if (algo == 4) return (int)launch_fwd_mfma(taps, la, make_lds_geo(lp, T, C, S, w_flags), dim3(lp.ncb * lp.nbt), s);
         const int run = K == 31 ? taps : K;
         const LdsGeo lg = make_lds_geo(lp, T, C, S, run == K ? w_flags : lds_w_flags);
         return (int)launch_fwd_split(run, bf16, la, lg, dim3(lp.ncb * lp.nbt), s);
@@ -598,7 +627,7 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
 
-    int algo = choose_algo(true, tune, bf16, T, C, K, bits);
+    int algo = choose_algo(true, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, bits);
     if (algo < 0) return algo;
     if (algo == 3 && !(dx && want_red)) {     // the role-split kernel is fused only: a partial request takes the others
         if (tune && tune->algo == 3) return -NPLM_DWCONV_ETUNING;
@@ -1205,7 +1234,7 @@ size_t nplm_dwconv_bwd_workspace_bytes(int64_t T, int32_t C, int32_t K, int32_t 
     Plan p;
     if (make_plan(true, bf16, T, C, K, 0, nullptr, &p)) return 0;
     int slabs = p.nbt;
-    if (choose_algo(true, nullptr, bf16, T, C, K, 0) == 2) {
+    if (choose_algo(true, nullptr, bf16, true, T, C, K, 0) == 2) {
         LdsPlan lp;
         if (make_lds_plan(true, bf16, T, C, K, nullptr, &lp) == 0 && lp.nbt > slabs) slabs = lp.nbt;
     }
@@ -1236,7 +1265,7 @@ int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype
     if (check_common(T, C, K, 0, act_dtype, NPLM_DWCONV_F32) || T == 0) return 0;
     K = exec_kernel_size(K);
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
-    const int algo = choose_algo(true, tune, bf16, T, C, K, 0);
+    const int algo = choose_algo(true, tune, bf16, true, T, C, K, 0);
     if (algo < 0) return 0;
     if (algo == 3) {
         LdsPlan lp;

@@ -8,6 +8,7 @@
 #include "dwconv_kernels.h"
 #include "dwconv_lds_kernels.h"
 #include "dwconv_lds_split_kernels.h"
+#include "dwconv_mfma_kernels.h"
 #include "dwconv_ln_kernels.h"
 
 #ifdef __cplusplus
@@ -25,7 +26,7 @@ typedef struct nplm_dwconv_tuning {
     int32_t xcd_remap;  // 1 = give each XCD a contiguous share of the token-blocks (off by default: measured slower)
     int32_t maxt;       // launch-bounds class (threads per block the kernel was compiled for)
     int32_t algo;       // 1 = sliding-window (register) kernels, 2 = LDS-staged pipelined kernels,
-                        // 3 = role-split LDS-staged kernels (K = 31, 15)
+                        // 3 = role-split LDS-staged kernels (K = 31, 15), 4 = matrix-core kernels (the same sizes, bf16)
     int32_t nwl;        // LDS kernels: loader waves per block
     int32_t nbuf;       // LDS forward: tile buffers (2 or 3)
     uint32_t flags;     // NPLM_DWCONV_RESIDUAL etc., as for the _ex entry points
@@ -136,6 +137,14 @@ hipError_t launch_fwd_split_k15(bool bf16, const ConvPtrs& p, const LdsGeo& g, d
 hipError_t launch_fwd_split_k21(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 hipError_t launch_fwd_split_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 #undef NPLM_DECLARE_SPLIT_K
+// matrix-core kernels of bf16 activations (dwconv_mfma_kernels.h), planned like the role-split ones
+#define NPLM_DECLARE_MFMA_K(KK) \
+    hipError_t launch_fwd_mfma_k##KK(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
+NPLM_DECLARE_MFMA_K(11)
+NPLM_DECLARE_MFMA_K(15)
+NPLM_DECLARE_MFMA_K(21)
+NPLM_DECLARE_MFMA_K(31)
+#undef NPLM_DECLARE_MFMA_K
 // LayerNorm-fused forward (dwconv_ln_kernels.h), K <= 9, fixed shape per dtype, see lds_ln_shape()
 hipError_t launch_ln_fwd_k3(bool bf16, const ConvPtrs& p, const LnArgs& ln, const LdsGeo& g, dim3 grid, hipStream_t s);
 hipError_t launch_ln_fwd_k5(bool bf16, const ConvPtrs& p, const LnArgs& ln, const LdsGeo& g, dim3 grid, hipStream_t s);

@@ -1,0 +1,87 @@
+"""The kernels of 11 to 31 taps on the matrix cores (bf16 activations and weights) against the oracle and the vector kernels."""
+import pytest
+import torch
+
+import nanoplm_amd as npa
+from nanoplm_amd import _lib
+from nanoplm_amd.workloads import cu_from_lengths
+from oracle import dwconv_ref as O
+
+from gpu_util import assert_act_close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# sequences shorter than four rows, than the halo and than a tile, empty ones, tile edges, and tiles without a boundary
+LENS = [1, 2, 3, 8, 0, 1, 150, 0, 5, 7, 6, 1, 64, 63, 65, 2, 300, 4, 15, 16, 17, 30, 31, 32, 33, 700, 1, 1, 1, 29, 0, 0, 45,
+        1200, 14]
+MFMA = dict(algo=4)
+
+
+def _case(lens, C, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    cu = cu_from_lengths(torch.tensor(lens))
+    T = int(cu[-1])
+    return (torch.randn(T, C, generator=g).bfloat16(), cu, (torch.randn(C, K, generator=g) * K ** -0.5).bfloat16(),
+            torch.randn(C, generator=g).bfloat16(), torch.randn(T, C, generator=g).bfloat16())
+
+
+# (the K that run on 11, 15, 21 and 31 taps; whole, partial and several column blocks; one, few and many tiles a block; a last
+# tile of 1, 63 and 64 rows)
+CASES = [(11, LENS, 264, 1), (13, LENS, 256, 0), (15, LENS * 4, 512, 2), (17, [700], 1000, 0), (21, LENS, 264, 1),
+         (25, LENS[::-1], 2056, 5), (29, [64, 1], 256, 0), (31, LENS * 4, 256, 1), (31, [127], 320, 0), (31, [1] * 130, 256, 0),
+         (31, LENS, 2056, 0)]
+
+
+@pytest.mark.parametrize("K,lens,C,nbt", CASES)
+def test_forward_on_the_matrix_cores_matches_the_oracle(K, lens, C, nbt):
+    """To one bf16 rounding of the oracle's y; the same bits again after a call that left NaN in every LDS byte it used, and
+    from the weights zero-padded to the planned size."""
+    print(f"[case] K={K} C={C} nbt={nbt}", flush=True)
+    x, cu, w, b, _ = _case(lens, C, K, C + K + nbt)
+    xd, cud, wd, bd = x.to(DEV), cu.to(DEV), w.to(DEV), b.to(DEV)
+    tn = _lib.Tuning(nbt=nbt, **MFMA)
+    y64 = O.c_oracle_fwd(x, cu, w, b)
+    y = npa.varlen_dwconv_fwd(xd, cud, wd, bd, tuning=tn)
+    assert_act_close(y, y64, torch.bfloat16, "y")
+    assert_act_close(npa.varlen_dwconv_fwd(xd, cud, wd, bd, residual=True, tuning=tn), y64 + x.double(), torch.bfloat16, "y + x")
+    npa.varlen_dwconv_fwd(torch.full_like(xd, float("nan")), cud, wd, bd, tuning=tn)
+    assert torch.equal(npa.varlen_dwconv_fwd(xd, cud, wd, bd, tuning=tn), y)
+    off = ((15 if K <= 15 else 31) - K) // 2
+    wide = torch.nn.functional.pad(wd, (off, off)).contiguous()
+    assert torch.equal(npa.varlen_dwconv_fwd(xd, cud, wide, bd, tuning=tn), y)
+
+
+def _plant_non_finite(t, cu):
+    for i in range(0, cu.numel() - 1, 5):
+        if cu[i + 1] - cu[i] < 10:
+            t[cu[i]:cu[i + 1], i % 7::7] = float("inf") if i % 2 else float("nan")
+
+
+@pytest.mark.parametrize("K", [11, 31])
+def test_forward_non_finite_rows_stay_in_their_sequence(K):
+    x, cu, w, b, _ = _case(LENS * 2, 512, K, K)
+    _plant_non_finite(x, cu)
+    xd, cud, wd, bd = x.to(DEV), cu.to(DEV), w.to(DEV), b.to(DEV)
+    y1 = npa.varlen_dwconv_fwd(xd, cud, wd, bd, tuning=_lib.Tuning(algo=1))
+    y4 = npa.varlen_dwconv_fwd(xd, cud, wd, bd, tuning=_lib.Tuning(**MFMA))
+    assert not bool(torch.isfinite(y1).all())
+    torch.testing.assert_close(y4, y1, rtol=2.0 ** -7, atol=1e-5, equal_nan=True)      # (two roundings of one sum)
+
+
+@pytest.mark.parametrize("T,C,K,wdt,served", [(4096, 256, 31, torch.bfloat16, True), (4095, 256, 31, torch.bfloat16, False),
+                                              (4096, 248, 31, torch.bfloat16, False), (4096, 260, 31, torch.bfloat16, False),
+                                              (4096, 256, 31, torch.float32, False), (4096, 256, 9, torch.bfloat16, False),
+                                              (4096, 264, 11, torch.bfloat16, True)])
+def test_which_forward_calls_the_matrix_cores_serve(T, C, K, wdt, served):
+    x, cu, w, b, _ = _case([T], C, K, T + C)
+    xd, cud, wd = x.to(DEV), cu.to(DEV), w.to(DEV).to(wdt)
+    y = npa.varlen_dwconv_fwd(xd, cud, wd, None)
+    y1 = npa.varlen_dwconv_fwd(xd, cud, wd, None, tuning=_lib.Tuning(algo=1))
+    if served:
+        assert torch.equal(y, npa.varlen_dwconv_fwd(xd, cud, wd, None, tuning=_lib.Tuning(**MFMA)))
+    else:
+        assert torch.equal(y, y1)
+        if T >= 4096:
+            with pytest.raises(RuntimeError):
+                npa.varlen_dwconv_fwd(xd, cud, wd, None, tuning=_lib.Tuning(**MFMA))
+    torch.testing.assert_close(y, y1, rtol=2.0 ** -7, atol=1e-5)                          # (two roundings of one sum)
