@@ -340,6 +340,7 @@ hipError_t launch_fwd_split(int taps, bool bf16, const ConvPtrs& a, const LdsGeo
         return hipErrorInvalidConfiguration;                                                  \
     }
 NPLM_LAUNCH_MFMA(launch_fwd_mfma)
+NPLM_LAUNCH_MFMA(launch_bwd_mfma)
 #undef NPLM_LAUNCH_MFMA
 
 bool split_eligible(bool bf16, long long T, int C, int K, uintptr_t align_bits) {
@@ -354,6 +355,20 @@ bool mfma_eligible(bool bf16, bool w_bf16, long long T, int C, int K, uintptr_t 
     return bf16 && w_bf16 && split_eligible(bf16, T, C, K, align_bits);
 }
 constexpr long long kMfmaMinRows = 4096;
+// A backward tile with sequence boundaries makes one pass over its rows per sequence for dw, so the gain goes with the length
+// of the sequences. Measured at T=131072, us, matrix cores against role-split, for lengths of 20 to 128 residues (mean 75), 20
+// to 512 (mean 263), log-normal (mean 333), one sequence:
+//   K=31, C=1024   276/288   209/249   198/246   153/238      (C=2048: 520/538, -, 372/511, 294/479; T=16384, C=512: 36/43,
+//   K=15, C=1024   202/228   158/168   154/167   136/159       33/38, 33/39, 28/36; T=4096: 26/30, 24/29, 24/28, 22/26)
+//   K=21, C=1024   275/234   197/197   192/195   147/183      (T=65536, C=512: 80/73, 68/64, 64/63, 49/59)
+//   K=11, C=1024   195/177   154/153   151/150   135/146
+// About 24 rows a sequence: K=31 627/575, 32: 560/574 (C=2048). 21 taps pay for the 32 lags of the plan, which short
+// sequences do not leave room for; 11 taps are bound by HBM on the vector ALU too.
+// Sequences of 522, 705, 1928 rows on average: K=21 181/196, 175/191, 160/186; K=11 150/150, 142/146, 139/144.
+bool mfma_bwd_preferred(long long T, int taps, int S) {
+    const int rows = taps == 31 ? 32 : taps == 15 ? 64 : 512;
+    return T >= (long long)S * rows;
+}
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
                     bool gated = false, int tile_rows = 0) {
     LdsPlan p{};
@@ -397,18 +412,19 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
 //     or two and what is measured is the launch (2048 rows, C=1024: K=31 11.8 / 12.5, K=15 10.0 / 10.2; 600 rows, C=512:
 //     12.2 / 11.8), while the others' sums are those of the sliding-window kernels bit for bit.
 //     fp32 weights would take three bf16 terms each: 280 us against 265 (K=31, C=2048), so they stay on the vector ALU.
-//   K=31 and K=15 backward (ALU-bound; one wave cannot hold the fused backward's registers): the role-split
+//   the same calls backward: matrix cores where a sequence has enough rows (mfma_bwd_preferred()).
+//   K=31 and K=15 backward of fp32 weights (ALU-bound; one wave cannot hold the fused backward's registers): the role-split
 //     kernel, when every output is asked for - C=2048, K=31: 510 us against 720 sliding-window on the log-normal length mix;
 //     K=15: 345 against 385 (C=1024: 177 against 205). A backward asked for dx alone or dw/db alone takes the
 //     sliding-window kernel, like everything the LDS kernels are not built for (other sizes, narrow or unaligned rows).
 //   K=31 forward of fp32 weights: the role-split kernel's dx role on every wave, 262 us against 299 LDS-staged with loader
 //     waves (C=2048); K=15: LDS-staged with loader waves, 190 us against 203 role-split and 227 sliding-window (C=2048).
-int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, bool w_bf16, long long T, int C, int K, uintptr_t align_bits) {
-    if (tune && tune->algo == 4) return !bwd && mfma_eligible(bf16, w_bf16, T, C, K, align_bits) ? 4 : -NPLM_DWCONV_ETUNING;
+int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, bool w_bf16, long long T, int C, int K, int taps, int S, uintptr_t align_bits) {
+    if (tune && tune->algo == 4) return mfma_eligible(bf16, w_bf16, T, C, K, align_bits) ? 4 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 3) return split_eligible(bf16, T, C, K, align_bits) ? 3 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 2) return lds_eligible(bf16, T, C, K, align_bits) ? 2 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 1) return 1;
-    if (mfma_eligible(bf16, w_bf16, T, C, K, align_bits) && T >= kMfmaMinRows && !bwd) return 4;
+    if (mfma_eligible(bf16, w_bf16, T, C, K, align_bits) && T >= kMfmaMinRows && (!bwd || mfma_bwd_preferred(T, taps, S))) return 4;
     if (split_eligible(bf16, T, C, K, align_bits) && (bwd || K == 31)) return 3;
     return lds_preferred(bwd, bf16, T, C, K, align_bits) ? 2 : 1;
 }
@@ -557,7 +573,7 @@ int fwd_impl(const void* x, const int32_t* cu, const void* w, const void* b, voi
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if (((uintptr_t)w | (uintptr_t)b) % WE || (uintptr_t)cu % 4) return -NPLM_DWCONV_EALIGN;
     hipStream_t s = (hipStream_t)stream;
-    const int algo = choose_algo(false, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, bits);
+    const int algo = choose_algo(false, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, bits);
     if (algo < 0) return algo;
     if (algo == 3 || algo == 4) {
         LdsPlan lp;
@@ -627,13 +643,13 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
 
-    int algo = choose_algo(true, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, bits);
+    int algo = choose_algo(true, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, bits);
     if (algo < 0) return algo;
-    if (algo == 3 && !(dx && want_red)) {     // the role-split kernel is fused only: a partial request takes the others
-        if (tune && tune->algo == 3) return -NPLM_DWCONV_ETUNING;
+    if (algo >= 3 && !(dx && want_red)) {     // these kernels are fused only: a partial request takes the others
+        if (tune && tune->algo >= 3) return -NPLM_DWCONV_ETUNING;
         algo = 1;
     }
-    if (algo == 3) {
+    if (algo == 3 || algo == 4) {
         LdsPlan lp;
         rc = make_split_plan(false, bf16, T, C, K, tune, &lp);
         if (rc) return rc;
@@ -642,9 +658,10 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
             return -NPLM_DWCONV_EWORKSPACE;
         float* part = reinterpret_cast<float*>(workspace);
         const ConvPtrs la{x, dy, cu, w, nullptr, dx, part};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | (lds_tap_off << W_TAP_OFF_SHIFT));
+        // (the matrix-core kernels place the caller's taps among those of K, the role-split ones among the taps that run)
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, algo == 4 ? w_flags : kernel_w_flags(w_dtype, flags) | (lds_tap_off << W_TAP_OFF_SHIFT));
         const dim3 grid(lp.ncb * lp.nbt);
-        hipError_t e = launch_bwd_split(taps, bf16, la, lg, grid, s);
+        hipError_t e = algo == 4 ? launch_bwd_mfma(taps, la, lg, grid, s) : launch_bwd_split(taps, bf16, la, lg, grid, s);
         if (e != hipSuccess) return (int)e;
         if (tune && tune->mid_event) {
             e = hipEventRecord((hipEvent_t)tune->mid_event, s);
@@ -1234,7 +1251,7 @@ size_t nplm_dwconv_bwd_workspace_bytes(int64_t T, int32_t C, int32_t K, int32_t 
     Plan p;
     if (make_plan(true, bf16, T, C, K, 0, nullptr, &p)) return 0;
     int slabs = p.nbt;
-    if (choose_algo(true, nullptr, bf16, true, T, C, K, 0) == 2) {
+    if (choose_algo(true, nullptr, bf16, true, T, C, K, K, 1, 0) == 2) {
         LdsPlan lp;
         if (make_lds_plan(true, bf16, T, C, K, nullptr, &lp) == 0 && lp.nbt > slabs) slabs = lp.nbt;
     }
@@ -1265,9 +1282,9 @@ int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype
     if (check_common(T, C, K, 0, act_dtype, NPLM_DWCONV_F32) || T == 0) return 0;
     K = exec_kernel_size(K);
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
-    const int algo = choose_algo(true, tune, bf16, true, T, C, K, 0);
+    const int algo = choose_algo(true, tune, bf16, true, T, C, K, K, 1, 0);
     if (algo < 0) return 0;
-    if (algo == 3) {
+    if (algo >= 3) {
         LdsPlan lp;
         if (make_split_plan(false, bf16, T, C, K, tune, &lp)) return 0;
         return lp.nbt;

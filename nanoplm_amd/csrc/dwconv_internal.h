@@ -138,8 +138,9 @@ hipError_t launch_fwd_split_k21(bool bf16, const ConvPtrs& p, const LdsGeo& g, d
 hipError_t launch_fwd_split_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 #undef NPLM_DECLARE_SPLIT_K
 // matrix-core kernels of bf16 activations (dwconv_mfma_kernels.h), planned like the role-split ones
-#define NPLM_DECLARE_MFMA_K(KK) \
-    hipError_t launch_fwd_mfma_k##KK(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
+#define NPLM_DECLARE_MFMA_K(KK)                                                                              \
+    hipError_t launch_fwd_mfma_k##KK(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);          \
+    hipError_t launch_bwd_mfma_k##KK(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 NPLM_DECLARE_MFMA_K(11)
 NPLM_DECLARE_MFMA_K(15)
 NPLM_DECLARE_MFMA_K(21)

@@ -527,4 +527,381 @@ dwconv_fwd_mfma_kernel(const void* __restrict__ x, const int32_t* __restrict__ c
     }
 }
 
+// ---- backward --------------------------------------------------------------------------------------------------------
+// dw of a plan tap m sums x[t] * dy[t - (KP-1)/2 + m] over the rows t of one sequence. As a contraction over rows:
+//     D[i][j] += sum over k of x[4c + k - i] * dy_staged[4(c + d + j) + k],  d = 0, 4:  the lag is m = 4 CK0 + 4d + 4j + i
+// so the four lanes of a block hold x at distance one row and dy at distance four rows, and 32 taps (16 at KP = 15) of 16
+// channels take two instructions (one) per four rows. db is the product of dy's chunks with ones. A tile's sums are formed
+// from zero and join the block's when they are finite; otherwise the tile is summed again one product at a time.
+template <int KT>
+struct MfmaDw {
+    using TP = MfmaTaps<KT>;
+    static constexpr int Q = kMfmaQ, R = 64;
+    static constexpr int ND = TP::KP == 15 ? 1 : 2;          // groups of 16 lags
+    static constexpr int NCX = R / 4 + 1;                    // x chunks: a lane's rows are shifted by up to 3
+    static constexpr int ROWB = kMfmaCb;
+    f32x4 tot[ND][Q];
+    float dbs[Q];              // the lane's share of db
+    uint32_t ady[4], ax[4];    // LDS addresses of the lane's slice: of dy chunk c by c & 3, of row k of an x chunk (chunk 0, the tile at hand)
+    int n, c0;
+    bool active;
+
+    __device__ __forceinline__ void init(const char* lds, int wc, int lane, int ch0, int nch, int x_at) {
+        n = lane & 3;
+        const int lc = (wc * 16 + (lane >> 2)) * Q;
+        active = lc < nch;
+        const int lcc = active ? lc : nch - Q;
+        c0 = ch0 + lcc;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
+            ady[k] = base + 4 * n * ROWB + ((lcc * 2) ^ (((n + k) & 3) << 6));
+            ax[k] = base + x_at + (k - n) * ROWB + ((lcc * 2) ^ (((k - n) & 3) << 6));
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            dbs[q] = 0.f;
+#pragma unroll
+            for (int d = 0; d < ND; ++d) tot[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    __device__ __forceinline__ void read_x(int chunk, MfmaRaw& o) const {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const u32x2 t = mfma_lds(ax[k] + chunk * 4 * ROWB);
+            o.r[k][0] = t.x; o.r[k][1] = t.y;
+        }
+    }
+    __device__ __forceinline__ void read_dy(int chunk, MfmaRaw& o) const {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const u32x2 t = mfma_lds(ady[chunk & 3] + (chunk * 4 + k) * ROWB);
+            o.r[k][0] = t.x; o.r[k][1] = t.y;
+        }
+    }
+    __device__ __forceinline__ void next_buffer(int by) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { ady[k] += by; ax[k] += by; }
+    }
+    // Packed masks of a lane's rows r0 + at .. r0 + at + 3 against [lo, hi); r0, lo, hi are uniform, at + 4 <= 16.
+    __device__ __forceinline__ static void row_masks(int r0, int at, int lo, int hi, uint32_t& m0, uint32_t& m1) {
+        const int o = lo > r0 ? lo - r0 : 0, e = hi - r0 < 16 ? hi - r0 : 16;
+        uint32_t in = (uint32_t)__builtin_amdgcn_readfirstlane((int)(e > o ? ((1u << e) - 1u) & ~((1u << o) - 1u) : 0u));
+        asm volatile("" : "+s"(in));                         // (not computed ahead of the tiles and kept in registers)
+        const uint32_t v = in >> at;
+        m0 = __builtin_amdgcn_perm((uint32_t)((int)(v << 30) >> 31), (uint32_t)((int)(v << 31) >> 31), 0x05040100);
+        m1 = __builtin_amdgcn_perm((uint32_t)((int)(v << 28) >> 31), (uint32_t)((int)(v << 29) >> 31), 0x05040100);
+    }
+    __device__ __forceinline__ static void mask(MfmaChunk& c, uint32_t m0, uint32_t m1) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) { c.b[q].x &= m0; c.b[q].y &= m1; }
+    }
+    __device__ __forceinline__ void add_db(const MfmaChunk& dy) {
+        const s16x4 one = {(short)0x3f80, (short)0x3f80, (short)0x3f80, (short)0x3f80};
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            dbs[q] += mfma4(one, dy.op(q), f32x4{0.f, 0.f, 0.f, 0.f})[0];
+            asm volatile("" : "+v"(dbs[q]));                 // one product's registers at a time
+        }
+    }
+
+    // words = the tile's boundary bits; nrow = its rows in front of T
+    __device__ __forceinline__ void tile(const uint32_t* words, int nrow) {
+        constexpr int SPAN = R + TP::HALO, NR = 4 * (ND - 1) + 1, NCD = NCX + 4 * (ND - 1);
+        uint64_t w0, w1;                                     // boundary bits of staged rows 0 .. 63 and 64 on
+        {
+            uint32_t v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)words[i]);
+            w0 = ((uint64_t)v[0] | (uint64_t)v[1] << 32) & ~1ull;
+            w1 = (uint64_t)v[2] | (uint64_t)v[3] << 32;
+        }
+        f32x4 acc[ND][Q];
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) acc[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if ((w0 | w1) == 0) {
+            MfmaRaw rd, rx;
+            MfmaChunk ring[NR];                           // x chunks c - 4 .. c (of one group of lags: c)
+            read_dy(0, rd);
+            read_x(0, rx);
+            static_for<NCD>([&](auto c_c) __attribute__((always_inline)) {
+                constexpr int c = decltype(c_c)::value;
+                MfmaChunk dy;
+                uint32_t m0, m1;
+                mfma_pack(rd, dy);
+                if constexpr (c < NCX) {
+                    mfma_pack(rx, ring[c % NR]);
+                    if constexpr (c == 0 || c == NCX - 1) {
+                        row_masks(4 * c - 3, 3 - n, 0, R, m0, m1);
+                        mask(ring[c % NR], m0, m1);
+                    }
+                }
+                if constexpr (4 * c + 16 > SPAN) {           // what follows the staged rows meets only masked x, but may hold a NaN
+                    row_masks(4 * c, 4 * n, 0, SPAN, m0, m1);
+                    mask(dy, m0, m1);
+                }
+                if constexpr (c + 1 < NCD) read_dy(c + 1, rd);
+                if constexpr (c + 1 < NCX) read_x(c + 1, rx);
+                if constexpr (c < NCX) {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) acc[0][q] = mfma4(ring[c % NR].op(q), dy.op(q), acc[0][q]);
+                }
+                if constexpr (ND == 2 && c >= 4) {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) acc[ND - 1][q] = mfma4(ring[(c - 4) % NR].op(q), dy.op(q), acc[ND - 1][q]);
+                }
+                if constexpr (c % 4 == 0 && c < NCX) {       // staged rows 4c .. 4c + 15 in the four columns
+                    if constexpr (c == 0 || c == NCX - 1) {
+                        row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + R, m0, m1);
+                        mask(dy, m0, m1);
+                    }
+                    add_db(dy);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } else {
+            const uint32_t col = ady[0] ^ (n << 6);          // the lane's address of dy chunk 0 without the permutation of its rows
+            uint32_t m0, m1;
+#pragma nounroll
+            for (int c = 0; c < NCX; c += 4) {
+                MfmaRaw raw;
+                MfmaChunk dy;
+                read_dy(c, raw);
+                mfma_pack(raw, dy);
+                row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + nrow, m0, m1);
+                mask(dy, m0, m1);
+                add_db(dy);
+            }
+            // one pass per sequence that owns rows of the tile, over the chunks that hold them; the next chunk is on its way
+            // while one is summed
+            int a = sequence_of(w0, w1, TP::FRONT);
+            while (a < TP::FRONT + nrow) {
+                int b = next_sequence(w0, w1, a);
+                if (b > SPAN) b = SPAN;                      // (staged rows end there)
+                const int t0 = a > TP::FRONT ? a - TP::FRONT : 0, t1 = b - TP::FRONT < nrow ? b - TP::FRONT : nrow;
+                const int c1 = (t1 + 2) >> 2;
+                MfmaRaw rx, rd[ND];
+                auto fetch = [&](int c) __attribute__((always_inline)) {
+                    const uint32_t at = (col + 4 * c * ROWB) ^ (((n + c) & 3) << 6);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        u32x2 t = mfma_lds(ax[k] + c * 4 * ROWB);
+                        rx.r[k][0] = t.x; rx.r[k][1] = t.y;
+#pragma unroll
+                        for (int d = 0; d < ND; ++d) {
+                            t = mfma_lds(at + (16 * d + k) * ROWB);
+                            rd[d].r[k][0] = t.x; rd[d].r[k][1] = t.y;
+                        }
+                    }
+                };
+                int c = t0 >> 2;
+                fetch(c);
+#pragma nounroll
+                for (; c <= c1; ++c) {
+                    MfmaChunk x, dy[ND];
+                    mfma_pack(rx, x);
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) mfma_pack(rd[d], dy[d]);
+                    fetch(c < c1 ? c + 1 : c);
+                    if (4 * c - 3 < t0 || 4 * c + 3 >= t1) {
+                        row_masks(4 * c - 3, 3 - n, t0, t1, m0, m1);
+                        mask(x, m0, m1);
+                    }
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        const int r0 = 4 * (c + 4 * d);
+                        if (r0 < a || r0 + 16 > b) {
+                            row_masks(r0, 4 * n, a, b, m0, m1);
+                            mask(dy[d], m0, m1);
+                        }
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) acc[d][q] = mfma4(x.op(q), dy[d].op(q), acc[d][q]);
+                    }
+                }
+                a = b;
+            }
+        }
+        float chk = 0.f;
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(acc[d][q][0], 0.f, chk);
+        if (__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) acc[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+            int a = sequence_of(w0, w1, TP::FRONT), b = next_sequence(w0, w1, a);
+#pragma nounroll
+            for (int t = 0; t < nrow; ++t) {
+                if (t + TP::FRONT >= b) { a = b; b = next_sequence(w0, w1, a); }
+                RowVec<true, Q> xr, gr;
+                float xv[Q], gv[Q];
+                auto row_of = [&](RowVec<true, Q>& v, uint32_t at) __attribute__((always_inline)) {
+                    const u32x2 t2 = mfma_lds(at);
+                    v.d[0] = t2.x; v.d[1] = t2.y;
+                };
+                // the lane's slice of row 0 of a tile, its pieces in order, and the permutation of the row at hand
+                const uint32_t x0 = (ax[0] + n * ROWB) ^ ((-n & 3) << 6), g0 = (ady[0] - 4 * n * ROWB) ^ (n << 6);
+                row_of(xr, (x0 + t * ROWB) ^ ((t & 3) << 6));
+                xr.to_f32(xv);
+#pragma unroll
+                for (int d = 0; d < ND; ++d)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int r = t + 16 * d + 4 * n + i;
+                        if (r >= a && r < b && r < SPAN) {
+                            row_of(gr, (g0 + r * ROWB) ^ (((r >> 2) & 3) << 6));
+                            gr.to_f32(gv);
+#pragma unroll
+                            for (int q = 0; q < Q; ++q) acc[d][q][i] = __builtin_fmaf(xv[q], gv[q], acc[d][q][i]);
+                        }
+                    }
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) tot[d][q][i] += acc[d][q][i];
+    }
+    // first staged row of the sequence that holds row `at` (0: it began before), at < 128
+    __device__ __forceinline__ static int sequence_of(uint64_t w0, uint64_t w1, int at) {
+        if (at >= 64) {
+            const uint64_t m = w1 & (~0ull >> (127 - at));
+            if (m) return 127 - (int)__builtin_clzll(m);
+            at = 63;
+        }
+        const uint64_t m = w0 & (~0ull >> (63 - at));
+        return m ? 63 - (int)__builtin_clzll(m) : 0;
+    }
+    // first staged row of the sequence after the one that holds row `at` (128: none)
+    __device__ __forceinline__ static int next_sequence(uint64_t w0, uint64_t w1, int at) {
+        if (at < 63) {
+            const uint64_t m = w0 & (~0ull << (at + 1));
+            if (m) return (int)__builtin_ctzll(m);
+            return w1 ? 64 + (int)__builtin_ctzll(w1) : 128;
+        }
+        const uint64_t m = at < 127 ? w1 & (~0ull << (at - 63)) : 0;
+        return m ? 64 + (int)__builtin_ctzll(m) : 128;
+    }
+    // the block's sums to its slab: rows of taps (the weight's order), then db
+    __device__ __forceinline__ void finish(float* __restrict__ slab, int C, int lane) const {
+        float db[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {                        // the four columns hold rows 0 .. 3, 4 .. 7, ... of every 16
+            float v = dbs[q];
+            v += __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ 1) * 4, __float_as_int(v)));
+            v += __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ 2) * 4, __float_as_int(v)));
+            db[q] = v;
+        }
+        if (!active) return;
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 4 * TP::CK0 + 16 * d + 4 * n + i - (TP::PP - TP::P);
+                if (m >= 0 && m < KT) *reinterpret_cast<float4*>(slab + (size_t)(KT - 1 - m) * C + c0) = make_float4(tot[d][0][i], tot[d][1][i], tot[d][2][i], tot[d][3][i]);
+            }
+        if (n == 0) *reinterpret_cast<float4*>(slab + (size_t)KT * C + c0) = make_float4(db[0], db[1], db[2], db[3]);
+    }
+};
+
+// Backward: 64-row tiles (a dy tile with its halo rows, an x tile without), 4 wave-columns; waves of three kinds: dx
+// (MfmaConv over dy), dw and db, loaders and boundaries.
+// T=131072, C=2048, 31 taps: 294 us on one sequence (the role-split kernel of the vector ALU 479; a copy of the bytes takes 313),
+// 372 on log-normal lengths (511), where the dw waves' passes at sequence boundaries show. Tried for those, all slower on
+// every mix: one sweep of unrolled chunks that branches at each (382 to 452), one sweep and a left-over per boundary (spills).
+template <int KT>
+struct MfmaBwdShape {
+    using TP = MfmaTaps<KT>;
+    static constexpr int NDX = kMfmaCh / (16 * kMfmaQ), NDW = NDX, NWC = NDX + NDW, NWL = 3;
+    static constexpr int NT = (NWC + NWL + 1) * 64;
+    static constexpr int R = 64, NROWS = R + TP::HALO;
+    static constexpr int X_AT = NROWS * kMfmaCb, BUF_BYTES = X_AT + R * kMfmaCb;
+    // lanes read up to four rows behind an x tile (masked); the boundary bits lie there behind the second one
+    static constexpr int LDS_BYTES = 2 * BUF_BYTES + 4 * kMfmaCb;
+    static_assert(2 * kMfmaWords * 4 <= 4 * kMfmaCb, "room for the boundary bits");
+    static_assert(LDS_BYTES <= kLdsBytes, "two pairs of tiles fit the LDS");
+    static_assert(kMfmaCh * TP::WSTR * 4 <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
+    static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords && NROWS <= 96, "boundary bits");
+};
+
+template <int KT, bool RES>
+__global__ void __launch_bounds__(MfmaBwdShape<KT>::NT)
+dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, const int32_t* __restrict__ cu,
+                       const void* __restrict__ w, void* __restrict__ dx, float* __restrict__ partial, const LdsGeo g) {
+    using SH = MfmaBwdShape<KT>;
+    using TP = MfmaTaps<KT>;
+    constexpr int R = SH::R;
+    extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+    uint32_t* words = reinterpret_cast<uint32_t*>(lds_raw + 2 * SH::BUF_BYTES);
+    uint32_t* tab = reinterpret_cast<uint32_t*>(lds_raw + SH::BUF_BYTES);
+    const int lane = (int)(threadIdx.x & 63);
+    const int wv = wave_id();
+    int cb, tb;
+    lds_block_coords(g, cb, tb);
+    const int T = g.T, S = g.S, C = g.C;
+    const int rowb = C * 2;
+    const int col_byte0 = cb * kMfmaCb;
+    const int valid_bytes = rowb - col_byte0 < kMfmaCb ? rowb - col_byte0 : kMfmaCb;
+    const int nch = valid_bytes / 2;
+    const int ntl = (g.ntiles + g.nbt - 1) / g.nbt;
+    int q = tb;
+
+    if (wv >= SH::NWC) {
+        __builtin_amdgcn_s_setprio(3);
+        const int lw = wv - SH::NWC;
+        auto prepare = [&](int par, int t0) __attribute__((always_inline)) {
+            char* buf = lds_raw + par * SH::BUF_BYTES;
+            if (lw < SH::NWL) {
+                mfma_stage<SH::NROWS, SH::NWL, false, kLoadAuxOnceBwd>(dy, buf, t0 - TP::FRONT, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, TP::HALO);
+                mfma_stage<R, SH::NWL, true, kLoadAuxOnceBwdX>(x, buf + SH::X_AT, t0, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, 0);
+            } else {
+                mfma_bounds(cu, S, T, t0 - TP::FRONT, SH::NROWS, words + par * kMfmaWords, lane);
+            }
+        };
+        prepare(0, tb * R);
+        lds_barrier();                       // the weight table is written
+        lds_barrier();                       // and has been read
+        for (int it = 0; it < ntl; ++it) {
+            if (lw < SH::NWL) wait_vmem_all();
+            lds_barrier();                   // tile `it` has landed, the buffer of the tile before is free
+            q = lds_next_slot(g, q);
+            const int t0 = it + 1 < ntl ? lds_tile_row0(g, it + 1, q, R) : T;
+            if (t0 < T) prepare((it + 1) & 1, t0);
+        }
+        return;
+    }
+    mfma_fill_weights<KT, true>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x, SH::NWC * 64);
+    lds_barrier();
+    if (wv < SH::NDX) {
+        MfmaConv<KT, R / 16, true, RES> conv;
+        conv.init(tab, w, g.w_flags, nullptr, wv, lane, cb * kMfmaCh, nch, rowb);
+        lds_barrier();
+        for (int it = 0; it < ntl; ++it) {
+            lds_barrier();
+            const int t0 = lds_tile_row0(g, it, q, R);
+            if (t0 < T)
+                conv.rows(lds_raw + (it & 1) * SH::BUF_BYTES, words + (it & 1) * kMfmaWords, 0, mfma_out_rsrc(dx, t0, T - t0 < R ? T - t0 : R, rowb), rowb);
+            q = lds_next_slot(g, q);
+        }
+    } else {
+        MfmaDw<KT> dw;
+        dw.init(lds_raw, wv - SH::NDX, lane, cb * kMfmaCh, nch, SH::X_AT);
+        lds_barrier();
+        for (int it = 0; it < ntl; ++it) {
+            lds_barrier();
+            const int t0 = lds_tile_row0(g, it, q, R);
+            if (t0 < T) dw.tile(words + (it & 1) * kMfmaWords, T - t0 < R ? T - t0 : R);
+            dw.next_buffer(it & 1 ? -SH::BUF_BYTES : SH::BUF_BYTES);
+            q = lds_next_slot(g, q);
+        }
+        dw.finish(partial + (size_t)tb * (KT + 1) * C, C, lane);
+    }
+}
+
 }  // namespace nplm

@@ -7,7 +7,7 @@ from nanoplm_amd import _lib
 from nanoplm_amd.workloads import cu_from_lengths
 from oracle import dwconv_ref as O
 
-from gpu_util import assert_act_close
+from gpu_util import assert_act_close, assert_red_close
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -85,3 +85,53 @@ def test_which_forward_calls_the_matrix_cores_serve(T, C, K, wdt, served):
             with pytest.raises(RuntimeError):
                 npa.varlen_dwconv_fwd(xd, cud, wd, None, tuning=_lib.Tuning(**MFMA))
     torch.testing.assert_close(y, y1, rtol=2.0 ** -7, atol=1e-5)                          # (two roundings of one sum)
+
+
+@pytest.mark.parametrize("K,lens,C,nbt", CASES)
+def test_backward_on_the_matrix_cores_matches_the_oracle(K, lens, C, nbt):
+    """dx to one bf16 rounding, dw and db to the reductions' tolerance; the same bits again after a call that left NaN in LDS."""
+    print(f"[case] K={K} C={C} nbt={nbt}", flush=True)
+    x, cu, w, _, dy = _case(lens, C, K, C + K + nbt)
+    xd, cud, wd, dyd = x.to(DEV), cu.to(DEV), w.to(DEV), dy.to(DEV)
+    tn = _lib.Tuning(nbt=nbt, **MFMA)
+    dx64, dw64, db64 = O.c_oracle_bwd(x, dy, cu, w)
+    got = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=tn)
+    assert_act_close(got[0], dx64, torch.bfloat16, "dx")
+    assert_red_close(got[1], dw64, "dw")
+    assert_red_close(got[2], db64, "db")
+    dxr, dwr, dbr = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, residual=True, tuning=tn)
+    assert_act_close(dxr, dx64 + dy.double(), torch.bfloat16, "dx + dy")
+    assert torch.equal(dwr, got[1]) and torch.equal(dbr, got[2])
+    nan = torch.full_like(xd, float("nan"))
+    npa.varlen_dwconv_bwd(nan, nan, cud, wd, tuning=tn)
+    again = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=tn)
+    assert all(torch.equal(a, c) for a, c in zip(again, got))
+
+
+@pytest.mark.parametrize("K", [15, 31])
+@pytest.mark.parametrize("which", ["x", "dy"])
+def test_backward_non_finite_rows_stay_in_their_sequence(K, which):
+    x, cu, w, _, dy = _case(LENS * 2, 512, K, K)
+    _plant_non_finite(x if which == "x" else dy, cu)
+    xd, cud, wd, dyd = x.to(DEV), cu.to(DEV), w.to(DEV), dy.to(DEV)
+    dx1, dw1, db1 = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(algo=1))
+    dx4, dw4, db4 = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(**MFMA))
+    assert not bool(torch.isfinite(dw1).all())
+    torch.testing.assert_close(dx4, dx1, rtol=2.0 ** -7, atol=1e-5, equal_nan=True)
+    for got, ref in ((dw4, dw1), (db4, db1)):                                             # assert_red_close's bar
+        torch.testing.assert_close(got, ref, rtol=0, atol=1e-5 * float(ref[torch.isfinite(ref)].abs().max()), equal_nan=True)
+
+
+@pytest.mark.parametrize("T,n,K,wdt,served", [(4096, 128, 31, torch.bfloat16, True), (4096, 129, 31, torch.bfloat16, False),
+                                              (4095, 1, 31, torch.bfloat16, False), (4096, 1, 31, torch.float32, False),
+                                              (4096, 64, 15, torch.bfloat16, True), (4096, 65, 15, torch.bfloat16, False),
+                                              (4096, 8, 21, torch.bfloat16, True), (4096, 9, 21, torch.bfloat16, False),
+                                              (4096, 8, 11, torch.bfloat16, True), (4096, 9, 11, torch.bfloat16, False)])
+def test_which_backward_calls_the_matrix_cores_serve(T, n, K, wdt, served):
+    x, cu, w, _, dy = _case([T // n] * (n - 1) + [T - T // n * (n - 1)], 256, K, T + n)
+    xd, cud, wd, dyd = x.to(DEV), cu.to(DEV), w.to(DEV).to(wdt), dy.to(DEV)
+    got = npa.varlen_dwconv_bwd(xd, dyd, cud, wd)
+    want = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(algo=4 if served else 3))
+    assert all(torch.equal(a, c) for a, c in zip(got, want))
+    assert torch.equal(npa.varlen_dwconv_bwd(xd, dyd, cud, wd, need_dw=False)[0],
+                       npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(algo=1))[0])
