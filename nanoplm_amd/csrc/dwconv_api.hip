@@ -369,14 +369,24 @@ bool mfma_bwd_preferred(long long T, int taps, int S) {
     const int rows = taps == 31 ? 32 : taps == 15 ? 64 : 512;
     return T >= (long long)S * rows;
 }
+// The gated backward with dz on the matrix cores: 31 taps. Measured, us, against role-split, for lengths of 20 to 128 residues
+// (mean 75), 20 to 512 (263), log-normal (333), short and long mixed (193), one sequence:
+//   T=131072, C=2048   886/807   705/737   673/721   673/724   619/674         T=32768, C=1024   125/117   100/105   95/105   97/108   87/100
+//   T=16384, C=1024    72/75     61/66     58/65     56/69     51/66           T=8192, C=512     29/39     27/37     27/38    26/39    24/34
+// A wave of dw makes one pass over its rows whatever begins there, but masked row by row: short sequences cost it more than the
+// role-split kernel's roles, which share the loss, once a call is longer than its first tiles. 15 taps (T=131072, C=1024: 302/264,
+// T=4096: 19/22) and 21 (306/299) have too few FMAs to save.
+bool mfma_gated_bwd_preferred(long long T, int taps, int S) {
+    return taps == 31 && (T <= 16384 || T >= 192ll * S);
+}
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
-                    bool gated = false, int tile_rows = 0) {
+                    bool gated = false, int tile_rows = 0, int block_bytes = 0) {
     LdsPlan p{};
     nplm_dwconv_tuning z{};
     if (!tune) tune = &z;
     const int E = bf16 ? 2 : 4;
     const SplitShapeSel sh = !gated ? lds_split_shape(fwd, bf16, K) : fwd ? lds_split_gated_fwd_shape(bf16, K) : lds_split_gated_shape(bf16, K);
-    const long long cb_bytes = (long long)sh.ncw * 64 * sh.vec * E;
+    const long long cb_bytes = block_bytes ? block_bytes : (long long)sh.ncw * 64 * sh.vec * E;
     const long long row_bytes = (long long)C * E;
     p.R = tile_rows ? tile_rows : sh.rw * sh.nrg;
     if ((long long)(p.R + K) * row_bytes * (gated ? 2 : 1) + 2 * row_bytes >= INT_MAX) return -NPLM_DWCONV_ESHAPE;
@@ -1147,15 +1157,17 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
     if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {
         LdsPlan lp;
-        rc = make_split_plan(false, bf16, T, C, K, nullptr, &lp, true);
+        const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 && T >= kMfmaMinRows && mfma_gated_bwd_preferred(T, taps, S);
+        rc = mfma ? make_split_plan(false, bf16, T, C, K, nullptr, &lp, true, kMfmaGatedRows, kMfmaGatedCb)
+                  : make_split_plan(false, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;
         const size_t slab = (size_t)(K + 1) * C * sizeof(float);
         if (!workspace || (uintptr_t)workspace % 256 || workspace_bytes < slab * (size_t)lp.nbt) return -NPLM_DWCONV_EWORKSPACE;
         float* part = reinterpret_cast<float*>(workspace);
         const ConvPtrs la{z, dy, cu, w, nullptr, dz, part};
-        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | (lds_tap_off << W_TAP_OFF_SHIFT));
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | (mfma ? tap_flags : lds_tap_off << W_TAP_OFF_SHIFT));
         const dim3 grid(lp.ncb * lp.nbt);
-        hipError_t e = launch_bwd_split_gated(taps, bf16, la, lg, grid, s);
+        hipError_t e = mfma ? launch_bwd_gated_mfma_k31(la, lg, grid, s) : launch_bwd_split_gated(taps, bf16, la, lg, grid, s);
         if (e != hipSuccess) return (int)e;
         const long long n_out = (long long)(taps + 1) * C;
         hipLaunchKernelGGL(dwconv_finalize_kernel<FIN_SPLIT>, dim3((unsigned)((n_out + 63) / 64)), dim3(64 * FIN_SPLIT), 0, s,

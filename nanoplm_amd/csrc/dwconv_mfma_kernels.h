@@ -49,6 +49,8 @@ struct MfmaTaps {
 
 constexpr int kMfmaCb = 512;           // bytes of a row in one column block: 256 channels
 constexpr int kMfmaCh = kMfmaCb / 2;
+constexpr int kMfmaGatedCb = 256;      // gated kernels: 128 channels (three tiles in each of two buffers)
+constexpr int kMfmaGatedRows = 64;
 constexpr int kMfmaQ = 4;              // channels of a lane: 8 bytes of a row
 constexpr int kMfmaFwdRows = 64;       // output rows of a forward tile
 // Offset of a store that is to be dropped: beyond the descriptor of a group of output rows (less than 2 GiB) whatever
@@ -60,27 +62,20 @@ __device__ __forceinline__ rsrc_t mfma_out_rsrc(void* out, int row0, int rows, i
 constexpr int kMfmaWords = 8;          // 32-bit words of a tile's boundary bits (lanes read up to 2 words past the last row)
 
 // One chunk (four rows) of a lane's Q channels as matrix operands: per channel rows 0, 1 and rows 2, 3.
+template <int Q = kMfmaQ>
 struct MfmaChunk {
-    u32x2 b[kMfmaQ];
+    u32x2 b[Q];
     __device__ __forceinline__ s16x4 op(int q) const { return __builtin_bit_cast(s16x4, b[q]); }
 };
-struct MfmaRaw { uint32_t r[4][kMfmaQ / 2]; };
+template <int Q = kMfmaQ> struct MfmaRaw { uint32_t r[4][Q / 2]; };
 
 // (lds_u32x2 loads: one ds_read_b64 per row, rows 512 bytes apart)
 typedef const __attribute__((address_space(3))) u32x2* lds_u32x2;
 __device__ __forceinline__ u32x2 mfma_lds(uint32_t at) { return *(lds_u32x2)(uintptr_t)at; }
-template <int ROWS = 4>
-__device__ __forceinline__ void mfma_read(const char* p, MfmaRaw& o) {
+template <int Q>
+__device__ __forceinline__ void mfma_pack(const MfmaRaw<Q>& r, MfmaChunk<Q>& c) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        u32x2 t = {0, 0};
-        if (r < ROWS) t = *(lds_u32x2)(p + r * kMfmaCb);
-        o.r[r][0] = t.x; o.r[r][1] = t.y;
-    }
-}
-__device__ __forceinline__ void mfma_pack(const MfmaRaw& r, MfmaChunk& c) {
-#pragma unroll
-    for (int h = 0; h < kMfmaQ / 2; ++h) {
+    for (int h = 0; h < Q / 2; ++h) {
         c.b[2 * h].x = __builtin_amdgcn_perm(r.r[1][h], r.r[0][h], 0x05040100);
         c.b[2 * h].y = __builtin_amdgcn_perm(r.r[3][h], r.r[2][h], 0x05040100);
         c.b[2 * h + 1].x = __builtin_amdgcn_perm(r.r[1][h], r.r[0][h], 0x07060302);
@@ -89,28 +84,32 @@ __device__ __forceinline__ void mfma_pack(const MfmaRaw& r, MfmaChunk& c) {
 }
 __device__ __forceinline__ f32x4 mfma4(s16x4 a, s16x4 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(a, b, c, 0, 0, 0); }
 
-// Staging: rows of a 512-byte column block, two per 1 KiB direct load. The 16-byte pieces of a row are permuted (by the
+// Staging: rows of a column block of CB = 512 (gated: 256) bytes, two (four) per 1 KiB direct load. The 16-byte pieces of a row are permuted (by the
 // lanes' global addresses, inside the row) so that lanes which read four rows at once read different banks: piece p of row
-// r lies at p ^ (swz(r) << 2). ROWSWZ: swz = r & 3 (readers at distance 1 row), else (r >> 2) & 3 (distance 4 rows).
-template <bool ROWSWZ>
-__device__ __forceinline__ int mfma_swz(int row) { return ROWSWZ ? row & 3 : (row >> 2) & 3; }
+// r lies at p ^ (swz(r) << 2). SWZ_ROW: swz = r & 3 (readers at distance 1 row); SWZ_QUAD: (r >> 2) & 3 (distance 4 rows);
+// SWZ_BOTH: (r + (r >> 2)) & 3 (distance 4 rows, and at most two on a bank at distance 1).
+enum MfmaSwz { SWZ_QUAD = 0, SWZ_ROW = 1, SWZ_BOTH = 2 };
+template <MfmaSwz SWZ>
+__device__ __forceinline__ int mfma_swz(int row) {
+    return (SWZ == SWZ_ROW ? row : SWZ == SWZ_QUAD ? row >> 2 : row + (row >> 2)) & 3;
+}
 // Every one of the NLW loader waves issues the same number of loads (a surplus one repeats the last rows), so that "all but
 // the newest tile's have landed" is a compile-time wait.
-template <int NROWS, int NLW, bool ROWSWZ, int ONCE_AUX>
+template <int NROWS, int NLW, MfmaSwz SWZ, int ONCE_AUX, int CB = kMfmaCb>
 __device__ __forceinline__ void mfma_stage(const void* __restrict__ src, char* dst, int first_row, int T, size_t row_bytes,
                                            int col_byte0, int valid_bytes, int lw, int lane, int edge) {
-    constexpr int RPL = 1024 / kMfmaCb, NL = (NROWS + RPL - 1) / RPL, CNT = (NL + NLW - 1) / NLW;
+    constexpr int RPL = 1024 / CB, NL = (NROWS + RPL - 1) / RPL, CNT = (NL + NLW - 1) / NLW;
     const int rb = first_row > 0 ? first_row : 0;
     const rsrc_t rs = rows_rsrc(src, rb, T, row_bytes);
     const int rowb = (int)row_bytes;
-    const int lrow = lane / (kMfmaCb / 16), lpiece = lane % (kMfmaCb / 16);
+    const int lrow = lane / (CB / 16), lpiece = lane % (CB / 16);
     // rows outside [0, T) are not clamped: their offsets fall outside the descriptor (or, on a tensor beyond 4 GiB, on other
     // rows of it), and what lands in LDS for them is never used
 #pragma unroll
     for (int i = 0; i < CNT; ++i) {
         const int gi = lw + i * NLW < NL ? lw + i * NLW : NL - 1;
         const int row = RPL * gi + lrow;
-        const int piece = lpiece ^ (mfma_swz<ROWSWZ>(row) << 2);
+        const int piece = lpiece ^ (mfma_swz<SWZ>(row) << 2);
         const bool once = gi * RPL >= edge && gi * RPL + RPL <= NROWS - edge;
         if ((NROWS % RPL == 0 || row < NROWS) && piece * 16 < valid_bytes)
             load_to_lds<ONCE_AUX>(rs, dst + gi * 1024, (first_row - rb + row) * rowb + col_byte0 + piece * 16, 0, once);
@@ -190,10 +189,10 @@ __device__ __forceinline__ float mfma_weight(const void* __restrict__ w, int w_f
 }
 
 // Weight table of a column block in LDS, [channel][WSTR] dwords of two bf16: entry e of a channel is plan tap e - 4 + 4 CK0.
-template <int KT, bool FLIP>
+template <int KT, bool FLIP, int CH = kMfmaCh>
 __device__ __forceinline__ void mfma_fill_weights(uint32_t* tab, const void* __restrict__ w, int w_flags, int ch0, int nch, int tid, int nthreads) {
     using TP = MfmaTaps<KT>;
-    for (int i = tid; i < kMfmaCh * TP::WSTR; i += nthreads) {
+    for (int i = tid; i < CH * TP::WSTR; i += nthreads) {
         const int c = i / TP::WSTR, p = i - c * TP::WSTR;
         uint32_t t = 0;
         if (c < nch) {
@@ -209,10 +208,13 @@ __device__ __forceinline__ void mfma_fill_weights(uint32_t* tab, const void* __r
 
 // One wave's conv over staged rows: 16 Q channels, groups of 16 NSTEP output rows. FLIP: dx from dy. RES: the identity is one
 // more band (a single 1 per row), since a bf16 weight plus one is not one in bf16.
-template <int KT, int NSTEP, bool FLIP, bool RES>
+// GATED (backward): the rows are dh; what is stored are the two halves of dz = [dh * silu(g) | dh * u * silu'(g)], with u and
+// g of the row out of their LDS tiles; 256-byte column blocks.
+template <int KT, int NSTEP, bool FLIP, bool RES, bool GATED = false>
 struct MfmaConv {
     using TP = MfmaTaps<KT>;
-    static constexpr int Q = kMfmaQ, NCK = TP::NCK;
+    static constexpr int Q = GATED ? 2 : kMfmaQ, NCK = TP::NCK, CB = GATED ? kMfmaGatedCb : kMfmaCb;
+    static constexpr MfmaSwz SWZ = GATED ? SWZ_BOTH : SWZ_QUAD;
     static constexpr int ROWS = 16 * NSTEP;                  // output rows of a group
     static_assert(ROWS % 32 == 0, "a group's boundary bits start at a word");
     static constexpr int NCHUNK = 4 * (NSTEP - 1) + NCK;     // chunks that the steps of a group read (per lane)
@@ -239,11 +241,11 @@ struct MfmaConv {
         c0 = ch0 + lcc;
         swap = ((lane >> 4) + 4 * (lane & 15)) * 4;
         const int lcs = (wc * 16 + (lane & 15)) * Q;
-        out_at = lcs < nch ? 4 * (lane >> 4) * rowb + (ch0 + lcs) * 2 : kMfmaNoStore;
+        out_at = lcs < nch ? 4 * (lane >> 4) * (GATED ? 2 * rowb : rowb) + (ch0 + lcs) * 2 : kMfmaNoStore;
         w = w_;
         w_flags = w_flags_;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) off[k] = 4 * n * kMfmaCb + ((lcc * 2) ^ (((n + k) & 3) << 6));
+        for (int k = 0; k < 4; ++k) off[k] = 4 * n * CB + ((lcc * 2) ^ (((n + k) & 3) << 6));
         const int p0 = (4 - n) >> 1, sh = (n & 1) * 16;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -278,7 +280,7 @@ struct MfmaConv {
     }
     // acc += the products of window chunk k
     template <int k>
-    __device__ __forceinline__ void taps(f32x4 (&acc)[Q], const MfmaChunk& x) const {
+    __device__ __forceinline__ void taps(f32x4 (&acc)[Q], const MfmaChunk<Q>& x) const {
 #pragma unroll
         for (int q = 0; q < Q; ++q) acc[q] = mfma4(A[k][q], x.op(q), acc[q]);
         if constexpr (RES && k >= IDC && k < IDC + IDN) {
@@ -286,15 +288,52 @@ struct MfmaConv {
             for (int q = 0; q < Q; ++q) acc[q] = mfma4(I[k - IDC], x.op(q), acc[q]);
         }
     }
+    // window chunk c of the lane, its first ROWS rows
+    template <int c, int ROWS = 4>
+    __device__ __forceinline__ void read(const char* lp, MfmaRaw<Q>& o) const {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (r < ROWS) {
+                RowVec<true, Q> t;
+                t.load(lp + off[(c + (SWZ == SWZ_BOTH ? r : 0)) & 3] + (c * 4 + r) * CB);
+#pragma unroll
+                for (int h = 0; h < Q / 2; ++h) o.r[r][h] = t.d[h];
+            } else {
+#pragma unroll
+                for (int h = 0; h < Q / 2; ++h) o.r[r][h] = 0;
+            }
+        }
+    }
     // Adjacent lanes of a sum are rows 0, 4, 8, 12; they trade places first, so that 16 adjacent lanes store the 32 Q bytes
     // of one row (as 4-row pieces of 8 bytes the memory pipeline takes four times the requests: T=131072, C=2048, 31 taps
     // 223 us against 200).
-    __device__ __forceinline__ void store(rsrc_t ro, int at, int rowb, int row, const float (&v)[Q]) const {
+    __device__ __forceinline__ void store_at(rsrc_t ro, int at, int soff, const float (&v)[Q]) const {
         RowVec<true, Q> o;
         o.from_f32(v);
 #pragma unroll
         for (int h = 0; h < Q / 2; ++h) o.d[h] = (uint32_t)__builtin_amdgcn_ds_bpermute(swap, (int)o.d[h]);
-        o.bstore(ro, at, row * rowb);
+        o.bstore(ro, at, soff);
+    }
+    // output row 4 n + row of the group; up = the group's first row in the u tile
+    __device__ __forceinline__ void store(rsrc_t ro, int at, int rowb, const char* up, int row, const float (&v)[Q]) const {
+        if constexpr (GATED) {
+            float u[Q], g[Q], du[Q], dg[Q];
+            RowVec<true, Q> ru, rg;
+            ru.load(up + off[0] + row * CB);
+            rg.load(up + off[0] + (row + kMfmaGatedRows) * CB);
+            ru.to_f32(u);
+            rg.to_f32(g);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const float sg = sigmoid_f32(g[q]);
+                du[q] = v[q] * (g[q] * sg);
+                dg[q] = v[q] * (u[q] * sg * (1.f + g[q] * (1.f - sg)));
+            }
+            store_at(ro, at, row * 2 * rowb, du);
+            store_at(ro, at, row * 2 * rowb + rowb, dg);
+        } else {
+            store_at(ro, at, row * rowb, v);
+        }
     }
 
     // boundary bits of this lane's window in step s (rows 16 s + 4 n on) of a group whose bits start at wp
@@ -307,7 +346,8 @@ struct MfmaConv {
 
     // One group of output rows: lp = the group's first window row in LDS, words = the tile's boundary bits, p0 = the window row's
     // place among them; ro = descriptor of the group's output rows (those in front of T).
-    __device__ __forceinline__ void rows(const char* lp, const uint32_t* words, int p0, rsrc_t ro, int rowb) const {
+    // GATED: up = the group's first row in the u tile; the g tile lies kMfmaGatedRows rows behind it.
+    __device__ __forceinline__ void rows(const char* lp, const uint32_t* words, int p0, rsrc_t ro, int rowb, const char* up = nullptr) const {
         constexpr int SPAN = 16 * NSTEP + TP::HALO;          // window rows of the group
         const uint32_t* wp = words + (p0 >> 5);              // p0 is a multiple of 32
         bool open;                                           // no boundary inside the window (a bit at its first row is none)
@@ -321,14 +361,14 @@ struct MfmaConv {
         if (open) {
             float chk = 0.f;
             f32x4 acc[(NCK + 3) / 4][Q];
-            MfmaRaw raw;
-            mfma_read(lp + off[0], raw);
+            MfmaRaw<Q> raw;
+            read<0>(lp, raw);
             static_for<NCHUNK>([&](auto c_c) __attribute__((always_inline)) {
                 constexpr int c = decltype(c_c)::value;
-                MfmaChunk x;
+                MfmaChunk<Q> x;
                 mfma_pack(raw, x);
                 if constexpr (c + 1 < NCHUNK)
-                    mfma_read<(c + 1 == NCHUNK - 1 ? TP::LASTROWS : 4)>(lp + off[(c + 1) & 3] + (c + 1) * 4 * kMfmaCb, raw);
+                    read<c + 1, (c + 1 == NCHUNK - 1 ? TP::LASTROWS : 4)>(lp, raw);
                 static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
                     constexpr int s = decltype(s_c)::value;
                     constexpr int k = c - 4 * s;
@@ -347,7 +387,7 @@ struct MfmaConv {
                                 float v[Q];
 #pragma unroll
                                 for (int q = 0; q < Q; ++q) v[q] = a[q][i];
-                                store(ro, out_at, rowb, 16 * s + i, v);
+                                store(ro, out_at, rowb, up, 16 * s + i, v);
                             }
                         }
                     }
@@ -359,7 +399,7 @@ struct MfmaConv {
 #pragma nounroll
             for (int s = 0; s < NSTEP; ++s) {
                 const MfmaBits bits = window_bits(wp, s);
-                const char* sp = lp + 16 * s * kMfmaCb;
+                const char* sp = lp + 16 * s * CB;
                 int i0 = 0;
                 do {
                     int lo, hi;
@@ -372,15 +412,15 @@ struct MfmaConv {
                     f32x4 acc[Q];
 #pragma unroll
                     for (int q = 0; q < Q; ++q) acc[q] = start(q);
-                    MfmaRaw raw;
-                    mfma_read(sp + off[0], raw);
+                    MfmaRaw<Q> raw;
+                    read<0>(sp, raw);
                     static_for<NCK>([&](auto k_c) __attribute__((always_inline)) {
                         constexpr int k = decltype(k_c)::value;
-                        const MfmaRaw cur = raw;
+                        const MfmaRaw<Q> cur = raw;
                         if constexpr (k + 1 < NCK)
-                            mfma_read<(k + 1 == NCK - 1 ? TP::LASTROWS : 4)>(sp + off[(k + 1) & 3] + (k + 1) * 4 * kMfmaCb, raw);
+                            read<k + 1, (k + 1 == NCK - 1 ? TP::LASTROWS : 4)>(sp, raw);
                         if ((some >> (4 * k)) & 15) {
-                            MfmaChunk x;
+                            MfmaChunk<Q> x;
                             mfma_pack(cur, x);
                             if (((every >> (4 * k)) & 15) != 15) {
                                 const uint32_t b4 = 4 * k < 32 ? in.lo >> (4 * k & 31) : in.hi >> (4 * k & 31);
@@ -404,7 +444,7 @@ struct MfmaConv {
                         float v[Q];
 #pragma unroll
                         for (int q = 0; q < Q; ++q) v[q] = acc[q][i];
-                        store(ro, i >= (range & 255) && i < (range >> 8) ? out_at : kMfmaNoStore, rowb, 16 * s + i, v);
+                        store(ro, i >= (range & 255) && i < (range >> 8) ? out_at : kMfmaNoStore, rowb, up, 16 * s + i, v);
                     }
                     i0 = i0 < 4 ? i1 : 4;
                 } while (__builtin_amdgcn_ballot_w64(i0 < 4) != 0);
@@ -414,12 +454,12 @@ struct MfmaConv {
 #pragma nounroll
         for (; redo != 0; redo &= redo - 1) {
             const int s = __builtin_ctz(redo);
-            exact_step(lp + 16 * s * kMfmaCb, window_bits(wp, s), ro, rowb, s);
+            exact_step(lp + 16 * s * CB, window_bits(wp, s), ro, rowb, s, up);
         }
     }
 
     // The 16 output rows of a step one product at a time, only the products that belong to them.
-    __device__ __forceinline__ void exact_step(const char* sp, MfmaBits bits, rsrc_t ro, int rowb, int s) const {
+    __device__ __forceinline__ void exact_step(const char* sp, MfmaBits bits, rsrc_t ro, int rowb, int s, const char* up) const {
         const int koff = w_tap_off(w_flags), kw = TP::KP - 2 * koff;
         const bool res = (w_flags & W_RESIDUAL) != 0;
 #pragma nounroll
@@ -434,7 +474,7 @@ struct MfmaConv {
                 const int p = TP::FRONT + i - TP::PP + m;       // window row of tap m
                 if (p < lo || p >= hi || !active) continue;
                 // (the lane's row 4 n + p of the step: its piece is where the chunk of that row has it)
-                const char* a = sp + (off[0] ^ (((((p >> 2) + n) & 3) ^ (n & 3)) << 6)) + p * kMfmaCb;
+                const char* a = sp + (off[0] ^ (((((p >> 2) + (SWZ == SWZ_BOTH ? p : 0) + n) & 3) ^ (n & 3)) << 6)) + p * CB;
                 RowVec<true, Q> x;
                 float f[Q];
                 x.load(a);
@@ -443,7 +483,7 @@ struct MfmaConv {
                 for (int q = 0; q < Q; ++q)
                     v[q] = __builtin_fmaf(mfma_weight<TP::KP, FLIP>(w, w_flags, c0 + q, m, res), f[q], v[q]);
             }
-            store(ro, out_at, rowb, 16 * s + i, v);
+            store(ro, out_at, rowb, up, 16 * s + i, v);
         }
     }
 };
@@ -494,7 +534,7 @@ dwconv_fwd_mfma_kernel(const void* __restrict__ x, const int32_t* __restrict__ c
         const int lw = wv - SH::NWC;
         auto prepare = [&](int par, int t0) __attribute__((always_inline)) {
             if (lw < SH::NWL) {
-                mfma_stage<SH::NROWS, SH::NWL, false, kLoadAuxOnceFwd>(x, lds_raw + par * SH::BUF_BYTES, t0 - TP::FRONT, T, (size_t)rowb,
+                mfma_stage<SH::NROWS, SH::NWL, SWZ_QUAD, kLoadAuxOnceFwd>(x, lds_raw + par * SH::BUF_BYTES, t0 - TP::FRONT, T, (size_t)rowb,
                                                                        col_byte0, valid_bytes, lw, lane, TP::HALO);
             } else {
                 mfma_bounds(cu, S, T, t0 - TP::FRONT, SH::NROWS, words + par * kMfmaWords, lane);
@@ -565,14 +605,14 @@ struct MfmaDw {
             for (int d = 0; d < ND; ++d) tot[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    __device__ __forceinline__ void read_x(int chunk, MfmaRaw& o) const {
+    __device__ __forceinline__ void read_x(int chunk, MfmaRaw<Q>& o) const {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const u32x2 t = mfma_lds(ax[k] + chunk * 4 * ROWB);
             o.r[k][0] = t.x; o.r[k][1] = t.y;
         }
     }
-    __device__ __forceinline__ void read_dy(int chunk, MfmaRaw& o) const {
+    __device__ __forceinline__ void read_dy(int chunk, MfmaRaw<Q>& o) const {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const u32x2 t = mfma_lds(ady[chunk & 3] + (chunk * 4 + k) * ROWB);
@@ -592,11 +632,11 @@ struct MfmaDw {
         m0 = __builtin_amdgcn_perm((uint32_t)((int)(v << 30) >> 31), (uint32_t)((int)(v << 31) >> 31), 0x05040100);
         m1 = __builtin_amdgcn_perm((uint32_t)((int)(v << 28) >> 31), (uint32_t)((int)(v << 29) >> 31), 0x05040100);
     }
-    __device__ __forceinline__ static void mask(MfmaChunk& c, uint32_t m0, uint32_t m1) {
+    __device__ __forceinline__ static void mask(MfmaChunk<Q>& c, uint32_t m0, uint32_t m1) {
 #pragma unroll
         for (int q = 0; q < Q; ++q) { c.b[q].x &= m0; c.b[q].y &= m1; }
     }
-    __device__ __forceinline__ void add_db(const MfmaChunk& dy) {
+    __device__ __forceinline__ void add_db(const MfmaChunk<Q>& dy) {
         const s16x4 one = {(short)0x3f80, (short)0x3f80, (short)0x3f80, (short)0x3f80};
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -622,13 +662,13 @@ struct MfmaDw {
 #pragma unroll
             for (int q = 0; q < Q; ++q) acc[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
         if ((w0 | w1) == 0) {
-            MfmaRaw rd, rx;
-            MfmaChunk ring[NR];                           // x chunks c - 4 .. c (of one group of lags: c)
+            MfmaRaw<Q> rd, rx;
+            MfmaChunk<Q> ring[NR];                           // x chunks c - 4 .. c (of one group of lags: c)
             read_dy(0, rd);
             read_x(0, rx);
             static_for<NCD>([&](auto c_c) __attribute__((always_inline)) {
                 constexpr int c = decltype(c_c)::value;
-                MfmaChunk dy;
+                MfmaChunk<Q> dy;
                 uint32_t m0, m1;
                 mfma_pack(rd, dy);
                 if constexpr (c < NCX) {
@@ -666,8 +706,8 @@ struct MfmaDw {
             uint32_t m0, m1;
 #pragma nounroll
             for (int c = 0; c < NCX; c += 4) {
-                MfmaRaw raw;
-                MfmaChunk dy;
+                MfmaRaw<Q> raw;
+                MfmaChunk<Q> dy;
                 read_dy(c, raw);
                 mfma_pack(raw, dy);
                 row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + nrow, m0, m1);
@@ -682,7 +722,7 @@ struct MfmaDw {
                 if (b > SPAN) b = SPAN;                      // (staged rows end there)
                 const int t0 = a > TP::FRONT ? a - TP::FRONT : 0, t1 = b - TP::FRONT < nrow ? b - TP::FRONT : nrow;
                 const int c1 = (t1 + 2) >> 2;
-                MfmaRaw rx, rd[ND];
+                MfmaRaw<Q> rx, rd[ND];
                 auto fetch = [&](int c) __attribute__((always_inline)) {
                     const uint32_t at = (col + 4 * c * ROWB) ^ (((n + c) & 3) << 6);
 #pragma unroll
@@ -700,7 +740,7 @@ struct MfmaDw {
                 fetch(c);
 #pragma nounroll
                 for (; c <= c1; ++c) {
-                    MfmaChunk x, dy[ND];
+                    MfmaChunk<Q> x, dy[ND];
                     mfma_pack(rx, x);
 #pragma unroll
                     for (int d = 0; d < ND; ++d) mfma_pack(rd[d], dy[d]);
@@ -858,8 +898,8 @@ dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, 
         auto prepare = [&](int par, int t0) __attribute__((always_inline)) {
             char* buf = lds_raw + par * SH::BUF_BYTES;
             if (lw < SH::NWL) {
-                mfma_stage<SH::NROWS, SH::NWL, false, kLoadAuxOnceBwd>(dy, buf, t0 - TP::FRONT, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, TP::HALO);
-                mfma_stage<R, SH::NWL, true, kLoadAuxOnceBwdX>(x, buf + SH::X_AT, t0, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, 0);
+                mfma_stage<SH::NROWS, SH::NWL, SWZ_QUAD, kLoadAuxOnceBwd>(dy, buf, t0 - TP::FRONT, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, TP::HALO);
+                mfma_stage<R, SH::NWL, SWZ_ROW, kLoadAuxOnceBwdX>(x, buf + SH::X_AT, t0, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, 0);
             } else {
                 mfma_bounds(cu, S, T, t0 - TP::FRONT, SH::NROWS, words + par * kMfmaWords, lane);
             }
@@ -901,6 +941,296 @@ dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, 
             q = lds_next_slot(g, q);
         }
         dw.finish(partial + (size_t)tb * (KT + 1) * C, C, lane);
+    }
+}
+
+// ---- gated backward --------------------------------------------------------------------------------------------------
+// z = [u | g] [T, 2C], the conv ran over h = u * silu(g). dz is MfmaConv over dy with the gate in its stores. dw needs h in
+// fp32, which the matrix cores take only as three bf16 terms: three instructions of 10.7 cycles per 1024 products, what the
+// vector ALU's FMAs take too, and the terms to be made (built and measured that way: 726 us, no gain). So dw stays on the
+// vector ALU: a wave has 128 channels (two per lane) of 8 rows of the tile, with KT sums per channel and 8 rows of h in
+// registers, and reads its KT + 7 rows of dy one after the other. What the role-split kernel spends on dx's FMAs is gone.
+// Bound by the dz waves (one per SIMD: 555 us without the dw waves, loads alone 276). T=131072, C=2048, 31 taps, before and
+// now: log-normal lengths 721 and 673 us, one sequence 674 to 729 and 619, 20 to 512 residues 737 and 705; T=8192, C=512 38 and
+// 27. Two dz and one dw wave of 16 rows per SIMD: 1028 us.
+// a[-i] += h[i] * d for the i < N whose bit of `in` is set (all lanes of the wave are on). Rows of another sequence are left out
+// by the execution mask, not multiplied by zero (their product may be with an Inf). In one instruction block: sums that two
+// branches of compiled code change come to lie in two sets of registers (56 spilled). The masked form lies behind the section's
+// other code, so that the usual one runs on without a jump (T=131072, C=2048, 31 taps, one sequence: 699 us with one, 627).
+template <int N>
+__device__ __forceinline__ void fmac_rows(float (*a)[2], const float (*h)[2], float d0, float d1, uint32_t in) {
+    uint32_t t;
+    if constexpr (N == 1)
+        asm volatile("s_and_b32 %[t], %[in], 1\n\ts_cmp_eq_u32 %[t], 1\n\ts_cbranch_scc0 .Lsome%=\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
+                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
+                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1])
+                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [d0] "v"(d0), [d1] "v"(d1)
+                     : "scc");
+    else if constexpr (N == 2)
+        asm volatile("s_and_b32 %[t], %[in], 3\n\ts_cmp_eq_u32 %[t], 3\n\ts_cbranch_scc0 .Lsome%=\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
+                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
+                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "s_bitcmp1_b32 %[in], 1\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
+                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
+                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1]), [a2] "+v"(a[-1][0]), [a3] "+v"(a[-1][1])
+                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [h2] "v"(h[1][0]), [h3] "v"(h[1][1]), [d0] "v"(d0), [d1] "v"(d1)
+                     : "scc");
+    else if constexpr (N == 3)
+        asm volatile("s_and_b32 %[t], %[in], 7\n\ts_cmp_eq_u32 %[t], 7\n\ts_cbranch_scc0 .Lsome%=\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
+                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
+                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
+                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "s_bitcmp1_b32 %[in], 1\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
+                     "s_bitcmp1_b32 %[in], 2\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
+                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
+                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1]), [a2] "+v"(a[-1][0]), [a3] "+v"(a[-1][1]), [a4] "+v"(a[-2][0]), [a5] "+v"(a[-2][1])
+                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [h2] "v"(h[1][0]), [h3] "v"(h[1][1]), [h4] "v"(h[2][0]), [h5] "v"(h[2][1]), [d0] "v"(d0), [d1] "v"(d1)
+                     : "scc");
+    else if constexpr (N == 4)
+        asm volatile("s_and_b32 %[t], %[in], 15\n\ts_cmp_eq_u32 %[t], 15\n\ts_cbranch_scc0 .Lsome%=\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
+                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
+                     "v_fmac_f32 %[a6], %[h6], %[d0]\n\tv_fmac_f32 %[a7], %[h7], %[d1]\n\t"
+                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
+                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
+                     "s_bitcmp1_b32 %[in], 1\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
+                     "s_bitcmp1_b32 %[in], 2\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
+                     "s_bitcmp1_b32 %[in], 3\n\ts_cselect_b64 exec, -1, 0\n\t"
+                     "v_fmac_f32 %[a6], %[h6], %[d0]\n\tv_fmac_f32 %[a7], %[h7], %[d1]\n\t"
+                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
+                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1]), [a2] "+v"(a[-1][0]), [a3] "+v"(a[-1][1]), [a4] "+v"(a[-2][0]), [a5] "+v"(a[-2][1]), [a6] "+v"(a[-3][0]), [a7] "+v"(a[-3][1])
+                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [h2] "v"(h[1][0]), [h3] "v"(h[1][1]), [h4] "v"(h[2][0]), [h5] "v"(h[2][1]), [h6] "v"(h[3][0]), [h7] "v"(h[3][1]), [d0] "v"(d0), [d1] "v"(d1)
+                     : "scc");
+}
+template <int KT>
+struct GatedDw {
+    using TP = MfmaTaps<KT>;
+    static constexpr int RW = 8, CB = kMfmaGatedCb, NJ = RW + KT - 1;
+    static constexpr int OFS = TP::PP - TP::P - 4 * TP::CK0; // staged row of tap 0 of output row 0 (below 4)
+    float acc[KT][2], db[2];
+    uint32_t ady[4], au;       // LDS addresses of the lane's slice of the wave's first staged row of dy (by the row's permutation) and of u
+
+    // lds: the first buffer; wr: the wave's first row
+    __device__ __forceinline__ void init(const char* lds, int wr, int lane, int x_at) {
+        const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds + wr * CB;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) ady[f] = base + ((lane * 4) ^ (((f + (wr >> 2)) & 3) << 6));
+        au = base + x_at + ((lane * 4) ^ (((wr >> 2) & 3) << 6));
+#pragma unroll
+        for (int m = 0; m < KT; ++m) acc[m][0] = acc[m][1] = 0.f;
+        db[0] = db[1] = 0.f;
+    }
+    __device__ __forceinline__ void next_buffer(int by) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) ady[f] += by;
+        au += by;
+    }
+    __device__ __forceinline__ static uint32_t lds32(uint32_t at) { return *(const __attribute__((address_space(3))) uint32_t*)(uintptr_t)at; }
+    template <int j>
+    __device__ __forceinline__ uint32_t read_dy() const {
+        constexpr int r = j + OFS;
+        return lds32(ady[(r + (r >> 2)) & 3] + r * CB);
+    }
+    // bits: boundaries of the wave's staged rows (bit p: a sequence begins at staged row p of the wave, p > 0)
+    __device__ __forceinline__ void sums(uint64_t bits) {
+        // the wave's rows of the sequence that staged row j + OFS belongs to, as bits; four to a register
+        uint32_t own[(NJ + 3) / 4];
+#pragma unroll
+        for (int i = 0; i < (NJ + 3) / 4; ++i) own[i] = ~0u;
+        if (bits != 0) {
+            static_for<NJ>([&](auto j_c) __attribute__((always_inline)) {
+                constexpr int j = decltype(j_c)::value, r = j + OFS, F = TP::FRONT;
+                int lo = 0;
+                if constexpr (r > 0) lo = 63 - (int)__builtin_clzll((bits & (~0ull >> (63 - r))) | 1ull);
+                int hi = (int)__builtin_ctzll((bits & (~0ull << (r + 1))) | 1ull << 63);
+                lo = lo > F ? lo - F : 0;
+                hi = hi - F < RW ? hi - F : RW;
+                const uint32_t in = hi > lo ? (1u << hi) - (1u << lo) : 0u;
+                own[j / 4] = (own[j / 4] & ~(255u << j % 4 * 8)) | in << j % 4 * 8;
+            });
+        }
+#pragma unroll
+        for (int i = 0; i < (NJ + 3) / 4; ++i) own[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)own[i]);
+        float h[RW][2];
+#pragma unroll
+        for (int u = 0; u < RW; ++u) {
+            const uint32_t at = u < 4 ? au : au ^ 64;        // rows 4 .. 7 have the next permutation
+            const uint32_t xu = lds32(at + u * CB), xg = lds32(at + (u + kMfmaGatedRows) * CB);
+            h[u][0] = gate_mul(bf16_lo(xu), bf16_lo(xg));
+            h[u][1] = gate_mul(bf16_hi(xu), bf16_hi(xg));
+        }
+        uint32_t nxt[2] = {read_dy<0>(), read_dy<1>()};
+        static_for<NJ>([&](auto j_c) __attribute__((always_inline)) {
+            constexpr int j = decltype(j_c)::value;
+            const float d0 = bf16_lo(nxt[j & 1]), d1 = bf16_hi(nxt[j & 1]);
+            if constexpr (j + 2 < NJ) nxt[j & 1] = read_dy<j + 2>();
+            if constexpr (j >= TP::P && j < TP::P + RW) { db[0] += d0; db[1] += d1; }
+            const uint32_t in = own[j / 4] >> j % 4 * 8;
+            constexpr int u0 = j >= KT ? j - KT + 1 : 0, nu = (j < RW ? j + 1 : RW) - u0;
+            fmac_rows<(nu < 4 ? nu : 4)>(&acc[j - u0], &h[u0], d0, d1, in >> u0);
+            if constexpr (nu > 4) fmac_rows<nu - 4>(&acc[j - u0 - 4], &h[u0 + 4], d0, d1, in >> (u0 + 4));
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
+    // words: the tile's boundary bits; wr: the wave's first row, in front of T
+    __device__ __forceinline__ void tile(const uint32_t* words, int wr) {
+        static_assert(NJ + OFS <= 62, "one word of bits");
+        uint32_t v[3];
+        const uint32_t* wp = words + (wr >> 5);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) v[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)wp[i]);
+        const int sh = wr & 31;
+        const uint64_t lo = ((uint64_t)v[0] | (uint64_t)v[1] << 32) >> sh;
+        const uint64_t bits = (lo | (sh ? (uint64_t)v[2] << (64 - sh) : 0)) & ~1ull & ((1ull << (NJ + OFS)) - 1ull);
+        sums(bits);
+    }
+    // the sums by way of LDS, [2 KT + 2][64] floats a wave
+    static constexpr int BOX = (2 * KT + 2) * 64;
+    __device__ __forceinline__ void give(float* box, int lane) const {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            box[c * 64 + lane] = db[c];
+#pragma unroll
+            for (int m = 0; m < KT; ++m) box[(2 + 2 * m + c) * 64 + lane] = acc[m][c];
+        }
+    }
+    __device__ __forceinline__ void take(const float* box, int lane) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            db[c] += box[c * 64 + lane];
+#pragma unroll
+            for (int m = 0; m < KT; ++m) acc[m][c] += box[(2 + 2 * m + c) * 64 + lane];
+        }
+    }
+    // the block's sums to its slab: rows of taps (the weight's order), then db
+    __device__ __forceinline__ void finish(float* __restrict__ slab, int C, int c0) const {
+#pragma unroll
+        for (int m = 0; m < KT; ++m) *reinterpret_cast<float2*>(slab + (size_t)(KT - 1 - m) * C + c0) = make_float2(acc[m][0], acc[m][1]);
+        *reinterpret_cast<float2*>(slab + (size_t)KT * C + c0) = make_float2(db[0], db[1]);
+    }
+};
+
+// 64-row tiles of dy (with its halo rows), u and g; waves of four kinds: dz (4 x 32 channels), dw and db (8 x 8 rows), loaders and
+// boundaries.
+template <int KT>
+struct MfmaGatedBwdShape {
+    using TP = MfmaTaps<KT>;
+    static constexpr int CB = kMfmaGatedCb, CH = CB / 2, R = kMfmaGatedRows, NROWS = R + TP::HALO;
+    static constexpr int NCW = 4, NDZ = NCW, NDW = R / GatedDw<KT>::RW, NWC = NDZ + NDW, NWL = 3;
+    static constexpr int NT = (NWC + NWL + 1) * 64;
+    static constexpr int X_AT = NROWS * CB, BUF_BYTES = X_AT + 2 * R * CB;
+    static constexpr int WORDS_AT = 2 * BUF_BYTES;
+    static constexpr int LDS_BYTES = WORDS_AT + 2 * kMfmaWords * 4;
+    static_assert(CH == 128, "a dw wave has two channels per lane");
+    static_assert(NDW == 8 && NDW / 2 * GatedDw<KT>::BOX * 4 <= WORDS_AT, "half of the sums in the buffers");
+    static_assert(LDS_BYTES <= kLdsBytes, "two buffers of three tiles and the terms of h fit the LDS");
+    static_assert(CH * TP::WSTR * 4 <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
+    static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords && NROWS <= 96, "boundary bits");
+};
+
+template <int KT, bool RES>
+__global__ void __launch_bounds__(MfmaGatedBwdShape<KT>::NT)
+dwconv_bwd_gated_mfma_kernel(const void* __restrict__ z, const void* __restrict__ dy, const int32_t* __restrict__ cu,
+                             const void* __restrict__ w, void* __restrict__ dz, float* __restrict__ partial, const LdsGeo g) {
+    using SH = MfmaGatedBwdShape<KT>;
+    using TP = MfmaTaps<KT>;
+    constexpr int R = SH::R;
+    extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+    uint32_t* words = reinterpret_cast<uint32_t*>(lds_raw + SH::WORDS_AT);
+    uint32_t* tab = reinterpret_cast<uint32_t*>(lds_raw + SH::BUF_BYTES);
+    const int lane = (int)(threadIdx.x & 63);
+    const int wv = wave_id();
+    int cb, tb;
+    lds_block_coords(g, cb, tb);
+    const int T = g.T, S = g.S, C = g.C;
+    const int rowb = C * 2;
+    const int col_byte0 = cb * SH::CB;
+    const int valid_bytes = rowb - col_byte0 < SH::CB ? rowb - col_byte0 : SH::CB;
+    const int nch = valid_bytes / 2;
+    const int ntl = (g.ntiles + g.nbt - 1) / g.nbt;
+    int q = tb;
+
+    if (wv >= SH::NWC) {
+        __builtin_amdgcn_s_setprio(3);
+        const int lw = wv - SH::NWC;
+        auto prepare = [&](int par, int t0) __attribute__((always_inline)) {
+            char* buf = lds_raw + par * SH::BUF_BYTES;
+            if (lw < SH::NWL) {
+                mfma_stage<SH::NROWS, SH::NWL, SWZ_BOTH, kLoadAuxOnceBwd, SH::CB>(dy, buf, t0 - TP::FRONT, T, (size_t)rowb, col_byte0, valid_bytes, lw, lane, TP::HALO);
+                mfma_stage<R, SH::NWL, SWZ_QUAD, kLoadAuxOnceBwdX, SH::CB>(z, buf + SH::X_AT, t0, T, 2 * (size_t)rowb, col_byte0, valid_bytes, lw, lane, 0);
+                mfma_stage<R, SH::NWL, SWZ_QUAD, kLoadAuxOnceBwdX, SH::CB>(z, buf + SH::X_AT + R * SH::CB, t0, T, 2 * (size_t)rowb, rowb + col_byte0, valid_bytes, lw, lane, 0);
+            } else {
+                mfma_bounds(cu, S, T, t0 - TP::FRONT, SH::NROWS, words + par * kMfmaWords, lane);
+            }
+        };
+        prepare(0, tb * R);
+        lds_barrier();                       // the weight table is written
+        lds_barrier();                       // and has been read
+        for (int it = 0; it < ntl; ++it) {
+            if (lw < SH::NWL) wait_vmem_all();
+            lds_barrier();                   // tile `it` has landed, the buffer of the tile before is free
+            q = lds_next_slot(g, q);
+            const int t0 = it + 1 < ntl ? lds_tile_row0(g, it + 1, q, R) : T;
+            if (t0 < T) prepare((it + 1) & 1, t0);
+        }
+        for (int k = 0; k < 6; ++k) lds_barrier();      // (the dw waves join their sums)
+        return;
+    }
+    mfma_fill_weights<KT, true, SH::CH>(tab, w, g.w_flags, cb * SH::CH, nch, (int)threadIdx.x, SH::NWC * 64);
+    lds_barrier();
+    if (wv < SH::NDZ) {
+        __builtin_amdgcn_s_setprio(2);       // a dz wave has the longest way through a tile (log-normal lengths: 682 us without, 673 with)
+        MfmaConv<KT, R / 16, true, RES, true> conv;
+        conv.init(tab, w, g.w_flags, nullptr, wv, lane, cb * SH::CH, nch, rowb);
+        lds_barrier();
+        for (int it = 0; it < ntl; ++it) {
+            lds_barrier();
+            const int t0 = lds_tile_row0(g, it, q, R);
+            const char* buf = lds_raw + (it & 1) * SH::BUF_BYTES;
+            if (t0 < T)
+                conv.rows(buf, words + (it & 1) * kMfmaWords, 0, mfma_out_rsrc(dz, t0, T - t0 < R ? T - t0 : R, 2 * rowb), rowb, buf + SH::X_AT);
+            q = lds_next_slot(g, q);
+        }
+        for (int k = 0; k < 6; ++k) lds_barrier();
+    } else {
+        using DW = GatedDw<KT>;
+        DW dw;
+        const int dv = wv - SH::NDZ, wr = dv * DW::RW;
+        dw.init(lds_raw, wr, lane, SH::X_AT);
+        lds_barrier();
+        for (int it = 0; it < ntl; ++it) {
+            lds_barrier();
+            if (lds_tile_row0(g, it, q, R) + wr < T) dw.tile(words + (it & 1) * kMfmaWords, wr);
+            dw.next_buffer(it & 1 ? -SH::BUF_BYTES : SH::BUF_BYTES);
+            q = lds_next_slot(g, q);
+        }
+        // the eight waves' sums in a fixed order: 0 + 4, 1 + 5, ...; then 0 + 2, 1 + 3; then 0 + 1
+        float* box = reinterpret_cast<float*>(lds_raw);
+#pragma nounroll
+        for (int half = SH::NDW / 2; half > 0; half /= 2) {
+            lds_barrier();
+            if (dv >= half && dv < 2 * half) dw.give(box + (dv - half) * DW::BOX, lane);
+            lds_barrier();
+            if (dv < half) dw.take(box + dv * DW::BOX, lane);
+        }
+        if (dv == 0 && 2 * lane < nch) dw.finish(partial + (size_t)tb * (KT + 1) * C, C, cb * SH::CH + 2 * lane);
     }
 }
 

@@ -135,3 +135,53 @@ def test_which_backward_calls_the_matrix_cores_serve(T, n, K, wdt, served):
     assert all(torch.equal(a, c) for a, c in zip(got, want))
     assert torch.equal(npa.varlen_dwconv_bwd(xd, dyd, cud, wd, need_dw=False)[0],
                        npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(algo=1))[0])
+
+
+@pytest.mark.parametrize("K,lens,C", [(31, LENS * 2, 512), (29, LENS[::-1] * 2, 520), (25, [4096], 1000), (31, [4095, 1, 63], 648),
+                                      (31, LENS * 4, 2056), (31, [1] * 4160, 512), (31, [4095], 512), (31, [16500] + [1] * 200, 512)])
+def test_gated_backward_of_31_taps_matches_the_oracle(K, lens, C):
+    """From 4096 rows on dz comes from the matrix cores and dw from waves of 8 rows that leave out the products across a
+    boundary (below, and with many short sequences in a long batch, from the role-split kernel): whole, partial and several
+    column blocks, rows of one sequence and of many in a wave, and the same bits after a call that left NaN in LDS."""
+    print(f"[case] gated K={K} C={C}", flush=True)
+    _, cu, w, b, dy = _case(lens, C, K, C + K)
+    z = torch.randn(dy.shape[0], 2 * C, generator=torch.Generator().manual_seed(C)).bfloat16()
+    zd, cud, wd, dyd = z.to(DEV), cu.to(DEV), w.to(DEV), dy.to(DEV)
+    for res in (False, True):
+        _, dz64, dw64, db64 = O.ref_gated_dwconv_grads(z, cu, w, b, dy, torch.float64, res)
+        got = npa.gated_dwconv_bwd(zd, dyd, cud, wd, residual=res)
+        assert_act_close(got[0], dz64, torch.bfloat16, "dz")
+        assert_red_close(got[1], dw64, "dw")
+        assert_red_close(got[2], db64, "db")
+    npa.gated_dwconv_bwd(torch.full_like(zd, float("nan")), torch.full_like(dyd, float("nan")), cud, wd, residual=True)
+    again = npa.gated_dwconv_bwd(zd, dyd, cud, wd, residual=True)
+    assert all(torch.equal(a, c) for a, c in zip(again, got))
+
+
+@pytest.mark.parametrize("which", ["z", "dy"])
+def test_gated_backward_non_finite_rows_stay_in_their_sequence(which):
+    """Rows of one-row sequences reach the centre tap (and, from dy, db) only; rows of other sequences keep their dz."""
+    C, K, lens = 512, 31, [40, 1, 700, 1, 213, 64, 1, 33, 1, 1500, 1, 1700]
+    _, cu, w, _, dy = _case(lens, C, K, 3)
+    z = torch.randn(dy.shape[0], 2 * C, generator=torch.Generator().manual_seed(5)).bfloat16()
+    bad = torch.zeros(dy.shape[0], dtype=torch.bool)
+    for i, n in enumerate(lens):
+        if n == 1:
+            bad[cu[i]] = True
+    cud, wd = cu.to(DEV), w.to(DEV)
+    dz0, dw0, db0 = npa.gated_dwconv_bwd(z.to(DEV), dy.to(DEV), cud, wd)
+    t = z if which == "z" else dy
+    t[bad, ::3] = float("inf")
+    dz, dw, db = npa.gated_dwconv_bwd(z.to(DEV), dy.to(DEV), cud, wd)
+    assert torch.equal(dz[~bad.to(DEV)], dz0[~bad.to(DEV)])
+    hit = torch.zeros(C, K, dtype=torch.bool, device=DEV)
+    hit[0::3 if which == "dy" else 1, K // 2] = True
+    if which == "z":                                                  # (u's columns 0, 3, ...; g's from where C leaves off)
+        hit[:, K // 2] = ((torch.arange(C) % 3 == 0) | ((torch.arange(C) + C) % 3 == 0)).to(DEV)
+    assert not bool(torch.isfinite(dw[hit]).any()) and bool(torch.isfinite(dw[~hit]).all())
+    torch.testing.assert_close(dw[~hit], dw0[~hit], rtol=0, atol=1e-5 * float(dw0.abs().max()))
+    keep = torch.ones(C, dtype=torch.bool, device=DEV)
+    if which == "dy":
+        keep[0::3] = False
+    assert not bool(torch.isfinite(db[~keep]).any())
+    torch.testing.assert_close(db[keep], db0[keep], rtol=0, atol=1e-5 * float(db0.abs().max()))
