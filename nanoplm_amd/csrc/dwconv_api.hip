@@ -355,6 +355,12 @@ bool mfma_eligible(bool bf16, bool w_bf16, long long T, int C, int K, uintptr_t 
     return bf16 && w_bf16 && split_eligible(bf16, T, C, K, align_bits);
 }
 constexpr long long kMfmaMinRows = 4096;
+// The library's own choice of them: their tiles of 64 rows reach make_split_plan()'s limit on a tile's bytes in rows that the
+// shorter tiles of other kernels still take (C beyond 13 million, gated 5.5 million, bf16); those rows keep the others.
+bool mfma_tile_fits(int C, int K, bool gated) {
+    const int tile_rows = gated ? kMfmaGatedRows : kMfmaFwdRows;
+    return ((long long)(tile_rows + K) * (gated ? 2 : 1) + 2) * C * 2 < INT_MAX;
+}
 // A backward tile with sequence boundaries makes one pass over its rows per sequence for dw, so the gain goes with the length
 // of the sequences. Measured at T=131072, us, matrix cores against role-split, for lengths of 20 to 128 residues (mean 75), 20
 // to 512 (mean 263), log-normal (mean 333), one sequence:
@@ -434,7 +440,8 @@ int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, bool w_bf16
     if (tune && tune->algo == 3) return split_eligible(bf16, T, C, K, align_bits) ? 3 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 2) return lds_eligible(bf16, T, C, K, align_bits) ? 2 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 1) return 1;
-    if (mfma_eligible(bf16, w_bf16, T, C, K, align_bits) && T >= kMfmaMinRows && (!bwd || mfma_bwd_preferred(T, taps, S))) return 4;
+    if (mfma_eligible(bf16, w_bf16, T, C, K, align_bits) && T >= kMfmaMinRows && mfma_tile_fits(C, K, false) &&
+        (!bwd || mfma_bwd_preferred(T, taps, S))) return 4;
     if (split_eligible(bf16, T, C, K, align_bits) && (bwd || K == 31)) return 3;
     return lds_preferred(bwd, bf16, T, C, K, align_bits) ? 2 : 1;
 }
@@ -1157,7 +1164,8 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
     if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {
         LdsPlan lp;
-        const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 && T >= kMfmaMinRows && mfma_gated_bwd_preferred(T, taps, S);
+        const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 && T >= kMfmaMinRows &&
+                          mfma_tile_fits(C, K, true) && mfma_gated_bwd_preferred(T, taps, S);
         rc = mfma ? make_split_plan(false, bf16, T, C, K, nullptr, &lp, true, kMfmaGatedRows, kMfmaGatedCb)
                   : make_split_plan(false, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;

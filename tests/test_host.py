@@ -100,6 +100,18 @@ def test_argument_errors_are_reported_before_any_launch():
     assert _bwd(dx=None, dw=None, db=None) == 0      # nothing requested
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the calls pass every check and would launch on made-up pointers")
+def test_rows_too_wide_for_the_matrix_cores_tiles_keep_their_kernels():
+    """Rows whose 64-row tiles pass the 2 GiB limit of a tile still take the kernels with shorter tiles, which refuse them at
+    a limit of their own: without a GPU an accepted call ends with the runtime's (positive) error."""
+    lib, p, bf16 = _lib.load(), 1 << 20, 1
+    for K, C in ((11, 14_000_000), (15, 17_000_000), (15, 13_000_000)):
+        assert lib.nplm_dwconv_fwd(p, p, p, None, p, 4096, C, K, 1, bf16, bf16, None) > 0
+    for K, C, ok in ((31, 5_500_000, True), (31, 6_000_000, True), (31, 7_400_000, True), (31, 7_500_000, False)):
+        rc = lib.nplm_dwconv_gated_bwd(p, p, p, p, p, p, p, p, 1 << 60, 4096, C, K, 1, bf16, bf16, 0, None)
+        assert rc > 0 if ok else rc == -2, (C, rc)
+
+
 def test_workspace_bytes_arithmetic():
     lib = _lib.load()
     for (T, C, K, act) in [(131072, 1024, 7, 1), (131072, 2048, 31, 1), (65536, 1024, 7, 1), (776, 64, 3, 0),
