@@ -1385,6 +1385,38 @@ int64_t nplm_dwconv_debug_intervals(const int32_t* cu_host, int32_t S, int64_t T
     return n;
 }
 
+int64_t nplm_dwconv_debug_starts(const int32_t* cu_host, int32_t S, int32_t a, int32_t n, uint32_t* marks_out) {
+    if (!cu_host || !marks_out || S < 0 || n < 1 || n > 256) return -1;
+    struct Lanes {
+        const int32_t* cu;
+        uint32_t* words;
+        int a, n;
+        int64_t reads;
+        uint64_t above(uint32_t lo, uint32_t step, uint32_t last, int row) {
+            ++reads;
+            uint64_t m = 0;
+            for (uint32_t l = 0; l < 64; ++l) {
+                const uint32_t i = lo + (l + 1) * step - 1;
+                m |= (uint64_t)(cu[i < last ? i : last] > row) << l;
+            }
+            return m;
+        }
+        int take(uint32_t lo, uint32_t last) {
+            ++reads;
+            int v = 0;
+            for (uint32_t l = 0; l < 64; ++l) {
+                v = cu[lo + l < last ? lo + l : last];
+                const uint32_t p = (uint32_t)v - (uint32_t)a;
+                if (v > a && p < (uint32_t)n) words[(p - 1) >> 5] |= 1u << ((p - 1) & 31);
+            }
+            return v;
+        }
+    } lanes{cu_host, marks_out, a, n, 0};
+    for (int i = 0; i < (n + 31) / 32; ++i) marks_out[i] = 0;
+    walk_starts(lanes, S, a, n);
+    return lanes.reads;
+}
+
 int nplm_dwconv_check_cu(const int32_t* cu, int32_t S, int64_t T, void* stream) {
     if (!cu) return -NPLM_DWCONV_ENULL;
     if (S < 0 || T < 0 || T > kMaxRows) return -NPLM_DWCONV_ESHAPE;

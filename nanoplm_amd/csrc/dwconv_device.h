@@ -227,7 +227,7 @@ struct SeqCursor {
         int lo = hint < 0 ? 0 : hint, hi = S;
         // first i in [lo, S) with cu[i+1] > t, else S
         while (lo < hi) {
-            int mid = (lo + hi) >> 1;
+            const int mid = (int)(((uint32_t)lo + (uint32_t)hi) >> 1);      // (the sum of two ints may need 32 bits)
             if (cu_at(cu, mid + 1) > t) hi = mid; else lo = mid + 1;
         }
         seq = lo;
@@ -245,6 +245,27 @@ struct SeqCursor {
         }
     }
 };
+
+// What one wave does to find every sequence that begins in rows (a, a + n): a search with 64 probes a step for the first entry of
+// cu beyond row a, then 64 entries at a time. Wave is the wave itself (dwconv_mfma_kernels.h) or 64 lanes on the host:
+//   above(lo, step, last, a)  the lanes l with cu[min(lo + (l + 1) * step - 1, last)] > a, as bits
+//   take(lo, last)            marks the rows cu[min(lo + l, last)] of all lanes, returns the last lane's
+// Entries are numbered 0 .. S with S up to 2^31 - 1, probes reach 63 beyond: unsigned. Indices stay in [0, S] whatever cu holds.
+template <typename Wave>
+__host__ __device__ __forceinline__ void walk_starts(Wave& wave, int S, int a, int n) {
+    uint32_t lo = 0, hi = (uint32_t)S + 1;       // the first i in [lo, hi) with cu[i] > a, else hi
+    while (hi - lo > 64) {
+        const uint32_t step = (hi - lo + 63) >> 6;
+        const uint64_t m = wave.above(lo, step, hi - 1, a);
+        if (m == 0) { lo = hi; break; }
+        const uint32_t f = (uint32_t)__builtin_ctzll(m), nhi = lo + (f + 1) * step;
+        lo += f * step;
+        hi = nhi < hi ? nhi : hi;
+    }
+    for (; lo <= (uint32_t)S; lo += 64) {
+        if ((long long)wave.take(lo, (uint32_t)S) >= (long long)a + n) break;
+    }
+}
 
 // Which of the K taps of output row t stay inside the cursor's interval: bit m is set iff row
 // t - P + m lies in [cs, ce). One scalar word (K <= 32) per row instead of two compares per tap;

@@ -887,7 +887,7 @@ dwconv_bwd_lds_kernel(const void* __restrict__ x, const void* __restrict__ dy, c
             int lo = 0, hi = S;     // first i in [0, S) with cu[i + 1] > t, else S
             while (__builtin_amdgcn_ballot_w64(lo < hi) != 0) {
                 if (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
+                    const int mid = (int)(((uint32_t)lo + (uint32_t)hi) >> 1);
                     if (cu[mid + 1] > t) hi = mid; else lo = mid + 1;
                 }
             }

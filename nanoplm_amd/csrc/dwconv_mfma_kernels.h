@@ -117,33 +117,32 @@ __device__ __forceinline__ void mfma_stage(const void* __restrict__ src, char* d
 }
 
 // Boundary bits of the rows [a, a + n): bit p of `words` is set iff a sequence begins at row a + p (0 < p < n); the tensor's
-// first and one-past-last row count. One whole wave; a search with 64 probes a step finds the first entry of cu beyond row
-// a, then entries are taken 64 at a time. Indices stay in [0, S] whatever cu holds.
-__device__ __forceinline__ void mfma_bounds(const int32_t* __restrict__ cu, int S, int T, int a, int n, uint32_t* words, int lane) {
-    if (lane < kMfmaWords) words[lane] = 0;
-    auto mark = [&](int row) __attribute__((always_inline)) {
+// first and one-past-last row count. One whole wave (walk_starts()).
+struct MfmaMarks {
+    const int32_t* __restrict__ cu;
+    uint32_t* words;
+    int a, n, lane;
+    __device__ __forceinline__ void mark(int row) const {
         const uint32_t p = (uint32_t)row - (uint32_t)a;      // (unsigned: cu may hold anything)
         if (row > a && p < (uint32_t)n) __hip_atomic_fetch_or(words + (p >> 5), 1u << (p & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    };
-    if (lane == 0) mark(0);
-    if (lane == 1) mark(T);
-    int lo = 0, hi = S + 1;              // the first i in [lo, hi) with cu[i] > a, else hi
-    while (hi - lo > 64) {
-        const int step = (hi - lo + 63) >> 6;
-        const int i = lo + (lane + 1) * step - 1;
-        const uint64_t m = __builtin_amdgcn_ballot_w64(cu[i < hi ? i : hi - 1] > a);
-        if (m == 0) { lo = hi; break; }
-        const int f = (int)__builtin_ctzll(m);
-        const int nhi = lo + (f + 1) * step;
-        lo += f * step;
-        hi = nhi < hi ? nhi : hi;
     }
-    for (; lo <= S; lo += 64) {
-        const int i = lo + lane <= S ? lo + lane : S;
-        const int v = cu[i];
+    __device__ __forceinline__ uint64_t above(uint32_t lo, uint32_t step, uint32_t last, int row) const {
+        const uint32_t i = lo + ((uint32_t)lane + 1) * step - 1;
+        return __builtin_amdgcn_ballot_w64(cu[i < last ? i : last] > row);
+    }
+    __device__ __forceinline__ int take(uint32_t lo, uint32_t last) const {
+        const uint32_t i = lo + (uint32_t)lane;
+        const int v = cu[i < last ? i : last];
         mark(v);
-        if (__builtin_amdgcn_readlane(v, 63) >= a + n) break;
+        return __builtin_amdgcn_readlane(v, 63);
     }
+};
+__device__ __forceinline__ void mfma_bounds(const int32_t* __restrict__ cu, int S, int T, int a, int n, uint32_t* words, int lane) {
+    if (lane < kMfmaWords) words[lane] = 0;
+    MfmaMarks m{cu, words, a, n, lane};
+    if (lane == 0) m.mark(0);
+    if (lane == 1) m.mark(T);
+    walk_starts(m, S, a, n);
 }
 
 // Boundary bits of a lane's window: bit r is set iff a sequence begins at window row r (r < 64).

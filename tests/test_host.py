@@ -210,6 +210,38 @@ def test_cursor_never_leaves_the_array_on_malformed_cu():
     _intervals([0, 50, 100], 12)             # entries beyond T
 
 
+# ---- boundary walk of the matrix-core kernels -----------------------------------------------------
+def _starts(cu, a, n):
+    words = np.zeros(8, dtype=np.uint32)
+    reads = _lib.load().nplm_dwconv_debug_starts(cu.ctypes.data, len(cu) - 1, a, n, words.ctypes.data)
+    assert reads >= 1
+    bits = np.unpackbits(words.view(np.uint8), bitorder="little")[:n - 1]
+    return (a + 1 + np.flatnonzero(bits)).tolist(), reads
+
+
+def test_boundary_walk_marks_every_start_in_the_window():
+    rng = np.random.default_rng(3)
+    for _ in range(200):
+        lens = rng.integers(0, rng.integers(2, 60), size=rng.integers(1, 400))
+        cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        T = int(cu[-1])
+        for a in (-15, 0, 1, T // 2, max(T - 20, 0), T):
+            n = int(rng.integers(2, 95))
+            rows, _ = _starts(cu, a, n)
+            assert rows == sorted({int(r) for r in cu if a < r < a + n})
+
+
+def test_boundary_walk_of_the_largest_number_of_sequences():
+    """S = 2^31 - 1, all but the last sequence empty: entry numbers of the probes need 32 bits. (The array is 8 GiB of address
+    space, of which the walk touches a few hundred pages.)"""
+    cu = np.zeros(2 ** 31, dtype=np.int32)
+    cu[-1] = 64
+    assert _starts(cu, 10, 60)[0] == [64]
+    cu[-3:-1] = 30
+    assert _starts(cu, 10, 60)[0] == [30, 64]
+    assert _starts(cu, 30, 40)[0] == [64]
+
+
 # ---- Python surface -----------------------------------------------------------------------------
 def test_cpu_tensors_are_refused():
     x = torch.randn(10, 8)
