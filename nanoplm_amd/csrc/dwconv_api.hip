@@ -1385,35 +1385,36 @@ int64_t nplm_dwconv_debug_intervals(const int32_t* cu_host, int32_t S, int64_t T
     return n;
 }
 
-int64_t nplm_dwconv_debug_starts(const int32_t* cu_host, int32_t S, int32_t a, int32_t n, uint32_t* marks_out) {
-    if (!cu_host || !marks_out || S < 0 || n < 1 || n > 256) return -1;
+int64_t nplm_dwconv_debug_starts(const int32_t* cu_host, int32_t S, int64_t T, int32_t a, int32_t n, uint32_t* marks_out) {
+    if (!cu_host || !marks_out || S < 0 || T < 0 || T > kMaxRows || n < 1 || n > 256) return -1;
     struct Lanes {
         const int32_t* cu;
         uint32_t* words;
         int a, n;
         int64_t reads;
-        uint64_t above(uint32_t lo, uint32_t step, uint32_t last, int row) {
+        void mark(int row) {
+            const uint32_t p = (uint32_t)row - (uint32_t)a;
+            if (row > a && p < (uint32_t)n) words[(p - 1) >> 5] |= 1u << ((p - 1) & 31);
+        }
+        uint64_t above(uint32_t lo, uint32_t step, uint32_t end, int row) {
             ++reads;
             uint64_t m = 0;
             for (uint32_t l = 0; l < 64; ++l) {
                 const uint32_t i = lo + (l + 1) * step - 1;
-                m |= (uint64_t)(cu[i < last ? i : last] > row) << l;
+                m |= (uint64_t)(cu[i < end ? i : end] > row) << l;
             }
             return m;
         }
-        int take(uint32_t lo, uint32_t last) {
+        int take(uint32_t lo, uint32_t end, int& first) {
             ++reads;
-            int v = 0;
-            for (uint32_t l = 0; l < 64; ++l) {
-                v = cu[lo + l < last ? lo + l : last];
-                const uint32_t p = (uint32_t)v - (uint32_t)a;
-                if (v > a && p < (uint32_t)n) words[(p - 1) >> 5] |= 1u << ((p - 1) & 31);
-            }
-            return v;
+            for (uint32_t l = 0; l < 64; ++l) mark(cu[lo + l < end ? lo + l : end]);
+            first = cu[lo < end ? lo : end];
+            return cu[lo + 63 < end ? lo + 63 : end];
         }
     } lanes{cu_host, marks_out, a, n, 0};
     for (int i = 0; i < (n + 31) / 32; ++i) marks_out[i] = 0;
-    walk_starts(lanes, S, a, n);
+    lanes.mark((int)T);
+    walk_starts(lanes, S, (int)T, a, n);
     return lanes.reads;
 }
 

@@ -66,9 +66,9 @@ int64_t nplm_dwconv_debug_intervals(const int32_t* cu_host, int32_t S, int64_t T
                                     int64_t relocate_every, int32_t* cs_out, int32_t* ce_out);
 
 // Host-side run of the matrix-core kernels' boundary walk (walk_starts()) over a HOST copy of cu, for the staged rows [a, a + n):
-// bit p - 1 of marks_out[(p - 1) / 32] for every sequence that begins at row a + p, 0 < p < n <= 256. Returns how many times 64
-// entries were read, -1 on bad arguments.
-int64_t nplm_dwconv_debug_starts(const int32_t* cu_host, int32_t S, int32_t a, int32_t n, uint32_t* marks_out);
+// bit p - 1 of marks_out[(p - 1) / 32] for every sequence that begins at row a + p, 0 < p < n <= 256, and for T. Returns how many
+// times 64 entries were read, -1 on bad arguments.
+int64_t nplm_dwconv_debug_starts(const int32_t* cu_host, int32_t S, int64_t T, int32_t a, int32_t n, uint32_t* marks_out);
 
 // Plain streaming copy of `bytes` bytes (multiple of 16, 16-byte aligned pointers) with one block
 // per contiguous 16 KiB: the measuring stick for what a 1-read-1-write kernel reaches on this GPU and

@@ -126,14 +126,15 @@ struct MfmaMarks {
         const uint32_t p = (uint32_t)row - (uint32_t)a;      // (unsigned: cu may hold anything)
         if (row > a && p < (uint32_t)n) __hip_atomic_fetch_or(words + (p >> 5), 1u << (p & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    __device__ __forceinline__ uint64_t above(uint32_t lo, uint32_t step, uint32_t last, int row) const {
+    __device__ __forceinline__ uint64_t above(uint32_t lo, uint32_t step, uint32_t end, int row) const {
         const uint32_t i = lo + ((uint32_t)lane + 1) * step - 1;
-        return __builtin_amdgcn_ballot_w64(cu[i < last ? i : last] > row);
+        return __builtin_amdgcn_ballot_w64(cu[i < end ? i : end] > row);
     }
-    __device__ __forceinline__ int take(uint32_t lo, uint32_t last) const {
+    __device__ __forceinline__ int take(uint32_t lo, uint32_t end, int& first) const {
         const uint32_t i = lo + (uint32_t)lane;
-        const int v = cu[i < last ? i : last];
+        const int v = cu[i < end ? i : end];
         mark(v);
+        first = __builtin_amdgcn_readfirstlane(v);
         return __builtin_amdgcn_readlane(v, 63);
     }
 };
@@ -142,7 +143,7 @@ __device__ __forceinline__ void mfma_bounds(const int32_t* __restrict__ cu, int 
     MfmaMarks m{cu, words, a, n, lane};
     if (lane == 0) m.mark(0);
     if (lane == 1) m.mark(T);
-    walk_starts(m, S, a, n);
+    walk_starts(m, S, T, a, n);
 }
 
 // Boundary bits of a lane's window: bit r is set iff a sequence begins at window row r (r < 64).

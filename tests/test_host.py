@@ -213,7 +213,7 @@ def test_cursor_never_leaves_the_array_on_malformed_cu():
 # ---- boundary walk of the matrix-core kernels -----------------------------------------------------
 def _starts(cu, a, n):
     words = np.zeros(8, dtype=np.uint32)
-    reads = _lib.load().nplm_dwconv_debug_starts(cu.ctypes.data, len(cu) - 1, a, n, words.ctypes.data)
+    reads = _lib.load().nplm_dwconv_debug_starts(cu.ctypes.data, len(cu) - 1, int(cu[-1]), a, n, words.ctypes.data)
     assert reads >= 1
     bits = np.unpackbits(words.view(np.uint8), bitorder="little")[:n - 1]
     return (a + 1 + np.flatnonzero(bits)).tolist(), reads
@@ -240,6 +240,20 @@ def test_boundary_walk_of_the_largest_number_of_sequences():
     cu[-3:-1] = 30
     assert _starts(cu, 10, 60)[0] == [30, 64]
     assert _starts(cu, 30, 40)[0] == [64]
+
+
+@pytest.mark.parametrize("front,inside,tail", [(0, 0, 70000), (0, 70000, 0), (70000, 0, 0), (5000, 3000, 9000)])
+def test_boundary_walk_does_not_walk_runs_of_empty_sequences(front, inside, tail):
+    """Empty sequences in front of the rows, between them and behind (the static collator's tail): read 64 at a time they would
+    be over a thousand reads in the tiles that hold them."""
+    T = 4096
+    lens = [0] * front + [1000, 30] + [0] * inside + [7] + [0] * inside + [3, 2000, T - 3040] + [0] * tail
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    for a in [-15, 0] + list(range(49, T, 64)):
+        rows, reads = _starts(cu, a, 94)
+        assert rows == sorted({int(r) for r in cu if a < r < a + 94})
+        # three probes find an entry among 2^18; the window has at most four starts, each with a read, a search and a read behind it
+        assert reads <= 4 + 4 * 5
 
 
 # ---- Python surface -----------------------------------------------------------------------------
