@@ -361,6 +361,28 @@ bool mfma_tile_fits(int C, int K, bool gated) {
     const int tile_rows = gated ? kMfmaGatedRows : kMfmaFwdRows;
     return ((long long)(tile_rows + K) * (gated ? 2 : 1) + 2) * C * 2 < INT_MAX;
 }
+// Output rows that do not begin on whole cache lines (128 bytes). A wave of the matrix-core kernels stores 128 bytes of a row
+// (gated 64) at a time where the others store 256 or 512; off the lines' grid each piece is two parts of lines, which other waves
+// complete later, and once the output is too large for the caches many of them reach HBM as parts. Measured with lengths of 20 to
+// 512 (backward at 11 taps: 700) residues, us, matrix cores against the best of the others, by MiB of T rows of C channels:
+//   forward, 11 / 15 taps: T=131072 C=1000 (250 MiB) 140 / 112, 139 / 111; C=648 (162) 106 / 99; T=65536 C=1160 (145) 89 / 80,
+//     C=840 (105) 61 / 59; T=32768 C=2008 (126) 72 / 63, C=1160 (72) 42 / 43, C=1000 (62) 36 / 38. Rows that fill the others'
+//     1 KiB column blocks to less than 3/5 stay: C=584 (0.57) T=98304 66 / 77, T=262144 173 / 180.
+//   backward, T=131072 C=1000 (250): 11 taps 228 / 184, 15 223 / 192; T=32768 C=648 (40) 47.6 / 45.1, 50.5 / 47.5, C=520 (32) 41.0 /
+//     41.0, 46.6 / 46.3; rows of less than 640 bytes stay: T=131072 C=264 (66) 71.7 / 72.8, 86.5 / 90.2.
+//   gated backward, 31 taps: T=131072 C=2008 (502) 1011 / 762, C=1000 518 / 392; T=65536 C=584 (73) 157 / 144; T=16384 C=1000 (31) 68 /
+//     65, C=648 (20) 53 / 54, C=520 (16) 47 / 53.
+// 31 taps save more FMAs than that costs (backward T=131072 C=1000 229 / 261, C=2040 509 / 517; forward 149 / 151, 346 / 326), 21
+// taps come out even (forward 145 / 144, backward 222 / 206, C=1800 351 / 377): both stay.
+bool mfma_lines_ok(bool bwd, bool gated, long long T, int C, int K, int taps, uintptr_t out_bits) {
+    const long long row_bytes = 2LL * C;
+    if (((uintptr_t)row_bytes | out_bits) % 128 == 0) return true;
+    const long long mib = T * row_bytes >> 20;
+    if (gated) return mib < 30;
+    if (taps > 15) return true;
+    if (bwd) return row_bytes < 640 || mib < 30;
+    return mib < 100 || !lds_preferred(false, true, T, C, K, 0) || row_bytes * 5 < ceil_div(row_bytes, kLdsDefaultCb) * 3LL * kLdsDefaultCb;
+}
 // A backward tile with sequence boundaries makes one pass over its rows per sequence for dw, so the gain goes with the length
 // of the sequences. Measured at T=131072, us, matrix cores against role-split, for lengths of 20 to 128 residues (mean 75), 20
 // to 512 (mean 263), log-normal (mean 333), one sequence:
@@ -429,19 +451,21 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
 //     12.2 / 11.8), while the others' sums are those of the sliding-window kernels bit for bit.
 //     fp32 weights would take three bf16 terms each: 280 us against 265 (K=31, C=2048), so they stay on the vector ALU.
 //   the same calls backward: matrix cores where a sequence has enough rows (mfma_bwd_preferred()).
+//   Large outputs whose rows are not whole cache lines keep the other kernels at 11 and 15 taps (mfma_lines_ok()).
 //   K=31 and K=15 backward of fp32 weights (ALU-bound; one wave cannot hold the fused backward's registers): the role-split
 //     kernel, when every output is asked for - C=2048, K=31: 510 us against 720 sliding-window on the log-normal length mix;
 //     K=15: 345 against 385 (C=1024: 177 against 205). A backward asked for dx alone or dw/db alone takes the
 //     sliding-window kernel, like everything the LDS kernels are not built for (other sizes, narrow or unaligned rows).
 //   K=31 forward of fp32 weights: the role-split kernel's dx role on every wave, 262 us against 299 LDS-staged with loader
 //     waves (C=2048); K=15: LDS-staged with loader waves, 190 us against 203 role-split and 227 sliding-window (C=2048).
-int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, bool w_bf16, long long T, int C, int K, int taps, int S, uintptr_t align_bits) {
+int choose_algo(bool bwd, const nplm_dwconv_tuning* tune, bool bf16, bool w_bf16, long long T, int C, int K, int taps, int S, uintptr_t align_bits,
+                uintptr_t out_bits) {
     if (tune && tune->algo == 4) return mfma_eligible(bf16, w_bf16, T, C, K, align_bits) ? 4 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 3) return split_eligible(bf16, T, C, K, align_bits) ? 3 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 2) return lds_eligible(bf16, T, C, K, align_bits) ? 2 : -NPLM_DWCONV_ETUNING;
     if (tune && tune->algo == 1) return 1;
     if (mfma_eligible(bf16, w_bf16, T, C, K, align_bits) && T >= kMfmaMinRows && mfma_tile_fits(C, K, false) &&
-        (!bwd || mfma_bwd_preferred(T, taps, S))) return 4;
+        mfma_lines_ok(bwd, false, T, C, K, taps, out_bits) && (!bwd || mfma_bwd_preferred(T, taps, S))) return 4;
     if (split_eligible(bf16, T, C, K, align_bits) && (bwd || K == 31)) return 3;
     return lds_preferred(bwd, bf16, T, C, K, align_bits) ? 2 : 1;
 }
@@ -590,7 +614,7 @@ int fwd_impl(const void* x, const int32_t* cu, const void* w, const void* b, voi
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if (((uintptr_t)w | (uintptr_t)b) % WE || (uintptr_t)cu % 4) return -NPLM_DWCONV_EALIGN;
     hipStream_t s = (hipStream_t)stream;
-    const int algo = choose_algo(false, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, bits);
+    const int algo = choose_algo(false, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, bits, (uintptr_t)y);
     if (algo < 0) return algo;
     if (algo == 3 || algo == 4) {
         LdsPlan lp;
@@ -660,7 +684,7 @@ int bwd_impl(const void* x, const void* dy, const int32_t* cu, const void* w, vo
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
 
-    int algo = choose_algo(true, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, bits);
+    int algo = choose_algo(true, tune, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, bits, (uintptr_t)dx);
     if (algo < 0) return algo;
     if (algo >= 3 && !(dx && want_red)) {     // these kernels are fused only: a partial request takes the others
         if (tune && tune->algo >= 3) return -NPLM_DWCONV_ETUNING;
@@ -1165,7 +1189,8 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
     if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {
         LdsPlan lp;
         const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 && T >= kMfmaMinRows &&
-                          mfma_tile_fits(C, K, true) && mfma_gated_bwd_preferred(T, taps, S);
+                          mfma_tile_fits(C, K, true) && mfma_lines_ok(true, true, T, C, K, taps, (uintptr_t)dz) &&
+                          mfma_gated_bwd_preferred(T, taps, S);
         rc = mfma ? make_split_plan(false, bf16, T, C, K, nullptr, &lp, true, kMfmaGatedRows, kMfmaGatedCb)
                   : make_split_plan(false, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;
@@ -1271,7 +1296,7 @@ size_t nplm_dwconv_bwd_workspace_bytes(int64_t T, int32_t C, int32_t K, int32_t 
     Plan p;
     if (make_plan(true, bf16, T, C, K, 0, nullptr, &p)) return 0;
     int slabs = p.nbt;
-    if (choose_algo(true, nullptr, bf16, true, T, C, K, K, 1, 0) == 2) {
+    if (choose_algo(true, nullptr, bf16, true, T, C, K, K, 1, 0, 0) == 2) {
         LdsPlan lp;
         if (make_lds_plan(true, bf16, T, C, K, nullptr, &lp) == 0 && lp.nbt > slabs) slabs = lp.nbt;
     }
@@ -1302,7 +1327,7 @@ int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype
     if (check_common(T, C, K, 0, act_dtype, NPLM_DWCONV_F32) || T == 0) return 0;
     K = exec_kernel_size(K);
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
-    const int algo = choose_algo(true, tune, bf16, true, T, C, K, K, 1, 0);
+    const int algo = choose_algo(true, tune, bf16, true, T, C, K, K, 1, 0, 0);
     if (algo < 0) return 0;
     if (algo >= 3) {
         LdsPlan lp;

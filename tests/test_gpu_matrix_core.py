@@ -137,6 +137,32 @@ def test_which_backward_calls_the_matrix_cores_serve(T, n, K, wdt, served):
                        npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(algo=1))[0])
 
 
+# (rows of 128-byte lines or not; outputs below and above the sizes from which the others take over: forward 100 MiB, backward 30)
+@pytest.mark.parametrize("bwd,T,C,K,offset,served", [
+    (False, 53248, 1000, 15, 0, False), (False, 52000, 1000, 15, 0, True), (False, 51200, 1024, 11, 0, True), (False, 53248, 1000, 21, 0, True),
+    (False, 94208, 584, 11, 0, True), (False, 51200, 1024, 11, 16, False),
+    (True, 15768, 1000, 15, 0, False), (True, 15700, 1000, 15, 0, True), (True, 15360, 1024, 15, 0, True), (True, 15768, 1000, 31, 0, True),
+    (True, 59904, 264, 11, 0, True), (True, 15360, 1024, 15, 8, False)])
+def test_which_rows_of_partial_cache_lines_the_matrix_cores_serve(bwd, T, C, K, offset, served):
+    lib = _lib.load()
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x, dy = (torch.empty(T, C, device=DEV, dtype=torch.bfloat16).normal_(generator=g) for _ in range(2))
+    w = torch.empty(C, K, device=DEV, dtype=torch.bfloat16).normal_(0, K ** -0.5, generator=g)
+    cu = cu_from_lengths(torch.tensor([T])).to(DEV)
+    out = torch.empty(T * C + offset, device=DEV, dtype=torch.bfloat16)[offset:].view(T, C)       # (allocations begin on a line)
+    st = torch.cuda.current_stream().cuda_stream
+    if not bwd:
+        _lib.check(lib.nplm_dwconv_fwd(x.data_ptr(), cu.data_ptr(), w.data_ptr(), None, out.data_ptr(), T, C, K, 1, _lib.BF16, _lib.BF16, st), "fwd")
+        assert torch.equal(out, npa.varlen_dwconv_fwd(x, cu, w, None, tuning=_lib.Tuning(algo=4 if served else 2)))
+        return
+    ws = torch.empty(int(lib.nplm_dwconv_bwd_workspace_bytes(T, C, K, _lib.BF16)), dtype=torch.uint8, device=DEV)
+    dw, db = torch.empty(C, K, device=DEV), torch.empty(C, device=DEV)
+    _lib.check(lib.nplm_dwconv_bwd(x.data_ptr(), dy.data_ptr(), cu.data_ptr(), w.data_ptr(), out.data_ptr(), dw.data_ptr(), db.data_ptr(),
+                                   ws.data_ptr(), ws.numel(), T, C, K, 1, _lib.BF16, _lib.BF16, st), "bwd")
+    want = npa.varlen_dwconv_bwd(x, dy, cu, w, tuning=_lib.Tuning(algo=4 if served else 3))
+    assert all(torch.equal(a, c) for a, c in zip((out, dw, db), want))
+
+
 @pytest.mark.parametrize("K,lens,C", [(31, LENS * 2, 512), (29, LENS[::-1] * 2, 520), (25, [4096], 1000), (31, [4095, 1, 63], 648),
                                       (31, LENS * 4, 2056), (31, [1] * 4160, 512), (31, [4095], 512), (31, [16500] + [1] * 200, 512)])
 def test_gated_backward_of_31_taps_matches_the_oracle(K, lens, C):
