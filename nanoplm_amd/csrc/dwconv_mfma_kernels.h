@@ -13,8 +13,9 @@
 // and packs pairs of rows per channel with v_perm_b32 (a 4 x 4 transpose of 16-bit values in registers).
 //
 // Zeros and non-finite values: the band's zeros multiply rows that are not in an output row's taps, so an Inf or NaN there
-// would reach it. Every sum that holds such a product is itself not finite; the kernels test their sums and form the rows
-// of a wave's group again, one product at a time and only the ones that belong, when one is not.
+// would reach it. Every sum that holds such a product is itself not finite; the kernels test their sums and form those of a pass
+// again without the factors that are not finite, then add the products with such factors that belong, one at a time. So sums
+// that none of them belongs to keep their bits, whatever shares a pass with them.
 //
 // Sequence boundaries: one wave of a block leaves for every tile a bit string, one bit per staged row, set where a sequence
 // begins. A wave whose window holds no bit runs unmasked; otherwise every lane finds the rows of its four output rows'
@@ -62,10 +63,21 @@ __device__ __forceinline__ rsrc_t mfma_out_rsrc(void* out, int row0, int rows, i
 constexpr int kMfmaWords = 8;          // 32-bit words of a tile's boundary bits (lanes read up to 2 words past the last row)
 
 // One chunk (four rows) of a lane's Q channels as matrix operands: per channel rows 0, 1 and rows 2, 3.
+// The two bf16 of a dword, zero in the place of one that is not finite.
+__device__ __forceinline__ uint32_t finite_bf16x2(uint32_t v) {
+    const uint32_t bad = ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u;       // sign bit of each half: its exponent is all ones
+    return v & ~((bad << 1) - (bad >> 15));                                     // (the bits spread over their halves)
+}
+__device__ __forceinline__ u32x2 finite_bf16x4(u32x2 v) { return u32x2{finite_bf16x2(v.x), finite_bf16x2(v.y)}; }
+
 template <int Q = kMfmaQ>
 struct MfmaChunk {
     u32x2 b[Q];
     __device__ __forceinline__ s16x4 op(int q) const { return __builtin_bit_cast(s16x4, b[q]); }
+    __device__ __forceinline__ void drop_non_finite() {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) b[q] = finite_bf16x4(b[q]);
+    }
 };
 template <int Q = kMfmaQ> struct MfmaRaw { uint32_t r[4][Q / 2]; };
 
@@ -175,15 +187,15 @@ __device__ __forceinline__ void mfma_columns(MfmaBits v, uint64_t& some, uint64_
     }
 }
 
-// The caller's weight of channel c at tap m of the plan (0 .. KP-1), as the conv takes it (FLIP: the transposed conv of dx).
+// The caller's weight (bf16) of channel c at tap m of the plan (0 .. KP-1), as the conv takes it (FLIP: the transposed conv of dx).
 template <int KP, bool FLIP>
 __device__ __forceinline__ float mfma_weight(const void* __restrict__ w, int w_flags, int c, int m, bool res) {
     const int off = w_tap_off(w_flags), kw = KP - 2 * off;
     const int r = (FLIP ? KP - 1 - m : m) - off;
     float v = 0.f;
     if (r >= 0 && r < kw) {
-        const size_t i = (size_t)c * kw + r;
-        v = (w_flags & W_BF16) ? bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[i]) : reinterpret_cast<const float*>(w)[i];
+        const uint32_t i = (uint32_t)(c * kw + r) * 2;       // bytes (bf16 weights; C * K is below 2^28)
+        v = bf16_to_f32(*reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(w) + i));
     }
     return v + (res && m == (KP - 1) / 2 ? 1.f : 0.f);
 }
@@ -270,6 +282,8 @@ struct MfmaConv {
             bias[q] = 0.f;
             if (b) bias[q] = (w_flags & W_BF16) ? bf16_to_f32(reinterpret_cast<const uint16_t*>(b)[c0 + q]) : reinterpret_cast<const float*>(b)[c0 + q];
         }
+        // here and not at every step, where stores are under way (T=131072, C=1024, 11 taps, 24 rows a sequence: 110 us there, 99)
+        if constexpr (!FLIP) wait_vmem_all();
     }
 
     __device__ __forceinline__ f32x4 start(int q) const {
@@ -278,11 +292,19 @@ struct MfmaConv {
         asm volatile("" : "+v"(b));                          // (else four copies of it stay in registers)
         return f32x4{b, b, b, b};
     }
-    // acc += the products of window chunk k
-    template <int k>
+    // acc += the products of window chunk k (FINITE: without the weights that are not finite)
+    template <int k, bool FINITE = false>
     __device__ __forceinline__ void taps(f32x4 (&acc)[Q], const MfmaChunk<Q>& x) const {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) acc[q] = mfma4(A[k][q], x.op(q), acc[q]);
+        for (int q = 0; q < Q; ++q) {
+            s16x4 w4 = A[k][q];
+            if constexpr (FINITE) {
+                u32x2 t = __builtin_bit_cast(u32x2, w4);
+                asm volatile("" : "+v"(t.x), "+v"(t.y));     // (not formed ahead of the steps and kept in registers)
+                w4 = __builtin_bit_cast(s16x4, finite_bf16x4(t));
+            }
+            acc[q] = mfma4(w4, x.op(q), acc[q]);
+        }
         if constexpr (RES && k >= IDC && k < IDC + IDN) {
 #pragma unroll
             for (int q = 0; q < Q; ++q) acc[q] = mfma4(I[k - IDC], x.op(q), acc[q]);
@@ -357,7 +379,6 @@ struct MfmaConv {
             for (int i = 0; i * 32 < SPAN; ++i) any |= wp[i] & (i == 0 ? ~1u : SPAN - i * 32 >= 32 ? ~0u : (1u << (SPAN & 31)) - 1u);
             open = __builtin_amdgcn_readfirstlane((int)any) == 0;
         }
-        uint32_t redo = 0;                                   // steps whose sums are not all finite
         if (open) {
             float chk = 0.f;
             f32x4 acc[(NCK + 3) / 4][Q];
@@ -394,50 +415,34 @@ struct MfmaConv {
                 });
                 __builtin_amdgcn_sched_barrier(0);
             });
-            if (__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0) redo = (1u << NSTEP) - 1;
-        } else {
+            if (__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) == 0) return;
+        }
 #pragma nounroll
-            for (int s = 0; s < NSTEP; ++s) {
-                const MfmaBits bits = window_bits(wp, s);
-                const char* sp = lp + 16 * s * CB;
-                int i0 = 0;
-                do {
-                    int lo, hi;
-                    mfma_row_bounds(bits, TP::FRONT + (i0 < 4 ? i0 : 3), lo, hi);
-                    const MfmaBits in = mfma_row_mask(lo, hi);
-                    // window rows that some lane's pass takes, and those that every lane's takes (lanes of a column hold the same):
-                    // a chunk that none takes is skipped, one that all take whole needs no mask
-                    uint64_t some, every;
-                    mfma_columns(in, some, every);
-                    f32x4 acc[Q];
+        for (int s = 0; s < NSTEP; ++s) {
+            const MfmaBits bits = window_bits(wp, s);
+            const char* sp = lp + 16 * s * CB;
+            int i0 = 0;
+            do {
+                int lo, hi;
+                mfma_row_bounds(bits, TP::FRONT + (i0 < 4 ? i0 : 3), lo, hi);
+                f32x4 acc[Q];
+                pass<false>(sp, lo, hi, acc);
+                const int i1 = hi - TP::FRONT < 4 ? hi - TP::FRONT : 4;
+                float chk = 0.f;
 #pragma unroll
-                    for (int q = 0; q < Q; ++q) acc[q] = start(q);
-                    MfmaRaw<Q> raw;
-                    read<0>(sp, raw);
-                    static_for<NCK>([&](auto k_c) __attribute__((always_inline)) {
-                        constexpr int k = decltype(k_c)::value;
-                        const MfmaRaw<Q> cur = raw;
-                        if constexpr (k + 1 < NCK)
-                            read<k + 1, (k + 1 == NCK - 1 ? TP::LASTROWS : 4)>(sp, raw);
-                        if ((some >> (4 * k)) & 15) {
-                            MfmaChunk<Q> x;
-                            mfma_pack(cur, x);
-                            if (((every >> (4 * k)) & 15) != 15) {
-                                const uint32_t b4 = 4 * k < 32 ? in.lo >> (4 * k & 31) : in.hi >> (4 * k & 31);
-                                const uint32_t m0 = __builtin_amdgcn_perm((uint32_t)((int)(b4 << 30) >> 31), (uint32_t)((int)(b4 << 31) >> 31), 0x05040100);
-                                const uint32_t m1 = __builtin_amdgcn_perm((uint32_t)((int)(b4 << 28) >> 31), (uint32_t)((int)(b4 << 29) >> 31), 0x05040100);
+                for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(acc[q][0], 0.f, chk);
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0, 0)) {
+                    pass<true>(sp, lo, hi, acc);
+                    const int range = __builtin_amdgcn_ds_bpermute(swap, i0 | i1 << 8);
+#pragma nounroll
+                    for (int i = 0; i < 4; ++i) {
+                        float v[Q];
 #pragma unroll
-                                for (int q = 0; q < Q; ++q) { x.b[q].x &= m0; x.b[q].y &= m1; }
-                            }
-                            taps<k>(acc, x);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    });
-                    const int i1 = hi - TP::FRONT < 4 ? hi - TP::FRONT : 4;
-                    float chk = 0.f;
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(acc[q][0], 0.f, chk);
-                    if (__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0) { redo |= 1u << s; break; }
+                        for (int q = 0; q < Q; ++q) v[q] = i < 2 ? (i == 0 ? acc[q][0] : acc[q][1]) : i == 2 ? acc[q][2] : acc[q][3];
+                        add_non_finite(sp, i, lo, hi, v);
+                        store(ro, i >= (range & 255) && i < (range >> 8) ? out_at : kMfmaNoStore, rowb, up, 16 * s + i, v);
+                    }
+                } else {
                     const int range = __builtin_amdgcn_ds_bpermute(swap, i0 | i1 << 8);     // rows of the pass in the lane that stores them
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -446,44 +451,68 @@ struct MfmaConv {
                         for (int q = 0; q < Q; ++q) v[q] = acc[q][i];
                         store(ro, i >= (range & 255) && i < (range >> 8) ? out_at : kMfmaNoStore, rowb, up, 16 * s + i, v);
                     }
-                    i0 = i0 < 4 ? i1 : 4;
-                } while (__builtin_amdgcn_ballot_w64(i0 < 4) != 0);
-            }
-        }
-        // one product at a time, only the products that belong to the row
-#pragma nounroll
-        for (; redo != 0; redo &= redo - 1) {
-            const int s = __builtin_ctz(redo);
-            exact_step(lp + 16 * s * CB, window_bits(wp, s), ro, rowb, s, up);
+                }
+                i0 = i0 < 4 ? i1 : 4;
+            } while (__builtin_amdgcn_ballot_w64(i0 < 4) != 0);
         }
     }
 
-    // The 16 output rows of a step one product at a time, only the products that belong to them.
-    __device__ __forceinline__ void exact_step(const char* sp, MfmaBits bits, rsrc_t ro, int rowb, int s, const char* up) const {
+    // The sums of a step (sp: its first window row) over the window rows [lo, hi) alone. FINITE: products of finite factors alone.
+    template <bool FINITE>
+    __device__ __forceinline__ void pass(const char* sp, int lo, int hi, f32x4 (&acc)[Q]) const {
+        const MfmaBits in = mfma_row_mask(lo, hi);
+        // window rows that some lane's pass takes, and those that every lane's takes (lanes of a column hold the same):
+        // a chunk that none takes is skipped, one that all take whole needs no mask
+        uint64_t some, every;
+        mfma_columns(in, some, every);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) acc[q] = start(q);
+        MfmaRaw<Q> raw;
+        if constexpr (!FINITE) {
+            read<0>(sp, raw);
+            asm volatile("" ::: "memory");                   // (else the reads move into the first chunk's branch, in front of their use)
+        }
+        static_for<NCK>([&](auto k_c) __attribute__((always_inline)) {
+            constexpr int k = decltype(k_c)::value;
+            if constexpr (FINITE) read<k, (k == NCK - 1 ? TP::LASTROWS : 4)>(sp, raw);      // (rarely run: few registers)
+            const MfmaRaw<Q> cur = raw;
+            if constexpr (!FINITE && k + 1 < NCK)
+                read<k + 1, (k + 1 == NCK - 1 ? TP::LASTROWS : 4)>(sp, raw);
+            if ((some >> (4 * k)) & 15) {
+                MfmaChunk<Q> x;
+                mfma_pack(cur, x);
+                if (((every >> (4 * k)) & 15) != 15) {
+                    const uint32_t b4 = 4 * k < 32 ? in.lo >> (4 * k & 31) : in.hi >> (4 * k & 31);
+                    const uint32_t m0 = __builtin_amdgcn_perm((uint32_t)((int)(b4 << 30) >> 31), (uint32_t)((int)(b4 << 31) >> 31), 0x05040100);
+                    const uint32_t m1 = __builtin_amdgcn_perm((uint32_t)((int)(b4 << 28) >> 31), (uint32_t)((int)(b4 << 29) >> 31), 0x05040100);
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) { x.b[q].x &= m0; x.b[q].y &= m1; }
+                }
+                if constexpr (FINITE) x.drop_non_finite();
+                taps<k, FINITE>(acc, x);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
+    // v += the products of output row 4 n + i of the step that are in its pass's window rows [lo, hi) and have a factor that is not finite
+    __device__ __forceinline__ void add_non_finite(const char* sp, int i, int lo, int hi, float (&v)[Q]) const {
         const int koff = w_tap_off(w_flags), kw = TP::KP - 2 * koff;
         const bool res = (w_flags & W_RESIDUAL) != 0;
 #pragma nounroll
-        for (int i = 0; i < 4; ++i) {
-            int lo, hi;
-            mfma_row_bounds(bits, TP::FRONT + i, lo, hi);
-            float v[Q];
+        for (int m = koff; m < koff + kw; ++m) {
+            const int p = TP::FRONT + i - TP::PP + m;           // window row of tap m
+            if (p < lo || p >= hi || !active) continue;
+            // (the lane's row 4 n + p of the step: its piece is where the chunk of that row has it)
+            const char* a = sp + (off[0] ^ (((((p >> 2) + (SWZ == SWZ_BOTH ? p : 0) + n) & 3) ^ (n & 3)) << 6)) + p * CB;
+            RowVec<true, Q> x;
+            float f[Q];
+            x.load(a);
+            x.to_f32(f);
 #pragma unroll
-            for (int q = 0; q < Q; ++q) v[q] = bias[q];
-#pragma nounroll
-            for (int m = koff; m < koff + kw; ++m) {
-                const int p = TP::FRONT + i - TP::PP + m;       // window row of tap m
-                if (p < lo || p >= hi || !active) continue;
-                // (the lane's row 4 n + p of the step: its piece is where the chunk of that row has it)
-                const char* a = sp + (off[0] ^ (((((p >> 2) + (SWZ == SWZ_BOTH ? p : 0) + n) & 3) ^ (n & 3)) << 6)) + p * CB;
-                RowVec<true, Q> x;
-                float f[Q];
-                x.load(a);
-                x.to_f32(f);
-#pragma unroll
-                for (int q = 0; q < Q; ++q)
-                    v[q] = __builtin_fmaf(mfma_weight<TP::KP, FLIP>(w, w_flags, c0 + q, m, res), f[q], v[q]);
+            for (int q = 0; q < Q; ++q) {
+                const float wq = mfma_weight<TP::KP, FLIP>(w, w_flags, c0 + q, m, res);
+                if (!__builtin_isfinite(f[q]) || !__builtin_isfinite(wq)) v[q] = __builtin_fmaf(wq, f[q], v[q]);
             }
-            store(ro, out_at, rowb, up, 16 * s + i, v);
         }
     }
 };
@@ -572,14 +601,15 @@ dwconv_fwd_mfma_kernel(const void* __restrict__ x, const int32_t* __restrict__ c
 //     D[i][j] += sum over k of x[4c + k - i] * dy_staged[4(c + d + j) + k],  d = 0, 4:  the lag is m = 4 CK0 + 4d + 4j + i
 // so the four lanes of a block hold x at distance one row and dy at distance four rows, and 32 taps (16 at KP = 15) of 16
 // channels take two instructions (one) per four rows. db is the product of dy's chunks with ones. A tile's sums are formed
-// from zero and join the block's when they are finite; otherwise the tile is summed again one product at a time.
+// from zero and join the block's when they are finite; otherwise the tile is summed again without the values that are not, and the
+// products with those are added one at a time (sums that none of them belongs to keep their bits).
 template <int KT>
 struct MfmaDw {
     using TP = MfmaTaps<KT>;
     static constexpr int Q = kMfmaQ, R = 64;
     static constexpr int ND = TP::KP == 15 ? 1 : 2;          // groups of 16 lags
     static constexpr int NCX = R / 4 + 1;                    // x chunks: a lane's rows are shifted by up to 3
-    static constexpr int ROWB = kMfmaCb;
+    static constexpr int ROWB = kMfmaCb, SPAN = R + TP::HALO; // (staged rows)
     f32x4 tot[ND][Q];
     float dbs[Q];              // the lane's share of db
     uint32_t ady[4], ax[4];    // LDS addresses of the lane's slice: of dy chunk c by c & 3, of row k of an x chunk (chunk 0, the tile at hand)
@@ -645,9 +675,64 @@ struct MfmaDw {
         }
     }
 
+    // acc += the sums of a tile with boundaries: one pass per sequence that owns rows of the tile, over the chunks that hold them; the
+    // next chunk is on its way while one is summed. FINITE: products of finite factors alone.
+    template <bool FINITE>
+    __device__ __forceinline__ void passes(uint64_t w0, uint64_t w1, int nrow, f32x4 (&acc)[ND][Q]) const {
+        const uint32_t col = ady[0] ^ (n << 6);              // the lane's address of dy chunk 0 without the permutation of its rows
+        uint32_t m0, m1;
+        int a = sequence_of(w0, w1, TP::FRONT);
+        while (a < TP::FRONT + nrow) {
+            int b = next_sequence(w0, w1, a);
+            if (b > SPAN) b = SPAN;                          // (staged rows end there)
+            const int t0 = a > TP::FRONT ? a - TP::FRONT : 0, t1 = b - TP::FRONT < nrow ? b - TP::FRONT : nrow;
+            const int c1 = (t1 + 2) >> 2;
+            MfmaRaw<Q> rx, rd[ND];
+            auto fetch = [&](int c) __attribute__((always_inline)) {
+                const uint32_t at = (col + 4 * c * ROWB) ^ (((n + c) & 3) << 6);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    u32x2 t = mfma_lds(ax[k] + c * 4 * ROWB);
+                    rx.r[k][0] = t.x; rx.r[k][1] = t.y;
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        t = mfma_lds(at + (16 * d + k) * ROWB);
+                        rd[d].r[k][0] = t.x; rd[d].r[k][1] = t.y;
+                    }
+                }
+            };
+            int c = t0 >> 2;
+            fetch(c);
+#pragma nounroll
+            for (; c <= c1; ++c) {
+                MfmaChunk<Q> x, dy[ND];
+                mfma_pack(rx, x);
+#pragma unroll
+                for (int d = 0; d < ND; ++d) mfma_pack(rd[d], dy[d]);
+                fetch(c < c1 ? c + 1 : c);
+                if (4 * c - 3 < t0 || 4 * c + 3 >= t1) {
+                    row_masks(4 * c - 3, 3 - n, t0, t1, m0, m1);
+                    mask(x, m0, m1);
+                }
+                if constexpr (FINITE) x.drop_non_finite();
+#pragma unroll
+                for (int d = 0; d < ND; ++d) {
+                    const int r0 = 4 * (c + 4 * d);
+                    if (r0 < a || r0 + 16 > b) {
+                        row_masks(r0, 4 * n, a, b, m0, m1);
+                        mask(dy[d], m0, m1);
+                    }
+                    if constexpr (FINITE) dy[d].drop_non_finite();
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) acc[d][q] = mfma4(x.op(q), dy[d].op(q), acc[d][q]);
+                }
+            }
+            a = b;
+        }
+    }
     // words = the tile's boundary bits; nrow = its rows in front of T
     __device__ __forceinline__ void tile(const uint32_t* words, int nrow) {
-        constexpr int SPAN = R + TP::HALO, NR = 4 * (ND - 1) + 1, NCD = NCX + 4 * (ND - 1);
+        constexpr int NR = 4 * (ND - 1) + 1, NCD = NCX + 4 * (ND - 1);
         uint64_t w0, w1;                                     // boundary bits of staged rows 0 .. 63 and 64 on
         {
             uint32_t v[4];
@@ -702,7 +787,6 @@ struct MfmaDw {
                 __builtin_amdgcn_sched_barrier(0);
             });
         } else {
-            const uint32_t col = ady[0] ^ (n << 6);          // the lane's address of dy chunk 0 without the permutation of its rows
             uint32_t m0, m1;
 #pragma nounroll
             for (int c = 0; c < NCX; c += 4) {
@@ -714,54 +798,7 @@ struct MfmaDw {
                 mask(dy, m0, m1);
                 add_db(dy);
             }
-            // one pass per sequence that owns rows of the tile, over the chunks that hold them; the next chunk is on its way
-            // while one is summed
-            int a = sequence_of(w0, w1, TP::FRONT);
-            while (a < TP::FRONT + nrow) {
-                int b = next_sequence(w0, w1, a);
-                if (b > SPAN) b = SPAN;                      // (staged rows end there)
-                const int t0 = a > TP::FRONT ? a - TP::FRONT : 0, t1 = b - TP::FRONT < nrow ? b - TP::FRONT : nrow;
-                const int c1 = (t1 + 2) >> 2;
-                MfmaRaw<Q> rx, rd[ND];
-                auto fetch = [&](int c) __attribute__((always_inline)) {
-                    const uint32_t at = (col + 4 * c * ROWB) ^ (((n + c) & 3) << 6);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        u32x2 t = mfma_lds(ax[k] + c * 4 * ROWB);
-                        rx.r[k][0] = t.x; rx.r[k][1] = t.y;
-#pragma unroll
-                        for (int d = 0; d < ND; ++d) {
-                            t = mfma_lds(at + (16 * d + k) * ROWB);
-                            rd[d].r[k][0] = t.x; rd[d].r[k][1] = t.y;
-                        }
-                    }
-                };
-                int c = t0 >> 2;
-                fetch(c);
-#pragma nounroll
-                for (; c <= c1; ++c) {
-                    MfmaChunk<Q> x, dy[ND];
-                    mfma_pack(rx, x);
-#pragma unroll
-                    for (int d = 0; d < ND; ++d) mfma_pack(rd[d], dy[d]);
-                    fetch(c < c1 ? c + 1 : c);
-                    if (4 * c - 3 < t0 || 4 * c + 3 >= t1) {
-                        row_masks(4 * c - 3, 3 - n, t0, t1, m0, m1);
-                        mask(x, m0, m1);
-                    }
-#pragma unroll
-                    for (int d = 0; d < ND; ++d) {
-                        const int r0 = 4 * (c + 4 * d);
-                        if (r0 < a || r0 + 16 > b) {
-                            row_masks(r0, 4 * n, a, b, m0, m1);
-                            mask(dy[d], m0, m1);
-                        }
-#pragma unroll
-                        for (int q = 0; q < Q; ++q) acc[d][q] = mfma4(x.op(q), dy[d].op(q), acc[d][q]);
-                    }
-                }
-                a = b;
-            }
+            passes<false>(w0, w1, nrow, acc);
         }
         float chk = 0.f;
 #pragma unroll
@@ -773,6 +810,7 @@ struct MfmaDw {
             for (int d = 0; d < ND; ++d)
 #pragma unroll
                 for (int q = 0; q < Q; ++q) acc[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+            passes<true>(w0, w1, nrow, acc);
             int a = sequence_of(w0, w1, TP::FRONT), b = next_sequence(w0, w1, a);
 #pragma nounroll
             for (int t = 0; t < nrow; ++t) {
@@ -796,7 +834,8 @@ struct MfmaDw {
                             row_of(gr, (g0 + r * ROWB) ^ (((r >> 2) & 3) << 6));
                             gr.to_f32(gv);
 #pragma unroll
-                            for (int q = 0; q < Q; ++q) acc[d][q][i] = __builtin_fmaf(xv[q], gv[q], acc[d][q][i]);
+                            for (int q = 0; q < Q; ++q)
+                                if (!__builtin_isfinite(xv[q]) || !__builtin_isfinite(gv[q])) acc[d][q][i] = __builtin_fmaf(xv[q], gv[q], acc[d][q][i]);
                         }
                     }
             }

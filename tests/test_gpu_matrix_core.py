@@ -211,3 +211,73 @@ def test_gated_backward_non_finite_rows_stay_in_their_sequence(which):
         keep[0::3] = False
     assert not bool(torch.isfinite(db[~keep]).any())
     torch.testing.assert_close(db[keep], db0[keep], rtol=0, atol=1e-5 * float(db0.abs().max()))
+
+
+@pytest.mark.parametrize("K", [11, 15, 21, 31])
+@pytest.mark.parametrize("seed", [0, 1, 2, 3])
+def test_what_non_finite_rows_do_not_feed_keeps_its_bits(K, seed):
+    """Inf and NaN in single rows (in front of, between and behind boundaries, in tiles without one) and in whole short sequences:
+    every y, dx, dw and db that no such value belongs to has the bits of the call without them, the others are not finite."""
+    x, cu, w, b, dy = _case(LENS[seed:] + LENS * 2, 512, K, 31 * K + seed)
+    T, P = x.shape[0], (K - 1) // 2
+    seq = torch.searchsorted(cu.long(), torch.arange(T), right=True)
+    bad = torch.zeros(T, 512, dtype=torch.bool)
+    g = torch.Generator().manual_seed(seed)
+    bad[torch.randint(T, (40,), generator=g), torch.randint(512, (40,), generator=g)] = True
+    for i in range(0, cu.numel() - 1, 7):
+        if cu[i + 1] - cu[i] < 10:
+            bad[cu[i]:cu[i + 1], i % 5::5] = True
+    value = torch.where(torch.arange(512) % 3 == 0, float("nan"), float("inf")).bfloat16().expand(T, 512)
+    reach, tap = torch.zeros_like(bad), torch.zeros(512, K, dtype=torch.bool)      # outputs a bad row belongs to; (x[t], dy[t + P - k])
+    for k in range(K):
+        d = k - P
+        o, i = slice(max(0, -d), T - max(0, d)), slice(max(0, d), T - max(0, -d))
+        reach[o] |= bad[i] & (seq[o] == seq[i])[:, None]
+    cud, wd, bd = cu.to(DEV), w.to(DEV), b.to(DEV)
+    tn = _lib.Tuning(**MFMA)
+    same = lambda got, ref, hit: torch.equal(got[~hit], ref[~hit]) and not bool(torch.isfinite(got[hit]).any())
+    xb, dyb = torch.where(bad, value, x), torch.where(bad, value, dy)
+    for res in (False, True):
+        y0, y = (npa.varlen_dwconv_fwd(t.to(DEV), cud, wd, bd, residual=res, tuning=tn) for t in (x, xb))
+        assert same(y, y0, reach.to(DEV))
+        dx0, dw0, db0 = npa.varlen_dwconv_bwd(x.to(DEV), dy.to(DEV), cud, wd, residual=res, tuning=tn)
+        for which in ("x", "dy"):
+            dx, dw, db = npa.varlen_dwconv_bwd((xb if which == "x" else x).to(DEV), (dyb if which == "dy" else dy).to(DEV), cud, wd,
+                                               residual=res, tuning=tn)
+            tap.zero_()
+            for k in range(K):              # dw[k] sums dy[t] * x[t + k - P]
+                d = k - P
+                o, i = slice(max(0, -d), T - max(0, d)), slice(max(0, d), T - max(0, -d))
+                tap[:, k] = (bad[i if which == "x" else o] & (seq[o] == seq[i])[:, None]).any(0)
+            assert same(dw, dw0, tap.to(DEV))
+            assert torch.equal(dx, dx0) if which == "x" else same(dx, dx0, reach.to(DEV))
+            assert torch.equal(db, db0) if which == "x" else same(db, db0, bad.any(0).to(DEV))
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_what_non_finite_rows_do_not_feed_keeps_its_bits_gated(seed):
+    C, K, lens = 512, 31, LENS + [1500, 3, 40, 1, 1, 700]
+    _, cu, w, _, dy = _case(lens, C, K, 100 + seed)
+    T = dy.shape[0]
+    assert T >= 4096
+    g = torch.Generator().manual_seed(seed)
+    z = torch.randn(T, 2 * C, generator=g).bfloat16()
+    bad = torch.zeros(T, C, dtype=torch.bool)
+    bad[torch.randint(T, (30,), generator=g), torch.randint(C, (30,), generator=g)] = True
+    seq = torch.searchsorted(cu.long(), torch.arange(T), right=True)
+    reach, tap = torch.zeros_like(bad), torch.zeros(C, K, dtype=torch.bool)
+    for k in range(K):
+        d = k - K // 2
+        o, i = slice(max(0, -d), T - max(0, d)), slice(max(0, d), T - max(0, -d))
+        reach[o] |= bad[i] & (seq[o] == seq[i])[:, None]
+        tap[:, k] = (bad[o] & (seq[o] == seq[i])[:, None]).any(0)
+    cud, wd = cu.to(DEV), w.to(DEV)
+    dz0, dw0, db0 = npa.gated_dwconv_bwd(z.to(DEV), dy.to(DEV), cud, wd)
+    dz, dw, db = npa.gated_dwconv_bwd(z.to(DEV), dy.masked_fill(bad, float("inf")).to(DEV), cud, wd)
+    for half in (slice(0, C), slice(C, None)):
+        keep = ~reach.to(DEV)
+        assert torch.equal(dz[:, half][keep], dz0[:, half][keep])
+    assert not bool(torch.isfinite(dz[:, :C][reach.to(DEV)]).any())
+    assert torch.equal(dw[~tap.to(DEV)], dw0[~tap.to(DEV)]) and not bool(torch.isfinite(dw[tap.to(DEV)]).any())
+    col = bad.any(0).to(DEV)
+    assert torch.equal(db[~col], db0[~col]) and not bool(torch.isfinite(db[col]).any())
