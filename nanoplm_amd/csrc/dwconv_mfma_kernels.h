@@ -200,23 +200,39 @@ __device__ __forceinline__ float mfma_weight(const void* __restrict__ w, int w_f
     return v + (res && m == (KP - 1) / 2 ? 1.f : 0.f);
 }
 
-// Weight table of a column block in LDS, [channel][WSTR] dwords of two bf16: entry e of a channel is plan tap e - 4 + 4 CK0.
-template <int KT, bool FLIP, int CH = kMfmaCh>
-__device__ __forceinline__ void mfma_fill_weights(uint32_t* tab, const void* __restrict__ w, int w_flags, int ch0, int nch, int tid, int nthreads) {
+// Weight table of a column block in LDS, [channel][WSTR] dwords of two bf16: entry e of a channel is plan tap e - 4 + 4 CK0. Behind it
+// one word of each of the NW waves that fill it, not zero where it met a weight that is not finite.
+template <int KT, int CH, int NW>
+struct MfmaWeights {
     using TP = MfmaTaps<KT>;
-    for (int i = tid; i < CH * TP::WSTR; i += nthreads) {
-        const int c = i / TP::WSTR, p = i - c * TP::WSTR;
-        uint32_t t = 0;
-        if (c < nch) {
+    static constexpr int MARKS_AT = CH * TP::WSTR, BYTES = (MARKS_AT + NW) * 4;
+    template <bool FLIP>
+    __device__ __forceinline__ static void fill(uint32_t* tab, const void* __restrict__ w, int w_flags, int ch0, int nch, int tid) {
+        bool odd = false;
+        for (int i = tid; i < CH * TP::WSTR; i += NW * 64) {
+            const int c = i / TP::WSTR, p = i - c * TP::WSTR;
+            uint32_t t = 0;
+            if (c < nch) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int m = 2 * p + h - 4 + 4 * TP::CK0;
-                if (m >= 0 && m < TP::KP) t |= (__float_as_uint(mfma_weight<TP::KP, FLIP>(w, w_flags, ch0 + c, m, false)) >> 16) << (16 * h);
+                for (int h = 0; h < 2; ++h) {
+                    const int m = 2 * p + h - 4 + 4 * TP::CK0;
+                    if (m >= 0 && m < TP::KP) t |= (__float_as_uint(mfma_weight<TP::KP, FLIP>(w, w_flags, ch0 + c, m, false)) >> 16) << (16 * h);
+                }
             }
+            odd |= finite_bf16x2(t) != t;
+            tab[i] = t;
         }
-        tab[i] = t;
+        const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
+        if ((tid & 63) == 0) tab[MARKS_AT + tid / 64] = any ? 1 : 0;
     }
-}
+    // whether one of the block's weights is not finite (after the barrier that follows fill())
+    __device__ __forceinline__ static bool odd(const uint32_t* tab) {
+        uint32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) any |= tab[MARKS_AT + i];
+        return __builtin_amdgcn_readfirstlane((int)any) != 0;
+    }
+};
 
 // One wave's conv over staged rows: 16 Q channels, groups of 16 NSTEP output rows. FLIP: dx from dy. RES: the identity is one
 // more band (a single 1 per row), since a bf16 weight plus one is not one in bf16.
@@ -241,10 +257,12 @@ struct MfmaConv {
     int swap;              // stores: the lane whose output goes out through this one (x 4)
     int out_at;            // byte offset of that lane's slice of output row 4 n, or kMfmaNoStore
     bool active;
+    bool odd;              // a weight of the block is not finite
     const void* w;
     int w_flags;
 
-    __device__ __forceinline__ void init(const uint32_t* tab, const void* w_, int w_flags_, const void* b, int wc, int lane, int ch0, int nch, int rowb) {
+    __device__ __forceinline__ void init(const uint32_t* tab, bool odd_, const void* w_, int w_flags_, const void* b, int wc, int lane, int ch0, int nch, int rowb) {
+        odd = odd_;
         n = lane & 3;
         const int blk = lane >> 2;
         const int lc = (wc * 16 + blk) * Q;
@@ -431,7 +449,8 @@ struct MfmaConv {
                 float chk = 0.f;
 #pragma unroll
                 for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(acc[q][0], 0.f, chk);
-                if (__builtin_expect(__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0, 0)) {
+                // (a row that is not finite meets all four sums; a weight meets each in another chunk, and chunks are left out here)
+                if (__builtin_expect(odd || __builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0, 0)) {
                     pass<true>(sp, lo, hi, acc);
                     const int range = __builtin_amdgcn_ds_bpermute(swap, i0 | i1 << 8);
 #pragma nounroll
@@ -530,7 +549,8 @@ struct MfmaFwdShape {
     static constexpr int R = kMfmaFwdRows, RW = R / NRG, NROWS = R + TP::HALO;
     static constexpr int BUF_BYTES = NROWS * kMfmaCb;
     static constexpr int TAB_AT = 2 * BUF_BYTES + 2 * kMfmaWords * 4;      // two tiles, their boundary bits, the weight table
-    static constexpr int LDS_BYTES = TAB_AT + kMfmaCh * TP::WSTR * 4;
+    using W = MfmaWeights<KT, kMfmaCh, NWC>;
+    static constexpr int LDS_BYTES = TAB_AT + W::BYTES;
     static_assert(LDS_BYTES <= kLdsBytes, "fits the LDS");
     static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords, "lanes read two words past the one of their window's first row");
 };
@@ -582,10 +602,10 @@ dwconv_fwd_mfma_kernel(const void* __restrict__ x, const int32_t* __restrict__ c
     }
     const int wc = wv % SH::NCW, r0 = wv / SH::NCW * SH::RW;
     const int nch = valid_bytes / 2;
-    mfma_fill_weights<KT, false>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x, SH::NWC * 64);
+    SH::W::template fill<false>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x);
     lds_barrier();
     MfmaConv<KT, SH::RW / 16, false, RES> conv;
-    conv.init(tab, w, g.w_flags, bias, wc, lane, cb * kMfmaCh, nch, rowb);
+    conv.init(tab, SH::W::odd(tab), w, g.w_flags, bias, wc, lane, cb * kMfmaCh, nch, rowb);
     for (int it = 0; it < ntl; ++it) {
         lds_barrier();
         const int tf = lds_tile_row0(g, it, q, R) + r0;
@@ -905,7 +925,8 @@ struct MfmaBwdShape {
     static constexpr int LDS_BYTES = 2 * BUF_BYTES + 4 * kMfmaCb;
     static_assert(2 * kMfmaWords * 4 <= 4 * kMfmaCb, "room for the boundary bits");
     static_assert(LDS_BYTES <= kLdsBytes, "two pairs of tiles fit the LDS");
-    static_assert(kMfmaCh * TP::WSTR * 4 <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
+    using W = MfmaWeights<KT, kMfmaCh, NWC>;
+    static_assert(W::BYTES <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
     static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords && NROWS <= 96, "boundary bits");
 };
 
@@ -955,11 +976,11 @@ dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, 
         }
         return;
     }
-    mfma_fill_weights<KT, true>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x, SH::NWC * 64);
+    SH::W::template fill<true>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x);
     lds_barrier();
     if (wv < SH::NDX) {
         MfmaConv<KT, R / 16, true, RES> conv;
-        conv.init(tab, w, g.w_flags, nullptr, wv, lane, cb * kMfmaCh, nch, rowb);
+        conv.init(tab, SH::W::odd(tab), w, g.w_flags, nullptr, wv, lane, cb * kMfmaCh, nch, rowb);
         lds_barrier();
         for (int it = 0; it < ntl; ++it) {
             lds_barrier();
@@ -1180,7 +1201,8 @@ struct MfmaGatedBwdShape {
     static_assert(CH == 128, "a dw wave has two channels per lane");
     static_assert(NDW == 8 && NDW / 2 * GatedDw<KT>::BOX * 4 <= WORDS_AT, "half of the sums in the buffers");
     static_assert(LDS_BYTES <= kLdsBytes, "two buffers of three tiles and the terms of h fit the LDS");
-    static_assert(CH * TP::WSTR * 4 <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
+    using W = MfmaWeights<KT, CH, NWC>;
+    static_assert(W::BYTES <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
     static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords && NROWS <= 96, "boundary bits");
 };
 
@@ -1232,12 +1254,12 @@ dwconv_bwd_gated_mfma_kernel(const void* __restrict__ z, const void* __restrict_
         for (int k = 0; k < 6; ++k) lds_barrier();      // (the dw waves join their sums)
         return;
     }
-    mfma_fill_weights<KT, true, SH::CH>(tab, w, g.w_flags, cb * SH::CH, nch, (int)threadIdx.x, SH::NWC * 64);
+    SH::W::template fill<true>(tab, w, g.w_flags, cb * SH::CH, nch, (int)threadIdx.x);
     lds_barrier();
     if (wv < SH::NDZ) {
         __builtin_amdgcn_s_setprio(2);       // a dz wave has the longest way through a tile (log-normal lengths: 682 us without, 673 with)
         MfmaConv<KT, R / 16, true, RES, true> conv;
-        conv.init(tab, w, g.w_flags, nullptr, wv, lane, cb * SH::CH, nch, rowb);
+        conv.init(tab, SH::W::odd(tab), w, g.w_flags, nullptr, wv, lane, cb * SH::CH, nch, rowb);
         lds_barrier();
         for (int it = 0; it < ntl; ++it) {
             lds_barrier();

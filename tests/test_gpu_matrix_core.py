@@ -281,3 +281,39 @@ def test_what_non_finite_rows_do_not_feed_keeps_its_bits_gated(seed):
     assert torch.equal(dw[~tap.to(DEV)], dw0[~tap.to(DEV)]) and not bool(torch.isfinite(dw[tap.to(DEV)]).any())
     col = bad.any(0).to(DEV)
     assert torch.equal(db[~col], db0[~col]) and not bool(torch.isfinite(db[col]).any())
+
+
+@pytest.mark.parametrize("K", [11, 15, 21, 31])
+def test_a_non_finite_weight_meets_the_rows_of_its_tap_only(K):
+    """Weights of Inf and NaN at one tap of every fifth channel, sequences of one row and a few among them: outputs whose sequence
+    has no row at that tap are those of a zero weight, bit for bit. Forward, dx and the gated dz."""
+    lens = [1] * 300 + LENS + [1, 2, 3, 1, 4, 1, 1, 5] * 40 + [500, 1, 1, 900, 2, 460]
+    C = 512
+    x, cu, w, b, dy = _case(lens, C, K, K)
+    T = x.shape[0]
+    assert T >= 4096
+    odd = w.clone()
+    for c in range(0, C, 5):
+        odd[c, c // 5 % K] = float("nan") if c % 2 else float("inf")
+    seq = torch.searchsorted(cu.long(), torch.arange(T), right=True)
+    fwd, bwd = torch.zeros(T, C, dtype=torch.bool), torch.zeros(T, C, dtype=torch.bool)      # outputs that such a weight belongs to
+    for k in range(K):
+        d = k - K // 2
+        o, i = slice(max(0, -d), T - max(0, d)), slice(max(0, d), T - max(0, -d))
+        both = (seq[o] == seq[i])[:, None] & ~torch.isfinite(odd[:, k])
+        fwd[o] |= both              # y[t] takes w[k] from x[t + d], dx[t + d] takes it from dy[t]
+        bwd[i] |= both
+    zeros = torch.where(torch.isfinite(odd), odd, 0.0)
+    xd, dyd, cud, od, zd, bd, fwd, bwd = (t.to(DEV) for t in (x, dy, cu, odd, zeros, b, fwd, bwd))
+    tn = _lib.Tuning(**MFMA)
+    g = torch.randn(T, 2 * C, generator=torch.Generator().manual_seed(K)).bfloat16().to(DEV)
+    for res in (False, True):
+        y, y0 = (npa.varlen_dwconv_fwd(xd, cud, v, bd, residual=res, tuning=tn) for v in (od, zd))
+        (dx, dw, db), (dx0, dw0, db0) = (npa.varlen_dwconv_bwd(xd, dyd, cud, v, residual=res, tuning=tn) for v in (od, zd))
+        for got, want, hit in ((y, y0, fwd), (dx, dx0, bwd)):
+            assert torch.equal(got[~hit], want[~hit]) and not bool(torch.isfinite(got[hit]).any())
+        assert torch.equal(dw, dw0) and torch.equal(db, db0)
+        if K == 31:
+            dz, dz0 = (npa.gated_dwconv_bwd(g, dyd, cud, v, residual=res)[0] for v in (od, zd))
+            assert torch.equal(dz[:, :C][~bwd], dz0[:, :C][~bwd]) and torch.equal(dz[:, C:][~bwd], dz0[:, C:][~bwd])
+            assert not bool(torch.isfinite(dz[:, :C][bwd]).any())
