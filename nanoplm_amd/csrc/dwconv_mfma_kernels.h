@@ -64,8 +64,9 @@ constexpr int kMfmaWords = 8;          // 32-bit words of a tile's boundary bits
 
 // One chunk (four rows) of a lane's Q channels as matrix operands: per channel rows 0, 1 and rows 2, 3.
 // The two bf16 of a dword, zero in the place of one that is not finite.
+__device__ __forceinline__ uint32_t non_finite_bf16x2(uint32_t v) { return ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u; }
 __device__ __forceinline__ uint32_t finite_bf16x2(uint32_t v) {
-    const uint32_t bad = ((v & 0x7f807f80u) + 0x00800080u) & 0x80008000u;       // sign bit of each half: its exponent is all ones
+    const uint32_t bad = non_finite_bf16x2(v);                                  // sign bit of each half: its exponent is all ones
     return v & ~((bad << 1) - (bad >> 15));                                     // (the bits spread over their halves)
 }
 __device__ __forceinline__ u32x2 finite_bf16x4(u32x2 v) { return u32x2{finite_bf16x2(v.x), finite_bf16x2(v.y)}; }
@@ -208,7 +209,7 @@ struct MfmaWeights {
     static constexpr int MARKS_AT = CH * TP::WSTR, BYTES = (MARKS_AT + NW) * 4;
     template <bool FLIP>
     __device__ __forceinline__ static void fill(uint32_t* tab, const void* __restrict__ w, int w_flags, int ch0, int nch, int tid) {
-        bool odd = false;
+        uint32_t odd = 0;
         for (int i = tid; i < CH * TP::WSTR; i += NW * 64) {
             const int c = i / TP::WSTR, p = i - c * TP::WSTR;
             uint32_t t = 0;
@@ -219,18 +220,18 @@ struct MfmaWeights {
                     if (m >= 0 && m < TP::KP) t |= (__float_as_uint(mfma_weight<TP::KP, FLIP>(w, w_flags, ch0 + c, m, false)) >> 16) << (16 * h);
                 }
             }
-            odd |= finite_bf16x2(t) != t;
+            odd |= non_finite_bf16x2(t);
             tab[i] = t;
         }
-        const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
+        const bool any = __builtin_amdgcn_ballot_w64(odd != 0) != 0;
         if ((tid & 63) == 0) tab[MARKS_AT + tid / 64] = any ? 1 : 0;
     }
     // whether one of the block's weights is not finite (after the barrier that follows fill())
-    __device__ __forceinline__ static bool odd(const uint32_t* tab) {
+    __device__ __forceinline__ static uint64_t odd(const uint32_t* tab) {
         uint32_t any = 0;
 #pragma unroll
         for (int i = 0; i < NW; ++i) any |= tab[MARKS_AT + i];
-        return __builtin_amdgcn_readfirstlane((int)any) != 0;
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)any);
     }
 };
 
@@ -257,11 +258,11 @@ struct MfmaConv {
     int swap;              // stores: the lane whose output goes out through this one (x 4)
     int out_at;            // byte offset of that lane's slice of output row 4 n, or kMfmaNoStore
     bool active;
-    bool odd;              // a weight of the block is not finite
+    uint64_t odd;          // not zero: a weight of the block is not finite
     const void* w;
     int w_flags;
 
-    __device__ __forceinline__ void init(const uint32_t* tab, bool odd_, const void* w_, int w_flags_, const void* b, int wc, int lane, int ch0, int nch, int rowb) {
+    __device__ __forceinline__ void init(const uint32_t* tab, uint64_t odd_, const void* w_, int w_flags_, const void* b, int wc, int lane, int ch0, int nch, int rowb) {
         odd = odd_;
         n = lane & 3;
         const int blk = lane >> 2;
@@ -450,7 +451,7 @@ struct MfmaConv {
 #pragma unroll
                 for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(acc[q][0], 0.f, chk);
                 // (a row that is not finite meets all four sums; a weight meets each in another chunk, and chunks are left out here)
-                if (__builtin_expect(odd || __builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0, 0)) {
+                if (__builtin_expect((odd | __builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk))) != 0, 0)) {
                     pass<true>(sp, lo, hi, acc);
                     const int range = __builtin_amdgcn_ds_bpermute(swap, i0 | i1 << 8);
 #pragma nounroll
