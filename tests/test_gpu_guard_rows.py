@@ -149,3 +149,55 @@ def test_layernorm_fused_conv_writes_its_outputs_only(C, K, dt):
     # ln_dwconv_bwd returns dx, d ln_weight, d ln_bias, dw, db
     for got, want, what in zip((dx, dg, dbt, dw, db), ref, ("dx", "d ln_weight", "d ln_bias", "dw", "db")):
         got.check(want, "layernorm " + what)
+
+
+# ---- the matrix-core kernels: from 4096 rows on, few sequences; a last tile of 1, 3 and 63 rows, partial column blocks ----
+def _long_inputs(T, C, K, seed, width=1):
+    g = torch.Generator().manual_seed(seed)
+    lens = [1300, 1, 17, 700, T - 2019, 1]
+    x = torch.randn(T, width * C, generator=g).bfloat16().to(DEV)
+    dy = torch.randn(T, C, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(C, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    b = (torch.randn(C, generator=g) * 0.02).bfloat16().to(DEV)
+    return x, dy, cu_from_lengths(torch.tensor(lens)).to(DEV), w, b
+
+
+@pytest.mark.parametrize("T,C,K", [(4097, 264, 11), (4099, 520, 15), (4159, 264, 21), (4097, 520, 31), (4099, 2048, 31), (4159, 1000, 31),
+                                   (4161, 256, 15), (4163, 512, 11), (4223, 648, 21)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_matrix_core_kernels_write_their_outputs_only(T, C, K, residual):
+    print(f"[case] guard rows, matrix cores T={T} C={C} K={K} residual={residual}", flush=True)
+    lib = _lib.load()
+    x, dy, cu, w, b = _long_inputs(T, C, K, T + C + K)
+    S, flags, code = cu.numel() - 1, _lib.RESIDUAL if residual else 0, _lib.BF16
+    stream = torch.cuda.current_stream().cuda_stream
+    tn = _lib.Tuning(algo=4)
+    y_ref = npa.varlen_dwconv_fwd(x, cu, w, b, residual=residual, tuning=tn)
+    dx_ref, dw_ref, db_ref = npa.varlen_dwconv_bwd(x, dy, cu, w, residual=residual, tuning=tn)
+    y, dx = Guarded(T, C, torch.bfloat16), Guarded(T, C, torch.bfloat16)
+    dw, db = Guarded(C * K, 1, torch.float32), Guarded(C, 1, torch.float32)
+    _lib.check(lib.nplm_dwconv_fwd_ex(x.data_ptr(), cu.data_ptr(), w.data_ptr(), b.data_ptr(), y.ptr(), T, C, K, S, code, code, flags, stream),
+               "nplm_dwconv_fwd_ex")
+    y.check(y_ref, "y")
+    ws = torch.empty(int(lib.nplm_dwconv_bwd_workspace_bytes(T, C, K, code)), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.nplm_dwconv_bwd_ex(x.data_ptr(), dy.data_ptr(), cu.data_ptr(), w.data_ptr(), dx.ptr(), dw.ptr(), db.ptr(), ws.data_ptr(),
+                                      ws.numel(), T, C, K, S, code, code, flags, stream), "nplm_dwconv_bwd_ex")
+    dx.check(dx_ref, "dx")
+    dw.check(dw_ref, "dw")
+    db.check(db_ref, "db")
+
+
+@pytest.mark.parametrize("T,C", [(4097, 520), (4099, 1024), (4159, 648), (4161, 1152)])
+def test_gated_matrix_core_backward_writes_its_outputs_only(T, C):
+    print(f"[case] guard rows, gated matrix cores T={T} C={C}", flush=True)
+    lib, K, code = _lib.load(), 31, _lib.BF16
+    z, dy, cu, w, b = _long_inputs(T, C, K, T + C, width=2)
+    stream = torch.cuda.current_stream().cuda_stream
+    dz_ref, dw_ref, db_ref = npa.gated_dwconv_bwd(z, dy, cu, w)
+    dz, dw, db = Guarded(T, 2 * C, torch.bfloat16), Guarded(C * K, 1, torch.float32), Guarded(C, 1, torch.float32)
+    ws = torch.empty(int(lib.nplm_dwconv_gated_bwd_workspace_bytes(T, C, K, code)), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.nplm_dwconv_gated_bwd(z.data_ptr(), dy.data_ptr(), cu.data_ptr(), w.data_ptr(), dz.ptr(), dw.ptr(), db.ptr(), ws.data_ptr(),
+                                         ws.numel(), T, C, K, cu.numel() - 1, code, code, 0, stream), "nplm_dwconv_gated_bwd")
+    dz.check(dz_ref, "dz")
+    dw.check(dw_ref, "gated dw")
+    db.check(db_ref, "gated db")

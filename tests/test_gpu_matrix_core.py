@@ -317,3 +317,56 @@ def test_a_non_finite_weight_meets_the_rows_of_its_tap_only(K):
             dz, dz0 = (npa.gated_dwconv_bwd(g, dyd, cud, v, residual=res)[0] for v in (od, zd))
             assert torch.equal(dz[:, :C][~bwd], dz0[:, :C][~bwd]) and torch.equal(dz[:, C:][~bwd], dz0[:, C:][~bwd])
             assert not bool(torch.isfinite(dz[:, :C][bwd]).any())
+
+
+@pytest.mark.parametrize("K,C", [(15, 512), (31, 264)])
+@pytest.mark.parametrize("seq_len,nbt", [(64, 0), (96, 24), (17, 10), (512, 7)])
+def test_equal_length_sequences_on_rotating_tile_slots(K, C, seq_len, nbt):
+    """Boundaries at a fixed period of tiles, grids whose last round is partial, empty sequences behind the last row."""
+    T = 2700
+    x, cu, w, b, dy = _case([seq_len] * (T // seq_len) + [T % seq_len] + [0] * 300, C, K, K + seq_len)
+    xd, cud, wd, dyd = x.to(DEV), cu.to(DEV), w.to(DEV), dy.to(DEV)
+    tn = _lib.Tuning(nbt=nbt, **MFMA)
+    assert_act_close(npa.varlen_dwconv_fwd(xd, cud, wd, b.to(DEV), tuning=tn), O.c_oracle_fwd(x, cu, w, b), torch.bfloat16, "y")
+    dx64, dw64, db64 = O.c_oracle_bwd(x, dy, cu, w)
+    dx, dw, db = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=tn)
+    assert_act_close(dx, dx64, torch.bfloat16, "dx")
+    assert_red_close(dw, dw64, "dw")
+    assert_red_close(db, db64, "db")
+
+
+def test_empty_sequences_do_not_change_the_bits():
+    """In front of the rows, between sequences and behind them, thousands at a time: the kernels mark the same starts."""
+    x, cu, w, b, dy = _case(LENS * 2, 512, 31, 8)
+    lens = []
+    for i, n in enumerate(LENS * 2):
+        lens += [n] + [0] * (3000 if i in (0, 7, 40) else i % 3)
+    many = cu_from_lengths(torch.tensor([0] * 5000 + lens + [0] * 20000))
+    xd, wd, bd, dyd, tn = x.to(DEV), w.to(DEV), b.to(DEV), dy.to(DEV), _lib.Tuning(**MFMA)
+    assert torch.equal(npa.varlen_dwconv_fwd(xd, cu.to(DEV), wd, bd, tuning=tn), npa.varlen_dwconv_fwd(xd, many.to(DEV), wd, bd, tuning=tn))
+    one, two = (npa.varlen_dwconv_bwd(xd, dyd, c.to(DEV), wd, tuning=tn) for c in (cu, many))
+    assert all(torch.equal(a, c) for a, c in zip(one, two))
+
+
+def test_rows_beyond_2_and_4_gib_offsets():
+    """1.1 M rows x 4 KiB: row offsets cross 2^31 and 2^32 bytes. Whole sequences cut out of the batch give the same y and dx alone:
+    their first row is a multiple of four, which is what the order of a row's sums goes by."""
+    T, C, K = 1_100_000, 2048, 31
+    g = torch.Generator().manual_seed(78)
+    lens = 4 * torch.randint(5, 129, (T // 200,), generator=g)
+    lens = lens[torch.cumsum(lens, 0) <= T]
+    cu = cu_from_lengths(torch.cat([lens, torch.tensor([T - int(lens.sum())])])).to(DEV)
+    x, dy = (torch.randn(T, C, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    w = (torch.randn(C, K, device=DEV) * K ** -0.5).bfloat16()
+    tn = _lib.Tuning(**MFMA)
+    y = npa.varlen_dwconv_fwd(x, cu, w, None)
+    dx, _, db = npa.varlen_dwconv_bwd(x, dy, cu, w)
+    cul = cu.tolist()
+    S = len(cul) - 1
+    assert cul[S // 2] * C * 2 > 2 ** 31 and cul[S - 40] * C * 2 > 2 ** 32
+    for first in (0, S // 2 - 20, S - 40):
+        s, e = cul[first], cul[first + 40]
+        sub = (cu[first:first + 41] - s).contiguous()
+        assert torch.equal(y[s:e], npa.varlen_dwconv_fwd(x[s:e], sub, w, None, tuning=tn)), f"rows {s}..{e}"
+        assert torch.equal(dx[s:e], npa.varlen_dwconv_bwd(x[s:e], dy[s:e], sub, w, tuning=tn)[0]), f"rows {s}..{e}"
+    torch.testing.assert_close(db, dy.float().sum(0), rtol=2e-5, atol=0.05)

@@ -79,3 +79,30 @@ def test_random_case_matches_oracle(case):
     assert_act_close(dx, dx64, dt, "dx")
     assert_red_close(dw, dw64, "dw")
     assert_red_close(db, db64, "db")
+
+
+def _matrix_core_cases():
+    rng = random.Random(20260608)
+    return [(i, rng.choice([11, 13, 15, 17, 21, 25, 31, 31]), rng.choice([256, 264, 320, 512, 520, 768, 1000, 1024, 2048]),
+             _lengths(rng, rng.choice([60, 700, 4200, 9000])), rng.choice([0, 0, 1, 5]), rng.random() < 0.4, rng.random() < 0.8) for i in range(32)]
+
+
+@pytest.mark.parametrize("case", _matrix_core_cases(), ids=lambda c: f"{c[0]}-K{c[1]}-C{c[2]}-nbt{c[4]}")
+def test_random_case_on_the_matrix_cores_matches_oracle(case):
+    i, K, C, lens, nbt, residual, with_bias = case
+    print(f"[case] matrix cores #{i} K={K} C={C} nbt={nbt} residual={residual} S={len(lens)} T={sum(lens)}", flush=True)
+    g = torch.Generator().manual_seed(2000 + i)
+    T = sum(lens)
+    x, dy = (torch.randn(T, C, generator=g).bfloat16() for _ in range(2))
+    w = (torch.randn(C, K, generator=g) * K ** -0.5).bfloat16()
+    b = (torch.randn(C, generator=g) * 0.02).bfloat16() if with_bias else None
+    cu = cu_from_lengths(torch.tensor(lens))
+    xd, dyd, wd, cud = x.to(DEV), dy.to(DEV), w.to(DEV), cu.to(DEV)
+    tn = _lib.Tuning(algo=4, nbt=nbt)
+    y = npa.varlen_dwconv_fwd(xd, cud, wd, None if b is None else b.to(DEV), residual=residual, tuning=tn)
+    dx, dw, db = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, residual=residual, tuning=tn)
+    dx64, dw64, db64 = O.c_oracle_bwd(x, dy, cu, w, residual=residual)
+    assert_act_close(y, O.c_oracle_fwd(x, cu, w, b, residual=residual), torch.bfloat16, "y")
+    assert_act_close(dx, dx64, torch.bfloat16, "dx")
+    assert_red_close(dw, dw64, "dw")
+    assert_red_close(db, db64, "db")

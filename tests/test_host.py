@@ -256,6 +256,16 @@ def test_boundary_walk_does_not_walk_runs_of_empty_sequences(front, inside, tail
         assert reads <= 4 + 4 * 5
 
 
+def test_boundary_walk_ends_on_malformed_cu():
+    rng = np.random.default_rng(4)
+    for _ in range(50):
+        cu = rng.integers(-2 ** 31, 2 ** 31, size=rng.integers(1, 2000)).astype(np.int32)
+        words = np.zeros(8, dtype=np.uint32)
+        for a in (-15, 0, 1000, 2 ** 31 - 2 ** 20 - 64):
+            reads = _lib.load().nplm_dwconv_debug_starts(cu.ctypes.data, len(cu) - 1, 2 ** 31 - 2 ** 20 - 1, a, 94, words.ctypes.data)
+            assert 1 <= reads <= 5 * len(cu)
+
+
 # ---- Python surface -----------------------------------------------------------------------------
 def test_cpu_tensors_are_refused():
     x = torch.randn(10, 8)
