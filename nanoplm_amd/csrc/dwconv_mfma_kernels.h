@@ -116,8 +116,9 @@ __device__ __forceinline__ void mfma_stage(const void* __restrict__ src, char* d
     const rsrc_t rs = rows_rsrc(src, rb, T, row_bytes);
     const int rowb = (int)row_bytes;
     const int lrow = lane / (CB / 16), lpiece = lane % (CB / 16);
-    // rows outside [0, T) are not clamped: their offsets fall outside the descriptor (or, on a tensor beyond 4 GiB, on other
-    // rows of it), and what lands in LDS for them is never used
+    // Rows outside [0, T) are not clamped. Those from T on lie outside the descriptor, which ends with the tensor's last row, and land
+    // as zeros: GatedDw's sums take them in (dy to db, h and dy to a sequence of their own). The offsets of rows in front of 0
+    // fall outside the descriptor too, or, on a tensor beyond 4 GiB, on other rows of it: what lands for them is never used.
 #pragma unroll
     for (int i = 0; i < CNT; ++i) {
         const int gi = lw + i * NLW < NL ? lw + i * NLW : NL - 1;
@@ -1018,68 +1019,39 @@ dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, 
 // by the execution mask, not multiplied by zero (their product may be with an Inf). In one instruction block: sums that two
 // branches of compiled code change come to lie in two sets of registers (56 spilled). The masked form lies behind the section's
 // other code, so that the usual one runs on without a jump (T=131072, C=2048, 31 taps, one sequence: 699 us with one, 627).
+#define NPLM_ROW_FMAC(i) "v_fmac_f32 %[a" #i "], %[h" #i "], %[d0]\n\tv_fmac_f32 %[b" #i "], %[g" #i "], %[d1]\n\t"
+#define NPLM_ROW_SOME(i) "s_bitcmp1_b32 %[in], " #i "\n\ts_cselect_b64 exec, -1, 0\n\t" NPLM_ROW_FMAC(i)
+#define NPLM_ROW_OUT(i) [a##i] "+v"(a[-i][0]), [b##i] "+v"(a[-i][1])
+#define NPLM_ROW_IN(i) [h##i] "v"(h[i][0]), [g##i] "v"(h[i][1])
+#define NPLM_FMAC_ROWS(ALL, FMAC, SOME, OUT, ...)                                                                              \
+    asm volatile("s_and_b32 %[t], %[in], " #ALL "\n\ts_cmp_eq_u32 %[t], " #ALL "\n\ts_cbranch_scc0 .Lsome%=\n\t" FMAC          \
+                 ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t" SOME "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"   \
+                 : [t] "=&s"(t), OUT : [in] "s"(in), __VA_ARGS__, [d0] "v"(d0), [d1] "v"(d1) : "scc")
+#define NPLM_COMMA ,
 template <int N>
 __device__ __forceinline__ void fmac_rows(float (*a)[2], const float (*h)[2], float d0, float d1, uint32_t in) {
+    static_assert(N >= 1 && N <= 4, "rows of a block");
     uint32_t t;
     if constexpr (N == 1)
-        asm volatile("s_and_b32 %[t], %[in], 1\n\ts_cmp_eq_u32 %[t], 1\n\ts_cbranch_scc0 .Lsome%=\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
-                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
-                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1])
-                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [d0] "v"(d0), [d1] "v"(d1)
-                     : "scc");
+        NPLM_FMAC_ROWS(1, NPLM_ROW_FMAC(0), NPLM_ROW_SOME(0), NPLM_ROW_OUT(0), NPLM_ROW_IN(0));
     else if constexpr (N == 2)
-        asm volatile("s_and_b32 %[t], %[in], 3\n\ts_cmp_eq_u32 %[t], 3\n\ts_cbranch_scc0 .Lsome%=\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
-                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
-                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "s_bitcmp1_b32 %[in], 1\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
-                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
-                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1]), [a2] "+v"(a[-1][0]), [a3] "+v"(a[-1][1])
-                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [h2] "v"(h[1][0]), [h3] "v"(h[1][1]), [d0] "v"(d0), [d1] "v"(d1)
-                     : "scc");
+        NPLM_FMAC_ROWS(3, NPLM_ROW_FMAC(0) NPLM_ROW_FMAC(1), NPLM_ROW_SOME(0) NPLM_ROW_SOME(1), NPLM_ROW_OUT(0) NPLM_COMMA NPLM_ROW_OUT(1),
+                       NPLM_ROW_IN(0), NPLM_ROW_IN(1));
     else if constexpr (N == 3)
-        asm volatile("s_and_b32 %[t], %[in], 7\n\ts_cmp_eq_u32 %[t], 7\n\ts_cbranch_scc0 .Lsome%=\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
-                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
-                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
-                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "s_bitcmp1_b32 %[in], 1\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
-                     "s_bitcmp1_b32 %[in], 2\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
-                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
-                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1]), [a2] "+v"(a[-1][0]), [a3] "+v"(a[-1][1]), [a4] "+v"(a[-2][0]), [a5] "+v"(a[-2][1])
-                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [h2] "v"(h[1][0]), [h3] "v"(h[1][1]), [h4] "v"(h[2][0]), [h5] "v"(h[2][1]), [d0] "v"(d0), [d1] "v"(d1)
-                     : "scc");
-    else if constexpr (N == 4)
-        asm volatile("s_and_b32 %[t], %[in], 15\n\ts_cmp_eq_u32 %[t], 15\n\ts_cbranch_scc0 .Lsome%=\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
-                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
-                     "v_fmac_f32 %[a6], %[h6], %[d0]\n\tv_fmac_f32 %[a7], %[h7], %[d1]\n\t"
-                     ".Ldone%=:\n\t.subsection 1\n.Lsome%=:\n\t"
-                     "s_bitcmp1_b32 %[in], 0\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a0], %[h0], %[d0]\n\tv_fmac_f32 %[a1], %[h1], %[d1]\n\t"
-                     "s_bitcmp1_b32 %[in], 1\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a2], %[h2], %[d0]\n\tv_fmac_f32 %[a3], %[h3], %[d1]\n\t"
-                     "s_bitcmp1_b32 %[in], 2\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a4], %[h4], %[d0]\n\tv_fmac_f32 %[a5], %[h5], %[d1]\n\t"
-                     "s_bitcmp1_b32 %[in], 3\n\ts_cselect_b64 exec, -1, 0\n\t"
-                     "v_fmac_f32 %[a6], %[h6], %[d0]\n\tv_fmac_f32 %[a7], %[h7], %[d1]\n\t"
-                     "s_mov_b64 exec, -1\n\ts_branch .Ldone%=\n\t.subsection 0"
-                     : [t] "=&s"(t), [a0] "+v"(a[-0][0]), [a1] "+v"(a[-0][1]), [a2] "+v"(a[-1][0]), [a3] "+v"(a[-1][1]), [a4] "+v"(a[-2][0]), [a5] "+v"(a[-2][1]), [a6] "+v"(a[-3][0]), [a7] "+v"(a[-3][1])
-                     : [in] "s"(in), [h0] "v"(h[0][0]), [h1] "v"(h[0][1]), [h2] "v"(h[1][0]), [h3] "v"(h[1][1]), [h4] "v"(h[2][0]), [h5] "v"(h[2][1]), [h6] "v"(h[3][0]), [h7] "v"(h[3][1]), [d0] "v"(d0), [d1] "v"(d1)
-                     : "scc");
+        NPLM_FMAC_ROWS(7, NPLM_ROW_FMAC(0) NPLM_ROW_FMAC(1) NPLM_ROW_FMAC(2), NPLM_ROW_SOME(0) NPLM_ROW_SOME(1) NPLM_ROW_SOME(2),
+                       NPLM_ROW_OUT(0) NPLM_COMMA NPLM_ROW_OUT(1) NPLM_COMMA NPLM_ROW_OUT(2), NPLM_ROW_IN(0), NPLM_ROW_IN(1), NPLM_ROW_IN(2));
+    else
+        NPLM_FMAC_ROWS(15, NPLM_ROW_FMAC(0) NPLM_ROW_FMAC(1) NPLM_ROW_FMAC(2) NPLM_ROW_FMAC(3),
+                       NPLM_ROW_SOME(0) NPLM_ROW_SOME(1) NPLM_ROW_SOME(2) NPLM_ROW_SOME(3),
+                       NPLM_ROW_OUT(0) NPLM_COMMA NPLM_ROW_OUT(1) NPLM_COMMA NPLM_ROW_OUT(2) NPLM_COMMA NPLM_ROW_OUT(3),
+                       NPLM_ROW_IN(0), NPLM_ROW_IN(1), NPLM_ROW_IN(2), NPLM_ROW_IN(3));
 }
+#undef NPLM_ROW_FMAC
+#undef NPLM_ROW_SOME
+#undef NPLM_ROW_OUT
+#undef NPLM_ROW_IN
+#undef NPLM_FMAC_ROWS
+#undef NPLM_COMMA
 template <int KT>
 struct GatedDw {
     using TP = MfmaTaps<KT>;
@@ -1142,7 +1114,7 @@ struct GatedDw {
             constexpr int j = decltype(j_c)::value;
             const float d0 = bf16_lo(nxt[j & 1]), d1 = bf16_hi(nxt[j & 1]);
             if constexpr (j + 2 < NJ) nxt[j & 1] = read_dy<j + 2>();
-            if constexpr (j >= TP::P && j < TP::P + RW) { db[0] += d0; db[1] += d1; }
+            if constexpr (j >= TP::P && j < TP::P + RW) { db[0] += d0; db[1] += d1; }         // (rows from T on are staged as zeros)
             const uint32_t in = own[j / 4] >> j % 4 * 8;
             constexpr int u0 = j >= KT ? j - KT + 1 : 0, nu = (j < RW ? j + 1 : RW) - u0;
             fmac_rows<(nu < 4 ? nu : 4)>(&acc[j - u0], &h[u0], d0, d1, in >> u0);
@@ -1201,7 +1173,7 @@ struct MfmaGatedBwdShape {
     static constexpr int LDS_BYTES = WORDS_AT + 2 * kMfmaWords * 4;
     static_assert(CH == 128, "a dw wave has two channels per lane");
     static_assert(NDW == 8 && NDW / 2 * GatedDw<KT>::BOX * 4 <= WORDS_AT, "half of the sums in the buffers");
-    static_assert(LDS_BYTES <= kLdsBytes, "two buffers of three tiles and the terms of h fit the LDS");
+    static_assert(LDS_BYTES <= kLdsBytes, "two buffers of three tiles fit the LDS");
     using W = MfmaWeights<KT, CH, NWC>;
     static_assert(W::BYTES <= BUF_BYTES, "the weight table lies in the second buffer until its tiles come");
     static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords && NROWS <= 96, "boundary bits");
