@@ -492,7 +492,7 @@ def main():
     def roof(nbytes, samples_us, kernel):
         """Roofline of one kernel against both ceilings it can meet: HBM on its algorithmic bytes and the fp32 vector
         ALU on its algorithmic flops (forward 2KTC, backward 4KTC + TC). `bound` names the ceiling that takes longer at its
-        peak, i.e. the one that binds - HBM where the products are on the matrix cores (11 to 31 taps in bf16);
+        peak, i.e. the one that binds - HBM where the call runs on the matrix cores (the library says which kernels it takes);
         achieved/peak/unit/frac are that ceiling's, and both ceilings' figures are kept under "hbm" and "valu"."""
         med = statistics.median(samples_us)
         gbps = nbytes / med / 1e3
@@ -505,8 +505,9 @@ def main():
                "algorithmic_bytes": nbytes, "us_at_peak": nbytes / HBM_PEAK_GBPS / 1e3}
         valu = {"achieved": tflops, "peak": VALU_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tflops / VALU_PEAK_TFLOPS,
                 "algorithmic_flops": flops, "us_at_peak": flops / VALU_PEAK_TFLOPS / 1e6}
-        valu_bound = valu["us_at_peak"] >= hbm["us_at_peak"] and not (args.gated or args.ln or (
-            d.x.dtype == torch.bfloat16 and 11 <= K <= 31))
+        code = [_lib.BF16 if t.dtype == torch.bfloat16 else _lib.F32 for t in (d.x, d.weight)]
+        matrix_cores = lib.nplm_dwconv_debug_algo(int(kernel == "backward"), T, C, K, S, *code) == 4
+        valu_bound = valu["us_at_peak"] >= hbm["us_at_peak"] and not (args.gated or args.ln or matrix_cores)
         top = valu if valu_bound else hbm
         r = {"bound": "valu" if valu_bound else "hbm", "achieved": top["achieved"], "peak": top["peak"], "unit": top["unit"],
              "frac": top["frac"], "flops_per_byte": flops / nbytes, "ridge_flops_per_byte": VALU_PEAK_TFLOPS * 1e3 / HBM_PEAK_GBPS,

@@ -1323,6 +1323,12 @@ int nplm_dwconv_mask_cu(const void* mask, int32_t kind, int64_t row_stride, int6
 
 int32_t nplm_dwconv_exec_kernel_size(int32_t K) { return exec_kernel_size(K); }
 
+int32_t nplm_dwconv_debug_algo(int32_t bwd, int64_t T, int32_t C, int32_t K, int32_t S, int32_t act_dtype, int32_t w_dtype) {
+    const int rc = check_common(T, C, K, S, act_dtype, w_dtype);
+    if (rc) return rc;
+    return choose_algo(bwd != 0, nullptr, act_dtype == NPLM_DWCONV_BF16, w_dtype == NPLM_DWCONV_BF16, T, C, exec_kernel_size(K), lds_taps(K), S, 0, 0);
+}
+
 int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype, const nplm_dwconv_tuning* tune) {
     if (check_common(T, C, K, 0, act_dtype, NPLM_DWCONV_F32) || T == 0) return 0;
     K = exec_kernel_size(K);
