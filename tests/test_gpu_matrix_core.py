@@ -370,3 +370,18 @@ def test_rows_beyond_2_and_4_gib_offsets():
         assert torch.equal(y[s:e], npa.varlen_dwconv_fwd(x[s:e], sub, w, None, tuning=tn)), f"rows {s}..{e}"
         assert torch.equal(dx[s:e], npa.varlen_dwconv_bwd(x[s:e], dy[s:e], sub, w, tuning=tn)[0]), f"rows {s}..{e}"
     torch.testing.assert_close(db, dy.float().sum(0), rtol=2e-5, atol=0.05)
+
+
+@pytest.mark.parametrize("K", [11, 31])
+def test_share_of_outputs_that_are_not_correctly_rounded(K):
+    """fp32 sums of K exact products are off by up to K 2^-24 of the products' absolute sum, about sqrt(K) times an output, and land on
+    the other side of a rounding boundary of bf16 (one every 2^-8 of the value) once in about 2^8 * sqrt(K) * sqrt(K) 2^-24 outputs, with errors that
+    add at random: 1.7e-4 at 11 taps, 4.7e-4 at 31 as a bound; not more than a few times the share of the vector kernels."""
+    x, cu, w, b, dy = _case([5000, 300, 12000, 64] + LENS, 512, K, K)
+    xd, dyd, cud, wd, bd = (t.to(DEV) for t in (x, dy, cu, w, b))
+    want = (O.c_oracle_fwd(x, cu, w, b).bfloat16(), O.c_oracle_bwd(x, dy, cu, w)[0].bfloat16())
+    for name, f, ref in (("y", lambda t: npa.varlen_dwconv_fwd(xd, cud, wd, bd, tuning=t), want[0]),
+                         ("dx", lambda t: npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=t)[0], want[1])):
+        share = [float((f(_lib.Tuning(algo=a)).cpu() != ref).double().mean()) for a in (4, 1)]
+        print(f"[share] K={K} {name}: matrix cores {share[0]:.2e}, vector {share[1]:.2e}", flush=True)
+        assert share[0] <= K * 2.0 ** -16 and share[0] <= 2 * share[1] + 2e-6
