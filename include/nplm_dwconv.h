@@ -20,10 +20,13 @@
  *   Kernel sizes: K = 3, 5, 7, 9, 15 and 31 have kernels of their own. Any other odd K <= 31 runs on the
  *   kernels of the next of 3, 15, 31 with zero taps on either side (w and dw keep rows of K taps; the
  *   workspace holds slabs of that size; K = 11 and 17 .. 21 leave part of the zero taps out where a call
- *   takes LDS-staged kernels): for finite inputs the same sums with exact zeros added, so the
- *   same results; a NaN/Inf in x or dy then reaches the rows within that larger half-width of its own
- *   sequence (0 * Inf), never another sequence, and never a tap of dw that its products do not belong
- *   to. Odd K from 33 to NPLM_DWCONV_MAX_K run untuned kernels (one wave per row). The gated entry
+ *   takes LDS-staged or matrix-core kernels): for finite inputs the same sums with exact zeros added,
+ *   so the results of a call of that size with padded taps, bit for bit where both take the same
+ *   kernels (from T = 4096 on a backward in bf16 may not: K = 11 and 17 .. 21 keep the vector ALU for
+ *   longer sequences than 15 and 31; the fp32 sums then differ in their order). A NaN/Inf in x or dy
+ *   then reaches the rows within that larger half-width of its own sequence (0 * Inf; on the matrix cores
+ *   those within its own K taps only), never another sequence, and never a tap of dw that its products do
+ *   not belong to. Odd K from 33 to NPLM_DWCONV_MAX_K run untuned kernels (one wave per row). The gated entry
  *   points take the same kernel sizes up to 31 the same way; the LayerNorm-fused ones K = 3, 5, 7, 9 only.
  *
  * Where this sits in the reference (peymanvahidi/nanoplm 0.1.6): the reference snapshot holds no
@@ -40,8 +43,17 @@
  *    device memory, keeps no pointer after return and has no mutable global state.
  *  - All work is enqueued asynchronously on `stream` (a hipStream_t passed as void*; NULL = the
  *    null stream). cu is read on the device: no host synchronisation.
- *  - Launch geometry depends only on (T, C, K, dtypes), never on timing: results are
- *    run-to-run bit-identical (no floating-point atomics anywhere).
+ *  - Which kernels run and their launch geometry depend only on (T, C, K, S, dtypes) and on whether
+ *    pointers are aligned to 16 bytes (outputs: to 128), never on timing or on what the tensors
+ *    hold: results are run-to-run bit-identical (no floating-point atomics anywhere).
+ *  - S counts every entry of cu, empty sequences too. It changes which kernels run in the backward with
+ *    bf16 activations and weights, K from 11 to 31 and T >= 4096 only: the matrix cores take calls of at
+ *    least 32 rows per sequence at K = 31 (64 at 15, 512 at 11 and 21; gated, K = 31 from T = 16385 on,
+ *    192), counted as T / S. A long tail of empty sequences therefore costs speed (and another order of
+ *    the fp32 sums of dx, dz, dw): pass S without it where its length is known on the host.
+ *  - On the matrix cores (bf16 activations and weights, K from 11 to 31, T >= 4096) the order of a row's
+ *    fp32 sum goes by the row's number modulo 4: a sequence alone and the same one inside a batch may
+ *    differ by one bf16 rounding in y, dx and dz. Other kernels give the same bits in both.
  *  - Return value: 0 on success; < 0 an NPLM_DWCONV_E* argument error (nothing was launched);
  *    > 0 a hipError_t from a launch.
  *  - Preconditions NOT checked on the fast path (they would need a device read-back):

@@ -393,6 +393,7 @@ bool mfma_lines_ok(bool bwd, bool gated, long long T, int C, int K, int taps, ui
 // About 24 rows a sequence: K=31 627/575, 32: 560/574 (C=2048). 21 taps pay for the 32 lags of the plan, which short
 // sequences do not leave room for; 11 taps are bound by HBM on the vector ALU too.
 // Sequences of 522, 705, 1928 rows on average: K=21 181/196, 175/191, 160/186; K=11 150/150, 142/146, 139/144.
+// S counts empty sequences too, which the device alone could tell apart: a cu with a long tail of them is taken for shorter ones.
 bool mfma_bwd_preferred(long long T, int taps, int S) {
     const int rows = taps == 31 ? 32 : taps == 15 ? 64 : 512;
     return T >= (long long)S * rows;
@@ -403,7 +404,8 @@ bool mfma_bwd_preferred(long long T, int taps, int S) {
 //   T=16384, C=1024    72/75     61/66     58/65     56/69     51/66           T=8192, C=512     29/39     27/37     27/38    26/39    24/34
 // A wave of dw makes one pass over its rows whatever begins there, but masked row by row: short sequences cost it more than the
 // role-split kernel's roles, which share the loss, once a call is longer than its first tiles. 15 taps (T=131072, C=1024: 302/264,
-// T=4096: 19/22) and 21 (306/299) have too few FMAs to save.
+// T=4096: 19/22) and 21 (306/299) have too few FMAs to save. Calls of up to 16384 rows take it whatever begins in them (C=1024):
+//   T=16384   1 row 138/228   4 71/96   16 66/82   32 63/77   75 67/65        T=4096   1 row 45/83   8 27/40   32 26/39   75 26/36
 bool mfma_gated_bwd_preferred(long long T, int taps, int S) {
     return taps == 31 && (T <= 16384 || T >= 192ll * S);
 }
@@ -449,6 +451,9 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
 //     T=16384 C=1024: 24.6 / 28.6 at K=31, 17.7 / 21.4 at K=11. From kMfmaMinRows rows on: below, every block has a tile
 //     or two and what is measured is the launch (2048 rows, C=1024: K=31 11.8 / 12.5, K=15 10.0 / 10.2; 600 rows, C=512:
 //     12.2 / 11.8), while the others' sums are those of the sliding-window kernels bit for bit.
+//     Whatever the length of the sequences (T=65536, C=1024, K=31: 1 row 160 / 252, 4 64 / 154, 16 69 / 69, 24 70 / 96, 48 67 / 76;
+//     K=11: 1 row 113 / 196, 16 55 / 62, 75 56 / 64) and also where rows fill their column blocks poorly (T=32768, K=31: C=264
+//     25 / 35, C=520 33 / 44; K=11: 18 / 22, 25 / 29).
 //     fp32 weights would take three bf16 terms each: 280 us against 265 (K=31, C=2048), so they stay on the vector ALU.
 //   the same calls backward: matrix cores where a sequence has enough rows (mfma_bwd_preferred()).
 //   Large outputs whose rows are not whole cache lines keep the other kernels at 11 and 15 taps (mfma_lines_ok()).
