@@ -363,25 +363,27 @@ bool mfma_tile_fits(int C, int K, bool gated) {
 }
 // Output rows that do not begin on whole cache lines (128 bytes). A wave of the matrix-core kernels stores 128 bytes of a row
 // (gated 64) at a time where the others store 256 or 512; off the lines' grid each piece is two parts of lines, which other waves
-// complete later, and once the output is too large for the caches many of them reach HBM as parts. Measured with lengths of 20 to
-// 512 (backward at 11 taps: 700) residues, us, matrix cores against the best of the others, by MiB of T rows of C channels:
-//   forward, 11 / 15 taps: T=131072 C=1000 (250 MiB) 140 / 112, 139 / 111; C=648 (162) 106 / 99; T=65536 C=1160 (145) 89 / 80,
-//     C=840 (105) 61 / 59; T=32768 C=2008 (126) 72 / 63, C=1160 (72) 42 / 43, C=1000 (62) 36 / 38. Rows that fill the others'
-//     1 KiB column blocks to less than 3/5 stay: C=584 (0.57) T=98304 66 / 77, T=262144 173 / 180.
-//   backward, T=131072 C=1000 (250): 11 taps 228 / 184, 15 223 / 192; T=32768 C=648 (40) 47.6 / 45.1, 50.5 / 47.5, C=520 (32) 41.0 /
-//     41.0, 46.6 / 46.3; rows of less than 640 bytes stay: T=131072 C=264 (66) 71.7 / 72.8, 86.5 / 90.2.
-//   gated backward, 31 taps: T=131072 C=2008 (502) 1011 / 762, C=1000 518 / 392; T=65536 C=584 (73) 157 / 144; T=16384 C=1000 (31) 68 /
-//     65, C=648 (20) 53 / 54, C=520 (16) 47 / 53.
-// 31 taps save more FMAs than that costs (backward T=131072 C=1000 229 / 261, C=2040 509 / 517; forward 149 / 151, 346 / 326), 21
-// taps come out even (forward 145 / 144, backward 222 / 206, C=1800 351 / 377): both stay.
+// complete later. mfma_lines() lets them meet in the L2; in outputs too large for it and the Infinity Cache many reach HBM as parts all
+// the same, and up to 15 taps the others are faster there. Measured with lengths of 20 to 512 (backward at 11 and 21 taps: 700) residues, us,
+// matrix cores / the best of the others, by MiB of output:
+//   forward, 11 taps: T=131072 C=1000 (250 MiB) 127 / 112, C=1160 (290) 154 / 152, C=2008 (502) 246 / 215; T=65536 C=1800 (225) 110 / 107,
+//     C=1160 (145) 70 / 78, C=1000 (125) 55 / 62; T=131072 C=648 (162) 85 / 100; 15 taps the same to 3 %. Rows that fill the others'
+//     1 KiB column blocks to less than 3/5 stay: C=584 (0.57) T=131072 78 / 90.
+//   backward, 11 / 15 taps: T=131072 C=2008 (502) 433 / 364, 432 / 367; C=1160 (290) 247 / 216, 249 / 226; C=1032 (258) 204 / 207, 212 / 222;
+//     C=648 (162) 118 / 132, 127 / 138; T=16384 C=1000 (31) 34 / 38, 37 / 41.
+//   gated backward, 31 taps (stores with `nt` always): T=131072 C=2008 (502) 1011 / 762, C=1000 518 / 392; T=65536 C=584 (73) 157 / 144;
+//     T=16384 C=1000 (31) 68 / 65, C=648 (20) 53 / 54, C=520 (16) 47 / 53.
+// 31 taps save more FMAs than that costs (T=131072 C=2040 forward 254 / 304, backward 434 / 517), and so do 21 forward (258 / 307); 21
+// backward come out even (C=2008 423 / 393, C=1160 255 / 246, C=1800 373 / 380, T=98304 262 / 293) and stay.
 bool mfma_lines_ok(bool bwd, bool gated, long long T, int C, int K, int taps, uintptr_t out_bits) {
     const long long row_bytes = 2LL * C;
     if (((uintptr_t)row_bytes | out_bits) % 128 == 0) return true;
     const long long mib = T * row_bytes >> 20;
     if (gated) return mib < 30;
     if (taps > 15) return true;
-    if (bwd) return row_bytes < 640 || mib < 30;
-    return mib < 100 || !lds_preferred(false, true, T, C, K, 0) || row_bytes * 5 < ceil_div(row_bytes, kLdsDefaultCb) * 3LL * kLdsDefaultCb;
+    if (bwd) return mib < 270;
+    return mib < 200 || !lds_preferred(false, true, T, C, K, 0) ||
+           row_bytes * 5 < ceil_div(row_bytes, kLdsDefaultCb) * 3LL * kLdsDefaultCb;
 }
 // A backward tile with sequence boundaries makes one pass over its rows per sequence for dw, so the gain goes with the length
 // of the sequences. Measured at T=131072, us, matrix cores against role-split, for lengths of 20 to 128 residues (mean 75), 20
@@ -456,7 +458,7 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
 //     25 / 35, C=520 33 / 44; K=11: 18 / 22, 25 / 29).
 //     fp32 weights would take three bf16 terms each: 280 us against 265 (K=31, C=2048), so they stay on the vector ALU.
 //   the same calls backward: matrix cores where a sequence has enough rows (mfma_bwd_preferred()).
-//   Large outputs whose rows are not whole cache lines keep the other kernels at 11 and 15 taps (mfma_lines_ok()).
+//   Very large outputs whose rows are not whole cache lines keep the other kernels (mfma_lines_ok()).
 //   K=31 and K=15 backward of fp32 weights (ALU-bound; one wave cannot hold the fused backward's registers): the role-split
 //     kernel, when every output is asked for - C=2048, K=31: 510 us against 720 sliding-window on the log-normal length mix;
 //     K=15: 345 against 385 (C=1024: 177 against 205). A backward asked for dx alone or dw/db alone takes the

@@ -146,6 +146,16 @@ hipError_t launch_fwd_split_k21(bool bf16, const ConvPtrs& p, const LdsGeo& g, d
 hipError_t launch_fwd_split_k31(bool bf16, const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 #undef NPLM_DECLARE_SPLIT_K
 // matrix-core kernels of bf16 activations (dwconv_mfma_kernels.h), planned like the role-split ones
+// Whether they store their output with `nt`. Of a cache line (128 bytes) that is written in parts, by several waves, the parts then reach
+// memory one by one; without, they meet in the L2, but whole lines are slower, and so are small outputs and short rows. Forward of
+// 11 / 31 taps, us, with / without: T=131072 C=1000 140 / 127, 146 / 131, C=2040 340 / 266, 338 / 254, C=1024 96 / 101, 108 / 112, C=264
+// 45 / 48, 58 / 60; T=65536 C=1000 70 / 55, 75 / 64, C=520 (65 MiB) 40 / 40, 50 / 50; T=16384 C=1160 (36 MiB) 24 / 22, 30 / 29, C=392 (12) 12 / 13,
+// 17 / 18. Backward of 15 / 31 taps: T=131072 C=1000 223 / 193, 229 / 221; T=65536 C=1000 112 / 91, 124 / 118.
+inline bool mfma_lines(long long T, int C, const void* out) {
+    const long long row_bytes = 2LL * C, mib = T * row_bytes >> 20;
+    if (((uintptr_t)row_bytes | (uintptr_t)out) % 128 == 0) return true;
+    return row_bytes >= 1280 ? mib < 30 : row_bytes < 640 || mib < 96;
+}
 #define NPLM_DECLARE_MFMA_K(KK)                                                                              \
     hipError_t launch_fwd_mfma_k##KK(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);          \
     hipError_t launch_bwd_mfma_k##KK(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);

@@ -240,7 +240,8 @@ struct MfmaWeights {
 // more band (a single 1 per row), since a bf16 weight plus one is not one in bf16.
 // GATED (backward): the rows are dh; what is stored are the two halves of dz = [dh * silu(g) | dh * u * silu'(g)], with u and
 // g of the row out of their LDS tiles; 256-byte column blocks.
-template <int KT, int NSTEP, bool FLIP, bool RES, bool GATED = false>
+// LINES: stores with `nt`, for output rows of whole cache lines (see mfma_lines()).
+template <int KT, int NSTEP, bool FLIP, bool RES, bool LINES, bool GATED = false>
 struct MfmaConv {
     using TP = MfmaTaps<KT>;
     static constexpr int Q = GATED ? 2 : kMfmaQ, NCK = TP::NCK, CB = GATED ? kMfmaGatedCb : kMfmaCb;
@@ -354,7 +355,9 @@ struct MfmaConv {
         o.from_f32(v);
 #pragma unroll
         for (int h = 0; h < Q / 2; ++h) o.d[h] = (uint32_t)__builtin_amdgcn_ds_bpermute(swap, (int)o.d[h]);
-        o.bstore(ro, at, soff);
+        constexpr int aux = LINES ? kStoreAux : 0;
+        if constexpr (Q == 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2{o.d[0], o.d[1]}, ro, at, soff, aux);
+        else __builtin_amdgcn_raw_buffer_store_b32(o.d[0], ro, at, soff, aux);
     }
     // output row 4 n + row of the group; up = the group's first row in the u tile
     __device__ __forceinline__ void store(rsrc_t ro, int at, int rowb, const char* up, int row, const float (&v)[Q]) const {
@@ -557,7 +560,7 @@ struct MfmaFwdShape {
     static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords, "lanes read two words past the one of their window's first row");
 };
 
-template <int KT, bool RES>
+template <int KT, bool RES, bool LINES>
 __global__ void __launch_bounds__(MfmaFwdShape<KT>::NT)
 dwconv_fwd_mfma_kernel(const void* __restrict__ x, const int32_t* __restrict__ cu, const void* __restrict__ w,
                        const void* __restrict__ bias, void* __restrict__ y, const LdsGeo g) {
@@ -606,7 +609,7 @@ dwconv_fwd_mfma_kernel(const void* __restrict__ x, const int32_t* __restrict__ c
     const int nch = valid_bytes / 2;
     SH::W::template fill<false>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x);
     lds_barrier();
-    MfmaConv<KT, SH::RW / 16, false, RES> conv;
+    MfmaConv<KT, SH::RW / 16, false, RES, LINES> conv;
     conv.init(tab, SH::W::odd(tab), w, g.w_flags, bias, wc, lane, cb * kMfmaCh, nch, rowb);
     for (int it = 0; it < ntl; ++it) {
         lds_barrier();
@@ -932,7 +935,7 @@ struct MfmaBwdShape {
     static_assert((NROWS + 31) / 32 + 2 <= kMfmaWords && NROWS <= 96, "boundary bits");
 };
 
-template <int KT, bool RES>
+template <int KT, bool RES, bool LINES>
 __global__ void __launch_bounds__(MfmaBwdShape<KT>::NT)
 dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, const int32_t* __restrict__ cu,
                        const void* __restrict__ w, void* __restrict__ dx, float* __restrict__ partial, const LdsGeo g) {
@@ -981,7 +984,7 @@ dwconv_bwd_mfma_kernel(const void* __restrict__ x, const void* __restrict__ dy, 
     SH::W::template fill<true>(tab, w, g.w_flags, cb * kMfmaCh, nch, (int)threadIdx.x);
     lds_barrier();
     if (wv < SH::NDX) {
-        MfmaConv<KT, R / 16, true, RES> conv;
+        MfmaConv<KT, R / 16, true, RES, LINES> conv;
         conv.init(tab, SH::W::odd(tab), w, g.w_flags, nullptr, wv, lane, cb * kMfmaCh, nch, rowb);
         lds_barrier();
         for (int it = 0; it < ntl; ++it) {
@@ -1231,7 +1234,7 @@ dwconv_bwd_gated_mfma_kernel(const void* __restrict__ z, const void* __restrict_
     lds_barrier();
     if (wv < SH::NDZ) {
         __builtin_amdgcn_s_setprio(2);       // a dz wave has the longest way through a tile (log-normal lengths: 682 us without, 673 with)
-        MfmaConv<KT, R / 16, true, RES, true> conv;
+        MfmaConv<KT, R / 16, true, RES, true, true> conv;
         conv.init(tab, SH::W::odd(tab), w, g.w_flags, nullptr, wv, lane, cb * SH::CH, nch, rowb);
         lds_barrier();
         for (int it = 0; it < ntl; ++it) {

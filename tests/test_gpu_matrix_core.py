@@ -137,12 +137,12 @@ def test_which_backward_calls_the_matrix_cores_serve(T, n, K, wdt, served):
                        npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=_lib.Tuning(algo=1))[0])
 
 
-# (rows of 128-byte lines or not; outputs below and above the sizes from which the others take over: forward 100 MiB, backward 30)
+# (rows of 128-byte lines or not; outputs below and above the sizes from which the others take over: forward 200 MiB, backward 270)
 @pytest.mark.parametrize("bwd,T,C,K,offset,served", [
-    (False, 53248, 1000, 15, 0, False), (False, 52000, 1000, 15, 0, True), (False, 51200, 1024, 11, 0, True), (False, 53248, 1000, 21, 0, True),
-    (False, 94208, 584, 11, 0, True), (False, 51200, 1024, 11, 16, False),
-    (True, 15768, 1000, 15, 0, False), (True, 15700, 1000, 15, 0, True), (True, 15360, 1024, 15, 0, True), (True, 15768, 1000, 31, 0, True),
-    (True, 59904, 264, 11, 0, True), (True, 15360, 1024, 15, 8, False)])
+    (False, 105984, 1000, 15, 0, False), (False, 104000, 1000, 15, 0, True), (False, 102400, 1024, 11, 0, True), (False, 105984, 1000, 21, 0, True),
+    (False, 180224, 584, 11, 0, True), (False, 102400, 1024, 11, 16, False), (False, 16384, 1000, 31, 0, True), (False, 15700, 1000, 31, 0, True),
+    (True, 141824, 1000, 15, 0, False), (True, 141000, 1000, 15, 0, True), (True, 138240, 1024, 15, 0, True), (True, 141824, 1000, 31, 0, True),
+    (True, 141824, 1000, 21, 0, True), (True, 138240, 1024, 15, 8, False)])
 def test_which_rows_of_partial_cache_lines_the_matrix_cores_serve(bwd, T, C, K, offset, served):
     lib = _lib.load()
     g = torch.Generator(device=DEV).manual_seed(T)

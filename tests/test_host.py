@@ -269,13 +269,13 @@ def test_boundary_walk_ends_on_malformed_cu():
 # ---- which kernels a call runs on ----------------------------------------------------------------
 @pytest.mark.parametrize("bwd,T,C,K,S,algo", [
     (0, 4096, 256, 31, 1, 4), (0, 4095, 256, 31, 1, 3), (0, 4096, 248, 31, 1, 1), (0, 131072, 1024, 7, 500, 2), (1, 131072, 1024, 7, 500, 2),
-    # rows of partial cache lines: forward of 11 and 15 taps from 100 MiB of output on, if their column blocks are filled to 3/5
-    (0, 131072, 1000, 11, 500, 2), (0, 131072, 1000, 15, 500, 2), (0, 52000, 1000, 15, 200, 4), (0, 131072, 584, 15, 500, 4), (0, 131072, 1000, 21, 500, 4),
+    # rows of partial cache lines: forward of 11 and 15 taps from 200 MiB of output on, if their column blocks are filled to 3/5
+    (0, 131072, 1000, 11, 500, 2), (0, 131072, 1000, 15, 500, 2), (0, 104000, 1000, 15, 400, 4), (0, 262144, 584, 15, 900, 4), (0, 131072, 1000, 21, 500, 4),
     (0, 131072, 1000, 31, 500, 4), (0, 131072, 1024, 11, 500, 4),
-    # backward: rows a sequence, and rows of partial cache lines from 30 MiB on
+    # backward: rows a sequence, and rows of partial cache lines from 270 MiB on
     (1, 131072, 2048, 31, 4096, 4), (1, 131072, 2048, 31, 4097, 3), (1, 131072, 1024, 15, 2048, 4), (1, 131072, 1024, 15, 2049, 3),
-    (1, 131072, 1024, 21, 256, 4), (1, 131072, 1024, 21, 257, 3), (1, 131072, 1000, 15, 500, 3), (1, 15700, 1000, 15, 50, 4), (1, 131072, 264, 15, 500, 4),
-    (1, 131072, 1000, 31, 500, 4), (1, 131072, 1000, 11, 100, 3)])
+    (1, 131072, 1024, 21, 256, 4), (1, 131072, 1024, 21, 257, 3), (1, 142000, 1000, 15, 500, 3), (1, 141000, 1000, 15, 500, 4), (1, 142000, 1000, 21, 100, 4),
+    (1, 142000, 1000, 31, 500, 4), (1, 142000, 1000, 11, 100, 3), (1, 131072, 1000, 11, 100, 4)])
 def test_which_kernels_a_bf16_call_takes(bwd, T, C, K, S, algo):
     assert _lib.load().nplm_dwconv_debug_algo(bwd, T, C, K, S, _lib.BF16, _lib.BF16) == algo
     assert _lib.load().nplm_dwconv_debug_algo(bwd, T, C, K, S, _lib.BF16, _lib.F32) in (1, 2, 3)
