@@ -227,12 +227,12 @@ struct MfmaWeights {
         const bool any = __builtin_amdgcn_ballot_w64(odd != 0) != 0;
         if ((tid & 63) == 0) tab[MARKS_AT + tid / 64] = any ? 1 : 0;
     }
-    // whether one of the block's weights is not finite (after the barrier that follows fill())
-    __device__ __forceinline__ static uint64_t odd(const uint32_t* tab) {
+    // NaN if one of the block's weights is not finite, else 0 (after the barrier that follows fill())
+    __device__ __forceinline__ static float odd(const uint32_t* tab) {
         uint32_t any = 0;
 #pragma unroll
         for (int i = 0; i < NW; ++i) any |= tab[MARKS_AT + i];
-        return (uint32_t)__builtin_amdgcn_readfirstlane((int)any);
+        return __int_as_float(__builtin_amdgcn_readfirstlane((int)(any ? 0x7fc00000u : 0u)));
     }
 };
 
@@ -260,11 +260,11 @@ struct MfmaConv {
     int swap;              // stores: the lane whose output goes out through this one (x 4)
     int out_at;            // byte offset of that lane's slice of output row 4 n, or kMfmaNoStore
     bool active;
-    uint64_t odd;          // not zero: a weight of the block is not finite
+    float odd;             // NaN: a weight of the block is not finite, else 0
     const void* w;
     int w_flags;
 
-    __device__ __forceinline__ void init(const uint32_t* tab, uint64_t odd_, const void* w_, int w_flags_, const void* b, int wc, int lane, int ch0, int nch, int rowb) {
+    __device__ __forceinline__ void init(const uint32_t* tab, float odd_, const void* w_, int w_flags_, const void* b, int wc, int lane, int ch0, int nch, int rowb) {
         odd = odd_;
         n = lane & 3;
         const int blk = lane >> 2;
@@ -451,11 +451,11 @@ struct MfmaConv {
                 f32x4 acc[Q];
                 pass<false>(sp, lo, hi, acc);
                 const int i1 = hi - TP::FRONT < 4 ? hi - TP::FRONT : 4;
-                float chk = 0.f;
+                // (a row that is not finite meets all four sums; a weight meets each in another chunk, and chunks are left out here)
+                float chk = odd;
 #pragma unroll
                 for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(acc[q][0], 0.f, chk);
-                // (a row that is not finite meets all four sums; a weight meets each in another chunk, and chunks are left out here)
-                if (__builtin_expect((odd | __builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk))) != 0, 0)) {
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) != 0, 0)) {
                     pass<true>(sp, lo, hi, acc);
                     const int range = __builtin_amdgcn_ds_bpermute(swap, i0 | i1 << 8);
 #pragma nounroll
