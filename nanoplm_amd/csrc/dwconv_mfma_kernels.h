@@ -393,11 +393,114 @@ struct MfmaConv {
         return MfmaBits{__builtin_amdgcn_alignbit(d1, d0, at & 31), __builtin_amdgcn_alignbit(d2, d1, at & 31)};
     }
 
+    // Boundaries among a group's window rows, read by the wave as scalars. wp: its boundary bits (bit 0 is no boundary).
+    static constexpr int SPAN = 16 * NSTEP + TP::HALO;       // window rows of the group
+    static constexpr int kFewSequences = NCK >= 7 ? 3 : 0;   // (up to 15 taps a step's passes have too few chunks to leave out)
+    // whether at most kFewSequences sequences own rows of the group
+    __device__ __forceinline__ static bool few_sequences(const uint32_t* wp) {
+        int n = 1;
+#pragma unroll
+        for (int i = 0; i * 32 < TP::FRONT + ROWS; ++i) {    // rows FRONT + 1 .. FRONT + ROWS - 1
+            constexpr int A = TP::FRONT + 1, B = TP::FRONT + ROWS;
+            const uint32_t from = A > 32 * i ? (A - 32 * i < 32 ? ~0u << (A & 31) : 0u) : ~0u;
+            const uint32_t to = B < 32 * i + 32 ? (1u << (B & 31)) - 1u : ~0u;
+            n += __builtin_popcount((uint32_t)__builtin_amdgcn_readfirstlane((int)(wp[i] & from & to)));
+        }
+        return n <= kFewSequences;
+    }
+    // first window row of the sequence that holds row `at` (0: it began before), at < 32
+    __device__ __forceinline__ static int start_of(const uint32_t* wp, int at) {
+        const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)wp[0]);
+        return 31 - (int)__builtin_clz((w & ((2u << at) - 1u)) | 1u);
+    }
+    // first window row behind row `at` where a sequence begins (SPAN: none)
+    __device__ __forceinline__ static int start_behind(const uint32_t* wp, int at) {
+        int r = SPAN;
+#pragma unroll
+        for (int i = (SPAN + 31) / 32 - 1; i >= 0; --i) {
+            const int sh = at + 1 - 32 * i;                  // bits from here on lie behind `at`
+            uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)wp[i]);
+            w = sh <= 0 ? w : sh < 32 ? w & (~0u << sh) : 0u;
+            if (w) r = 32 * i + (int)__builtin_ctz(w);
+        }
+        return r < SPAN ? r : SPAN;
+    }
+    // Packed masks of a lane's window rows 4 (c + n) .. + 3 against [lo, hi) (uniform).
+    __device__ __forceinline__ void chunk_masks(int c, int lo, int hi, uint32_t& m0, uint32_t& m1) const {
+        const int o = lo > 4 * c ? lo - 4 * c : 0, e = hi - 4 * c < 16 ? hi - 4 * c : 16;      // (o < 16, e > 0: some rows are in)
+        const uint32_t v = (((1u << e) - 1u) & (~0u << o)) >> (4 * n);
+        m0 = __builtin_amdgcn_perm((uint32_t)((int)(v << 30) >> 31), (uint32_t)((int)(v << 31) >> 31), 0x05040100);
+        m1 = __builtin_amdgcn_perm((uint32_t)((int)(v << 28) >> 31), (uint32_t)((int)(v << 29) >> 31), 0x05040100);
+    }
+    // The group's output rows, chunk after chunk of its window, each chunk for all the steps it belongs to. PART: only the rows of one
+    // sequence, window rows [lo, hi): chunks without any of its rows are left out, those at its ends masked, rows outside it not
+    // stored. Returns whether all sums are finite (those that are not have to be formed again).
+    template <bool PART>
+    __device__ __forceinline__ bool sweep(const char* lp, int lo, int hi, rsrc_t ro, int rowb, const char* up) const {
+        float chk = PART ? odd : 0.f;
+        f32x4 acc[(NCK + 3) / 4][Q];
+        MfmaRaw<Q> raw;
+        read<0>(lp, raw);
+        int range = 0;                                       // output rows [o, e) of the group, relative to the storing lane's first
+        if constexpr (PART) range = __builtin_amdgcn_ds_bpermute(swap, 4 * n);
+        static_for<NCHUNK>([&](auto c_c) __attribute__((always_inline)) {
+            constexpr int c = decltype(c_c)::value;
+            const MfmaRaw<Q> cur = raw;
+            if constexpr (c + 1 < NCHUNK)
+                read<c + 1, (c + 1 == NCHUNK - 1 ? TP::LASTROWS : 4)>(lp, raw);
+            static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
+                constexpr int s = decltype(s_c)::value;
+                if constexpr (c == 4 * s) {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) acc[s % ((NCK + 3) / 4)][q] = start(q);
+                }
+            });
+            if (!PART || (4 * c < hi && 4 * c + 16 > lo)) {
+                MfmaChunk<Q> x;
+                mfma_pack(cur, x);
+                if (PART && (4 * c < lo || 4 * c + 16 > hi)) {
+                    uint32_t m0, m1;
+                    chunk_masks(c, lo, hi, m0, m1);
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) { x.b[q].x &= m0; x.b[q].y &= m1; }
+                }
+                static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
+                    constexpr int s = decltype(s_c)::value;
+                    constexpr int k = c - 4 * s;
+                    if constexpr (k >= 0 && k < NCK) taps<k>(acc[s % ((NCK + 3) / 4)], x);
+                });
+            }
+            static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
+                constexpr int s = decltype(s_c)::value;
+                if constexpr (c - 4 * s == NCK - 1) {
+                    const f32x4 (&a)[Q] = acc[s % ((NCK + 3) / 4)];
+                    if (!PART || (lo < TP::FRONT + 16 * s + 16 && hi > TP::FRONT + 16 * s)) {
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(a[q][0], 0.f, chk);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float v[Q];
+#pragma unroll
+                            for (int q = 0; q < Q; ++q) v[q] = a[q][i];
+                            int at = out_at;
+                            if constexpr (PART) {
+                                const int r = TP::FRONT + 16 * s + i + range;
+                                at = r >= lo && r < hi ? out_at : kMfmaNoStore;
+                            }
+                            store(ro, at, rowb, up, 16 * s + i, v);
+                        }
+                    }
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        return __builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) == 0;
+    }
+
     // One group of output rows: lp = the group's first window row in LDS, words = the tile's boundary bits, p0 = the window row's
     // place among them; ro = descriptor of the group's output rows (those in front of T).
     // GATED: up = the group's first row in the u tile; the g tile lies kMfmaGatedRows rows behind it.
     __device__ __forceinline__ void rows(const char* lp, const uint32_t* words, int p0, rsrc_t ro, int rowb, const char* up = nullptr) const {
-        constexpr int SPAN = 16 * NSTEP + TP::HALO;          // window rows of the group
         const uint32_t* wp = words + (p0 >> 5);              // p0 is a multiple of 32
         bool open;                                           // no boundary inside the window (a bit at its first row is none)
         {
@@ -407,42 +510,17 @@ struct MfmaConv {
             open = __builtin_amdgcn_readfirstlane((int)any) == 0;
         }
         if (open) {
-            float chk = 0.f;
-            f32x4 acc[(NCK + 3) / 4][Q];
-            MfmaRaw<Q> raw;
-            read<0>(lp, raw);
-            static_for<NCHUNK>([&](auto c_c) __attribute__((always_inline)) {
-                constexpr int c = decltype(c_c)::value;
-                MfmaChunk<Q> x;
-                mfma_pack(raw, x);
-                if constexpr (c + 1 < NCHUNK)
-                    read<c + 1, (c + 1 == NCHUNK - 1 ? TP::LASTROWS : 4)>(lp, raw);
-                static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
-                    constexpr int s = decltype(s_c)::value;
-                    constexpr int k = c - 4 * s;
-                    if constexpr (k >= 0 && k < NCK) {
-                        f32x4 (&a)[Q] = acc[s % ((NCK + 3) / 4)];
-                        if constexpr (k == 0) {
-#pragma unroll
-                            for (int q = 0; q < Q; ++q) a[q] = start(q);
-                        }
-                        taps<k>(a, x);
-                        if constexpr (k == NCK - 1) {
-#pragma unroll
-                            for (int q = 0; q < Q; ++q) chk = __builtin_fmaf(a[q][0], 0.f, chk);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) {
-                                float v[Q];
-#pragma unroll
-                                for (int q = 0; q < Q; ++q) v[q] = a[q][i];
-                                store(ro, out_at, rowb, up, 16 * s + i, v);
-                            }
-                        }
-                    }
-                });
-                __builtin_amdgcn_sched_barrier(0);
-            });
-            if (__builtin_amdgcn_ballot_w64(active && !__builtin_isfinite(chk)) == 0) return;
+            if (sweep<false>(lp, 0, SPAN, ro, rowb, up)) return;
+        } else if (kFewSequences > 0 && few_sequences(wp)) {
+            // One sweep per sequence that owns rows of the group.
+            int lo = start_of(wp, TP::FRONT);
+            bool done = true;
+            do {
+                const int hi = start_behind(wp, lo > TP::FRONT ? lo : TP::FRONT);
+                done = sweep<true>(lp, lo, hi, ro, rowb, up) && done;
+                lo = hi;
+            } while (lo < TP::FRONT + ROWS);
+            if (done) return;
         }
 #pragma nounroll
         for (int s = 0; s < NSTEP; ++s) {
@@ -547,7 +625,8 @@ struct MfmaConv {
 
 // Forward: 64-row tiles, 8 compute waves (4 wave-columns x 2 groups of 32 rows), 3 loader waves and one that finds the
 // boundaries of the next tile; two tile buffers.
-// Bound by HBM from 64 row tiles on: T=131072, C=2048, 31 taps, one sequence 184 us (5.8 TB/s), 248 on the vector ALU. More rows
+// Bound by HBM from 64 row tiles on: T=131072, C=2048, 31 taps, one sequence 182 us (5.9 TB/s), 248 on the vector ALU; log-normal
+// lengths 203 (216 before the sweeps over single sequences). More rows
 // per tile, three buffers or 1 KiB column blocks measured the same or slower (a tile's compute already hides the next one's
 // loads); one scout wave costs nothing that the loaders would use.
 template <int KT>
@@ -759,9 +838,81 @@ struct MfmaDw {
             a = b;
         }
     }
+    // Whether at most kFewSequences sequences own rows of the tile.
+    static constexpr int kFewSequences = ND == 2 ? 2 : 0;    // (with one group of lags the loop of passes() is as fast)
+    __device__ __forceinline__ static bool few_sequences(uint64_t w0, uint64_t w1) {
+        return __builtin_popcountll(w0 >> (TP::FRONT + 1)) + __builtin_popcountll(w1 & ((1ull << TP::FRONT) - 1ull)) < kFewSequences;
+    }
+    // acc += a tile's sums, chunk after chunk of dy, db with them; each chunk of x is packed once and meets the chunks of dy of both groups of lags.
+    // PART: those of one sequence alone, staged rows [a, b): chunks that hold none of its rows are left out, those at its ends masked.
+    // Every chunk is a place of its own in the code, so that neither addresses nor registers are moved: with one wave per SIMD
+    // every instruction counts, and the loop of passes() spends 170 on a chunk where this spends 45.
+    template <bool PART>
+    __device__ __forceinline__ void sweep(int a, int b, int nrow, f32x4 (&acc)[ND][Q]) {
+        constexpr int NR = 4 * (ND - 1) + 1, NCD = NCX + 4 * (ND - 1);
+        // rows of x and the chunks they lie in (a lane's rows are shifted by up to 3)
+        const int t0 = PART && a > TP::FRONT ? a - TP::FRONT : 0, t1 = !PART ? R : b - TP::FRONT < nrow ? b - TP::FRONT : nrow;
+        // (PART, db: the chunks 0, 4, ... that hold the sequence's rows of the tile are among those visited, x0 .. x1 + 4: the first of
+        // these rows is FRONT + t0)
+        const int d0 = (TP::FRONT + t0) >> 4 << 2;
+        const int x0 = !PART ? 0 : TP::FRONT < 15 && d0 < t0 >> 2 ? d0 : t0 >> 2, x1 = PART ? (t1 + 2) >> 2 : NCX - 1;
+        MfmaRaw<Q> rd, rx;
+        MfmaChunk<Q> ring[NR];                               // x chunks c - 4 .. c (of one group of lags: c)
+        if (!PART || x0 == 0) {
+            read_dy(0, rd);
+            read_x(0, rx);
+        }
+        static_for<NCD>([&](auto c_c) __attribute__((always_inline)) {
+            constexpr int c = decltype(c_c)::value;
+            auto next = [&]() __attribute__((always_inline)) {
+                if constexpr (c + 1 < NCD) read_dy(c + 1, rd);
+                if constexpr (c + 1 < NCX) read_x(c + 1, rx);
+            };
+            if (!PART || (c >= x0 && c <= x1 + 4 * (ND - 1))) {
+                MfmaChunk<Q> dy;
+                uint32_t m0, m1;
+                mfma_pack(rd, dy);
+                if constexpr (c < NCX) {
+                    mfma_pack(rx, ring[c % NR]);
+                    if (PART ? 4 * c - 3 < t0 || 4 * c + 3 >= t1 : c == 0 || c == NCX - 1) {
+                        row_masks(4 * c - 3, 3 - n, t0, t1, m0, m1);
+                        mask(ring[c % NR], m0, m1);
+                    }
+                }
+                // (what follows the staged rows meets only masked x, but may hold a NaN)
+                if (PART ? 4 * c < a || 4 * c + 16 > b : 4 * c + 16 > SPAN) {
+                    row_masks(4 * c, 4 * n, PART ? a : 0, PART ? b : SPAN, m0, m1);
+                    mask(dy, m0, m1);
+                }
+                next();
+                if constexpr (c < NCX) {
+                    if (!PART || c <= x1) {
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) acc[0][q] = mfma4(ring[c % NR].op(q), dy.op(q), acc[0][q]);
+                    }
+                }
+                if constexpr (ND == 2 && c >= 4) {
+                    if (!PART || c - 4 >= x0) {
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) acc[ND - 1][q] = mfma4(ring[(c - 4) % NR].op(q), dy.op(q), acc[ND - 1][q]);
+                    }
+                }
+                // db: staged rows 4c .. 4c + 15 in the four columns
+                if constexpr (c % 4 == 0 && c < NCX) {
+                    if constexpr (c == 0 || c == NCX - 1) {
+                        row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + R, m0, m1);
+                        mask(dy, m0, m1);
+                    }
+                    add_db(dy);
+                }
+            } else if (c + 1 == x0) {
+                next();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
     // words = the tile's boundary bits; nrow = its rows in front of T
     __device__ __forceinline__ void tile(const uint32_t* words, int nrow) {
-        constexpr int NR = 4 * (ND - 1) + 1, NCD = NCX + 4 * (ND - 1);
         uint64_t w0, w1;                                     // boundary bits of staged rows 0 .. 63 and 64 on
         {
             uint32_t v[4];
@@ -776,58 +927,32 @@ struct MfmaDw {
 #pragma unroll
             for (int q = 0; q < Q; ++q) acc[d][q] = f32x4{0.f, 0.f, 0.f, 0.f};
         if ((w0 | w1) == 0) {
-            MfmaRaw<Q> rd, rx;
-            MfmaChunk<Q> ring[NR];                           // x chunks c - 4 .. c (of one group of lags: c)
-            read_dy(0, rd);
-            read_x(0, rx);
-            static_for<NCD>([&](auto c_c) __attribute__((always_inline)) {
-                constexpr int c = decltype(c_c)::value;
-                MfmaChunk<Q> dy;
+            sweep<false>(0, SPAN, R, acc);
+        } else {
+            const bool few = kFewSequences > 0 && few_sequences(w0, w1);
+            if (!few) {
                 uint32_t m0, m1;
-                mfma_pack(rd, dy);
-                if constexpr (c < NCX) {
-                    mfma_pack(rx, ring[c % NR]);
-                    if constexpr (c == 0 || c == NCX - 1) {
-                        row_masks(4 * c - 3, 3 - n, 0, R, m0, m1);
-                        mask(ring[c % NR], m0, m1);
-                    }
-                }
-                if constexpr (4 * c + 16 > SPAN) {           // what follows the staged rows meets only masked x, but may hold a NaN
-                    row_masks(4 * c, 4 * n, 0, SPAN, m0, m1);
+#pragma nounroll
+                for (int c = 0; c < NCX; c += 4) {
+                    MfmaRaw<Q> raw;
+                    MfmaChunk<Q> dy;
+                    read_dy(c, raw);
+                    mfma_pack(raw, dy);
+                    row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + nrow, m0, m1);
                     mask(dy, m0, m1);
-                }
-                if constexpr (c + 1 < NCD) read_dy(c + 1, rd);
-                if constexpr (c + 1 < NCX) read_x(c + 1, rx);
-                if constexpr (c < NCX) {
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) acc[0][q] = mfma4(ring[c % NR].op(q), dy.op(q), acc[0][q]);
-                }
-                if constexpr (ND == 2 && c >= 4) {
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) acc[ND - 1][q] = mfma4(ring[(c - 4) % NR].op(q), dy.op(q), acc[ND - 1][q]);
-                }
-                if constexpr (c % 4 == 0 && c < NCX) {       // staged rows 4c .. 4c + 15 in the four columns
-                    if constexpr (c == 0 || c == NCX - 1) {
-                        row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + R, m0, m1);
-                        mask(dy, m0, m1);
-                    }
                     add_db(dy);
                 }
-                __builtin_amdgcn_sched_barrier(0);
-            });
-        } else {
-            uint32_t m0, m1;
-#pragma nounroll
-            for (int c = 0; c < NCX; c += 4) {
-                MfmaRaw<Q> raw;
-                MfmaChunk<Q> dy;
-                read_dy(c, raw);
-                mfma_pack(raw, dy);
-                row_masks(4 * c, 4 * n, TP::FRONT, TP::FRONT + nrow, m0, m1);
-                mask(dy, m0, m1);
-                add_db(dy);
             }
-            passes<false>(w0, w1, nrow, acc);
+            if (few) {
+                int a = sequence_of(w0, w1, TP::FRONT);
+                do {
+                    const int b = next_sequence(w0, w1, a > TP::FRONT ? a : TP::FRONT);
+                    sweep<true>(a, b < SPAN ? b : SPAN, nrow, acc);
+                    a = b;
+                } while (a < TP::FRONT + nrow);
+            } else {
+                passes<false>(w0, w1, nrow, acc);
+            }
         }
         float chk = 0.f;
 #pragma unroll
@@ -920,9 +1045,11 @@ struct MfmaDw {
 
 // Backward: 64-row tiles (a dy tile with its halo rows, an x tile without), 4 wave-columns; waves of three kinds: dx
 // (MfmaConv over dy), dw and db, loaders and boundaries.
-// T=131072, C=2048, 31 taps: 294 us on one sequence (the role-split kernel of the vector ALU 479; a copy of the bytes takes 313),
-// 372 on log-normal lengths (511), where the dw waves' passes at sequence boundaries show. Tried for those, all slower on
-// every mix: one sweep of unrolled chunks that branches at each (382 to 452), one sweep and a left-over per boundary (spills).
+// T=131072, C=2048, 31 taps: 272 us on one sequence (the role-split kernel of the vector ALU 479; a copy of the bytes takes 313),
+// 340 on log-normal lengths (511). A SIMD has one wave of dx and one of dw, each of which issues an instruction every 5 cycles or
+// so: what tiles with boundaries cost goes with the instructions they run (without the sweeps over single sequences 356 us;
+// sequences of 320 rows 303 against 353). Tried for dw, all slower: one sweep of unrolled chunks that branches at each, one sweep and
+// a left-over per boundary (spills), bit masks per chunk in place of the compares of sweep() (spills).
 template <int KT>
 struct MfmaBwdShape {
     using TP = MfmaTaps<KT>;

@@ -51,6 +51,22 @@ def test_forward_on_the_matrix_cores_matches_the_oracle(K, lens, C, nbt):
     assert torch.equal(npa.varlen_dwconv_fwd(xd, cud, wide, bd, tuning=tn), y)
 
 
+@pytest.mark.parametrize("K", [15, 21, 31])
+@pytest.mark.parametrize("step", [63, 95, 191])
+def test_one_to_three_sequences_a_tile_with_a_boundary_at_every_row_of_it(K, step):
+    """Sequences of `step` rows begin at every row of the 64-row tiles and the 32-row groups in turn: the sweeps over single sequences."""
+    print(f"[case] K={K} step={step}", flush=True)
+    x, cu, w, b, dy = _case([step] * 65 + [7], 264, K, K + step)
+    xd, cud, wd, bd, dyd = x.to(DEV), cu.to(DEV), w.to(DEV), b.to(DEV), dy.to(DEV)
+    tn = _lib.Tuning(**MFMA)
+    assert_act_close(npa.varlen_dwconv_fwd(xd, cud, wd, bd, tuning=tn), O.c_oracle_fwd(x, cu, w, b), torch.bfloat16, "y")
+    dx64, dw64, db64 = O.c_oracle_bwd(x, dy, cu, w)
+    dx, dw, db = npa.varlen_dwconv_bwd(xd, dyd, cud, wd, tuning=tn)
+    assert_act_close(dx, dx64, torch.bfloat16, "dx")
+    assert_red_close(dw, dw64, "dw")
+    assert_red_close(db, db64, "db")
+
+
 def _plant_non_finite(t, cu):
     for i in range(0, cu.numel() - 1, 5):
         if cu[i + 1] - cu[i] < 10:
