@@ -6,10 +6,12 @@ There is no fallback: if the shared object is missing, every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libnplm_dwconv.so")
+NODE_PATH = os.path.join(_HERE, "_node.so")
 
 F32 = 0
 BF16 = 1
@@ -39,6 +41,7 @@ PUBLIC_SYMBOLS = (
 )
 
 _lib = None
+_node = None
 
 
 class Tuning(ctypes.Structure):
@@ -113,6 +116,17 @@ def load():
     lib.nplm_dwconv_check_cu.restype = ctypes.c_int
     _lib = lib
     return lib
+
+
+def load_node():
+    """The native autograd nodes (``csrc/node.cpp``), built beside the library and linked to it."""
+    global _node
+    load()
+    if _node is None:
+        if not os.path.exists(NODE_PATH):
+            raise RuntimeError(f"{NODE_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}`")
+        _node = importlib.import_module("nanoplm_amd._node")
+    return _node
 
 
 def strerror(code: int) -> str:

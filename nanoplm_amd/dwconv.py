@@ -214,10 +214,12 @@ class VarlenDWConv1dFunction(torch.autograd.Function):
 def varlen_dwconv(x, cu_seqlens, weight, bias=None, residual: bool = False):
     """Functional form of :class:`VarlenDWConv1dFunction`. While ``torch.compile`` is tracing, the call goes
     through the registered custom ops instead (same kernels), so that callers of this function (the padded-batch
-    door among them) never break the graph."""
+    door among them) never break the graph. Otherwise the native node takes the call (same kernels, same gradients, no Python in
+    either direction) or, for a call that is not of its form, leaves it to the Function."""
     if torch.compiler.is_compiling():
         return varlen_dwconv_fwd_op(x, cu_seqlens, weight, bias, residual)
-    return VarlenDWConv1dFunction.apply(x, cu_seqlens, weight, bias, residual)
+    y = _lib.load_node().dwconv(x, cu_seqlens, weight, bias, residual)
+    return VarlenDWConv1dFunction.apply(x, cu_seqlens, weight, bias, residual) if y is None else y
 
 
 class VarlenDWConv1d(nn.Module):

@@ -146,10 +146,12 @@ def gated_varlen_dwconv(z: torch.Tensor, cu_seqlens: torch.Tensor, weight: torch
     """``conv(z[:, :C] * silu(z[:, C:]))`` over packed sequences, ``[T, 2C] -> [T, C]``.
 
     Under ``torch.compile`` the call goes through the registered custom ops (opaque to the tracer, no graph
-    break, any shape); otherwise through the autograd Function. Both run the same two raw entry points."""
+    break, any shape); otherwise the native node takes it (see :func:`nanoplm_amd.varlen_dwconv`) or, where the library has
+    no fused kernel or the call is not of the node's form, the autograd Function. All run the same kernels."""
     if torch.compiler.is_compiling():
         return gated_dwconv_fwd_op(z, cu_seqlens, weight, bias, residual)
-    return GatedVarlenDWConv1dFunction.apply(z, cu_seqlens, weight, bias, residual)
+    y = _lib.load_node().gated_dwconv(z, cu_seqlens, weight, bias, residual)
+    return GatedVarlenDWConv1dFunction.apply(z, cu_seqlens, weight, bias, residual) if y is None else y
 
 
 # ---------------------------------------------------------------------------------------------

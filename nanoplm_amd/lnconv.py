@@ -250,7 +250,12 @@ ln_dwconv_fwd_op.register_autograd(_ln_backward, setup_context=_ln_setup_context
 
 def ln_varlen_dwconv_compilable(x, cu_seqlens, ln_weight, ln_bias, weight, bias=None, *, eps: float = 1e-5,
                                 residual: bool = False):
-    """Same result as :func:`ln_varlen_dwconv`, routed through the registered custom ops (traceable)."""
+    """Same result as :func:`ln_varlen_dwconv`, traceable: through the registered custom ops, or, where nothing traces and the
+    library has the fused kernels, through the native node (see :func:`nanoplm_amd.varlen_dwconv`)."""
+    if not torch.compiler.is_compiling():
+        y = _lib.load_node().ln_dwconv(x, cu_seqlens, ln_weight, ln_bias, weight, bias, eps, residual)
+        if y is not None:
+            return y
     return ln_dwconv_fwd_op(x, cu_seqlens, ln_weight, ln_bias, weight, bias, eps, residual)[0]
 
 

@@ -197,3 +197,76 @@ def test_the_integration_guides_ctypes_binding_runs_as_written():
         assert torch.equal(y, npa.varlen_dwconv_fwd(d.x, d.cu_seqlens, d.weight, d.bias))
         dx, dw, db = npa.varlen_dwconv_bwd(d.x, d.dy, d.cu_seqlens, d.weight)
         assert torch.equal(x.grad, dx) and torch.equal(w.grad, dw.to(w.dtype)) and torch.equal(b.grad, db.to(b.dtype))
+
+
+# ---- native nodes ---------------------------------------------------------------------------------
+def _door(form, act, par, bias, residual):
+    """(call through the public door, the same call as a Python Function, its tensors) for T=600 rows of 512 channels, 7 taps."""
+    C, K = 512, 7
+    g = torch.Generator().manual_seed(7)
+    rnd = lambda *s, dt: torch.randn(*s, generator=g).to(dt).to(DEV)
+    cu = torch.tensor([0, 3, 3, 200, 600], dtype=torch.int32, device=DEV)
+    x = rnd(600, 2 * C if form == "gated" else C, dt=act)
+    w, b = rnd(C, K, dt=par), rnd(C, dt=par) if bias else None
+    if form == "ln":
+        lw, lb = rnd(C, dt=par), rnd(C, dt=par) if bias else None
+        return (lambda x, lw, lb, w, b: npa.ln_varlen_dwconv_compilable(x, cu, lw, lb, w, b, residual=residual),
+                lambda x, lw, lb, w, b: npa.ln_varlen_dwconv(x, cu, lw, lb, w, b, residual=residual), [x, lw, lb, w, b])
+    public, function = ((npa.gated_varlen_dwconv, npa.GatedVarlenDWConv1dFunction) if form == "gated" else
+                        (npa.varlen_dwconv, npa.VarlenDWConv1dFunction))
+    return (lambda x, w, b: public(x, cu, w, b, residual), lambda x, w, b: function.apply(x, cu, w, b, residual), [x, w, b])
+
+
+@pytest.mark.parametrize("form", ["plain", "gated", "ln"])
+@pytest.mark.parametrize("act,par", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("bias,residual,frozen", [(True, False, ()), (False, True, ()), (True, True, (0,)), (True, False, (-1, -2))])
+def test_native_nodes_give_the_bits_of_the_python_functions(form, act, par, bias, residual, frozen):
+    door, function, args = _door(form, act, par, bias, residual)
+    frozen = [args[i] for i in frozen]
+    leaves = [None if t is None else t.clone().requires_grad_(all(t is not f for f in frozen)) for t in args]
+    wanted = [t for t in leaves if t is not None and t.requires_grad]
+    y, y1 = door(*leaves), function(*leaves)
+    assert "Backward" not in type(y.grad_fn).__name__ and "Backward" in type(y1.grad_fn).__name__
+    dy = torch.randn(y.shape, device=DEV).to(y.dtype)
+    got, want = torch.autograd.grad(y, wanted, dy), torch.autograd.grad(y1, wanted, dy)
+    assert torch.equal(y, y1) and y.dtype == y1.dtype
+    for a, c, t in zip(got, want, wanted):
+        assert a.dtype == c.dtype == t.dtype and torch.equal(a, c)
+    with torch.no_grad():
+        y0 = door(*leaves)
+    assert torch.equal(y0, y1) and not y0.requires_grad
+
+
+@pytest.mark.parametrize("form", ["plain", "gated", "ln"])
+def test_native_nodes_leave_other_forms_of_call_to_the_python_route(form):
+    """Strided and unaligned tensors, mixed parameter dtypes, saved-tensor hooks, dy that is no dense tensor, transforms, forward mode."""
+    bf16, f32 = torch.bfloat16, torch.float32
+    door, function, args = _door(form, bf16, bf16, True, False)
+    y = function(*args)
+    x, rest = args[0], args[1:]
+    wide = torch.empty(600, 2 * x.shape[1], dtype=bf16, device=DEV)
+    wide[:, :x.shape[1]] = x
+    assert torch.equal(door(wide[:, :x.shape[1]], *rest), y)
+    odd = torch.empty(x.numel() + 1, dtype=bf16, device=DEV)[1:].view(x.shape).copy_(x)
+    torch.testing.assert_close(door(odd, *rest), function(odd, *rest), rtol=0, atol=0)
+    mixed = [x] + rest[:-1] + [rest[-1].to(f32)]
+    assert torch.equal(door(*mixed), function(*mixed))
+    xg = x.clone().requires_grad_()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t.clone(), lambda t: t):
+        yg = door(xg, *rest)
+    assert any(t is xg or t.data_ptr() == xg.data_ptr() for t in packed)
+    dy = torch.ones(1, dtype=bf16, device=DEV).expand(y.shape)
+    got = torch.autograd.grad(yg, xg, dy)[0]
+    assert torch.equal(got, torch.autograd.grad(function(xg, *rest), xg, dy.contiguous())[0])
+    batch = lambda: torch.func.vmap(lambda x: door(x, *rest))(x[None].expand(2, *x.shape))
+    if form == "ln":                                         # (a registered op, which vmap takes apart)
+        assert torch.equal(batch(), y[None].expand(2, *y.shape))
+    else:
+        pytest.raises(RuntimeError, batch)                   # (a Function without a rule for it)
+    import torch.autograd.forward_ad as fwd
+    with fwd.dual_level(), pytest.raises(Exception):
+        door(fwd.make_dual(xg, x), *rest)
+    with pytest.raises(RuntimeError):                        # not differentiable twice
+        g = torch.autograd.grad(door(xg, *rest).float().sum(), xg, create_graph=True)[0]
+        torch.autograd.grad(g.float().sum(), xg)
