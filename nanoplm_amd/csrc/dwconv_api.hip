@@ -411,6 +411,30 @@ bool mfma_bwd_preferred(long long T, int taps, int S) {
 bool mfma_gated_bwd_preferred(long long T, int taps, int S) {
     return taps == 31 && (T <= 16384 || T >= 192ll * S);
 }
+// The gated forward on the matrix cores: steps of 64 rows in a run, which a block walks down without staging or gating a halo again.
+// All of a block's runs are of one length, the longest that deals the call out evenly (T=65536, C=1152, 15 taps: runs of 16 steps,
+// three rounds for two and a bit, 115 us, of 13 95).
+int mfma_gated_fwd_steps(long long T, int C) {
+    const int ncb = ceil_div(2LL * C, kMfmaGatedCb), nbt = ncb < kNumCU ? kNumCU / ncb : 1;
+    const long long per_block = ceil_div(ceil_div(T, kMfmaGatedRows), nbt);
+    return ceil_div(per_block, ceil_div(per_block, kMfmaGatedSteps));
+}
+// Which gated forwards take it, measured by the mean rows of a sequence, us, role-split / matrix cores:
+//   31 taps              16 rows      32           75           300          one sequence
+//   T=131072, C=2048     639 / 692    581 / 561    488 / 476    432 / 387    405 / 361
+//   T=131072, C=1152     377 / 410    344 / 334    280 / 278    255 / 225    239 / 208
+//   T=32768, C=768       86 / 83      82 / 68      69 / 58      57 / 43      54 / 38
+//   T=16384, C=1024      59 / 56      -            49 / 40      44 / 33      40 / 31
+//   T=8192, C=512        27 / 22      -            26 / 18      24 / 16      23 / 14
+//   15 taps, T=16384, C=768 44 / 40, -, 34 / 32, 31 / 25, 30 / 22; T=65536, C=1024 139 / 148, 122 / 123, 100 / 105, 90 / 96, 83 / 93
+//   (C=768 115 / 120, 96 / 99, 83 / 81, 75 / 68, 68 / 63; T=131072, C=2048 517 / 551, 441 / 457, 376 / 384, 358 / 335, 353 / 333)
+//   21 taps as 31, 11 as 15: T=16384, C=1152 58 / 66, 54 / 55, 45 / 46, 40 / 37, 39 / 32; C=1024 41 / 45, 37 / 40, 32 / 34, 31 / 28, 29 / 25.
+// A boundary costs the consumers a sweep of their own; short calls gain on every mix because a run begins without a full tile of halo.
+bool mfma_gated_fwd_preferred(long long T, int taps, int S) {
+    if (T < kMfmaMinRows) return false;
+    if (taps == 31) return T <= 16384 || T >= 32ll * S;
+    return T <= 16384 && (taps == 15 || T >= 256ll * S);
+}
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
                     bool gated = false, int tile_rows = 0, int block_bytes = 0) {
     LdsPlan p{};
@@ -921,6 +945,16 @@ int nplm_dwconv_gated_fwd(const void* z, const int32_t* cu, const void* w, const
     if (!gated_supported(false, bf16, T, C, K, (uintptr_t)z | (uintptr_t)y)) return -NPLM_DWCONV_EUNSUPPORTED;
     LdsPlan lp;
     if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)y)) {
+        const int steps = mfma_gated_fwd_steps(T, C);
+        if (bf16 && w_dtype == NPLM_DWCONV_BF16 && mfma_gated_fwd_preferred(T, taps, S) &&
+            make_split_plan(true, bf16, T, C, K, nullptr, &lp, true, steps * kMfmaGatedRows, kMfmaGatedCb) == 0 &&
+            MfmaGatedFwdShape<31>::lds_bytes(ceil_div(lp.ntiles, lp.nbt)) <= kLdsBytes) {
+            const ConvPtrs la{z, nullptr, cu, w, b, y, nullptr};
+            const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | tap_flags);
+            const dim3 grid(lp.ncb * lp.nbt);
+            return (int)(K == 15 ? launch_fwd_gated_mfma_k15(la, lg, steps, grid, (hipStream_t)stream)
+                                 : launch_fwd_gated_mfma_k31(la, lg, steps, grid, (hipStream_t)stream));
+        }
         rc = make_split_plan(true, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;
         const ConvPtrs la{z, nullptr, cu, w, b, y, nullptr};

@@ -164,6 +164,8 @@ NPLM_DECLARE_MFMA_K(15)
 NPLM_DECLARE_MFMA_K(21)
 NPLM_DECLARE_MFMA_K(31)
 #undef NPLM_DECLARE_MFMA_K
+hipError_t launch_fwd_gated_mfma_k15(const ConvPtrs& p, const LdsGeo& g, int steps, dim3 grid, hipStream_t s);
+hipError_t launch_fwd_gated_mfma_k31(const ConvPtrs& p, const LdsGeo& g, int steps, dim3 grid, hipStream_t s);
 hipError_t launch_bwd_gated_mfma_k31(const ConvPtrs& p, const LdsGeo& g, dim3 grid, hipStream_t s);
 // LayerNorm-fused forward (dwconv_ln_kernels.h), K <= 9, fixed shape per dtype, see lds_ln_shape()
 hipError_t launch_ln_fwd_k3(bool bf16, const ConvPtrs& p, const LnArgs& ln, const LdsGeo& g, dim3 grid, hipStream_t s);

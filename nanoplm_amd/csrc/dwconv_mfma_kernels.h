@@ -52,6 +52,7 @@ constexpr int kMfmaCb = 512;           // bytes of a row in one column block: 25
 constexpr int kMfmaCh = kMfmaCb / 2;
 constexpr int kMfmaGatedCb = 256;      // gated kernels: 128 channels (three tiles in each of two buffers)
 constexpr int kMfmaGatedRows = 64;
+constexpr int kMfmaGatedSteps = 16;    // gated forward: steps of 64 rows in a run, at most
 constexpr int kMfmaQ = 4;              // channels of a lane: 8 bytes of a row
 constexpr int kMfmaFwdRows = 64;       // output rows of a forward tile
 // Offset of a store that is to be dropped: beyond the descriptor of a group of output rows (less than 2 GiB) whatever
@@ -156,8 +157,9 @@ struct MfmaMarks {
         return __builtin_amdgcn_readlane(v, 63);
     }
 };
+template <int NWORDS = kMfmaWords>
 __device__ __forceinline__ void mfma_bounds(const int32_t* __restrict__ cu, int S, int T, int a, int n, uint32_t* words, int lane) {
-    if (lane < kMfmaWords) words[lane] = 0;
+    if (lane < NWORDS) words[lane] = 0;
     MfmaMarks m{cu, words, a, n, lane};
     if (lane == 0) m.mark(0);
     if (lane == 1) m.mark(T);
@@ -240,24 +242,72 @@ struct MfmaWeights {
     }
 };
 
+// Ring of chunks (four rows of 128 channels) of h = u * silu(g) in the LDS, as matrix operands: a record holds, per term and channel,
+// the four rows' bf16. Records lie 64 bytes off a multiple of 256 apart, so that the four lanes of a block, which read records one
+// apart, are on different banks (LDS conflict cycles a call of T=131072, C=2048, 31 taps by that offset: 16 8.6e7, 32 4.2e7, 64 1.1e7,
+// which are the stores' ds_bpermute; 397, 379 and 357 us).
+// In phase p the producers write records 16 p - PRE on, 16 of them, and the consumers read the window of the step that begins at
+// record 16 (p - 2): the two ranges are adjacent and fill the ring.
+template <int KT>
+struct MfmaRing {
+    using TP = MfmaTaps<KT>;
+    static constexpr int R = kMfmaGatedRows, CH = kMfmaGatedCb / 2;
+    static constexpr int TERM = CH * 8, REC = 3 * TERM + 64;
+    static constexpr int NWIN = (R + TP::HALO + 3) / 4, PRE = 2 * (R / 4) - NWIN, LEN = NWIN + R / 4;
+    static constexpr int BYTES = LEN * REC;
+    static_assert(PRE >= 0, "a run's first window is written in two phases");
+    // LDS address of an offset that may lie up to one length behind the ring's end (the ring begins the kernel's LDS)
+    __device__ __forceinline__ static uint32_t at(uint32_t x) {
+        const uint32_t w = x - BYTES;                        // (huge in front of the end)
+        return w < x ? w : x;
+    }
+    __device__ __forceinline__ static int next(int slot) { return slot + R / 4 < LEN ? slot + R / 4 : slot + R / 4 - LEN; }
+};
+
 // One wave's conv over staged rows: 16 Q channels, groups of 16 NSTEP output rows. FLIP: dx from dy. RES: the identity is one
 // more band (a single 1 per row), since a bf16 weight plus one is not one in bf16.
 // GATED (backward): the rows are dh; what is stored are the two halves of dz = [dh * silu(g) | dh * u * silu'(g)], with u and
 // g of the row out of their LDS tiles; 256-byte column blocks.
 // LINES: stores with `nt`, for output rows of whole cache lines (see mfma_lines()).
-template <int KT, int NSTEP, bool FLIP, bool RES, bool LINES, bool GATED = false>
+// TERMS = 3 (gated forward): the rows are h in fp32, as three bf16 terms that add up to it, out of a ring of chunks that are
+// already packed (MfmaRing).
+template <int KT, int NSTEP, bool FLIP, bool RES, bool LINES, bool GATED = false, int TERMS = 1>
 struct MfmaConv {
     using TP = MfmaTaps<KT>;
-    static constexpr int Q = GATED ? 2 : kMfmaQ, NCK = TP::NCK, CB = GATED ? kMfmaGatedCb : kMfmaCb;
+    static constexpr bool RING = TERMS > 1;
+    using RG = MfmaRing<KT>;
+    static constexpr int Q = GATED || RING ? 2 : kMfmaQ, NCK = TP::NCK, CB = GATED ? kMfmaGatedCb : kMfmaCb;
     static constexpr MfmaSwz SWZ = GATED ? SWZ_BOTH : SWZ_QUAD;
     static constexpr int ROWS = 16 * NSTEP;                  // output rows of a group
     static_assert(ROWS % 32 == 0, "a group's boundary bits start at a word");
     static constexpr int NCHUNK = 4 * (NSTEP - 1) + NCK;     // chunks that the steps of a group read (per lane)
     static constexpr int IDC = (TP::FRONT + 0) / 4;          // chunk of the identity's first row
     static constexpr int IDN = (TP::FRONT + 3) / 4 - IDC + 1;
+    struct Chunk {
+        MfmaChunk<Q> t[TERMS];
+        __device__ __forceinline__ void mask(uint32_t m0, uint32_t m1) {
+#pragma unroll
+            for (int i = 0; i < TERMS; ++i)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) { t[i].b[q].x &= m0; t[i].b[q].y &= m1; }
+        }
+        __device__ __forceinline__ void drop_non_finite() {
+#pragma unroll
+            for (int i = 0; i < TERMS; ++i) t[i].drop_non_finite();
+        }
+    };
+    using Raw = std::conditional_t<RING, Chunk, MfmaRaw<Q>>;
+    // a group's (or step's) first window row: its address in the tile (RING: the offset in the ring of the lane's slice of its chunk,
+    // or that plus the ring's length)
+    using At = std::conditional_t<RING, uint32_t, const char*>;
+    __device__ __forceinline__ static At step_at(At lp, int s) { return lp + (RING ? 4 * s * RG::REC : 16 * s * CB); }
+    __device__ __forceinline__ static void pack(const Raw& r, Chunk& c) {
+        if constexpr (RING) c = r; else mfma_pack(r, c.t[0]);
+    }
     s16x4 A[NCK][Q];
     s16x4 I[RES ? IDN : 1];
     f32x4 bias;            // where the sums start (dx: 0)
+    uint32_t slice;        // RING: the lane's slice of chunk n from the ring's start
     int off[4];            // LDS offset of the lane's slice of chunk c, by c & 3 (without c * 4 rows)
     int n;                 // the lane's column: output rows 4 n .. 4 n + 3 of a step
     int c0;                // its first channel
@@ -282,7 +332,8 @@ struct MfmaConv {
         w = w_;
         w_flags = w_flags_;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) off[k] = 4 * n * CB + ((lcc * 2) ^ mfma_place((n + k) & 3));
+        for (int k = 0; k < 4; ++k) off[k] = RING ? 0 : 4 * n * CB + ((lcc * 2) ^ mfma_place((n + k) & 3));
+        slice = n * RG::REC + lcc * 8;
         const int p0 = (4 - n) >> 1, sh = (n & 1) * 16;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -318,26 +369,38 @@ struct MfmaConv {
         return f32x4{b, b, b, b};
     }
     // acc += the products of window chunk k (FINITE: without the weights that are not finite)
+    // (term and channel i of the TERMS * Q alone)
     template <int k, bool FINITE = false>
-    __device__ __forceinline__ void taps(f32x4 (&acc)[Q], const MfmaChunk<Q>& x) const {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            s16x4 w4 = A[k][q];
-            if constexpr (FINITE) {
-                u32x2 t = __builtin_bit_cast(u32x2, w4);
-                asm volatile("" : "+v"(t.x), "+v"(t.y));     // (not formed ahead of the steps and kept in registers)
-                w4 = __builtin_bit_cast(s16x4, finite_bf16x4(t));
-            }
-            acc[q] = mfma4(w4, x.op(q), acc[q]);
+    __device__ __forceinline__ void tap(f32x4 (&acc)[Q], const Chunk& x, int i) const {
+        const int q = i % Q;
+        s16x4 w4 = A[k][q];
+        if constexpr (FINITE) {
+            u32x2 t = __builtin_bit_cast(u32x2, w4);
+            asm volatile("" : "+v"(t.x), "+v"(t.y));         // (not formed ahead of the steps and kept in registers)
+            w4 = __builtin_bit_cast(s16x4, finite_bf16x4(t));
         }
-        if constexpr (RES && k >= IDC && k < IDC + IDN) {
+        acc[q] = mfma4(w4, x.t[i / Q].op(q), acc[q]);
+        if constexpr (RES && k >= IDC && k < IDC + IDN) acc[q] = mfma4(I[k - IDC], x.t[i / Q].op(q), acc[q]);
+    }
+    template <int k, bool FINITE = false>
+    __device__ __forceinline__ void taps(f32x4 (&acc)[Q], const Chunk& x) const {
 #pragma unroll
-            for (int q = 0; q < Q; ++q) acc[q] = mfma4(I[k - IDC], x.op(q), acc[q]);
-        }
+        for (int i = TERMS * Q - 1; i >= 0; --i) tap<k, FINITE>(acc, x, i);      // (the smaller terms first)
     }
     // window chunk c of the lane, its first ROWS rows
     template <int c, int ROWS = 4>
-    __device__ __forceinline__ void read(const char* lp, MfmaRaw<Q>& o) const {
+    __device__ __forceinline__ void read(At lp, Raw& o) const {
+        if constexpr (RING) {
+            const uint32_t at = RG::at(lp + c * RG::REC);
+#pragma unroll
+            for (int i = 0; i < TERMS; ++i) {
+                const u32x4 v = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(at + i * RG::TERM);
+                o.t[i].b[0] = u32x2{v.x, v.y};
+                o.t[i].b[1] = u32x2{v.z, v.w};
+            }
+            if constexpr (ROWS < 4) o.mask(ROWS == 1 ? 0xffffu : ~0u, ROWS == 3 ? 0xffffu : 0u);
+            return;
+        } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if (r < ROWS) {
@@ -349,6 +412,7 @@ struct MfmaConv {
 #pragma unroll
                 for (int h = 0; h < Q / 2; ++h) o.r[r][h] = 0;
             }
+        }
         }
     }
     // Adjacent lanes of a sum are rows 0, 4, 8, 12; they trade places first, so that 16 adjacent lanes store the 32 Q bytes
@@ -436,16 +500,16 @@ struct MfmaConv {
     // sequence, window rows [lo, hi): chunks without any of its rows are left out, those at its ends masked, rows outside it not
     // stored. Returns whether all sums are finite (those that are not have to be formed again).
     template <bool PART>
-    __device__ __forceinline__ bool sweep(const char* lp, int lo, int hi, rsrc_t ro, int rowb, const char* up) const {
+    __device__ __forceinline__ bool sweep(At lp, int lo, int hi, rsrc_t ro, int rowb, const char* up) const {
         float chk = PART ? odd : 0.f;
         f32x4 acc[(NCK + 3) / 4][Q];
-        MfmaRaw<Q> raw;
+        Raw raw;
         read<0>(lp, raw);
         int range = 0;                                       // output rows [o, e) of the group, relative to the storing lane's first
         if constexpr (PART) range = __builtin_amdgcn_ds_bpermute(swap, 4 * n);
         static_for<NCHUNK>([&](auto c_c) __attribute__((always_inline)) {
             constexpr int c = decltype(c_c)::value;
-            const MfmaRaw<Q> cur = raw;
+            const Raw cur = raw;
             if constexpr (c + 1 < NCHUNK)
                 read<c + 1, (c + 1 == NCHUNK - 1 ? TP::LASTROWS : 4)>(lp, raw);
             static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
@@ -456,19 +520,21 @@ struct MfmaConv {
                 }
             });
             if (!PART || (4 * c < hi && 4 * c + 16 > lo)) {
-                MfmaChunk<Q> x;
-                mfma_pack(cur, x);
+                Chunk x;
+                pack(cur, x);
                 if (PART && (4 * c < lo || 4 * c + 16 > hi)) {
                     uint32_t m0, m1;
                     chunk_masks(c, lo, hi, m0, m1);
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) { x.b[q].x &= m0; x.b[q].y &= m1; }
+                    x.mask(m0, m1);
                 }
-                static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
-                    constexpr int s = decltype(s_c)::value;
-                    constexpr int k = c - 4 * s;
-                    if constexpr (k >= 0 && k < NCK) taps<k>(acc[s % ((NCK + 3) / 4)], x);
-                });
+                // (the sums of all steps by turns: a product waits for the one before it in its sum)
+#pragma unroll
+                for (int i = TERMS * Q - 1; i >= 0; --i)
+                    static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
+                        constexpr int s = decltype(s_c)::value;
+                        constexpr int k = c - 4 * s;
+                        if constexpr (k >= 0 && k < NCK) tap<k>(acc[s % ((NCK + 3) / 4)], x, i);
+                    });
             }
             static_for<NSTEP>([&](auto s_c) __attribute__((always_inline)) {
                 constexpr int s = decltype(s_c)::value;
@@ -500,7 +566,7 @@ struct MfmaConv {
     // One group of output rows: lp = the group's first window row in LDS, words = the tile's boundary bits, p0 = the window row's
     // place among them; ro = descriptor of the group's output rows (those in front of T).
     // GATED: up = the group's first row in the u tile; the g tile lies kMfmaGatedRows rows behind it.
-    __device__ __forceinline__ void rows(const char* lp, const uint32_t* words, int p0, rsrc_t ro, int rowb, const char* up = nullptr) const {
+    __device__ __forceinline__ void rows(At lp, const uint32_t* words, int p0, rsrc_t ro, int rowb, const char* up = nullptr) const {
         const uint32_t* wp = words + (p0 >> 5);              // p0 is a multiple of 32
         bool open;                                           // no boundary inside the window (a bit at its first row is none)
         {
@@ -525,7 +591,7 @@ struct MfmaConv {
 #pragma nounroll
         for (int s = 0; s < NSTEP; ++s) {
             const MfmaBits bits = window_bits(wp, s);
-            const char* sp = lp + 16 * s * CB;
+            const At sp = step_at(lp, s);
             int i0 = 0;
             do {
                 int lo, hi;
@@ -565,7 +631,7 @@ struct MfmaConv {
 
     // The sums of a step (sp: its first window row) over the window rows [lo, hi) alone. FINITE: products of finite factors alone.
     template <bool FINITE>
-    __device__ __forceinline__ void pass(const char* sp, int lo, int hi, f32x4 (&acc)[Q]) const {
+    __device__ __forceinline__ void pass(At sp, int lo, int hi, f32x4 (&acc)[Q]) const {
         const MfmaBits in = mfma_row_mask(lo, hi);
         // window rows that some lane's pass takes, and those that every lane's takes (lanes of a column hold the same):
         // a chunk that none takes is skipped, one that all take whole needs no mask
@@ -573,7 +639,7 @@ struct MfmaConv {
         mfma_columns(in, some, every);
 #pragma unroll
         for (int q = 0; q < Q; ++q) acc[q] = start(q);
-        MfmaRaw<Q> raw;
+        Raw raw;
         if constexpr (!FINITE) {
             read<0>(sp, raw);
             asm volatile("" ::: "memory");                   // (else the reads move into the first chunk's branch, in front of their use)
@@ -581,18 +647,17 @@ struct MfmaConv {
         static_for<NCK>([&](auto k_c) __attribute__((always_inline)) {
             constexpr int k = decltype(k_c)::value;
             if constexpr (FINITE) read<k, (k == NCK - 1 ? TP::LASTROWS : 4)>(sp, raw);      // (rarely run: few registers)
-            const MfmaRaw<Q> cur = raw;
+            const Raw cur = raw;
             if constexpr (!FINITE && k + 1 < NCK)
                 read<k + 1, (k + 1 == NCK - 1 ? TP::LASTROWS : 4)>(sp, raw);
             if ((some >> (4 * k)) & 15) {
-                MfmaChunk<Q> x;
-                mfma_pack(cur, x);
+                Chunk x;
+                pack(cur, x);
                 if (((every >> (4 * k)) & 15) != 15) {
                     const uint32_t b4 = 4 * k < 32 ? in.lo >> (4 * k & 31) : in.hi >> (4 * k & 31);
                     const uint32_t m0 = __builtin_amdgcn_perm((uint32_t)((int)(b4 << 30) >> 31), (uint32_t)((int)(b4 << 31) >> 31), 0x05040100);
                     const uint32_t m1 = __builtin_amdgcn_perm((uint32_t)((int)(b4 << 28) >> 31), (uint32_t)((int)(b4 << 29) >> 31), 0x05040100);
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) { x.b[q].x &= m0; x.b[q].y &= m1; }
+                    x.mask(m0, m1);
                 }
                 if constexpr (FINITE) x.drop_non_finite();
                 taps<k, FINITE>(acc, x);
@@ -601,7 +666,7 @@ struct MfmaConv {
         });
     }
     // v += the products of output row 4 n + i of the step that are in its pass's window rows [lo, hi) and have a factor that is not finite
-    __device__ __forceinline__ void add_non_finite(const char* sp, int i, int lo, int hi, float (&v)[Q]) const {
+    __device__ __forceinline__ void add_non_finite(At sp, int i, int lo, int hi, float (&v)[Q]) const {
         const int koff = w_tap_off(w_flags), kw = TP::KP - 2 * koff;
         const bool res = (w_flags & W_RESIDUAL) != 0;
 #pragma nounroll
@@ -609,11 +674,24 @@ struct MfmaConv {
             const int p = TP::FRONT + i - TP::PP + m;           // window row of tap m
             if (p < lo || p >= hi || !active) continue;
             // (the lane's row 4 n + p of the step: its piece is where the chunk of that row has it)
+            float f[Q];
+            if constexpr (RING) {
+                const uint32_t at = RG::at(sp + (p >> 2) * RG::REC) + (p & 3) * 2;
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    f[q] = 0.f;
+#pragma unroll
+                    for (int t = TERMS - 1; t >= 0; --t) {   // (of a value that is not finite the first term is it)
+                        const float v = bf16_to_f32(*(const __attribute__((address_space(3))) uint16_t*)(uintptr_t)(at + t * RG::TERM + q * 8));
+                        f[q] = t == 0 && !__builtin_isfinite(v) ? v : f[q] + v;
+                    }
+                }
+            } else {
             const char* a = sp + (off[0] ^ mfma_place((((p >> 2) + (SWZ == SWZ_BOTH ? p : 0) + n) & 3) ^ n)) + p * CB;
             RowVec<true, Q> x;
-            float f[Q];
             x.load(a);
             x.to_f32(f);
+            }
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
                 const float wq = mfma_weight<TP::KP, FLIP>(w, w_flags, c0 + q, m, res);
@@ -1399,6 +1477,172 @@ dwconv_bwd_gated_mfma_kernel(const void* __restrict__ z, const void* __restrict_
             if (dv < half) dw.take(box + dv * DW::BOX, lane);
         }
         if (dv == 0 && 2 * lane < nch) dw.finish(partial + (size_t)tb * (KT + 1) * C, C, cb * SH::CH + 2 * lane);
+    }
+}
+
+// ---- gated forward ---------------------------------------------------------------------------------------------------
+// y = conv(h), h = u * silu(g) of z = [u | g] [T, 2C]. h is fp32 and stays it: the producers split it into three bf16 terms that add
+// up to it exactly (8 significant bits each, by truncation), and the consumers take the products of all three with the taps, which are
+// exact as well. So the sums differ from the vector ALU's by their order alone. (The third term of an h below 2^-109 is cut off at
+// bf16's smallest subnormal, 2^-133.)
+// What bounds it: on the vector ALU the 31 FMAs an element (0.8 of all issue slots); here the gate and the split, 14
+// instructions an element of which two are quarter-rate, each evaluated once: a block walks down a run of steps of 64 rows, and a
+// step's window takes over the halo rows from the step before in the ring. The producers alone take 201 us, the consumers alone 257
+// with one of 64 rows per SIMD (boundaries then cost twice what they do with two of 32: 430 and 395 us on log-normal lengths).
+// T=131072, C=2048, 31 taps, before and now: one sequence 393 to 413 and 357 to 369 us, log-normal lengths 415 to 444 and 387 to 406;
+// T=32768, C=768, 300 rows a sequence 57 and 43; T=8192, C=512 24 and 16. Outputs that are not the correctly rounded value 6.3e-5 (7.8e-5). Waves: 8 consumers (32 channels x 32 rows of a step; no packing, no gate), 8 producers (a
+// chunk of 4 rows x 128 channels at a time, z straight into registers two phases ahead). The boundary bits of all the block's runs are
+// found before the first.
+template <int KT>
+struct MfmaGatedFwdShape {
+    using TP = MfmaTaps<KT>;
+    using RG = MfmaRing<KT>;
+    static constexpr int NCW = 4, NCONS = 8, RW = RG::R * NCW / NCONS, NPROD = 8, UNITS = RG::R / 4 / NPROD, NW = NCONS + NPROD, NT = NW * 64;
+    static constexpr int WORDS = (kMfmaGatedSteps * RG::R + TP::HALO + 31) / 32 + 2;     // boundary bits of a run (lanes read two words further)
+    static_assert(WORDS <= 64, "a wave clears them in one go");
+    using W = MfmaWeights<KT, RG::CH, NCONS>;
+    static_assert(W::BYTES <= RG::BYTES, "the weight table lies in the ring until it is written");
+    static_assert(RG::BYTES + 64 * WORDS * 4 <= kLdsBytes, "fits the LDS");
+    // LDS of a call whose blocks have up to this many runs; the words begin behind the ring
+    static constexpr long long lds_bytes(long long runs) { return RG::BYTES + runs * WORDS * 4; }
+};
+
+template <int KT, bool RES>
+__global__ void __launch_bounds__(MfmaGatedFwdShape<KT>::NT)
+dwconv_fwd_gated_mfma_kernel(const void* __restrict__ z, const int32_t* __restrict__ cu, const void* __restrict__ w,
+                             const void* __restrict__ bias, void* __restrict__ y, const LdsGeo g, const int steps) {
+    using SH = MfmaGatedFwdShape<KT>;
+    using TP = MfmaTaps<KT>;
+    using RG = MfmaRing<KT>;
+    constexpr int R = RG::R;
+    extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+    uint32_t* words = reinterpret_cast<uint32_t*>(lds_raw + RG::BYTES);
+    uint32_t* tab = reinterpret_cast<uint32_t*>(lds_raw);
+    const int lane = (int)(threadIdx.x & 63);
+    const int wv = wave_id();
+    int cb, tb;
+    lds_block_coords(g, cb, tb);
+    const int T = g.T, C = g.C;
+    const int rowb = C * 2;
+    const int col_byte0 = cb * kMfmaGatedCb;
+    const int valid_bytes = rowb - col_byte0 < kMfmaGatedCb ? rowb - col_byte0 : kMfmaGatedCb;
+    const int nch = valid_bytes / 2;
+    // the block's runs: one a round, none in the last round where the slot lies past the last run
+    const int rounds = (g.ntiles + g.nbt - 1) / g.nbt;
+    const int last = (int)((tb + (long long)(rounds - 1) * g.rot_step) % g.nbt);
+    const int runs = lds_tile_row0(g, rounds - 1, last, R * steps) < T ? rounds : rounds - 1;
+    const int phases = runs > 0 ? runs * (steps + 1) + 1 : 0;
+    auto bounds = [&]() __attribute__((always_inline)) {
+        int q = tb;
+        for (int it = 0; it < runs; ++it) {
+            if (it % SH::NW == wv)
+                mfma_bounds<SH::WORDS>(cu, g.S, T, lds_tile_row0(g, it, q, R * steps) - TP::FRONT, R * steps + TP::HALO, words + it * SH::WORDS, lane);
+            q = lds_next_slot(g, q);
+        }
+    };
+
+    if (wv < SH::NCONS) {
+        __builtin_amdgcn_s_setprio(1);       // (the longer way through a phase)
+        SH::W::template fill<false>(tab, w, g.w_flags, cb * RG::CH, nch, (int)threadIdx.x);
+        bounds();
+        lds_barrier();
+        const int rg = wv / SH::NCW, r0 = rg * SH::RW;
+        MfmaConv<KT, SH::RW / 16, false, RES, false, false, 3> conv;      // (stores without `nt`: 64 bytes of a row at a time)
+        conv.init(tab, SH::W::odd(tab), w, g.w_flags, bias, wv % SH::NCW, lane, cb * RG::CH, nch, rowb);
+        lds_barrier();                       // the table has been read
+        int slot = 0, it = 0, s = 0, q = tb, row0 = lds_tile_row0(g, 0, q, R * steps);
+        for (int p = 0; p < phases; ++p) {
+            if (p >= 2) {
+                const int t0 = row0 + s * R + r0;
+                if (s < steps && t0 < T)
+                    conv.rows(conv.slice + (slot + r0 / 4) * RG::REC, words + it * SH::WORDS, s * R + r0,
+                              mfma_out_rsrc(y, t0, T - t0 < SH::RW ? T - t0 : SH::RW, rowb), rowb);
+                slot = RG::next(slot);
+                if (++s > steps) {           // (the phase between two runs has no step)
+                    s = 0;
+                    q = lds_next_slot(g, q);
+                    row0 = lds_tile_row0(g, ++it, q, R * steps);
+                }
+            }
+            lds_barrier();
+        }
+    } else {
+        const int pw = wv - SH::NCONS;
+        struct Unit { uint32_t u[4], g[4]; };
+        struct Step { Unit a[SH::UNITS]; };
+        const int zrow = 2 * rowb, at_lane = lane * 4 < valid_bytes ? col_byte0 + lane * 4 : (int)0xc0000000;
+        int it = 0, j = 0, q = tb, row0 = runs > 0 ? lds_tile_row0(g, 0, q, R * steps) : T;
+        // the loads of the next phase in the order of phases; rows that do not exist land as zeros (or, in front of row 0 of a
+        // tensor beyond 4 GiB, as other rows: what becomes of them is never used)
+        auto fetch = [&](Step& o) __attribute__((always_inline)) {
+            const int first = row0 - TP::FRONT, rb = first > 0 ? first : 0;
+            const bool live = it < runs;
+            const rsrc_t rs = live ? rows_rsrc(z, rb, T, (size_t)zrow) : make_rsrc(z, 0);
+#pragma unroll
+            for (int i = 0; i < SH::UNITS; ++i) {
+                const int k = 16 * j - RG::PRE + pw + i * SH::NPROD;         // chunk of the run (below 0: none)
+                const int at = k >= 0 ? (first - rb + 4 * k) * zrow + at_lane : (int)0xc0000000;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    o.a[i].u[r] = __builtin_amdgcn_raw_buffer_load_b32(rs, at + r * zrow, 0, 0);
+                    o.a[i].g[r] = __builtin_amdgcn_raw_buffer_load_b32(rs, at + r * zrow + rowb, 0, 0);
+                }
+            }
+            if (++j > steps) {
+                j = 0;
+                q = lds_next_slot(g, q);
+                row0 = ++it < runs ? lds_tile_row0(g, it, q, R * steps) : 0;
+            }
+        };
+        auto make = [&](const Step& v, int slot) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < SH::UNITS; ++i) {
+                int rec = slot + pw + i * SH::NPROD;
+                rec = rec < RG::LEN ? rec : rec - RG::LEN;
+                float h[2][4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    h[0][r] = gate_mul(bf16_lo(v.a[i].u[r]), bf16_lo(v.a[i].g[r]));
+                    h[1][r] = gate_mul(bf16_hi(v.a[i].u[r]), bf16_hi(v.a[i].g[r]));
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(h[0][r]), "+v"(h[1][r]));     // (h rounded: no product is contracted into the differences)
+                const uint32_t at = rec * RG::REC + lane * 16;
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    u32x4 o;
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        o[2 * c] = __builtin_amdgcn_perm(__float_as_uint(h[c][1]), __float_as_uint(h[c][0]), 0x07060302);
+                        o[2 * c + 1] = __builtin_amdgcn_perm(__float_as_uint(h[c][3]), __float_as_uint(h[c][2]), 0x07060302);
+                        if (t < 2) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) h[c][r] -= bf16_hi(__float_as_uint(h[c][r]));
+                        }
+                    }
+                    *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(at + t * RG::TERM) = o;
+                }
+            }
+        };
+        Step a, b;
+        fetch(a);
+        fetch(b);
+        bounds();
+        lds_barrier();
+        lds_barrier();
+        int slot = (RG::LEN - RG::PRE) % RG::LEN;
+        // (the way out in the middle of the body keeps "all but the other step's loads have landed" a wait for a count)
+        for (int p = 0; p < phases; ++p) {
+            make(a, slot);
+            slot = RG::next(slot);
+            fetch(a);
+            lds_barrier();
+            if (++p == phases) break;
+            make(b, slot);
+            slot = RG::next(slot);
+            fetch(b);
+            lds_barrier();
+        }
     }
 }
 

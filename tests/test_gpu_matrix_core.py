@@ -401,3 +401,58 @@ def test_share_of_outputs_that_are_not_correctly_rounded(K):
         share = [float((f(_lib.Tuning(algo=a)).cpu() != ref).double().mean()) for a in (4, 1)]
         print(f"[share] K={K} {name}: matrix cores {share[0]:.2e}, vector {share[1]:.2e}", flush=True)
         assert share[0] <= K * 2.0 ** -16 and share[0] <= 2 * share[1] + 2e-6
+
+
+# (built as 15 and 31 taps; whole, partial and several column blocks; one run a block, and with C=8200 two; runs that end inside a
+# step; a boundary at every row of the 32-row groups, one to many in a group)
+@pytest.mark.parametrize("K,lens,C", [(31, LENS * 2, 512), (29, LENS[::-1] * 2, 520), (25, [4096], 1000), (31, [95] * 44, 520),
+                                      (31, [191] * 22, 8200), (15, LENS * 2, 776), (13, [63] * 66, 1160), (21, [4095, 1], 512),
+                                      (11, [2500, 1, 1700], 520), (31, [1] * 4100, 512), (15, [17] * 260, 512)])
+def test_gated_forward_on_the_matrix_cores_matches_the_oracle(K, lens, C):
+    """To one bf16 rounding of the oracle's y: the three bf16 terms add up to the fp32 h. The same bits again after a call that left NaN
+    in the LDS; rows in front of and behind y keep theirs."""
+    print(f"[case] gated forward K={K} C={C}", flush=True)
+    _, cu, w, b, dy = _case(lens, C, K, C + K)
+    T = dy.shape[0]
+    z = torch.randn(T, 2 * C, generator=torch.Generator().manual_seed(C)).bfloat16()
+    zd, cud, wd, bd = z.to(DEV), cu.to(DEV), w.to(DEV), b.to(DEV)
+    lib = _lib.load()
+    for res in (False, True):
+        y64 = O.ref_gated_dwconv_grads(z, cu, w, b, None, torch.float64, res)
+        y = npa.gated_dwconv_fwd(zd, cud, wd, bd, residual=res)
+        assert_act_close(y, y64, torch.bfloat16, "y")
+        npa.gated_dwconv_fwd(torch.full_like(zd, float("nan")), cud, wd, bd, residual=res)
+        room = torch.full((T + 4, C), 7.0, dtype=torch.bfloat16, device=DEV)
+        _lib.check(lib.nplm_dwconv_gated_fwd(zd.data_ptr(), cud.data_ptr(), wd.data_ptr(), bd.data_ptr(), room[2:].data_ptr(), T, C, K,
+                                             len(lens), _lib.BF16, _lib.BF16, _lib.RESIDUAL if res else 0,
+                                             torch.cuda.current_stream().cuda_stream), "gated_fwd")
+        assert torch.equal(room[2:T + 2], y) and bool((room[:2] == 7).all()) and bool((room[T + 2:] == 7).all())
+
+
+@pytest.mark.parametrize("K", [15, 31])
+@pytest.mark.parametrize("where", ["u", "gate", "weight"])
+def test_gated_forward_non_finite_values_reach_the_rows_of_their_taps_only(K, where):
+    """Against the vector ALU's kernel (which takes the same weights in fp32): the same outputs are not finite, in the same way, and
+    the others differ by a rounding; rows of other sequences keep the bits of a clean call."""
+    C, lens = 512, [40, 1, 700, 1, 213, 64, 1, 33, 2, 1500, 1, 1700]
+    _, cu, w, b, dy = _case(lens, C, K, 3)
+    z = torch.randn(dy.shape[0], 2 * C, generator=torch.Generator().manual_seed(5)).bfloat16()
+    cud, bd = cu.to(DEV), b.to(DEV)
+    clean = npa.gated_dwconv_fwd(z.to(DEV), cud, w.to(DEV), bd)
+    hit = torch.zeros(dy.shape[0], dtype=torch.bool)
+    if where == "weight":
+        w[5::7, K // 2 - 3], w[6::7, K // 2] = float("inf"), float("nan")
+    else:
+        off = 0 if where == "u" else C
+        for i, n in enumerate(lens):
+            if n <= 2:
+                hit[cu[i]:cu[i + 1]] = True
+                z[cu[i], off + i % 7:off + C:7] = float("nan") if i % 2 else float("inf")
+        z[1700:1701, off:off + C:5] = -float("inf")          # inside a long sequence
+        hit[1055:2555] = True
+    y = npa.gated_dwconv_fwd(z.to(DEV), cud, w.to(DEV), bd)
+    want = npa.gated_dwconv_fwd(z.to(DEV), cud, w.to(DEV).float(), bd.float())
+    assert not bool(torch.isfinite(want).all())
+    torch.testing.assert_close(y, want, rtol=2.0 ** -7, atol=1e-5, equal_nan=True)
+    if where != "weight":
+        assert torch.equal(y[~hit.to(DEV)], clean[~hit.to(DEV)])
