@@ -529,15 +529,15 @@ __device__ __forceinline__ void finalize_block(float (&red)[SPLIT][64], int bloc
     if (on) {
         const float* src = partial + o;
         const size_t stride = (size_t)n_out;
-        int p = p0;
-        for (; p + 8 <= p1; p += 8) {
+        // Eight loads at a time whatever the group's share (those past its end repeat its last slab and are not added): one after the
+        // other a share of six took 6 times the latency of memory.
+        for (int p = p0; p < p1; p += 8) {
             float t[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) t[i] = src[(size_t)(p + i) * stride];
+            for (int i = 0; i < 8; ++i) t[i] = src[(size_t)(p + i < p1 ? p + i : p1 - 1) * stride];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s += t[i];
+            for (int i = 0; i < 8; ++i) s = p + i < p1 ? s + t[i] : s;
         }
-        for (; p < p1; ++p) s += src[(size_t)p * stride];
     }
     red[grp][lane] = s;
     __syncthreads();
