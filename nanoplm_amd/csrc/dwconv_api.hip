@@ -408,6 +408,7 @@ bool mfma_bwd_preferred(long long T, int taps, int S) {
 // role-split kernel's roles, which share the loss, once a call is longer than its first tiles. 15 taps (T=131072, C=1024: 302/264,
 // T=4096: 19/22) and 21 (306/299) have too few FMAs to save. Calls of up to 16384 rows take it whatever begins in them (C=1024):
 //   T=16384   1 row 138/228   4 71/96   16 66/82   32 63/77   75 67/65        T=4096   1 row 45/83   8 27/40   32 26/39   75 26/36
+// and so do the shortest: T=2048, C=768 1 row 30/49, 16 25/30, 75 21/29, 300 19/27, one sequence 18/26; T=20, C=512 18/21.
 bool mfma_gated_bwd_preferred(long long T, int taps, int S) {
     return taps == 31 && (T <= 16384 || T >= 192ll * S);
 }
@@ -426,14 +427,15 @@ int mfma_gated_fwd_steps(long long T, int C) {
 //   T=32768, C=768       86 / 83      82 / 68      69 / 58      57 / 43      54 / 38
 //   T=16384, C=1024      59 / 56      -            49 / 40      44 / 33      40 / 31
 //   T=8192, C=512        27 / 22      -            26 / 18      24 / 16      23 / 14
+//   T=2048, C=768        26 / 15      -            26 / 13      24 / 12      23 / 12     (one of the role-split tiles of 128 rows takes 22)
+//   T=20, C=512          22 / 12      -            -            -            21 / 12
 //   15 taps, T=16384, C=768 44 / 40, -, 34 / 32, 31 / 25, 30 / 22; T=65536, C=1024 139 / 148, 122 / 123, 100 / 105, 90 / 96, 83 / 93
 //   (C=768 115 / 120, 96 / 99, 83 / 81, 75 / 68, 68 / 63; T=131072, C=2048 517 / 551, 441 / 457, 376 / 384, 358 / 335, 353 / 333)
-//   21 taps as 31, 11 as 15: T=16384, C=1152 58 / 66, 54 / 55, 45 / 46, 40 / 37, 39 / 32; C=1024 41 / 45, 37 / 40, 32 / 34, 31 / 28, 29 / 25.
+//   21 taps as 31, 11 as 15: T=2048, C=768 (21 taps) 26 / 15, -, 20 / 13, 19 / 13, 19 / 12; T=4000, C=2048 31 / 34, -, 27 / 26, 25 / 23, 24 / 21; T=16384, C=1152 58 / 66, 54 / 55, 45 / 46, 40 / 37, 39 / 32; C=1024 41 / 45, 37 / 40, 32 / 34, 31 / 28, 29 / 25.
 // A boundary costs the consumers a sweep of their own; short calls gain on every mix because a run begins without a full tile of halo.
 bool mfma_gated_fwd_preferred(long long T, int taps, int S) {
-    if (T < kMfmaMinRows) return false;
     if (taps == 31) return T <= 16384 || T >= 32ll * S;
-    return T <= 16384 && (taps == 15 || T >= 256ll * S);
+    return T <= 2048 || (T <= 16384 && (taps == 15 || T >= 256ll * S));
 }
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
                     bool gated = false, int tile_rows = 0, int block_bytes = 0) {
@@ -1229,7 +1231,7 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
     if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {
         LdsPlan lp;
-        const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 && T >= kMfmaMinRows &&
+        const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 &&
                           mfma_tile_fits(C, K, true) && mfma_lines_ok(true, true, T, C, K, taps, (uintptr_t)dz) &&
                           mfma_gated_bwd_preferred(T, taps, S);
         rc = mfma ? make_split_plan(false, bf16, T, C, K, nullptr, &lp, true, kMfmaGatedRows, kMfmaGatedCb)
