@@ -49,6 +49,10 @@ int dtype_code(const at::Tensor& t) {
 bool dense(const at::Tensor& t, const at::Device& dev) {
     return t.layout() == at::kStrided && t.device() == dev && t.is_contiguous();
 }
+// a parameter of one value a channel, in w's dtype on its device
+bool vector_as(const at::Tensor& t, const at::Tensor& w, int32_t C) {
+    return dense(t, w.device()) && t.dim() == 1 && t.size(0) == C && t.scalar_type() == w.scalar_type();
+}
 
 struct Sizes {
     int64_t T;
@@ -64,7 +68,7 @@ bool sizes_of(const at::Tensor& x, int width, const at::Tensor& cu, const at::Te
     if (s->act < 0 || s->wdt < 0) return false;
     const int64_t C = x.size(1) / width, K = w.size(1);
     if (x.size(1) % width || w.size(0) != C || K % 2 == 0 || C > INT_MAX || K > INT_MAX || cu.numel() > INT_MAX) return false;
-    if (b && !(dense(*b, dev) && b->dim() == 1 && b->size(0) == C && b->scalar_type() == w.scalar_type())) return false;
+    if (b && !vector_as(*b, w, (int32_t)C)) return false;
     s->T = x.size(0);
     s->C = (int32_t)C;
     s->K = (int32_t)K;
@@ -96,12 +100,19 @@ at::Tensor as(const at::Tensor& t, bool wanted, at::ScalarType dt) {
 
 // The Python route of a backward whose call turns out to be of another form (its result as a list of tensors).
 template <typename... Args>
-variable_list python_backward(const char* module, const char* name, const Args&... args) {
+variable_list python_backward(const char* module, const char* name, Args&&... args) {
     pybind11::gil_scoped_acquire gil;
-    pybind11::object out = pybind11::module_::import(module).attr(name)(args...);
+    pybind11::object out = pybind11::module_::import(module).attr(name)(std::forward<Args>(args)...);
     variable_list r;
     for (pybind11::handle h : out) r.push_back(h.is_none() ? at::Tensor() : h.cast<at::Tensor>());
     return r;
+}
+
+// The tensors of a backward are what saved-tensor hooks gave back, which need not be what was saved: whether they still are as the
+// kernels take them. If not, the Python route makes them so or refuses them.
+bool usual_backward(const at::Tensor& x, int width, const at::Tensor& cu, const at::Tensor& w, const at::Tensor& dy, Sizes* s) {
+    return x.defined() && cu.defined() && w.defined() && sizes_of(x, width, cu, w, std::nullopt, s) && dense(dy, x.device()) &&
+           dy.dim() == 2 && dy.size(0) == s->T && dy.size(1) == s->C;
 }
 
 struct Plain : torch::autograd::Function<Plain> {
@@ -127,12 +138,18 @@ struct Plain : torch::autograd::Function<Plain> {
         const bool has_bias = ctx->saved_data["bias"].toBool(), residual = ctx->saved_data["residual"].toBool();
         const bool need_dx = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(2), need_b = has_bias && ctx->needs_input_grad(3);
         Sizes s;
-        sizes_of(x, 1, cu, w, std::nullopt, &s);
         const c10::DeviceGuard guard(x.device());
         const at::Tensor dy = incoming(grads[0], x);
-        const bool bf16 = s.wdt == NPLM_DWCONV_BF16;
+        const bool bf16 = w.scalar_type() == at::kBFloat16;
         const at::ScalarType gdt = w.scalar_type();          // (fp32 or bf16: what the reduction kernel writes)
         at::Tensor dx, dw, db, ws;
+        if (!usual_backward(x, 1, cu, w, dy, &s)) {
+            using namespace pybind11::literals;
+            pybind11::gil_scoped_acquire gil;
+            const variable_list r = python_backward("nanoplm_amd.dwconv", "varlen_dwconv_bwd", x, dy, cu, w, "need_dx"_a = need_dx,
+                                                    "need_dw"_a = need_w || need_b, "residual"_a = residual, "grads_bf16"_a = bf16);
+            return {r[0], at::Tensor(), need_w ? r[1] : at::Tensor(), need_b ? r[2] : at::Tensor(), at::Tensor()};
+        }
         if (need_dx) dx = at::empty({s.T, s.C}, x.options());
         size_t bytes = 0;
         if (need_w || need_b) {
@@ -171,12 +188,12 @@ struct Gated : torch::autograd::Function<Gated> {
         const at::Tensor &z = saved[0], &cu = saved[1], &w = saved[2];
         const bool has_bias = ctx->saved_data["bias"].toBool(), residual = ctx->saved_data["residual"].toBool();
         Sizes s;
-        sizes_of(z, 2, cu, w, std::nullopt, &s);
         const c10::DeviceGuard guard(z.device());
         const at::Tensor dy = incoming(grads[0], z);
-        const bool bf16 = s.wdt == NPLM_DWCONV_BF16;
+        const bool bf16 = w.scalar_type() == at::kBFloat16;
         const at::ScalarType gdt = w.scalar_type();
-        const size_t bytes = nplm_dwconv_gated_bwd_workspace_bytes(s.T, s.C, s.K, s.act);
+        const bool usual = usual_backward(z, 2, cu, w, dy, &s);
+        const size_t bytes = usual ? nplm_dwconv_gated_bwd_workspace_bytes(s.T, s.C, s.K, s.act) : 0;
         at::Tensor dz, dw, db;
         int rc = -NPLM_DWCONV_EUNSUPPORTED;
         if (bytes > 0) {
@@ -229,12 +246,14 @@ struct Prenorm : torch::autograd::Function<Prenorm> {
         const at::Tensor &x = saved[0], &cu = saved[1], &g = saved[2], &beta = saved[3], &w = saved[4], &stats = saved[5];
         const bool has_bias = ctx->saved_data["bias"].toBool(), residual = ctx->saved_data["residual"].toBool();
         Sizes s;
-        sizes_of(x, 1, cu, w, std::nullopt, &s);
         const c10::DeviceGuard guard(x.device());
         const at::Tensor dy = incoming(grads[0], x);
-        const bool bf16 = s.wdt == NPLM_DWCONV_BF16;
+        const bool bf16 = w.scalar_type() == at::kBFloat16;
         const at::ScalarType gdt = w.scalar_type();
-        const size_t bytes = nplm_dwconv_ln_bwd_workspace_bytes(s.T, s.C, s.K, s.act);
+        const bool usual = usual_backward(x, 1, cu, w, dy, &s) && vector_as(g, w, s.C) && (!beta.defined() || vector_as(beta, w, s.C)) &&
+                           dense(stats, x.device()) && stats.scalar_type() == at::kFloat && stats.dim() == 2 && stats.size(0) == s.T &&
+                           stats.size(1) == 2;
+        const size_t bytes = usual ? nplm_dwconv_ln_bwd_workspace_bytes(s.T, s.C, s.K, s.act) : 0;
         at::Tensor dx, dw, db, dg, dbeta;
         int rc = -NPLM_DWCONV_EUNSUPPORTED;
         // (under create_graph the op records itself, and says so if it is differentiated once more)
@@ -321,7 +340,7 @@ PyObject* prenorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (residual < 0) return nullptr;
     if (!sizes_of(x, 1, cu, w, b, &s) || s.T == 0 || !aligned16(x)) Py_RETURN_NONE;
     for (const at::Tensor& t : {g, beta ? *beta : g})        // (one dtype for all parameters)
-        if (!dense(t, x.device()) || t.dim() != 1 || t.size(0) != s.C || t.scalar_type() != w.scalar_type()) Py_RETURN_NONE;
+        if (!vector_as(t, w, s.C)) Py_RETURN_NONE;
     if (nplm_dwconv_ln_bwd_workspace_bytes(s.T, s.C, s.K, s.act) == 0) Py_RETURN_NONE;
     try {
         pybind11::gil_scoped_release no_gil;

@@ -270,3 +270,30 @@ def test_native_nodes_leave_other_forms_of_call_to_the_python_route(form):
     with pytest.raises(RuntimeError):                        # not differentiable twice
         g = torch.autograd.grad(door(xg, *rest).float().sum(), xg, create_graph=True)[0]
         torch.autograd.grad(g.float().sum(), xg)
+
+
+@pytest.mark.parametrize("form", ["plain", "gated", "ln"])
+def test_native_nodes_take_what_saved_tensor_hooks_give_back(form):
+    """Hooks may hand back other strides than were saved (made dense by the Python route), or another size (refused by it). An incoming
+    gradient that is not aligned goes the same way where the kernels want it aligned."""
+    door, function, args = _door(form, torch.bfloat16, torch.bfloat16, True, False)
+    dy = torch.randn(args[0].shape[0], 512, device=DEV).to(torch.bfloat16)
+
+    def grads(call, unpack, dy=dy):
+        leaves = [t.clone().requires_grad_() for t in args]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = call(*leaves)
+        return torch.autograd.grad(y, leaves, dy)
+
+    def strided(t):
+        wide = torch.empty(*t.shape, 2, dtype=t.dtype, device=t.device)
+        wide[..., 0] = t
+        return wide[..., 0]
+
+    for a, c in zip(grads(door, strided), grads(function, lambda t: t)):
+        assert torch.equal(a, c)
+    odd = torch.empty(dy.numel() + 1, dtype=dy.dtype, device=DEV)[1:].view(dy.shape).copy_(dy)
+    for a, c in zip(grads(door, lambda t: t, odd), grads(function, lambda t: t, odd)):
+        torch.testing.assert_close(a, c, rtol=0, atol=0)
+    with pytest.raises((ValueError, RuntimeError)):
+        grads(door, lambda t: t[:300] if t.shape[0] == 600 else t)
