@@ -407,7 +407,8 @@ def test_share_of_outputs_that_are_not_correctly_rounded(K):
 # step; a boundary at every row of the 32-row groups, one to many in a group)
 @pytest.mark.parametrize("K,lens,C", [(31, LENS * 2, 512), (29, LENS[::-1] * 2, 520), (25, [4096], 1000), (31, [95] * 44, 520),
                                       (31, [191] * 22, 8200), (15, LENS * 2, 776), (13, [63] * 66, 1160), (21, [4095, 1], 512),
-                                      (11, [2500, 1, 1700], 520), (31, [1] * 4100, 512), (15, [17] * 260, 512)])
+                                      (11, [2500, 1, 1700], 520), (31, [1] * 4100, 512), (15, [17] * 260, 512),
+                                      (15, [17] * 120, 512), (13, [63] * 32, 1160), (11, [1] * 1900, 512)])
 def test_gated_forward_on_the_matrix_cores_matches_the_oracle(K, lens, C):
     """To one bf16 rounding of the oracle's y: the three bf16 terms add up to the fp32 h. The same bits again after a call that left NaN
     in the LDS; rows in front of and behind y keep theirs."""
