@@ -431,7 +431,9 @@ int mfma_gated_fwd_steps(long long T, int C) {
 //   T=20, C=512          22 / 12      -            -            -            21 / 12
 //   15 taps, T=16384, C=768 44 / 40, -, 34 / 32, 31 / 25, 30 / 22; T=65536, C=1024 139 / 148, 122 / 123, 100 / 105, 90 / 96, 83 / 93
 //   (C=768 115 / 120, 96 / 99, 83 / 81, 75 / 68, 68 / 63; T=131072, C=2048 517 / 551, 441 / 457, 376 / 384, 358 / 335, 353 / 333)
-//   21 taps as 31, 11 as 15: T=2048, C=768 (21 taps) 26 / 15, -, 20 / 13, 19 / 13, 19 / 12; T=4000, C=2048 31 / 34, -, 27 / 26, 25 / 23, 24 / 21; T=16384, C=1152 58 / 66, 54 / 55, 45 / 46, 40 / 37, 39 / 32; C=1024 41 / 45, 37 / 40, 32 / 34, 31 / 28, 29 / 25.
+//   21 taps as 31, 11 as 15: T=2048, C=768 (21 taps) 26 / 15, -, 20 / 13, 19 / 13, 19 / 12;
+//   T=4000, C=2048 31 / 34, -, 27 / 26, 25 / 23, 24 / 21; T=16384, C=1152 58 / 66, 54 / 55, 45 / 46, 40 / 37, 39 / 32;
+//   C=1024 41 / 45, 37 / 40, 32 / 34, 31 / 28, 29 / 25.
 // A boundary costs the consumers a sweep of their own; short calls gain on every mix because a run begins without a full tile of halo.
 // Where 11 taps break even (between 75 and 300 rows) 15 would still gain a tenth, but 11 taps and the same taps padded to 15 have to
 // give the same bits, so both go by the one line.

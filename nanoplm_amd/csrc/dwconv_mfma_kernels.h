@@ -1490,8 +1490,8 @@ dwconv_bwd_gated_mfma_kernel(const void* __restrict__ z, const void* __restrict_
 // step's window takes over the halo rows from the step before in the ring. The producers alone take 201 us, the consumers alone 257
 // with one of 64 rows per SIMD (boundaries then cost twice what they do with two of 32: 430 and 395 us on log-normal lengths).
 // T=131072, C=2048, 31 taps, before and now: one sequence 393 to 413 and 357 to 369 us, log-normal lengths 415 to 444 and 387 to 406;
-// T=32768, C=768, 300 rows a sequence 57 and 43; T=8192, C=512 24 and 16. Outputs that are not the correctly rounded value 6.3e-5 (7.8e-5). Waves: 8 consumers (32 channels x 32 rows of a step; no packing, no gate), 8 producers (a
-// chunk of 4 rows x 128 channels at a time, z straight into registers two phases ahead). The boundary bits of all the block's runs are
+// T=32768, C=768, 300 rows a sequence 57 and 43; T=8192, C=512 24 and 16. Outputs that are not the correctly rounded value
+// 6.3e-5 (7.8e-5). Waves: 8 consumers (32 channels x 32 rows of a step; no packing, no gate), 8 producers (a chunk of 4 rows x 128 channels at a time, z straight into registers two phases ahead). The boundary bits of all the block's runs are
 // found before the first.
 template <int KT>
 struct MfmaGatedFwdShape {
