@@ -208,9 +208,19 @@ __device__ __forceinline__ float mfma_weight(const void* __restrict__ w, int w_f
     return v + (res && m == (KP - 1) / 2 ? 1.f : 0.f);
 }
 
+// Gated forward: h is taken kGateUp times as large, weights (and the identity) as much smaller.
+constexpr float kGateUp = 65536.f, kGateDown = 1.f / kGateUp;
+// kGateUp * u * silu(g), in the steps of gate_mul()
+__device__ __forceinline__ float gate_mul_up(float u, float g) {
+    return u * g * __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_amdgcn_exp2f(-1.44269504088896341f * g), kGateDown, kGateDown));
+}
+// A weight as the gated forward's table holds it
+__device__ __forceinline__ uint32_t mfma_weight_down(float w) { return __float_as_uint(w * kGateDown) & 0xffff0000u; }
+
 // Weight table of a column block in LDS, [channel][WSTR] dwords of two bf16: entry e of a channel is plan tap e - 4 + 4 CK0. Behind it
-// one word of each of the NW waves that fill it, not zero where it met a weight that is not finite.
-template <int KT, int CH, int NW>
+// one word of each of the NW waves that fill it, not zero where it met a weight that is not finite. DOWN: weights for gate_mul_up(), and
+// those below 2^-110, which lose bits there, count with the ones that are not finite.
+template <int KT, int CH, int NW, bool DOWN = false>
 struct MfmaWeights {
     using TP = MfmaTaps<KT>;
     static constexpr int MARKS_AT = CH * TP::WSTR, BYTES = (MARKS_AT + NW) * 4;
@@ -224,7 +234,11 @@ struct MfmaWeights {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const int m = 2 * p + h - 4 + 4 * TP::CK0;
-                    if (m >= 0 && m < TP::KP) t |= (__float_as_uint(mfma_weight<TP::KP, FLIP>(w, w_flags, ch0 + c, m, false)) >> 16) << (16 * h);
+                    if (m >= 0 && m < TP::KP) {
+                        const float v = mfma_weight<TP::KP, FLIP>(w, w_flags, ch0 + c, m, false);
+                        t |= ((DOWN ? mfma_weight_down(v) : __float_as_uint(v)) >> 16) << (16 * h);
+                        if constexpr (DOWN) odd |= __float_as_uint(v * kGateDown) & 0xffffu;
+                    }
                 }
             }
             odd |= non_finite_bf16x2(t);
@@ -233,7 +247,7 @@ struct MfmaWeights {
         const bool any = __builtin_amdgcn_ballot_w64(odd != 0) != 0;
         if ((tid & 63) == 0) tab[MARKS_AT + tid / 64] = any ? 1 : 0;
     }
-    // NaN if one of the block's weights is not finite, else 0 (after the barrier that follows fill())
+    // NaN if one of the block's weights is not finite (DOWN: or too small), else 0 (after the barrier that follows fill())
     __device__ __forceinline__ static float odd(const uint32_t* tab) {
         uint32_t any = 0;
 #pragma unroll
@@ -269,8 +283,8 @@ struct MfmaRing {
 // GATED (backward): the rows are dh; what is stored are the two halves of dz = [dh * silu(g) | dh * u * silu'(g)], with u and
 // g of the row out of their LDS tiles; 256-byte column blocks.
 // LINES: stores with `nt`, for output rows of whole cache lines (see mfma_lines()).
-// TERMS = 3 (gated forward): the rows are h in fp32, as three bf16 terms that add up to it, out of a ring of chunks that are
-// already packed (MfmaRing).
+// TERMS = 3 (gated forward): the rows are kGateUp * h in fp32, as three bf16 terms that add up to it, out of a ring of chunks that are
+// already packed (MfmaRing); the weights are kGateDown times the caller's.
 template <int KT, int NSTEP, bool FLIP, bool RES, bool LINES, bool GATED = false, int TERMS = 1>
 struct MfmaConv {
     using TP = MfmaTaps<KT>;
@@ -279,6 +293,7 @@ struct MfmaConv {
     static constexpr int Q = GATED || RING ? 2 : kMfmaQ, NCK = TP::NCK, CB = GATED ? kMfmaGatedCb : kMfmaCb;
     static constexpr MfmaSwz SWZ = GATED ? SWZ_BOTH : SWZ_QUAD;
     static constexpr int ROWS = 16 * NSTEP;                  // output rows of a group
+    struct Source { const void* z; int row0, T; };           // RING: z [T, 2C] and the row of the group's first output row
     static_assert(ROWS % 32 == 0, "a group's boundary bits start at a word");
     static constexpr int NCHUNK = 4 * (NSTEP - 1) + NCK;     // chunks that the steps of a group read (per lane)
     static constexpr int IDC = (TP::FRONT + 0) / 4;          // chunk of the identity's first row
@@ -314,7 +329,7 @@ struct MfmaConv {
     int swap;              // stores: the lane whose output goes out through this one (x 4)
     int out_at;            // byte offset of that lane's slice of output row 4 n, or kMfmaNoStore
     bool active;
-    float odd;             // NaN: a weight of the block is not finite, else 0
+    float odd;             // NaN: a weight of the block is not finite (MfmaWeights::odd), else 0
     const void* w;
     int w_flags;
 
@@ -351,7 +366,7 @@ struct MfmaConv {
 #pragma unroll
             for (int k = 0; k < IDN; ++k)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) I[k][e] = (4 * (IDC + k) + e == TP::FRONT + n) ? (short)0x3f80 : (short)0;
+                for (int e = 0; e < 4; ++e) I[k][e] = (4 * (IDC + k) + e == TP::FRONT + n) ? (short)(RING ? 0x3780 : 0x3f80) : (short)0;      // (RING: kGateDown)
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -501,7 +516,7 @@ struct MfmaConv {
     // stored. Returns whether all sums are finite (those that are not have to be formed again).
     template <bool PART>
     __device__ __forceinline__ bool sweep(At lp, int lo, int hi, rsrc_t ro, int rowb, const char* up) const {
-        float chk = PART ? odd : 0.f;
+        float chk = PART || RING ? odd : 0.f;
         f32x4 acc[(NCK + 3) / 4][Q];
         Raw raw;
         read<0>(lp, raw);
@@ -565,8 +580,9 @@ struct MfmaConv {
 
     // One group of output rows: lp = the group's first window row in LDS, words = the tile's boundary bits, p0 = the window row's
     // place among them; ro = descriptor of the group's output rows (those in front of T).
-    // GATED: up = the group's first row in the u tile; the g tile lies kMfmaGatedRows rows behind it.
-    __device__ __forceinline__ void rows(At lp, const uint32_t* words, int p0, rsrc_t ro, int rowb, const char* up = nullptr) const {
+    // GATED: up = the group's first row in the u tile; the g tile lies kMfmaGatedRows rows behind it. RING: src = where h comes from.
+    __device__ __forceinline__ void rows(At lp, const uint32_t* words, int p0, rsrc_t ro, int rowb, const char* up = nullptr,
+                                         const Source& src = Source{}) const {
         const uint32_t* wp = words + (p0 >> 5);              // p0 is a multiple of 32
         bool open;                                           // no boundary inside the window (a bit at its first row is none)
         {
@@ -611,7 +627,8 @@ struct MfmaConv {
                         float v[Q];
 #pragma unroll
                         for (int q = 0; q < Q; ++q) v[q] = i < 2 ? (i == 0 ? acc[q][0] : acc[q][1]) : i == 2 ? acc[q][2] : acc[q][3];
-                        add_non_finite(sp, i, lo, hi, v);
+                        if constexpr (RING) add_apart(src, rowb, 16 * s + i, i, lo, hi, v);
+                        else add_non_finite(sp, i, lo, hi, v);
                         store(ro, i >= (range & 255) && i < (range >> 8) ? out_at : kMfmaNoStore, rowb, up, 16 * s + i, v);
                     }
                 } else {
@@ -675,27 +692,37 @@ struct MfmaConv {
             if (p < lo || p >= hi || !active) continue;
             // (the lane's row 4 n + p of the step: its piece is where the chunk of that row has it)
             float f[Q];
-            if constexpr (RING) {
-                const uint32_t at = RG::at(sp + (p >> 2) * RG::REC) + (p & 3) * 2;
-#pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    f[q] = 0.f;
-#pragma unroll
-                    for (int t = TERMS - 1; t >= 0; --t) {   // (of a value that is not finite the first term is it)
-                        const float v = bf16_to_f32(*(const __attribute__((address_space(3))) uint16_t*)(uintptr_t)(at + t * RG::TERM + q * 8));
-                        f[q] = t == 0 && !__builtin_isfinite(v) ? v : f[q] + v;
-                    }
-                }
-            } else {
             const char* a = sp + (off[0] ^ mfma_place((((p >> 2) + (SWZ == SWZ_BOTH ? p : 0) + n) & 3) ^ n)) + p * CB;
             RowVec<true, Q> x;
             x.load(a);
             x.to_f32(f);
-            }
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
                 const float wq = mfma_weight<TP::KP, FLIP>(w, w_flags, c0 + q, m, res);
                 if (!__builtin_isfinite(f[q]) || !__builtin_isfinite(wq)) v[q] = __builtin_fmaf(wq, f[q], v[q]);
+            }
+        }
+    }
+    // The same for the gated forward, h once more from z: products that the finite terms and weights lack are those with a kGateUp * h or a
+    // weight that is not finite and, of weights too small for the table, what it holds too little. (row: output row 4 n + row of the group)
+    __device__ __forceinline__ void add_apart(const Source& src, int rowb, int row, int i, int lo, int hi, float (&v)[Q]) const {
+        const int koff = w_tap_off(w_flags), kw = TP::KP - 2 * koff;
+        const bool res = (w_flags & W_RESIDUAL) != 0;
+#pragma nounroll
+        for (int m = koff; m < koff + kw; ++m) {
+            const int p = TP::FRONT + i - TP::PP + m;           // window row of tap m
+            const int t = src.row0 + 4 * n + row + m - TP::PP;  // its row of z
+            if (p < lo || p >= hi || !active || t < 0 || t >= src.T) continue;
+            const char* a = reinterpret_cast<const char*>(src.z) + (size_t)t * 2 * (size_t)rowb + (size_t)c0 * 2;
+            const uint32_t u = *reinterpret_cast<const uint32_t*>(a), g = *reinterpret_cast<const uint32_t*>(a + rowb);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const float uq = q == 0 ? bf16_lo(u) : bf16_hi(u), gq = q == 0 ? bf16_lo(g) : bf16_hi(g), h = gate_mul(uq, gq);
+                const float wq = mfma_weight<TP::KP, FLIP>(w, w_flags, c0 + q, m, false);
+                if (!__builtin_isfinite(gate_mul_up(uq, gq)) || !__builtin_isfinite(wq))
+                    v[q] = __builtin_fmaf(wq + (res && m == TP::PP ? 1.f : 0.f), h, v[q]);
+                else
+                    v[q] = __builtin_fmaf(wq - __uint_as_float(mfma_weight_down(wq)) * kGateUp, h, v[q]);
             }
         }
     }
@@ -1483,8 +1510,11 @@ dwconv_bwd_gated_mfma_kernel(const void* __restrict__ z, const void* __restrict_
 // ---- gated forward ---------------------------------------------------------------------------------------------------
 // y = conv(h), h = u * silu(g) of z = [u | g] [T, 2C]. h is fp32 and stays it: the producers split it into three bf16 terms that add
 // up to it exactly (8 significant bits each, by truncation), and the consumers take the products of all three with the taps, which are
-// exact as well. So the sums differ from the vector ALU's by their order alone. (The third term of an h below 2^-109 is cut off at
-// bf16's smallest subnormal, 2^-133.)
+// exact as well. So the sums differ from the vector ALU's by their order alone.
+// bf16 ends at 2^-133 and fp32 at 2^-149, so the producers form 2^16 h (the factor rides in the sigmoid's sum and costs nothing) and the
+// weights are taken 2^-16 times: the same products, and terms that end where fp32 does. What that leaves out at the other ends, an h of
+// 2^112 on and weights below 2^-110, goes the way of values that are not finite. (Marking the chunks whose terms lack bits, for the
+// consumers to add them from z, took 366 us of the 359 without and 394 of 389 at 300 rows a sequence, T=131072, C=2048, 31 taps.)
 // What bounds it: on the vector ALU the 31 FMAs an element (0.8 of all issue slots); here the gate and the split, 14
 // instructions an element of which two are quarter-rate, each evaluated once: a block walks down a run of steps of 64 rows, and a
 // step's window takes over the halo rows from the step before in the ring. The producers alone take 201 us, the consumers alone 257
@@ -1500,7 +1530,7 @@ struct MfmaGatedFwdShape {
     static constexpr int NCW = 4, NCONS = 8, RW = RG::R * NCW / NCONS, NPROD = 8, UNITS = RG::R / 4 / NPROD, NW = NCONS + NPROD, NT = NW * 64;
     static constexpr int WORDS = (kMfmaGatedSteps * RG::R + TP::HALO + 31) / 32 + 2;     // boundary bits of a run (lanes read two words further)
     static_assert(WORDS <= 64, "a wave clears them in one go");
-    using W = MfmaWeights<KT, RG::CH, NCONS>;
+    using W = MfmaWeights<KT, RG::CH, NCONS, true>;
     static_assert(W::BYTES <= RG::BYTES, "the weight table lies in the ring until it is written");
     static_assert(RG::BYTES + 64 * WORDS * 4 <= kLdsBytes, "fits the LDS");
     // LDS of a call whose blocks have up to this many runs; the words begin behind the ring
@@ -1556,7 +1586,7 @@ dwconv_fwd_gated_mfma_kernel(const void* __restrict__ z, const int32_t* __restri
                 const int t0 = row0 + s * R + r0;
                 if (s < steps && t0 < T)
                     conv.rows(conv.slice + (slot + r0 / 4) * RG::REC, words + it * SH::WORDS, s * R + r0,
-                              mfma_out_rsrc(y, t0, T - t0 < SH::RW ? T - t0 : SH::RW, rowb), rowb);
+                              mfma_out_rsrc(y, t0, T - t0 < SH::RW ? T - t0 : SH::RW, rowb), rowb, nullptr, {z, t0, T});
                 slot = RG::next(slot);
                 if (++s > steps) {           // (the phase between two runs has no step)
                     s = 0;
@@ -1602,8 +1632,8 @@ dwconv_fwd_gated_mfma_kernel(const void* __restrict__ z, const int32_t* __restri
                 float h[2][4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    h[0][r] = gate_mul(bf16_lo(v.a[i].u[r]), bf16_lo(v.a[i].g[r]));
-                    h[1][r] = gate_mul(bf16_hi(v.a[i].u[r]), bf16_hi(v.a[i].g[r]));
+                    h[0][r] = gate_mul_up(bf16_lo(v.a[i].u[r]), bf16_lo(v.a[i].g[r]));
+                    h[1][r] = gate_mul_up(bf16_hi(v.a[i].u[r]), bf16_hi(v.a[i].g[r]));
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(h[0][r]), "+v"(h[1][r]));     // (h rounded: no product is contracted into the differences)

@@ -457,3 +457,42 @@ def test_gated_forward_non_finite_values_reach_the_rows_of_their_taps_only(K, wh
     torch.testing.assert_close(y, want, rtol=2.0 ** -7, atol=1e-5, equal_nan=True)
     if where != "weight":
         assert torch.equal(y[~hit.to(DEV)], clean[~hit.to(DEV)])
+
+
+@pytest.mark.parametrize("K", [15, 31])
+@pytest.mark.parametrize("what,h_exp,w_exp", [("small h", -100, 90), ("large h", 123, -90), ("small weights", 60, -103)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_gated_forward_keeps_the_range_of_fp32(K, what, h_exp, w_exp, residual):
+    """|h| from 2^-100 to 2^-135 and from 2^123 down, weights from 2^-103 to 2^-133, by channel; every seventh channel ordinary. A bf16
+    term ends at 2^-133, fp32 does not. Boundaries in most windows and in none. To one bf16 rounding of y, the fp32 sums' noise and the last
+    bits of a subnormal h or product; non-finite values among them reach what they reach on the vector ALU (which takes the same weights
+    in fp32)."""
+    C, lens = 520, LENS[:25] + [700, 1, 300]
+    _, cu, w, _, dy = _case(lens, C, K, K)
+    T = dy.shape[0]
+    g = torch.Generator().manual_seed(K)
+    ch = torch.arange(C, dtype=torch.float64)
+    usual = ch % 7 == 3
+    size = torch.where(usual, 1.0, 2.0 ** (h_exp - (0 if what == "small weights" else ch % 27)))
+    z = torch.cat([torch.randn(T, C, generator=g) * size, torch.randn(T, C, generator=g)], 1).bfloat16()
+    w = (w.double() * torch.where(usual, 1.0, 2.0 ** (w_exp - (ch % 27 if what == "small weights" else 0)))[:, None]).bfloat16()
+    cud, wd = cu.to(DEV), w.to(DEV)
+    ref, mass = (O.ref_gated_dwconv_grads(a, cu, b, None, None, torch.float64, residual)
+                 for a, b in ((z.double(), w.double()), (z.double().abs(), w.double().abs())))
+    y = npa.gated_dwconv_fwd(z.to(DEV), cud, wd, None, residual=residual).cpu().double()
+    # (gate_mul() is off by up to 4 roundings, K sums by one each; an h or a product below 2^-126 by 2^-149)
+    bound = ref.abs() * 2.0 ** -8 + (K + 8) * 2.0 ** -23 * mass + (w.double().abs().sum(1) + K) * 2.0 ** -148 + 2.0 ** -134
+    assert bool(((y - ref).abs() <= bound).all()), float(((y - ref).abs() / bound).max())
+    for where in ("z", "w"):
+        zo, wo = z.clone(), w.clone()
+        if where == "z":
+            zo[500, 5::11], zo[2, 1::13], zo[900, 2::17] = float("inf"), float("nan"), -float("inf")
+        else:
+            wo[5::11, 2], wo[4::13, K // 2], wo[2::17, K - 1] = float("inf"), float("nan"), -float("inf")
+        got = npa.gated_dwconv_fwd(zo.to(DEV), cud, wo.to(DEV), None, residual=residual)
+        want = npa.gated_dwconv_fwd(zo.to(DEV), cud, wo.to(DEV).float(), None, residual=residual)
+        fin = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), fin) and not bool(fin.all())
+        torch.testing.assert_close(got[~fin], want[~fin], rtol=0, atol=0, equal_nan=True)
+        if where == "z":
+            assert bool(((got.cpu().double() - ref).abs() <= bound)[fin.cpu()].all())
