@@ -17,6 +17,7 @@
 #include <torch/extension.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -46,8 +47,11 @@ int dtype_code(const at::Tensor& t) {
     if (t.scalar_type() == at::kBFloat16) return NPLM_DWCONV_BF16;
     return -1;
 }
+// Whether t's values are what lies at its data pointer, one after the other: not so for wrappers (of a batch, of another tensor), for a
+// tensor known to be zero, and for a view that negates its values when they are read.
 bool dense(const at::Tensor& t, const at::Device& dev) {
-    return t.layout() == at::kStrided && t.device() == dev && t.is_contiguous();
+    return t.layout() == at::kStrided && t.device() == dev && !at::isTensorSubclassLike(t) && !t.is_neg() && !t._is_zerotensor() &&
+           t.is_contiguous();
 }
 // a parameter of one value a channel, in w's dtype on its device
 bool vector_as(const at::Tensor& t, const at::Tensor& w, int32_t C) {
@@ -108,10 +112,17 @@ variable_list python_backward(const char* module, const char* name, Args&&... ar
     return r;
 }
 
-// The tensors of a backward are what saved-tensor hooks gave back, which need not be what was saved: whether they still are as the
-// kernels take them. If not, the Python route makes them so or refuses them.
+// Calls (and backwards) that something else records, rewrites or looks into go the Python way.
+bool observed() {
+    return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing() ||
+           torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr;
+}
+
+// The tensors of a backward are what saved-tensor hooks gave back, which need not be what was saved, and a gradient of whatever kind its
+// caller has: whether they are as the kernels take them. If not, the Python route makes them so, takes them apart or refuses them.
 bool usual_backward(const at::Tensor& x, int width, const at::Tensor& cu, const at::Tensor& w, const at::Tensor& dy, Sizes* s) {
-    return x.defined() && cu.defined() && w.defined() && sizes_of(x, width, cu, w, std::nullopt, s) && dense(dy, x.device()) &&
+    return !observed() && x.defined() && cu.defined() && w.defined() && sizes_of(x, width, cu, w, std::nullopt, s) && dense(dy, x.device()) &&
            dy.dim() == 2 && dy.size(0) == s->T && dy.size(1) == s->C;
 }
 
@@ -282,12 +293,6 @@ struct Prenorm : torch::autograd::Function<Prenorm> {
     }
 };
 
-// Calls that something else records, rewrites or looks into go the Python way.
-bool observed() {
-    return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0 ||
-           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing() ||
-           torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr;
-}
 bool tensor_arg(PyObject* o, at::Tensor* t) {
     if (!THPVariable_CheckExact(o)) return false;
     *t = THPVariable_Unpack(o);

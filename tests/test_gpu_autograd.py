@@ -297,3 +297,55 @@ def test_native_nodes_take_what_saved_tensor_hooks_give_back(form):
         torch.testing.assert_close(a, c, rtol=0, atol=0)
     with pytest.raises((ValueError, RuntimeError)):
         grads(door, lambda t: t[:300] if t.shape[0] == 600 else t)
+
+
+class _Wrapper(torch.Tensor):
+    """A tensor that holds another one and hands every operation on to it."""
+    @staticmethod
+    def __new__(cls, inner):
+        return torch.Tensor._make_wrapper_subclass(cls, inner.shape, strides=inner.stride(), dtype=inner.dtype, device=inner.device)
+
+    def __init__(self, inner):
+        self.inner = inner
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        from torch.utils._pytree import tree_map_only
+        out = func(*tree_map_only(cls, lambda t: t.inner, args), **tree_map_only(cls, lambda t: t.inner, kwargs or {}))
+        return tree_map_only(torch.Tensor, cls, out)
+
+
+def test_native_prenorm_node_takes_gradients_and_tensors_of_every_kind():
+    """What reached the registered ops of the pre-norm door reaches them still: incoming gradients that are a batch of gradients, wrap
+    another tensor, are known to be zero or are negated as they are read, negated inputs and weights, and a backward that a mode watches."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    door, function, args = _door("ln", torch.bfloat16, torch.bfloat16, True, False)
+    leaves = [t.clone().requires_grad_() for t in args]
+    dy = torch.randn(args[0].shape, device=DEV).bfloat16()
+    grads = lambda d, **kw: torch.autograd.grad(door(*leaves), leaves, d, **kw)
+    want, want2 = grads(dy), grads(-2 * dy)
+    same = lambda got, ref: all(torch.equal(a, c) for a, c in zip(got, ref))
+    assert same(want, torch.autograd.grad(function(*leaves), leaves, dy))
+    batch = grads(torch.stack([dy, -2 * dy]), is_grads_batched=True)
+    assert same([t[0] for t in batch], want) and same([t[1] for t in batch], want2)
+    y = door(*leaves)
+    batch = torch.func.vmap(lambda d: torch.autograd.grad(y, leaves[0], d, retain_graph=True)[0])(torch.stack([dy, -2 * dy]))
+    assert torch.equal(batch[0], want[0]) and torch.equal(batch[1], want2[0])
+    assert same([t.inner for t in grads(_Wrapper(dy))], want)
+    assert all(not bool(t.any()) for t in grads(torch._efficientzerotensor(dy.shape, dtype=dy.dtype, device=DEV)))
+    assert same(grads(torch._neg_view(dy)), grads(-dy))
+    for i in range(len(args)):
+        neg = [torch._neg_view(t) if j == i else t for j, t in enumerate(args)]
+        assert torch.equal(door(*neg), door(*[-t if j == i else t for j, t in enumerate(args)]))
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    y = door(*leaves)
+    with Watch():
+        got = torch.autograd.grad(y, leaves, dy)
+    assert same(got, want) and any("ln_dwconv_bwd" in f for f in seen)
