@@ -18,6 +18,7 @@
 
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -126,11 +127,16 @@ bool usual_backward(const at::Tensor& x, int width, const at::Tensor& cu, const 
            dy.dim() == 2 && dy.size(0) == s->T && dy.size(1) == s->C;
 }
 
-struct Plain : torch::autograd::Function<Plain> {
+}  // namespace
+
+// The nodes, by the names that profiles and autograd's messages give them; their calls are recorded there as the registered ops are.
+namespace nanoplm_amd {
+struct VarlenDWConv1d : torch::autograd::Function<VarlenDWConv1d> {
     static at::Tensor run(const at::Tensor& x, const at::Tensor& cu, const at::Tensor& w, const OptTensor& b, bool residual) {
+        RECORD_FUNCTION("nanoplm_amd::varlen_dwconv_fwd", {});
         Sizes s;
         sizes_of(x, 1, cu, w, b, &s);
-        const c10::DeviceGuard guard(x.device());
+        const c10::DeviceGuard on(x.device());
         at::Tensor y = at::empty({s.T, s.C}, x.options());
         check(nplm_dwconv_fwd_ex(x.const_data_ptr(), ints(cu), w.const_data_ptr(), ptr(b), y.mutable_data_ptr(), s.T, s.C, s.K, s.S, s.act,
                                  s.wdt, flags_of(residual, false), stream_of(x)), "nplm_dwconv_fwd");
@@ -144,12 +150,13 @@ struct Plain : torch::autograd::Function<Plain> {
         return run(x, cu, w, b, residual);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        RECORD_FUNCTION("nanoplm_amd::varlen_dwconv_bwd", {});
         const variable_list saved = ctx->get_saved_variables();
         const at::Tensor &x = saved[0], &cu = saved[1], &w = saved[2];
         const bool has_bias = ctx->saved_data["bias"].toBool(), residual = ctx->saved_data["residual"].toBool();
         const bool need_dx = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(2), need_b = has_bias && ctx->needs_input_grad(3);
         Sizes s;
-        const c10::DeviceGuard guard(x.device());
+        const c10::DeviceGuard on(x.device());
         const at::Tensor dy = incoming(grads[0], x);
         const bool bf16 = w.scalar_type() == at::kBFloat16;
         const at::ScalarType gdt = w.scalar_type();          // (fp32 or bf16: what the reduction kernel writes)
@@ -177,11 +184,12 @@ struct Plain : torch::autograd::Function<Plain> {
     }
 };
 
-struct Gated : torch::autograd::Function<Gated> {
+struct GatedVarlenDWConv1d : torch::autograd::Function<GatedVarlenDWConv1d> {
     static at::Tensor run(const at::Tensor& z, const at::Tensor& cu, const at::Tensor& w, const OptTensor& b, bool residual) {
+        RECORD_FUNCTION("nanoplm_amd::gated_dwconv_fwd", {});
         Sizes s;
         sizes_of(z, 2, cu, w, b, &s);
-        const c10::DeviceGuard guard(z.device());
+        const c10::DeviceGuard on(z.device());
         at::Tensor y = at::empty({s.T, s.C}, z.options());
         check(nplm_dwconv_gated_fwd(z.const_data_ptr(), ints(cu), w.const_data_ptr(), ptr(b), y.mutable_data_ptr(), s.T, s.C, s.K, s.S,
                                     s.act, s.wdt, flags_of(residual, false), stream_of(z)), "nplm_dwconv_gated_fwd");
@@ -195,11 +203,12 @@ struct Gated : torch::autograd::Function<Gated> {
         return run(z, cu, w, b, residual);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        RECORD_FUNCTION("nanoplm_amd::gated_dwconv_bwd", {});
         const variable_list saved = ctx->get_saved_variables();
         const at::Tensor &z = saved[0], &cu = saved[1], &w = saved[2];
         const bool has_bias = ctx->saved_data["bias"].toBool(), residual = ctx->saved_data["residual"].toBool();
         Sizes s;
-        const c10::DeviceGuard guard(z.device());
+        const c10::DeviceGuard on(z.device());
         const at::Tensor dy = incoming(grads[0], z);
         const bool bf16 = w.scalar_type() == at::kBFloat16;
         const at::ScalarType gdt = w.scalar_type();
@@ -229,13 +238,14 @@ struct Gated : torch::autograd::Function<Gated> {
     }
 };
 
-struct Prenorm : torch::autograd::Function<Prenorm> {
+struct LnVarlenDWConv1d : torch::autograd::Function<LnVarlenDWConv1d> {
     // stats [T, 2] come back for the backward
     static at::Tensor run(const at::Tensor& x, const at::Tensor& cu, const at::Tensor& g, const OptTensor& beta, const at::Tensor& w,
                           const OptTensor& b, double eps, bool residual, at::Tensor* stats) {
+        RECORD_FUNCTION("nanoplm_amd::ln_dwconv_fwd", {});
         Sizes s;
         sizes_of(x, 1, cu, w, b, &s);
-        const c10::DeviceGuard guard(x.device());
+        const c10::DeviceGuard on(x.device());
         at::Tensor y = at::empty({s.T, s.C}, x.options());
         *stats = at::empty({s.T, 2}, x.options().dtype(at::kFloat));
         check(nplm_dwconv_ln_fwd(x.const_data_ptr(), ints(cu), g.const_data_ptr(), ptr(beta), (float)eps, w.const_data_ptr(), ptr(b),
@@ -253,11 +263,12 @@ struct Prenorm : torch::autograd::Function<Prenorm> {
         return y;
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        RECORD_FUNCTION("nanoplm_amd::ln_dwconv_bwd", {});
         const variable_list saved = ctx->get_saved_variables();
         const at::Tensor &x = saved[0], &cu = saved[1], &g = saved[2], &beta = saved[3], &w = saved[4], &stats = saved[5];
         const bool has_bias = ctx->saved_data["bias"].toBool(), residual = ctx->saved_data["residual"].toBool();
         Sizes s;
-        const c10::DeviceGuard guard(x.device());
+        const c10::DeviceGuard on(x.device());
         const at::Tensor dy = incoming(grads[0], x);
         const bool bf16 = w.scalar_type() == at::kBFloat16;
         const at::ScalarType gdt = w.scalar_type();
@@ -292,6 +303,9 @@ struct Prenorm : torch::autograd::Function<Prenorm> {
         return {dx, at::Tensor(), dg, beta.defined() ? dbeta : at::Tensor(), dw, has_bias ? db : at::Tensor(), at::Tensor(), at::Tensor()};
     }
 };
+}  // namespace nanoplm_amd
+
+namespace {
 
 bool tensor_arg(PyObject* o, at::Tensor* t) {
     if (!THPVariable_CheckExact(o)) return false;
@@ -350,7 +364,7 @@ PyObject* prenorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     try {
         pybind11::gil_scoped_release no_gil;
         const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad() || g.requires_grad() || wants_grad(beta) || wants_grad(b));
-        y = grad ? Prenorm::apply(x, cu, g, beta, w, b, eps, residual != 0) : Prenorm::run(x, cu, g, beta, w, b, eps, residual != 0, &stats);
+        y = grad ? nanoplm_amd::LnVarlenDWConv1d::apply(x, cu, g, beta, w, b, eps, residual != 0) : nanoplm_amd::LnVarlenDWConv1d::run(x, cu, g, beta, w, b, eps, residual != 0, &stats);
     } catch (const Unsupported&) {
         Py_RETURN_NONE;
     }
@@ -359,8 +373,8 @@ PyObject* prenorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 PyMethodDef methods[] = {
-    {"dwconv", (PyCFunction)(void (*)(void))&conv<Plain, 1>, METH_FASTCALL, "y = conv(x), differentiable; None: take the Python route"},
-    {"gated_dwconv", (PyCFunction)(void (*)(void))&conv<Gated, 2>, METH_FASTCALL, "y = conv(u * silu(g)), differentiable; None: take the Python route"},
+    {"dwconv", (PyCFunction)(void (*)(void))&conv<nanoplm_amd::VarlenDWConv1d, 1>, METH_FASTCALL, "y = conv(x), differentiable; None: take the Python route"},
+    {"gated_dwconv", (PyCFunction)(void (*)(void))&conv<nanoplm_amd::GatedVarlenDWConv1d, 2>, METH_FASTCALL, "y = conv(u * silu(g)), differentiable; None: take the Python route"},
     {"ln_dwconv", (PyCFunction)(void (*)(void))&prenorm, METH_FASTCALL, "y = conv(layer_norm(x)), differentiable; None: take the Python route"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_node", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -349,3 +349,18 @@ def test_native_prenorm_node_takes_gradients_and_tensors_of_every_kind():
     with Watch():
         got = torch.autograd.grad(y, leaves, dy)
     assert same(got, want) and any("ln_dwconv_bwd" in f for f in seen)
+
+
+@pytest.mark.parametrize("form,name", [("plain", "varlen_dwconv"), ("gated", "gated_dwconv"), ("ln", "ln_dwconv")])
+def test_profiles_and_messages_name_the_native_nodes(form, name):
+    """A profile lists an eager call and its backward by the names of the registered ops; autograd's messages name the function."""
+    door, _, args = _door(form, torch.bfloat16, torch.bfloat16, True, False)
+    leaves = [t.clone().requires_grad_() for t in args]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as p:
+        y = door(*leaves)
+        torch.autograd.grad(y, leaves, torch.ones_like(y))
+    keys = {e.key for e in p.key_averages()}
+    assert {f"nanoplm_amd::{name}_fwd", f"nanoplm_amd::{name}_bwd"} <= keys
+    with pytest.raises(RuntimeError, match="VarlenDWConv1d.* returned nan"), torch.autograd.set_detect_anomaly(True):
+        y = door(*leaves)
+        torch.autograd.grad(y, leaves, torch.full_like(y, float("nan")))
