@@ -332,7 +332,8 @@ PyObject* conv(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int residual = PyObject_IsTrue(a[4]);
     if (residual < 0) return nullptr;
     if (!sizes_of(x, WIDTH, cu, w, b, &s)) Py_RETURN_NONE;
-    if (WIDTH == 2 && (s.T == 0 || !aligned16(x))) Py_RETURN_NONE;
+    // (asked first: a forward of the composed route would start with an allocation and an exception here, 4 us)
+    if (WIDTH == 2 && (s.T == 0 || !aligned16(x) || nplm_dwconv_gated_bwd_workspace_bytes(s.T, s.C, s.K, s.act) == 0)) Py_RETURN_NONE;
     try {
         pybind11::gil_scoped_release no_gil;
         const bool grad = at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad() || wants_grad(b));

@@ -364,3 +364,18 @@ def test_profiles_and_messages_name_the_native_nodes(form, name):
     with pytest.raises(RuntimeError, match="VarlenDWConv1d.* returned nan"), torch.autograd.set_detect_anomaly(True):
         y = door(*leaves)
         torch.autograd.grad(y, leaves, torch.full_like(y, float("nan")))
+
+
+@pytest.mark.parametrize("form", ["gated", "ln"])
+def test_native_nodes_leave_calls_without_a_fused_kernel_before_they_begin(form):
+    """Rows that the fused kernels are not built for: no output is allocated for a call that the Python route takes."""
+    from nanoplm_amd import _lib
+    C, K = (24, 7) if form == "gated" else (24, 11)
+    x = torch.randn(64, 2 * C if form == "gated" else C, device=DEV)
+    cu = torch.tensor([0, 64], dtype=torch.int32, device=DEV)
+    w, v = torch.randn(C, K, device=DEV), torch.randn(C, device=DEV)
+    node = _lib.load_node()
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = count()
+    assert (node.gated_dwconv(x, cu, w, v, False) if form == "gated" else node.ln_dwconv(x, cu, v, None, w, v, 1e-5, False)) is None
+    assert count() == before
