@@ -108,6 +108,8 @@ def load():
     lib.nplm_dwconv_debug_intervals.restype = i64
     lib.nplm_dwconv_debug_algo.argtypes = [i32, i64, i32, i32, i32, i32, i32]
     lib.nplm_dwconv_debug_algo.restype = i32
+    lib.nplm_dwconv_debug_gated_algo.argtypes = [i32, i64, i32, i32, i32, i32, i32]
+    lib.nplm_dwconv_debug_gated_algo.restype = i32
     lib.nplm_dwconv_debug_starts.argtypes = [vp, i32, i64, i32, i32, vp]
     lib.nplm_dwconv_debug_starts.restype = i64
     lib.nplm_dwconv_debug_copy.argtypes = [vp, vp, sz, vp]

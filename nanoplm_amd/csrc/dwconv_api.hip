@@ -415,9 +415,12 @@ bool mfma_gated_bwd_preferred(long long T, int taps, int S) {
 // The gated forward on the matrix cores: steps of 64 rows in a run, which a block walks down without staging or gating a halo again.
 // All of a block's runs are of one length, the longest that deals the call out evenly (T=65536, C=1152, 15 taps: runs of 16 steps,
 // three rounds for two and a bit, 115 us, of 13 95).
-int mfma_gated_fwd_steps(long long T, int C) {
+long long mfma_gated_fwd_steps_of_a_block(long long T, int C) {
     const int ncb = ceil_div(2LL * C, kMfmaGatedCb), nbt = ncb < kNumCU ? kNumCU / ncb : 1;
-    const long long per_block = ceil_div(ceil_div(T, kMfmaGatedRows), nbt);
+    return ceil_div(ceil_div(T, kMfmaGatedRows), nbt);
+}
+int mfma_gated_fwd_steps(long long T, int C) {
+    const long long per_block = mfma_gated_fwd_steps_of_a_block(T, C);
     return ceil_div(per_block, ceil_div(per_block, kMfmaGatedSteps));
 }
 // Which gated forwards take it, measured by the mean rows of a sequence, us, role-split / matrix cores:
@@ -437,9 +440,26 @@ int mfma_gated_fwd_steps(long long T, int C) {
 // A boundary costs the consumers a sweep of their own; short calls gain on every mix because a run begins without a full tile of halo.
 // Where 11 taps break even (between 75 and 300 rows) 15 would still gain a tenth, but 11 taps and the same taps padded to 15 have to
 // give the same bits, so both go by the one line.
-bool mfma_gated_fwd_preferred(long long T, int taps, int S) {
+// Up to 2048 rows what counts is how many steps a block gets, which goes by C too. With one (two at 21 taps) a block is done before the
+// role-split one has staged its tile; with more it is not, but for sequences so short that the others' masked passes take over:
+//   rows a sequence       4            8            16           24           75           150          300          one
+//   11 taps, 2 steps: T=2048, C=1536    18.1 / 17.1  16.4 / 16.8  15.0 / 16.7  14.8 / 16.7  13.4 / 14.2  13.2 / 14.1  12.7 / 12.8  11.7 / 11.8
+//   3: T=2048, C=3072     29.3 / 26.5  24.8 / 26.1  23.1 / 26.0  21.3 / 25.4  18.8 / 21.3  17.9 / 19.2  17.6 / 18.5  16.4 / 16.5
+//   4: T=2048, C=4096     30.8 / 27.9  25.7 / 28.1  23.5 / 28.4  22.5 / 26.7  20.2 / 22.5  19.9 / 21.3  19.2 / 19.9  18.4 / 19.1
+//   15 taps, 2: T=2048, C=1536          20.5 / 16.9  18.5 / 16.8  17.5 / 16.7  16.8 / 16.4  15.6 / 14.2  15.4 / 13.2  15.1 / 13.0  13.9 / 11.8
+//   4: T=2048, C=4096     34.4 / 29.4  28.7 / 28.9  26.8 / 28.9  25.7 / 26.4  23.1 / 23.7  22.5 / 21.4  22.2 / 21.0  20.9 / 19.4
+//   21 taps, 2: T=1536, C=2048          25.3 / 20.1  22.8 / 20.0  21.3 / 20.7  21.3 / 19.9  19.8 / 16.5  19.1 / 16.2  18.7 / 14.6  17.8 / 13.5
+//   4: T=2048, C=4096     40.0 / 34.6  33.8 / 33.6  30.8 / 36.2  30.0 / 33.1  27.1 / 27.5  26.8 / 25.3  26.0 / 24.9  24.7 / 22.5
+// 31 taps of up to 16384 rows gain everywhere but at 16 rows a sequence (T=16384, C=4096 4 rows 263 / 170, 8 203 / 171, 16 173 / 184, 24 164 / 163).
+// Rows of partial cache lines change none of this: a wave stores 64 bytes of a row without `nt`, and the pieces meet in the L2. 31 taps,
+// T=131072, 75 rows, 300 rows, one sequence: C=1000 253 / 251, 234 / 214, 226 / 208; C=1160 315 / 313, 287 / 262, 277 / 245; C=2008 489 / 496,
+// 450 / 418, 436 / 407; T=16384, C=520 40 / 33, 38 / 28, 34 / 25; C=1160 62 / 52, 58 / 43, 55 / 40; 15 taps, T=16384, 300 rows, one sequence C=1000
+// 39 / 33, 37 / 31; C=2008 63 / 57, 61 / 57; 11 taps C=2008 60 / 57, 59 / 56.
+bool mfma_gated_fwd_preferred(long long T, int C, int taps, int S) {
     if (taps == 31) return T <= 16384 || T >= 32ll * S;
-    return T <= 2048 || (T <= 16384 && T >= 192ll * S);
+    if (T > 2048) return T <= 16384 && T >= 192ll * S;
+    const long long steps = mfma_gated_fwd_steps_of_a_block(T, C);
+    return steps <= (taps == 21 ? 2 : 1) || T < 6ll * S || (T >= 192ll * S && (taps == 21 || steps == 2));
 }
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
                     bool gated = false, int tile_rows = 0, int block_bytes = 0) {
@@ -625,6 +645,20 @@ int make_long_gated_plan(bool bf16, long long T, int C, int K, Plan* out) {
     nplm_dwconv_tuning t{};
     t.vec = 1;
     return make_plan(true, bf16, T, C, K, 0, &t, out);
+}
+
+// algo of a gated call: 4 matrix cores, 3 role-split, 2 LDS-staged, 1 sliding-window; align_bits: of z, dy and the output, out_bits: of dz.
+int choose_gated_algo(bool bwd, bool bf16, bool w_bf16, long long T, int C, int K, int taps, int S, uintptr_t align_bits, uintptr_t out_bits) {
+    const bool supported = gated_supported(false, bf16, T, C, K, align_bits);
+    const bool role_split = long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, align_bits);
+    if (!supported && !(bwd && role_split)) return -NPLM_DWCONV_EUNSUPPORTED;
+    if (!role_split) return bwd && long_gated_kernel_size(K) ? 1 : 2;
+    if (!bf16 || !w_bf16) return 3;
+    if (bwd) return mfma_tile_fits(C, K, true) && mfma_lines_ok(true, true, T, C, K, taps, out_bits) && mfma_gated_bwd_preferred(T, taps, S) ? 4 : 3;
+    LdsPlan lp;
+    return mfma_gated_fwd_preferred(T, C, taps, S) &&
+           make_split_plan(true, bf16, T, C, K, nullptr, &lp, true, mfma_gated_fwd_steps(T, C) * kMfmaGatedRows, kMfmaGatedCb) == 0 &&
+           MfmaGatedFwdShape<31>::lds_bytes(ceil_div(lp.ntiles, lp.nbt)) <= kLdsBytes ? 4 : 3;
 }
 
 // launch flags of the kernels (W_BF16 | W_RESIDUAL) from the ABI's weight dtype and flags
@@ -948,19 +982,20 @@ int nplm_dwconv_gated_fwd(const void* z, const int32_t* cu, const void* w, const
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if (((uintptr_t)w | (uintptr_t)b) % WE || (uintptr_t)cu % 4) return -NPLM_DWCONV_EALIGN;
-    if (!gated_supported(false, bf16, T, C, K, (uintptr_t)z | (uintptr_t)y)) return -NPLM_DWCONV_EUNSUPPORTED;
+    const int algo = choose_gated_algo(false, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, (uintptr_t)z | (uintptr_t)y, 0);
+    if (algo < 0) return algo;
     LdsPlan lp;
-    if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)y)) {
+    if (algo == 4) {
         const int steps = mfma_gated_fwd_steps(T, C);
-        if (bf16 && w_dtype == NPLM_DWCONV_BF16 && mfma_gated_fwd_preferred(T, taps, S) &&
-            make_split_plan(true, bf16, T, C, K, nullptr, &lp, true, steps * kMfmaGatedRows, kMfmaGatedCb) == 0 &&
-            MfmaGatedFwdShape<31>::lds_bytes(ceil_div(lp.ntiles, lp.nbt)) <= kLdsBytes) {
-            const ConvPtrs la{z, nullptr, cu, w, b, y, nullptr};
-            const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | tap_flags);
-            const dim3 grid(lp.ncb * lp.nbt);
-            return (int)(K == 15 ? launch_fwd_gated_mfma_k15(la, lg, steps, grid, (hipStream_t)stream)
-                                 : launch_fwd_gated_mfma_k31(la, lg, steps, grid, (hipStream_t)stream));
-        }
+        rc = make_split_plan(true, bf16, T, C, K, nullptr, &lp, true, steps * kMfmaGatedRows, kMfmaGatedCb);
+        if (rc) return rc;
+        const ConvPtrs la{z, nullptr, cu, w, b, y, nullptr};
+        const LdsGeo lg = make_lds_geo(lp, T, C, S, kernel_w_flags(w_dtype, flags) | tap_flags);
+        const dim3 grid(lp.ncb * lp.nbt);
+        return (int)(K == 15 ? launch_fwd_gated_mfma_k15(la, lg, steps, grid, (hipStream_t)stream)
+                             : launch_fwd_gated_mfma_k31(la, lg, steps, grid, (hipStream_t)stream));
+    }
+    if (algo == 3) {
         rc = make_split_plan(true, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;
         const ConvPtrs la{z, nullptr, cu, w, b, y, nullptr};
@@ -1233,11 +1268,12 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
     const bool bf16 = act_dtype == NPLM_DWCONV_BF16;
     const uintptr_t WE = (w_dtype == NPLM_DWCONV_BF16) ? 2 : 4;
     if ((uintptr_t)w % WE || (uintptr_t)cu % 4 || ((uintptr_t)dw | (uintptr_t)db) % (out_bf16 ? 2 : 4)) return -NPLM_DWCONV_EALIGN;
-    if (long_gated_kernel_size(K) && split_gated_eligible(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {
+    const int algo = choose_gated_algo(true, bf16, w_dtype == NPLM_DWCONV_BF16, T, C, K, taps, S, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz,
+                                       (uintptr_t)dz);
+    if (algo < 0) return algo;
+    if (algo >= 3) {
         LdsPlan lp;
-        const bool mfma = bf16 && w_dtype == NPLM_DWCONV_BF16 &&
-                          mfma_tile_fits(C, K, true) && mfma_lines_ok(true, true, T, C, K, taps, (uintptr_t)dz) &&
-                          mfma_gated_bwd_preferred(T, taps, S);
+        const bool mfma = algo == 4;
         rc = mfma ? make_split_plan(false, bf16, T, C, K, nullptr, &lp, true, kMfmaGatedRows, kMfmaGatedCb)
                   : make_split_plan(false, bf16, T, C, K, nullptr, &lp, true);
         if (rc) return rc;
@@ -1254,7 +1290,7 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
                            (const float*)part, lp.nbt, C, taps, dw, db, out_bf16, lds_tap_off);
         return (int)hipGetLastError();
     }
-    if (long_gated_bwd_supported(bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) {
+    if (algo == 1) {
         Plan p;
         rc = make_long_gated_plan(bf16, T, C, K, &p);
         if (rc) return rc;
@@ -1273,7 +1309,6 @@ int nplm_dwconv_gated_bwd(const void* z, const void* dy, const int32_t* cu, cons
                            (const float*)part, p.nbt, C, K, dw, db, out_bf16, tap_off);
         return (int)hipGetLastError();
     }
-    if (!gated_supported(true, bf16, T, C, K, (uintptr_t)z | (uintptr_t)dy | (uintptr_t)dz)) return -NPLM_DWCONV_EUNSUPPORTED;
     LdsPlan lp;
     rc = make_lds_plan(true, bf16, T, C, K, nullptr, &lp, true);
     if (rc) return rc == -NPLM_DWCONV_ETUNING ? -NPLM_DWCONV_EUNSUPPORTED : rc;
@@ -1374,6 +1409,12 @@ int32_t nplm_dwconv_debug_algo(int32_t bwd, int64_t T, int32_t C, int32_t K, int
     const int rc = check_common(T, C, K, S, act_dtype, w_dtype);
     if (rc) return rc;
     return choose_algo(bwd != 0, nullptr, act_dtype == NPLM_DWCONV_BF16, w_dtype == NPLM_DWCONV_BF16, T, C, exec_kernel_size(K), lds_taps(K), S, 0, 0);
+}
+
+int32_t nplm_dwconv_debug_gated_algo(int32_t bwd, int64_t T, int32_t C, int32_t K, int32_t S, int32_t act_dtype, int32_t w_dtype) {
+    const int rc = check_common(T, C, K, S, act_dtype, w_dtype);
+    if (rc) return rc;
+    return choose_gated_algo(bwd != 0, act_dtype == NPLM_DWCONV_BF16, w_dtype == NPLM_DWCONV_BF16, T, C, exec_kernel_size(K), lds_taps(K), S, 0, 0);
 }
 
 int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype, const nplm_dwconv_tuning* tune) {

@@ -53,6 +53,8 @@ int32_t nplm_dwconv_bwd_slabs(int64_t T, int32_t C, int32_t K, int32_t act_dtype
 // The kernel family (nplm_dwconv_tuning.algo) the library takes a call of these sizes to, for pointers aligned to cache lines: plain
 // forward (bwd = 0) or a plain backward that asks for every gradient (1). Negative: an argument error.
 int32_t nplm_dwconv_debug_algo(int32_t bwd, int64_t T, int32_t C, int32_t K, int32_t S, int32_t act_dtype, int32_t w_dtype);
+// The same for the gated entry points; -NPLM_DWCONV_EUNSUPPORTED: none.
+int32_t nplm_dwconv_debug_gated_algo(int32_t bwd, int64_t T, int32_t C, int32_t K, int32_t S, int32_t act_dtype, int32_t w_dtype);
 // The kernel size K' a plain or gated conv of K taps is planned as, and its workspace made for (K itself for 3, 5, 7, 9, 15, 31
 // and above 31); K = 11 and 17 .. 21 run kernels of 11 and 21 taps where they take LDS-staged or role-split ones.
 int32_t nplm_dwconv_exec_kernel_size(int32_t K);

@@ -281,6 +281,34 @@ def test_which_kernels_a_bf16_call_takes(bwd, T, C, K, S, algo):
     assert _lib.load().nplm_dwconv_debug_algo(bwd, T, C, K, S, _lib.BF16, _lib.F32) in (1, 2, 3)
 
 
+@pytest.mark.parametrize("bwd,T,C,K,S,algo", [
+    # forward, up to 2048 rows: steps of 64 rows a block (T * C / 2^21), then rows a sequence (below 6; from 192 on)
+    (0, 2048, 1024, 11, 100, 4), (0, 2048, 1152, 11, 100, 3), (0, 2048, 1152, 15, 100, 3), (0, 2048, 1152, 15, 342, 4), (0, 2048, 1152, 15, 341, 3),
+    (0, 2048, 2048, 15, 10, 4), (0, 2048, 2048, 15, 11, 3), (0, 2048, 4096, 11, 128, 3), (0, 2048, 4096, 11, 1, 3), (0, 512, 8192, 11, 32, 3),
+    (0, 1024, 2048, 13, 100, 4), (0, 2048, 2048, 21, 100, 4), (0, 2048, 2176, 21, 100, 3), (0, 2048, 4096, 21, 10, 4), (0, 2048, 4096, 21, 11, 3),
+    (0, 1, 512, 15, 1, 4),
+    # up to 16384 rows, and 31 taps
+    (0, 2049, 512, 15, 10, 4), (0, 2049, 512, 15, 11, 3), (0, 16384, 4096, 21, 85, 4), (0, 16384, 512, 11, 86, 3), (0, 16385, 512, 15, 1, 3),
+    (0, 16384, 8192, 31, 16384, 4), (0, 16385, 512, 31, 512, 4), (0, 16385, 512, 31, 513, 3), (0, 131072, 1000, 31, 500, 4), (0, 64, 512, 29, 64, 4),
+    # backward: 31 taps, short calls and long sequences, whole cache lines from 30 MiB of output on
+    (1, 1, 512, 31, 1, 4), (1, 16384, 512, 31, 16384, 4), (1, 16385, 512, 31, 85, 4), (1, 16385, 512, 31, 86, 3), (1, 16385, 512, 21, 1, 3),
+    (1, 16384, 1000, 31, 1, 3), (1, 15700, 1000, 31, 1, 4), (1, 4096, 512, 15, 1, 3),
+    # rows of less than 1 KiB, sizes with other kernels, none
+    (0, 4096, 256, 31, 1, -10), (1, 4096, 256, 31, 1, 4), (0, 4096, 512, 7, 1, 2), (1, 4096, 512, 7, 1, 2), (0, 4096, 512, 33, 1, -10)])
+def test_which_kernels_a_bf16_gated_call_takes(bwd, T, C, K, S, algo):
+    assert _lib.load().nplm_dwconv_debug_gated_algo(bwd, T, C, K, S, _lib.BF16, _lib.BF16) == algo
+    assert _lib.load().nplm_dwconv_debug_gated_algo(bwd, T, C, K, S, _lib.BF16, _lib.F32) == min(algo, 3)
+
+
+@pytest.mark.parametrize("K", [11, 13])
+def test_gated_forwards_of_11_to_15_taps_take_one_kernel_as_the_same_taps_padded_to_15(K):
+    lib, rng = _lib.load(), np.random.default_rng(K)
+    for _ in range(4000):
+        T, C = int(np.exp(rng.uniform(0, np.log(200000)))), 8 * int(rng.integers(64, 1100))
+        S = int(np.exp(rng.uniform(0, np.log(2 * T + 1))))
+        assert lib.nplm_dwconv_debug_gated_algo(0, T, C, K, S, 1, 1) == lib.nplm_dwconv_debug_gated_algo(0, T, C, 15, S, 1, 1), (T, C, S)
+
+
 # ---- Python surface -----------------------------------------------------------------------------
 def test_cpu_tensors_are_refused():
     x = torch.randn(10, 8)
