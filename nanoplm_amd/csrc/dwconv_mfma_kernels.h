@@ -474,16 +474,29 @@ struct MfmaConv {
 
     // Boundaries among a group's window rows, read by the wave as scalars. wp: its boundary bits (bit 0 is no boundary).
     static constexpr int SPAN = 16 * NSTEP + TP::HALO;       // window rows of the group
-    static constexpr int kFewSequences = NCK >= 7 ? 3 : 0;   // (up to 15 taps a step's passes have too few chunks to leave out)
+    // Up to 15 taps a step's passes have too few chunks to leave out. With three sequences the plain kernels' steps are as fast as three
+    // sweeps and faster where sequences are short (T=131072, C=2048, 16 rows a sequence, none / two / three swept: 21 taps 289 / 287 / 307 us, 31 taps
+    // 326 / 328 / 340; 32 rows 253 / 243 / 244 and 289 / 268 / 266); the gated ones gain (forward of 31 taps, T=16384, C=1024, 24 rows, two / three: 55 / 50,
+    // backward, C=2048, 48 rows 127 / 124).
+    static constexpr int kFewSequences = NCK < 7 ? 0 : GATED || RING ? 3 : 2;
     // whether at most kFewSequences sequences own rows of the group
     __device__ __forceinline__ static bool few_sequences(const uint32_t* wp) {
         int n = 1;
+        if constexpr (GATED || RING) {                       // (short sequences, 4 rows: gated forward 54.5 and 53.2 us, T=16384, C=1024)
+            constexpr int A = TP::FRONT + 1;                 // rows FRONT + 1 .. FRONT + ROWS - 1
 #pragma unroll
-        for (int i = 0; i * 32 < TP::FRONT + ROWS; ++i) {    // rows FRONT + 1 .. FRONT + ROWS - 1
-            constexpr int A = TP::FRONT + 1, B = TP::FRONT + ROWS;
-            const uint32_t from = A > 32 * i ? (A - 32 * i < 32 ? ~0u << (A & 31) : 0u) : ~0u;
-            const uint32_t to = B < 32 * i + 32 ? (1u << (B & 31)) - 1u : ~0u;
-            n += __builtin_popcount((uint32_t)__builtin_amdgcn_readfirstlane((int)(wp[i] & from & to)));
+            for (int i = 0; i < ROWS; i += 32) {
+                const uint32_t w = __builtin_amdgcn_alignbit(wp[(A + i) / 32 + 1], wp[(A + i) / 32], (A + i) & 31);
+                n += __builtin_popcount((uint32_t)__builtin_amdgcn_readfirstlane((int)(i + 32 < ROWS ? w : w & 0x7fffffffu)));
+            }
+        } else {                                             // (plain forward of 21 taps, 75 rows, T=131072, C=2048: that way 211, this one 209)
+#pragma unroll
+            for (int i = 0; i * 32 < TP::FRONT + ROWS; ++i) {    // rows FRONT + 1 .. FRONT + ROWS - 1
+                constexpr int A = TP::FRONT + 1, B = TP::FRONT + ROWS;
+                const uint32_t from = A > 32 * i ? (A - 32 * i < 32 ? ~0u << (A & 31) : 0u) : ~0u;
+                const uint32_t to = B < 32 * i + 32 ? (1u << (B & 31)) - 1u : ~0u;
+                n += __builtin_popcount((uint32_t)__builtin_amdgcn_readfirstlane((int)(wp[i] & from & to)));
+            }
         }
         return n <= kFewSequences;
     }
