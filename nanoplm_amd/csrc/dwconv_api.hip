@@ -400,6 +400,11 @@ bool mfma_bwd_preferred(long long T, int taps, int S) {
     const int rows = taps == 31 ? 32 : taps == 15 ? 64 : 512;
     return T >= (long long)S * rows;
 }
+// Steps (backward: tiles) of 64 rows that a block of the gated matrix-core kernels gets.
+long long mfma_gated_steps_of_a_block(long long T, int C) {
+    const int ncb = ceil_div(2LL * C, kMfmaGatedCb), nbt = ncb < kNumCU ? kNumCU / ncb : 1;
+    return ceil_div(ceil_div(T, kMfmaGatedRows), nbt);
+}
 // The gated backward with dz on the matrix cores: 31 taps. Measured, us, against role-split, for lengths of 20 to 128 residues
 // (mean 75), 20 to 512 (263), log-normal (333), short and long mixed (193), one sequence:
 //   T=131072, C=2048   886/807   705/737   673/721   673/724   619/674         T=32768, C=1024   125/117   100/105   95/105   97/108   87/100
@@ -408,19 +413,23 @@ bool mfma_bwd_preferred(long long T, int taps, int S) {
 // role-split kernel's roles, which share the loss, once a call is longer than its first tiles. 15 taps (T=131072, C=1024: 302/264,
 // T=4096: 19/22) and 21 (306/299) have too few FMAs to save. Calls of up to 16384 rows take it whatever begins in them (C=1024):
 //   T=16384   1 row 138/228   4 71/96   16 66/82   32 63/77   75 67/65        T=4096   1 row 45/83   8 27/40   32 26/39   75 26/36
-// and so do the shortest: T=2048, C=768 1 row 30/49, 16 25/30, 75 21/29, 300 19/27, one sequence 18/26; T=20, C=512 18/21.
-bool mfma_gated_bwd_preferred(long long T, int taps, int S) {
-    return taps == 31 && (T <= 16384 || T >= 192ll * S);
+// and so do the shortest: T=2048, C=768 1 row 30/49, 16 25/30, 75 21/29, 300 19/27, one sequence 18/26; T=20, C=512 18/21. Below 4096 rows
+// only where a block has up to four tiles of 64 rows, which goes by C; with more of them short sequences cost what they do in long calls:
+//   rows a sequence   4         8        16       24       32       48       75       300
+//   T=2048, C=4096 (4 tiles)    58/74    54/63    53/57    55/57    47/54    44/55    41/51    38/49
+//   T=4000, C=2560 (6)          -        70/61    70/57    67/57    61/56    55/53    -        -
+//   T=4000, C=4096 (8)          97/108   91/88    94/81    85/79    76/78    71/76    64/74    57/69
+//   T=4000, C=8192 (16)         -        168/145  163/132  154/131  144/131  123/124  -        -
+bool mfma_gated_bwd_preferred(long long T, int C, int taps, int S) {
+    if (taps != 31) return false;
+    if (T >= kMfmaMinRows) return T <= 16384 || T >= 192ll * S;
+    return mfma_gated_steps_of_a_block(T, C) <= 4 || T < 5ll * S || T >= 64ll * S;
 }
 // The gated forward on the matrix cores: steps of 64 rows in a run, which a block walks down without staging or gating a halo again.
 // All of a block's runs are of one length, the longest that deals the call out evenly (T=65536, C=1152, 15 taps: runs of 16 steps,
 // three rounds for two and a bit, 115 us, of 13 95).
-long long mfma_gated_fwd_steps_of_a_block(long long T, int C) {
-    const int ncb = ceil_div(2LL * C, kMfmaGatedCb), nbt = ncb < kNumCU ? kNumCU / ncb : 1;
-    return ceil_div(ceil_div(T, kMfmaGatedRows), nbt);
-}
 int mfma_gated_fwd_steps(long long T, int C) {
-    const long long per_block = mfma_gated_fwd_steps_of_a_block(T, C);
+    const long long per_block = mfma_gated_steps_of_a_block(T, C);
     return ceil_div(per_block, ceil_div(per_block, kMfmaGatedSteps));
 }
 // Which gated forwards take it, measured by the mean rows of a sequence, us, role-split / matrix cores:
@@ -458,7 +467,7 @@ int mfma_gated_fwd_steps(long long T, int C) {
 bool mfma_gated_fwd_preferred(long long T, int C, int taps, int S) {
     if (taps == 31) return T <= 16384 || T >= 32ll * S;
     if (T > 2048) return T <= 16384 && T >= 192ll * S;
-    const long long steps = mfma_gated_fwd_steps_of_a_block(T, C);
+    const long long steps = mfma_gated_steps_of_a_block(T, C);
     return steps <= (taps == 21 ? 2 : 1) || T < 6ll * S || (T >= 192ll * S && (taps == 21 || steps == 2));
 }
 int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_dwconv_tuning* tune, LdsPlan* out,
@@ -654,7 +663,7 @@ int choose_gated_algo(bool bwd, bool bf16, bool w_bf16, long long T, int C, int 
     if (!supported && !(bwd && role_split)) return -NPLM_DWCONV_EUNSUPPORTED;
     if (!role_split) return bwd && long_gated_kernel_size(K) ? 1 : 2;
     if (!bf16 || !w_bf16) return 3;
-    if (bwd) return mfma_tile_fits(C, K, true) && mfma_lines_ok(true, true, T, C, K, taps, out_bits) && mfma_gated_bwd_preferred(T, taps, S) ? 4 : 3;
+    if (bwd) return mfma_tile_fits(C, K, true) && mfma_lines_ok(true, true, T, C, K, taps, out_bits) && mfma_gated_bwd_preferred(T, C, taps, S) ? 4 : 3;
     LdsPlan lp;
     return mfma_gated_fwd_preferred(T, C, taps, S) &&
            make_split_plan(true, bf16, T, C, K, nullptr, &lp, true, mfma_gated_fwd_steps(T, C) * kMfmaGatedRows, kMfmaGatedCb) == 0 &&

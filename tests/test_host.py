@@ -290,7 +290,9 @@ def test_which_kernels_a_bf16_call_takes(bwd, T, C, K, S, algo):
     # up to 16384 rows, and 31 taps
     (0, 2049, 512, 15, 10, 4), (0, 2049, 512, 15, 11, 3), (0, 16384, 4096, 21, 85, 4), (0, 16384, 512, 11, 86, 3), (0, 16385, 512, 15, 1, 3),
     (0, 16384, 8192, 31, 16384, 4), (0, 16385, 512, 31, 512, 4), (0, 16385, 512, 31, 513, 3), (0, 131072, 1000, 31, 500, 4), (0, 64, 512, 29, 64, 4),
-    # backward: 31 taps, short calls and long sequences, whole cache lines from 30 MiB of output on
+    # backward: 31 taps; up to 4 tiles a block below 4096 rows, short calls and long sequences, whole cache lines from 30 MiB of output on
+    (1, 2048, 4096, 31, 128, 4), (1, 4000, 4096, 31, 800, 3), (1, 4000, 4096, 31, 801, 4), (1, 4000, 4096, 31, 62, 4), (1, 4000, 4096, 31, 63, 3),
+    (1, 4095, 2048, 31, 256, 4), (1, 4095, 2560, 31, 256, 3), (1, 4096, 2560, 31, 256, 4),
     (1, 1, 512, 31, 1, 4), (1, 16384, 512, 31, 16384, 4), (1, 16385, 512, 31, 85, 4), (1, 16385, 512, 31, 86, 3), (1, 16385, 512, 21, 1, 3),
     (1, 16384, 1000, 31, 1, 3), (1, 15700, 1000, 31, 1, 4), (1, 4096, 512, 15, 1, 3),
     # rows of less than 1 KiB, sizes with other kernels, none
