@@ -529,14 +529,25 @@ __device__ __forceinline__ void finalize_block(float (&red)[SPLIT][64], int bloc
     if (on) {
         const float* src = partial + o;
         const size_t stride = (size_t)n_out;
-        // Eight loads at a time whatever the group's share (those past its end repeat its last slab and are not added): one after the
-        // other a share of six took 6 times the latency of memory.
-        for (int p = p0; p < p1; p += 8) {
+        int p = p0;
+        for (; p + 8 <= p1; p += 8) {
             float t[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) t[i] = src[(size_t)(p + i < p1 ? p + i : p1 - 1) * stride];
+            for (int i = 0; i < 8; ++i) t[i] = src[(size_t)(p + i) * stride];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s = p + i < p1 ? s + t[i] : s;
+            for (int i = 0; i < 8; ++i) s += t[i];
+        }
+        // What is left is loaded at once too, where it is three or more (those past the end repeat the last slab and are not added): one
+        // after the other a share of six took 6 times the latency of memory (T=2048, C=768, 7 taps, fp32 12.1 and 11.1 us). Whole eights
+        // that way would cost what they gain there (T=131072, C=64 28.6 and 29.4).
+        if (p + 2 < p1) {
+            float t[7];
+#pragma unroll
+            for (int i = 0; i < 7; ++i) t[i] = src[(size_t)(p + i < p1 ? p + i : p1 - 1) * stride];
+#pragma unroll
+            for (int i = 0; i < 7; ++i) s = p + i < p1 ? s + t[i] : s;
+        } else {
+            for (; p < p1; ++p) s += src[(size_t)p * stride];
         }
     }
     red[grp][lane] = s;
