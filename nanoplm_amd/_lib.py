@@ -1,13 +1,15 @@
 """ctypes binding of libnplm_dwconv.so (the C ABI declared in include/nplm_dwconv.h).
 
 The library is built in-tree by ``make -C nanoplm_amd/csrc`` (or ``__graft_entry__.build()``).
-There is no fallback: if the shared object is missing, every call raises.
+There is no fallback: if the shared object is missing, every call raises. The native autograd nodes beside it are a shorter way to
+the same kernels: where they cannot be loaded, calls reach the library through the Python Functions.
 """
 from __future__ import annotations
 
 import ctypes
 import importlib
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libnplm_dwconv.so")
@@ -120,14 +122,39 @@ def load():
     return lib
 
 
+class _NoNode:
+    """Stands for the native nodes where they cannot be loaded: leaves every call to the Python route, as they leave some."""
+
+    @staticmethod
+    def dwconv(*args):
+        return None
+
+    gated_dwconv = ln_dwconv = dwconv
+
+
+def _import_node():
+    import torch
+    built = f"build them with `make -C {os.path.join(_HERE, 'csrc')}`"
+    if not os.path.exists(NODE_PATH):
+        why = f"{NODE_PATH} is missing: {built}"
+    else:
+        try:
+            node = importlib.import_module("nanoplm_amd._node")
+            if node.torch_version == torch.__version__.split("+")[0]:
+                return node
+            why = f"they were built for torch {node.torch_version}, this is {torch.__version__}: {built}"
+        except ImportError as e:                # (symbols of another torch)
+            why = f"{e}: {built}"
+    warnings.warn(f"nanoplm_amd: the native autograd nodes are not in use, calls take more time on the host ({why})", RuntimeWarning)
+    return _NoNode
+
+
 def load_node():
-    """The native autograd nodes (``csrc/node.cpp``), built beside the library and linked to it."""
+    """The native autograd nodes (``csrc/node.cpp``), built beside the library and linked to it, for the torch they were built with."""
     global _node
-    load()
     if _node is None:
-        if not os.path.exists(NODE_PATH):
-            raise RuntimeError(f"{NODE_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}`")
-        _node = importlib.import_module("nanoplm_amd._node")
+        load()
+        _node = _import_node()
     return _node
 
 

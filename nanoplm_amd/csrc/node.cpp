@@ -382,4 +382,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_node", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__node() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__node() {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -346,6 +346,31 @@ def test_missing_library_fails_loudly(monkeypatch):
         _lib.load()
 
 
+@pytest.mark.parametrize("case", ["missing", "other symbols", "other version"])
+def test_without_loadable_native_nodes_calls_are_left_to_the_python_route(monkeypatch, case):
+    import types
+    monkeypatch.setattr(_lib, "_node", None)
+    if case == "missing":
+        monkeypatch.setattr(_lib, "NODE_PATH", "/nonexistent/_node.so")
+    else:
+        def other(name):
+            if case == "other symbols":
+                raise ImportError("_node.so: undefined symbol: _ZN5torch3jit")
+            return types.SimpleNamespace(torch_version="2.0.0")
+        monkeypatch.setattr(_lib.importlib, "import_module", other)
+    with pytest.warns(RuntimeWarning, match="native autograd nodes are not in use"):
+        node = _lib.load_node()
+    assert node.dwconv(*range(5)) is None and node.gated_dwconv(*range(5)) is None and node.ln_dwconv(*range(8)) is None
+    assert _lib.load_node() is node
+    with pytest.raises(RuntimeError, match="no CPU implementation"):          # (the Python route's own message)
+        nanoplm_amd.VarlenDWConv1d(8, 3)(torch.randn(10, 8), torch.tensor([0, 10], dtype=torch.int32))
+
+
+def test_native_nodes_are_for_the_torch_that_runs():
+    node = _lib.load_node()
+    assert node.__name__ == "nanoplm_amd._node" and node.torch_version == torch.__version__.split("+")[0]
+
+
 def test_product_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "nanoplm_amd")
     for dirpath, _, files in os.walk(pkg):
