@@ -371,6 +371,14 @@ def test_native_nodes_are_for_the_torch_that_runs():
     assert node.__name__ == "nanoplm_amd._node" and node.torch_version == torch.__version__.split("+")[0]
 
 
+@pytest.mark.parametrize("args", [["lib"], ["PYTHON=/nonexistent/python"], ["CXX=/nonexistent/g++"]])
+def test_the_library_builds_without_python_torch_or_a_host_compiler(args):
+    import subprocess
+    out = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "nanoplm_amd", "csrc"), *args], capture_output=True, text=True)
+    assert out.returncode == 0 and not out.stderr.strip(), out.stderr
+    assert "-o ../libnplm_dwconv.so" in out.stdout and "node" not in out.stdout
+
+
 def test_product_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "nanoplm_amd")
     for dirpath, _, files in os.walk(pkg):
