@@ -351,6 +351,7 @@ def test_native_prenorm_node_takes_gradients_and_tensors_of_every_kind():
     assert same(got, want) and any("ln_dwconv_bwd" in f for f in seen)
 
 
+@pytest.mark.filterwarnings("ignore:Error detected in")
 @pytest.mark.parametrize("form,name", [("plain", "varlen_dwconv"), ("gated", "gated_dwconv"), ("ln", "ln_dwconv")])
 def test_profiles_and_messages_name_the_native_nodes(form, name):
     """A profile lists an eager call and its backward by the names of the registered ops; autograd's messages name the function."""
@@ -379,3 +380,94 @@ def test_native_nodes_leave_calls_without_a_fused_kernel_before_they_begin(form)
     before = count()
     assert (node.gated_dwconv(x, cu, w, v, False) if form == "gated" else node.ln_dwconv(x, cu, v, None, w, v, 1e-5, False)) is None
     assert count() == before
+
+
+def _kernel_door(form, K):
+    """The door with kernels of K taps (on the matrix cores where they exist) on 4500 rows of 512 channels; its tensors, x first."""
+    C, T = 512, 4500
+    g = torch.Generator().manual_seed(K)
+    rnd = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).bfloat16().to(DEV)
+    cu = torch.tensor([0, 1000, 1001, 2500, T], dtype=torch.int32, device=DEV)
+    x, w, b = rnd(T, 2 * C if form == "gated" else C), rnd(C, K, scale=K ** -0.5), rnd(C)
+    if form == "ln":
+        return lambda x, lw, lb, w, b: npa.ln_varlen_dwconv_compilable(x, cu, lw, lb, w, b, residual=True), [x, rnd(C), rnd(C), w, b]
+    f = npa.gated_varlen_dwconv if form == "gated" else npa.varlen_dwconv
+    return lambda x, w, b: f(x, cu, w, b, True), [x, w, b]
+
+
+_NODE_CASES = [("plain", 7), ("plain", 31), ("gated", 7), ("gated", 31), ("ln", 7)]
+
+
+def _step(door, leaves, dy):
+    y = door(*leaves)
+    return (y.detach(), *torch.autograd.grad(y, leaves, dy))
+
+
+@pytest.mark.parametrize("form,K", _NODE_CASES)
+def test_native_nodes_on_a_side_stream_and_from_several_threads(form, K):
+    """Forwards on streams of their own (the engine runs their backwards there), temporaries freed and reused meanwhile; then two threads."""
+    import threading
+    door, args = _kernel_door(form, K)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    calls = []
+    for _ in range(6):
+        leaves = [torch.empty_like(args[0]).normal_(generator=g)] + [t.clone() for t in args[1:]]
+        leaves = [t.requires_grad_() for t in leaves]
+        calls.append((leaves, torch.empty(args[0].shape[0], 512, dtype=torch.bfloat16, device=DEV).normal_(generator=g)))
+    want = [_step(door, *c) for c in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    got = []
+    for i, c in enumerate(calls):
+        with torch.cuda.stream(streams[i % 3]):
+            got.append(_step(door, *c))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, r) for gs, ws in zip(got, want) for a, r in zip(gs, ws))
+    out = [None] * len(calls)
+
+    def work(k):
+        with torch.cuda.stream(streams[k]):
+            for i in range(k, len(calls), 2):
+                out[i] = _step(door, *calls[i])
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, r) for gs, ws in zip(out, want) for a, r in zip(gs, ws))
+
+
+@pytest.mark.parametrize("form,K", _NODE_CASES)
+def test_native_nodes_replay_from_a_hip_graph_and_run_under_checkpointing(form, K):
+    """A captured forward and backward of the door, replayed on new contents with eager work and synchronization between the replays; and
+    the same step under activation checkpointing, reentrant and not."""
+    from torch.utils.checkpoint import checkpoint
+    door, args = _kernel_door(form, K)
+    leaves = [t.clone().requires_grad_() for t in args]
+    dy = torch.randn(args[0].shape[0], 512, device=DEV).bfloat16()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _step(door, leaves, dy)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = _step(door, leaves, dy)
+    for it in range(4):
+        with torch.no_grad():
+            leaves[0].normal_()
+            dy.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = _step(door, leaves, dy)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, r) for a, r in zip(captured, eager)), f"replay {it}"
+    for reentrant in (False, True):
+        y = checkpoint(door, *leaves, use_reentrant=reentrant)
+        for t in leaves:
+            t.grad = None
+        y.backward(dy)
+        assert torch.equal(y, eager[0]) and all(torch.equal(t.grad, r) for t, r in zip(leaves, eager[1:]))

@@ -54,11 +54,10 @@ LENS_LONG = LENS_MIX + [40, 33, 31, 30, 29, 16, 15, 14, 0, 1, 1, 700]
                                        (torch.bfloat16, torch.bfloat16, 520), (torch.float32, torch.float32, 256),
                                        (torch.float32, torch.float32, 776), (torch.bfloat16, torch.bfloat16, 1152)])
 def test_long_gated_kernel_sizes_and_widths(K, dt, wdt, C):
-    """K = 15 and 31 (the intermediate-width configuration is C = 2048, K = 31): the forward forms the gate product in
-    LDS once per staged element (rows of at least 512 bytes: every wave gates its share of a 128-row tile and then runs
-    the taps; narrower rows: loader waves gate 32-row tiles); the backward is the role-split kernel with the gate in
-    both roles (rows of at least 512 bytes) or the sliding-window kernel with the gate on its centre rows (C = 256 in
-    bf16 would be; 520 takes column blocks of which the last is nearly empty)."""
+    """K = 15 and 31 (the intermediate-width configuration is C = 2048, K = 31). With bf16 weights both passes of 31 taps take the matrix cores
+    here, with fp32 weights (and the backward of 15 taps) the role-split kernels: every wave gates its share of a 128-row tile in LDS once per
+    staged element and then runs the taps; the backward has the gate in both roles. 520 takes column blocks of which the last is
+    nearly empty."""
     print(f"[case] long gated K={K} C={C} {dt} w {wdt}", flush=True)
     _check(*_case(LENS_LONG, C, K, dt, wdt, seed=K + C), f"gated K={K} C={C} {dt}")
     _check(*_case(LENS_LONG[::-1], C, K, dt, wdt, seed=K + C + 1), f"gated residual K={K} C={C} {dt}", residual=True)

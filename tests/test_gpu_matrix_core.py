@@ -179,14 +179,23 @@ def test_which_rows_of_partial_cache_lines_the_matrix_cores_serve(bwd, T, C, K, 
     assert all(torch.equal(a, c) for a, c in zip((out, dw, db), want))
 
 
-@pytest.mark.parametrize("K,lens,C", [(31, LENS * 2, 512), (29, LENS[::-1] * 2, 520), (25, [4096], 1000), (31, [4095, 1, 63], 648),
-                                      (31, LENS * 4, 2056), (31, [1] * 4160, 512), (31, [4095], 512), (31, [16500] + [1] * 200, 512)])
-def test_gated_backward_of_31_taps_matches_the_oracle(K, lens, C):
-    """From 4096 rows on dz comes from the matrix cores and dw from waves of 8 rows that leave out the products across a
-    boundary (below, and with many short sequences in a long batch, from the role-split kernel): whole, partial and several
-    column blocks, rows of one sequence and of many in a wave, and the same bits after a call that left NaN in LDS."""
+def _gated_algo(bwd, T, C, K, S):
+    """4: matrix cores, 3: role-split."""
+    return _lib.load().nplm_dwconv_debug_gated_algo(bwd, T, C, K, S, _lib.BF16, _lib.BF16)
+
+
+@pytest.mark.parametrize("K,lens,C,algo", [
+    (31, LENS * 2, 512, 4), (29, LENS[::-1] * 2, 520, 4), (25, [4096], 1000, 4), (31, [4095, 1, 63], 648, 4), (31, LENS * 4, 2056, 3), (31, LENS * 4, 2048, 4),
+    (31, [1] * 4160, 512, 4), (31, [4095], 512, 4), (31, [16500] + [1] * 200, 512, 3),
+    # both sides of the lines: 16384 rows, five to 63 rows a sequence in more than four tiles a block
+    (31, [100] * 163 + [84], 512, 4), (31, [100] * 163 + [85], 512, 3), (31, [16] * 160, 2560, 4), (31, [16] * 210, 2560, 3), (31, [64] * 52, 2560, 4)])
+def test_gated_backward_of_31_taps_matches_the_oracle(K, lens, C, algo):
+    """dz comes from the matrix cores and dw from waves of 8 rows that leave out the products across a boundary (with short sequences in
+    long batches, or in wide rows, from the role-split kernel): whole, partial and several column blocks, rows of one sequence and of
+    many in a wave, and the same bits after a call that left NaN in LDS."""
     print(f"[case] gated K={K} C={C}", flush=True)
     _, cu, w, b, dy = _case(lens, C, K, C + K)
+    assert _gated_algo(1, dy.shape[0], C, K, len(lens)) == algo
     z = torch.randn(dy.shape[0], 2 * C, generator=torch.Generator().manual_seed(C)).bfloat16()
     zd, cud, wd, dyd = z.to(DEV), cu.to(DEV), w.to(DEV), dy.to(DEV)
     for res in (False, True):
@@ -404,17 +413,20 @@ def test_share_of_outputs_that_are_not_correctly_rounded(K):
 
 
 # (built as 15 and 31 taps; whole, partial and several column blocks; one run a block, and with C=8200 two; runs that end inside a
-# step; a boundary at every row of the 32-row groups, one to many in a group)
-@pytest.mark.parametrize("K,lens,C", [(31, LENS * 2, 512), (29, LENS[::-1] * 2, 520), (25, [4096], 1000), (31, [95] * 44, 520),
-                                      (31, [191] * 22, 8200), (15, LENS * 2, 776), (13, [63] * 66, 1160), (21, [4095, 1], 512),
-                                      (11, [2500, 1, 1700], 520), (31, [1] * 4100, 512), (15, [17] * 260, 512),
-                                      (15, [17] * 120, 512), (13, [63] * 32, 1160), (11, [1] * 1900, 512)])
-def test_gated_forward_on_the_matrix_cores_matches_the_oracle(K, lens, C):
+# step; a boundary at every row of the 32-row groups, one to many in a group; some calls that the role-split kernel keeps)
+@pytest.mark.parametrize("K,lens,C,algo", [
+    (31, LENS * 2, 512, 4), (29, LENS[::-1] * 2, 520, 4), (25, [4096], 1000, 4), (31, [95] * 44, 520, 4), (31, [191] * 22, 8200, 4),
+    (15, LENS * 2, 776, 3), (13, [63] * 66, 1160, 3), (21, [4095, 1], 512, 4), (11, [2500, 1, 1700], 520, 4), (31, [1] * 4100, 512, 4),
+    (15, [17] * 260, 512, 3), (15, [17] * 120, 512, 4), (13, [63] * 32, 1160, 3), (11, [1] * 1900, 512, 4),
+    (15, LENS[:30], 776, 4), (13, [63] * 32, 1000, 4), (15, [63] * 10 + [1500, 2, 3, 1700, 1, 700], 776, 4), (15, [3] * 600, 1160, 4),
+    (21, [95] * 21, 2048, 4), (17, [31] * 60, 1544, 4)])
+def test_gated_forward_on_the_matrix_cores_matches_the_oracle(K, lens, C, algo):
     """To one bf16 rounding of the oracle's y: the three bf16 terms add up to the fp32 h. The same bits again after a call that left NaN
     in the LDS; rows in front of and behind y keep theirs."""
     print(f"[case] gated forward K={K} C={C}", flush=True)
     _, cu, w, b, dy = _case(lens, C, K, C + K)
     T = dy.shape[0]
+    assert _gated_algo(0, T, C, K, len(lens)) == algo
     z = torch.randn(T, 2 * C, generator=torch.Generator().manual_seed(C)).bfloat16()
     zd, cud, wd, bd = z.to(DEV), cu.to(DEV), w.to(DEV), b.to(DEV)
     lib = _lib.load()
@@ -496,3 +508,96 @@ def test_gated_forward_keeps_the_range_of_fp32(K, what, h_exp, w_exp, residual):
         torch.testing.assert_close(got[~fin], want[~fin], rtol=0, atol=0, equal_nan=True)
         if where == "z":
             assert bool(((got.cpu().double() - ref).abs() <= bound)[fin.cpu()].all())
+
+
+@pytest.mark.parametrize("K", [15, 21, 31])
+@pytest.mark.parametrize("C", [512, 520])
+def test_gated_calls_of_fewer_rows_than_a_tile_or_a_halo(K, C):
+    """One sequence, and a boundary behind every third row; forward, and (31 taps on the matrix cores) backward. Rows around the outputs keep
+    their values."""
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    for T in (1, 2, 15, 16, 31, 63, 64, 65, 129):
+        for lens in ([T], [3] * (T // 3) + [T % 3]):
+            _, cu, w, b, dy = _case(lens, C, K, C + K + T)
+            z = torch.randn(T, 2 * C, generator=torch.Generator().manual_seed(T)).bfloat16()
+            assert _gated_algo(0, T, C, K, len(lens)) == 4 and _gated_algo(1, T, C, K, len(lens)) == (4 if K == 31 else 3)
+            y64, dz64, dw64, db64 = O.ref_gated_dwconv_grads(z, cu, w, b, dy, torch.float64)
+            zd, cud, wd, bd, dyd = (t.to(DEV) for t in (z, cu, w, b, dy))
+            y, dz = (torch.full((T + 4, n), 7.0, dtype=torch.bfloat16, device=DEV) for n in (C, 2 * C))
+            dw, db = torch.full((C + 2, K), 7.0, device=DEV), torch.full((C + 2,), 7.0, device=DEV)
+            ws = torch.empty(int(lib.nplm_dwconv_gated_bwd_workspace_bytes(T, C, K, _lib.BF16)), dtype=torch.uint8, device=DEV)
+            sizes = (T, C, K, len(lens), _lib.BF16, _lib.BF16, 0, st)
+            _lib.check(lib.nplm_dwconv_gated_fwd(zd.data_ptr(), cud.data_ptr(), wd.data_ptr(), bd.data_ptr(), y[2:].data_ptr(), *sizes), "fwd")
+            _lib.check(lib.nplm_dwconv_gated_bwd(zd.data_ptr(), dyd.data_ptr(), cud.data_ptr(), wd.data_ptr(), dz[2:].data_ptr(), dw[1:].data_ptr(),
+                                                 db[1:].data_ptr(), ws.data_ptr(), ws.numel(), *sizes), "bwd")
+            assert_act_close(y[2:-2], y64, torch.bfloat16, f"y T={T}")
+            assert_act_close(dz[2:-2], dz64, torch.bfloat16, f"dz T={T}")
+            assert_red_close(dw[1:-1], dw64, f"dw T={T}")
+            assert_red_close(db[1:-1], db64, f"db T={T}")
+            for t, n in ((y, 2), (dz, 2), (dw, 1), (db, 1)):
+                assert bool((t[:n] == 7).all()) and bool((t[-n:] == 7).all())
+
+
+# runs of the gated forward: T, C -> steps a run, runs and slots: (16347, 2176) 9, 29 on 15 (a slot without a run in the last round), the last run
+# cut inside a step; (65500, 768) 13, 79 on 42; (131072, 2048) 16, 128 on 16
+@pytest.mark.parametrize("K,T,C", [(15, 16347, 2176), (31, 16347, 2176), (31, 65500, 768), (31, 131072, 2048)])
+def test_gated_forward_in_several_runs_a_block(K, T, C):
+    """Boundaries at a run's first rows, in front of and behind them (a run of 9 steps begins every 576 rows, of 13 every 832, of 16 every 1024);
+    a few channels of every column block against the oracle, all against the role-split kernel (which takes the same weights in fp32)."""
+    run = {16347: 576, 65500: 832, 131072: 1024}[T]
+    starts = sorted({run * i + d for i in range(1, T // run + 1) for d in ((0,), (1,), (-1,), (0, 3), (-2, 2), (15,), (-15, 31))[i % 7] if i % 3})
+    cu = torch.tensor([0] + [t for t in starts if t < T] + [T], dtype=torch.int32)
+    S = cu.numel() - 1
+    assert _gated_algo(0, T, C, K, S) == 4
+    g = torch.Generator(device=DEV).manual_seed(T)
+    z = torch.empty(T, 2 * C, device=DEV, dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(C, K, device=DEV, dtype=torch.bfloat16).normal_(0, K ** -0.5, generator=g)
+    b = torch.empty(C, device=DEV, dtype=torch.bfloat16).normal_(generator=g)
+    y = npa.gated_dwconv_fwd(z, cu.to(DEV), w, b)
+    torch.testing.assert_close(y, npa.gated_dwconv_fwd(z, cu.to(DEV), w.float(), b.float()), rtol=2.0 ** -7, atol=1e-5)
+    ch = torch.arange(37, C, 128, device=DEV)
+    want = O.ref_gated_dwconv_grads(z[:, torch.cat([ch, ch + C])].cpu(), cu, w[ch].cpu(), b[ch].cpu(), None, torch.float64)
+    assert_act_close(y[:, ch], want, torch.bfloat16, "y")
+
+
+def test_gated_forward_rows_beyond_2_and_4_gib_offsets():
+    """1.2 M rows of z of 4 KiB: whole sequences cut out of the batch give the same y alone (their first row is a multiple of four, which is
+    what the order of a row's sums goes by)."""
+    T, C, K = 1_200_000, 1024, 31
+    g = torch.Generator().manual_seed(79)
+    lens = 4 * torch.randint(5, 129, (T // 200,), generator=g)
+    lens = lens[torch.cumsum(lens, 0) <= T]
+    cu = cu_from_lengths(torch.cat([lens, torch.tensor([T - int(lens.sum())])])).to(DEV)
+    z = torch.randn(T, 2 * C, device=DEV, dtype=torch.bfloat16)
+    w = (torch.randn(C, K, device=DEV) * K ** -0.5).bfloat16()
+    cul = cu.tolist()
+    S = len(cul) - 1
+    assert _gated_algo(0, T, C, K, S) == 4
+    y = npa.gated_dwconv_fwd(z, cu, w, None, residual=True)
+    assert cul[S // 2] * C * 4 > 2 ** 31 and cul[S - 40] * C * 4 > 2 ** 32
+    for first in (0, S // 2 - 20, S - 40):
+        s, e = cul[first], cul[first + 40]
+        sub = (cu[first:first + 41] - s).contiguous()
+        assert _gated_algo(0, e - s, C, K, 40) == 4
+        assert torch.equal(y[s:e], npa.gated_dwconv_fwd(z[s:e], sub, w, None, residual=True)), f"rows {s}..{e}"
+
+
+@pytest.mark.parametrize("K,Kx,lens,same", [(11, 15, [17] * 120, True), (11, 15, [200] * 12, True), (21, 31, [300] * 10, True),
+                                            (21, 31, [20] * 300, False), (17, 31, [20] * 300, False)])
+def test_gated_taps_padded_to_the_planned_size(K, Kx, lens, same):
+    """The same bits where both sizes take the same kernels; 17 to 21 taps and 31 part where short sequences keep the smaller one on the
+    role-split kernel, and in the backward: there to the two roundings of one sum."""
+    C = 512
+    _, cu, w, b, dy = _case(lens, C, K, K)
+    z = torch.randn(dy.shape[0], 2 * C, generator=torch.Generator().manual_seed(K)).bfloat16().to(DEV)
+    wide = torch.nn.functional.pad(w, ((Kx - K) // 2,) * 2).contiguous().to(DEV)
+    cu, w, b, dy = (t.to(DEV) for t in (cu, w, b, dy))
+    assert (_gated_algo(0, dy.shape[0], C, K, len(lens)) == _gated_algo(0, dy.shape[0], C, Kx, len(lens))) == same
+    y, yx = npa.gated_dwconv_fwd(z, cu, w, b), npa.gated_dwconv_fwd(z, cu, wide, b)
+    assert torch.equal(y, yx) or not same
+    torch.testing.assert_close(y, yx, rtol=2.0 ** -7, atol=1e-5)
+    bwd = [npa.gated_dwconv_bwd(z, dy, cu, v) for v in (w, wide)]
+    equal = _gated_algo(1, dy.shape[0], C, K, len(lens)) == _gated_algo(1, dy.shape[0], C, Kx, len(lens))
+    assert equal == (Kx == 15)
+    assert torch.equal(bwd[0][0], bwd[1][0]) or not equal
+    torch.testing.assert_close(bwd[0][0], bwd[1][0], rtol=2.0 ** -7, atol=1e-5)
