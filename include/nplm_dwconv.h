@@ -22,8 +22,10 @@
  *   workspace holds slabs of that size; K = 11 and 17 .. 21 leave part of the zero taps out where a call
  *   takes LDS-staged or matrix-core kernels): for finite inputs the same sums with exact zeros added,
  *   so the results of a call of that size with padded taps, bit for bit where both take the same
- *   kernels (from T = 4096 on a backward in bf16 may not: K = 11 and 17 .. 21 keep the vector ALU for
- *   longer sequences than 15 and 31; the fp32 sums then differ in their order). A NaN/Inf in x or dy
+ *   kernels. In bf16 they may not: backward from T = 4096 on, where K = 11 and 17 .. 21 keep the vector
+ *   ALU for longer sequences than 15 and 31; gated forward, where 17 .. 21 keep it for shorter sequences
+ *   than 31; gated backward, where 17 .. 21 always keep it (see S below). The fp32 sums then differ in
+ *   their order. A NaN/Inf in x or dy
  *   then reaches the rows within that larger half-width of its own sequence (0 * Inf; on the matrix cores
  *   those within its own K taps only), never another sequence, and never a tap of dw that its products do
  *   not belong to. Odd K from 33 to NPLM_DWCONV_MAX_K run untuned kernels (one wave per row). The gated entry
@@ -46,14 +48,23 @@
  *  - Which kernels run and their launch geometry depend only on (T, C, K, S, dtypes) and on whether
  *    pointers are aligned to 16 bytes (outputs: to 128), never on timing or on what the tensors
  *    hold: results are run-to-run bit-identical (no floating-point atomics anywhere).
- *  - S counts every entry of cu, empty sequences too. It changes which kernels run in the backward with
- *    bf16 activations and weights, K from 11 to 31 and T >= 4096 only: the matrix cores take calls of at
- *    least 32 rows per sequence at K = 31 (64 at 15, 512 at 11 and 21; gated, K = 31 from T = 16385 on,
- *    192), counted as T / S. A long tail of empty sequences therefore costs speed (and another order of
- *    the fp32 sums of dx, dz, dw): pass S without it where its length is known on the host.
- *  - On the matrix cores (bf16 activations and weights, K from 11 to 31, T >= 4096) the order of a row's
- *    fp32 sum goes by the row's number modulo 4: a sequence alone and the same one inside a batch may
- *    differ by one bf16 rounding in y, dx and dz. Other kernels give the same bits in both.
+ *  - S counts every entry of cu, empty sequences too. With bf16 activations and weights and K from 11 to
+ *    31 it has a say in which kernels run, by T / S, the rows per sequence. The matrix cores take
+ *      plain forward    whatever S, from T = 4096 on;
+ *      plain backward   from T = 4096 on: K = 23 .. 31 from 32 rows on, 13 and 15 from 64, 11 and 17 .. 21
+ *                       from 512;
+ *      gated forward    K = 23 .. 31 up to T = 16384, beyond from 32 rows on; smaller K up to T = 16384 from
+ *                       192 rows on, and up to T = 2048 narrow calls (T * C up to 2^21; 2^22 from K = 17 on)
+ *                       and sequences of less than 6 rows too (but K < 17 beyond 2^22 those alone);
+ *      gated backward   K = 23 .. 31 up to T = 16384, beyond from 192 rows on; below T = 4096 wide calls
+ *                       (T * C beyond 2^23) of 5 to 63 rows stay away.
+ *    (roughly: tiles are whole, and large outputs of partial cache lines stay away as well). A long tail
+ *    of empty sequences can therefore cost speed, and another order of the fp32 sums of a gated y, of dx,
+ *    dz and dw: pass S without it where its length is known on the host.
+ *  - On the matrix cores (plain calls from T = 4096 on, gated calls of any T) the order of a row's fp32
+ *    sum goes by the row's number modulo 4: a sequence alone and the same one inside a batch may differ
+ *    by one bf16 rounding in y, dx and dz, and so may they where one of the two calls takes other kernels.
+ *    The other kernels give the same bits in both.
  *  - Return value: 0 on success; < 0 an NPLM_DWCONV_E* argument error (nothing was launched);
  *    > 0 a hipError_t from a launch.
  *  - Preconditions NOT checked on the fast path (they would need a device read-back):
