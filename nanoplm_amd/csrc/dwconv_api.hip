@@ -366,15 +366,15 @@ bool mfma_tile_fits(int C, int K, bool gated) {
 // complete later. mfma_lines() lets them meet in the L2; in outputs too large for it and the Infinity Cache many reach HBM as parts all
 // the same, and up to 15 taps the others are faster there. Measured with lengths of 20 to 512 (backward at 11 and 21 taps: 700) residues, us,
 // matrix cores / the best of the others, by MiB of output:
-//   forward, 11 taps: T=131072 C=1000 (250 MiB) 127 / 112, C=1160 (290) 154 / 152, C=2008 (502) 246 / 215; T=65536 C=1800 (225) 110 / 107,
-//     C=1160 (145) 70 / 78, C=1000 (125) 55 / 62; T=131072 C=648 (162) 85 / 100; 15 taps the same to 3 %. Rows that fill the others'
-//     1 KiB column blocks to less than 3/5 stay: C=584 (0.57) T=131072 78 / 90.
-//   backward, 11 / 15 taps: T=131072 C=2008 (502) 433 / 364, 432 / 367; C=1160 (290) 247 / 216, 249 / 226; C=1032 (258) 204 / 207, 212 / 222;
-//     C=648 (162) 118 / 132, 127 / 138; T=16384 C=1000 (31) 34 / 38, 37 / 41.
-//   gated backward, 31 taps (stores with `nt` always): T=131072 C=2008 (502) 1011 / 762, C=1000 518 / 392; T=65536 C=584 (73) 157 / 144;
-//     T=16384 C=1000 (31) 68 / 65, C=648 (20) 53 / 54, C=520 (16) 47 / 53.
-// 31 taps save more FMAs than that costs (T=131072 C=2040 forward 254 / 304, backward 434 / 517), and so do 21 forward (258 / 307); 21
-// backward come out even (C=2008 423 / 393, C=1160 255 / 246, C=1800 373 / 380, T=98304 262 / 293) and stay.
+//   forward, 11 taps: T=131072 C=1000 (250 MiB) 125 / 103, C=1160 (290) 152 / 147, C=2008 (502) 243 / 216; T=65536 C=1800 (225) 110 / 107,
+//     C=1160 (145) 69 / 80, C=1000 (125) 56 / 61; T=131072 C=648 (162) 83 / 98; 15 taps the same to 3 %. Rows that fill the others'
+//     1 KiB column blocks to less than 3/5 stay: C=584 (0.57) T=131072 77 / 96.
+//   backward, 11 / 15 taps: T=131072 C=2008 (502) 424 / 359, 427 / 369; C=1160 (290) 235 / 212, 242 / 227; C=1032 (258) 200 / 213, 210 / 219;
+//     C=648 (162) 118 / 129, 129 / 139; T=16384 C=1000 (31) 34 / 38, 37 / 41.
+//   gated backward, 31 taps (stores with `nt` always): T=131072 C=2008 (502) 1015 / 778, C=1000 507 / 384; T=65536 C=584 (73) 151 / 145;
+//     T=16384 C=1000 (31) 64 / 69, C=648 (20) 51 / 52, C=520 (16) 45 / 51.
+// 31 taps save more FMAs than that costs (T=131072 C=2040 forward 254 / 331, backward 430 / 509), and so do 21 forward (259 / 303); 21
+// backward come out even (C=2008 423 / 394, C=1160 257 / 247, C=1800 378 / 383, T=98304 C=1160 179 / 190) and stay.
 bool mfma_lines_ok(bool bwd, bool gated, long long T, int C, int K, int taps, uintptr_t out_bits) {
     const long long row_bytes = 2LL * C;
     if (((uintptr_t)row_bytes | out_bits) % 128 == 0) return true;
@@ -388,13 +388,14 @@ bool mfma_lines_ok(bool bwd, bool gated, long long T, int C, int K, int taps, ui
 // A backward tile with sequence boundaries makes one pass over its rows per sequence for dw, so the gain goes with the length
 // of the sequences. Measured at T=131072, us, matrix cores against role-split, for lengths of 20 to 128 residues (mean 75), 20
 // to 512 (mean 263), log-normal (mean 333), one sequence:
-//   K=31, C=1024   276/288   209/249   198/246   153/238      (C=2048: 520/538, -, 372/511, 294/479; T=16384, C=512: 36/43,
-//   K=15, C=1024   202/228   158/168   154/167   136/159       33/38, 33/39, 28/36; T=4096: 26/30, 24/29, 24/28, 22/26)
-//   K=21, C=1024   275/234   197/197   192/195   147/183      (T=65536, C=512: 80/73, 68/64, 64/63, 49/59)
-//   K=11, C=1024   195/177   154/153   151/150   135/146
-// About 24 rows a sequence: K=31 627/575, 32: 560/574 (C=2048). 21 taps pay for the 32 lags of the plan, which short
-// sequences do not leave room for; 11 taps are bound by HBM on the vector ALU too.
-// Sequences of 522, 705, 1928 rows on average: K=21 181/196, 175/191, 160/186; K=11 150/150, 142/146, 139/144.
+//   K=31, C=1024   257/279   198/257   188/251   139/240      (C=2048: 488/541, 346/488, -, 274/467; T=16384, C=512: 33/39, 31/37,
+//                                                              32/38, 24/35)
+//   K=15, C=1024   200/193   156/171   152/172   132/162      (T=16384, C=512: 25/28, 24/25, 23/25, 20/23; T=4096: 17/20, 16/18, 16/18, 16/16)
+//   K=21, C=1024   245/224   180/202   183/205   135/188      (T=65536, C=512: 77/73, 64/63, 58/61, 46/57)
+//   K=11, C=1024   198/175   159/157   159/149   136/146
+// About 24 rows a sequence: K=31 671/628, 32: 613/608 (C=2048). 21 taps pay for the 32 lags of the plan, which short
+// sequences do not leave room for (from 200 rows on they would gain where C = 1024, not where C = 512); 11 taps are bound by HBM on the
+// vector ALU too. Sequences of 522, 705, 1928 rows on average: K=21 164/195, 157/191, 144/189; K=11 151/150, 151/149, 142/145.
 // S counts empty sequences too, which the device alone could tell apart: a cu with a long tail of them is taken for shorter ones.
 bool mfma_bwd_preferred(long long T, int taps, int S) {
     const int rows = taps == 31 ? 32 : taps == 15 ? 64 : 512;
@@ -407,13 +408,13 @@ long long mfma_gated_steps_of_a_block(long long T, int C) {
 }
 // The gated backward with dz on the matrix cores: 31 taps. Measured, us, against role-split, for lengths of 20 to 128 residues
 // (mean 75), 20 to 512 (263), log-normal (333), short and long mixed (193), one sequence:
-//   T=131072, C=2048   886/807   705/737   673/721   673/724   619/674         T=32768, C=1024   125/117   100/105   95/105   97/108   87/100
-//   T=16384, C=1024    72/75     61/66     58/65     56/69     51/66           T=8192, C=512     29/39     27/37     27/38    26/39    24/34
+//   T=131072, C=2048   793/793   683/737   676/737   698/750   624/705         T=32768, C=1024   112/114   96/106   96/104   -   88/103
+//   T=16384, C=1024    62/70     53/68     -         -         51/64           T=8192, C=512     26/37     25/35     -        -        23/33
 // A wave of dw makes one pass over its rows whatever begins there, but masked row by row: short sequences cost it more than the
 // role-split kernel's roles, which share the loss, once a call is longer than its first tiles. 15 taps (T=131072, C=1024: 302/264,
 // T=4096: 19/22) and 21 (306/299) have too few FMAs to save. Calls of up to 16384 rows take it whatever begins in them (C=1024):
-//   T=16384   1 row 138/228   4 71/96   16 66/82   32 63/77   75 67/65        T=4096   1 row 45/83   8 27/40   32 26/39   75 26/36
-// and so do the shortest: T=2048, C=768 1 row 30/49, 16 25/30, 75 21/29, 300 19/27, one sequence 18/26; T=20, C=512 18/21. Below 4096 rows
+//   T=16384   1 row 143/226   4 94/108   16 86/81   32 76/78   75 62/70       T=4096   1 row 45/79   8 32/42   32 29/38   75 26/36
+// and so do the shortest: T=2048, C=768 1 row 28/47, 16 22/29, 75 19/27, 300 18/26, one sequence 17/24; T=20, C=512 15/20. Below 4096 rows
 // only where a block has up to four tiles of 64 rows, which goes by C; with more of them short sequences cost what they do in long calls:
 //   rows a sequence   4         8        16       24       32       48       75       300
 //   T=2048, C=4096 (4 tiles)    58/74    54/63    53/57    55/57    47/54    44/55    41/51    38/49
@@ -507,13 +508,13 @@ int make_split_plan(bool fwd, bool bf16, long long T, int C, int K, const nplm_d
 //     tile issued at once).
 //   11 to 31 taps, bf16 weights too, forward: matrix cores. On the vector ALU these sizes are bound by their FMAs (K=31, one
 //     sequence: 248 us where a copy of the same bytes takes 208); in us, matrix cores against the best of the others:
-//     K=31 C=2048: 202 against 260 (log-normal lengths), 184 / 248 (one sequence), 250 / 289 (20 to 128 residues);
-//     K=21 C=1024: 102 / 112; K=15: 182 / 192 at C=2048, 97 / 101 at C=1024; K=11 C=1024: 95 / 100;
-//     T=16384 C=1024: 24.6 / 28.6 at K=31, 17.7 / 21.4 at K=11. From kMfmaMinRows rows on: below, every block has a tile
+//     K=31 C=2048: 189 against 256 (log-normal lengths), 184 / 247 (one sequence), 232 / 293 (20 to 128 residues);
+//     K=21 C=1024: 88 / 107; K=15: 182 / 191 at C=2048, 85 / 91 at C=1024; K=11 C=1024: 85 / 93;
+//     T=16384 C=1024: 21.2 / 31.4 at K=31, 16.0 / 20.0 at K=11. From kMfmaMinRows rows on: below, every block has a tile
 //     or two and what is measured is the launch (2048 rows, C=1024: K=31 11.8 / 12.5, K=15 10.0 / 10.2; 600 rows, C=512:
 //     12.2 / 11.8), while the others' sums are those of the sliding-window kernels bit for bit.
-//     Whatever the length of the sequences (T=65536, C=1024, K=31: 1 row 160 / 252, 4 64 / 154, 16 69 / 69, 24 70 / 96, 48 67 / 76;
-//     K=11: 1 row 113 / 196, 16 55 / 62, 75 56 / 64) and also where rows fill their column blocks poorly (T=32768, K=31: C=264
+//     Whatever the length of the sequences (lengths spread by half around the mean, T=65536, C=1024, K=31: 4 rows 92 / 211, 16 92 / 115, 24
+//     87 / 108, 48 72 / 101; K=21: 16 81 / 99, 32 71 / 89; K=11: 16 69 / 94, 75 54 / 71) and also where rows fill their column blocks poorly (T=32768, K=31: C=264
 //     25 / 35, C=520 33 / 44; K=11: 18 / 22, 25 / 29).
 //     fp32 weights would take three bf16 terms each: 280 us against 265 (K=31, C=2048), so they stay on the vector ALU.
 //   the same calls backward: matrix cores where a sequence has enough rows (mfma_bwd_preferred()).

@@ -744,7 +744,7 @@ struct MfmaConv {
 // Forward: 64-row tiles, 8 compute waves (4 wave-columns x 2 groups of 32 rows), 3 loader waves and one that finds the
 // boundaries of the next tile; two tile buffers.
 // Bound by HBM from 64 row tiles on: T=131072, C=2048, 31 taps, one sequence 182 us (5.9 TB/s), 248 on the vector ALU; log-normal
-// lengths 203 (216 before the sweeps over single sequences). More rows
+// lengths 189 (216 with neither the sweeps over single sequences nor rows 32 bytes apart). More rows
 // per tile, three buffers or 1 KiB column blocks measured the same or slower (a tile's compute already hides the next one's
 // loads); one scout wave costs nothing that the loaders would use.
 template <int KT>

@@ -4,9 +4,10 @@
 // What bounds a small training step is the host. As torch.autograd.Function the backward runs Python on the engine's
 // thread, which first has to get the interpreter lock from the thread that waits for it; as torch.library custom ops (the
 // pre-norm door's eager route before) both directions go through Python dispatch as well. Here neither direction runs Python.
-// Forward + backward of one call after another, T=2048, 7 taps, bf16, before and now: plain, C=768 68 to 126 us (by how the threads
-// meet at the lock) and 37; gated, C=1152, fp32 parameters 122 and 37; pre-norm, C=1024 210 and 43. A multiplication by a constant
-// takes 24 to 47. Inference, T=776, C=64, 3 taps 15.3 and 7.4; padded door, 32 x 512 rows 24.6 and 15.5.
+// Forward + backward of one call after another, T=2048, 7 taps, bf16, before and now: plain, C=768 65 to 126 us (by how the threads
+// meet at the lock) and 34 to 67 (by how soon the waiting thread and the engine's wake each other); gated 124 to 129 and 38 to 68; pre-norm
+// 217 to 223 and 79 to 83. A multiplication by a constant takes 24 to 47. Inference, T=776, C=64, 3 taps 15.2 and 7.0; padded door, 32 x 512
+// rows 23.9 and 15.8.
 //
 // A call that is not of the usual form - arguments that the checks below do not settle, tensor subclasses, modes, transforms,
 // tracing, forward-mode AD - is answered with None, and the Python route takes it with its own messages. So nothing
